@@ -1,9 +1,9 @@
 // Matrix products y = x W^T (+ bias) for weights stored [N, K] with K contiguous,
 // which is how every linear layer of a checkpoint is stored.
 //
-//   * sgemm_nt_kernel: float32 in, float32 FMA over runs of 16, float64 over the
-//     runs, float32 out.  The true 32-bit path: no matrix-core shortcut, no
-//     reduced-precision inputs.
+//   * sgemm_nt_kernel: bfloat16 in, float32 FMA over runs of 16, float64 over the
+//     runs: the sizes that the matrix-core kernels refuse.  (The product of
+//     float32 rows is sgemm.hip's.)
 //   * gemm_bf16_kernel: bfloat16 in, MFMA 16x16x32 with float32 accumulation,
 //     bfloat16 or float32 out; LDS-tiled 128x128x32.  Any M and N; K % 8 == 0.
 //   * skinny_bf16_kernel: M <= 16 rows of x (decode).  Weight-streaming: a
@@ -17,17 +17,17 @@
 #include "gemm_epilogue.h"
 
 // ==========================================================================
-// float32
+// bfloat16 rows that are not 16-byte aligned
 // ==========================================================================
 #define SG_BM 64
 #define SG_BN 64
 #define SG_BK 16
 
-// InT float: the true 32-bit product.  InT bf16: the product for sizes the MFMA kernels refuse (K or a row
-// stride that is no multiple of 8, so that rows are not 16-byte aligned): element loads, float32 FMA.
-template <typename InT, typename BiasT, typename OutT>
+// The product for sizes the MFMA kernels refuse (K or a row stride that is no multiple of 8, so that rows are not
+// 16-byte aligned): element loads, float32 FMA.
+template <typename BiasT, typename OutT>
 __global__ void __launch_bounds__(256)
-    sgemm_nt_kernel(const InT* __restrict__ a, long lda, const InT* __restrict__ w, const BiasT* __restrict__ bias,
+    sgemm_nt_kernel(const bf16* __restrict__ a, long lda, const bf16* __restrict__ w, const BiasT* __restrict__ bias,
                     OutT* __restrict__ c, long ldc, int M, int N, int K) {
   __shared__ float as[SG_BK][SG_BM + 1];
   __shared__ float ws[SG_BK][SG_BN + 1];
@@ -79,18 +79,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
-                               int N, int K, hipStream_t stream) {
-  if (M == 0 || N == 0) return 0;
-  FMS_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
-  FMS_REQUIRE(lda >= K && ldc >= N, "gemm_f32: leading dimensions too small");
-  dim3 grid(ceil_div(N, SG_BN), ceil_div(M, SG_BM));
-  FMS_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d exceeds one launch", M);
-  sgemm_nt_kernel<float, float, float><<<grid, 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K);
-  FMS_LAUNCH_CHECK("gemm_f32");
-  return 0;
-}
-
 extern "C" int fmsamd_gemm_bf16_any(const void* a, long lda, const void* w, const void* bias, int bias_dtype, void* c,
                                     int out_dtype, long ldc, int M, int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;
@@ -100,7 +88,7 @@ extern "C" int fmsamd_gemm_bf16_any(const void* a, long lda, const void* w, cons
   FMS_REQUIRE(grid.y <= 65535, "gemm_bf16_any: M=%d exceeds one launch", M);
   const bool fb = bias != nullptr && bias_dtype == FMS_F32;
 #define FMS_SG(B, O)                                                                                                 \
-  sgemm_nt_kernel<bf16, B, O><<<grid, 256, 0, stream>>>((const bf16*)a, lda, (const bf16*)w, (const B*)bias, (O*)c, \
+  sgemm_nt_kernel<B, O><<<grid, 256, 0, stream>>>((const bf16*)a, lda, (const bf16*)w, (const B*)bias, (O*)c, \
                                                         ldc, M, N, K)
   if (out_dtype == FMS_BF16 && !fb)
     FMS_SG(bf16, bf16);

@@ -576,7 +576,7 @@ def linear(
     """act(x [M, K] @ weight[N, K]^T (+ bias)) -> [M, N].  The skinny kernels finish with relu and its square themselves; every
     other activation and kernel is followed by the activation kernel.
 
-    float32 x float32: the FMA kernel (true 32-bit).  bfloat16 x bfloat16: the weight-streaming
+    float32 x float32: the float32 matrix-core kernel (true 32-bit).  bfloat16 x bfloat16: the weight-streaming
     skinny kernels up to 192 rows; above that the vendor library (hipBLASLt through torch.matmul,
     as the reference's nn.Linear does; for float32 output with the float32 sums as they are), or this
     package's MFMA kernel when allow_library is False.

@@ -452,6 +452,21 @@ def test_gemm_f32(ops, M, N, K):
     torch.testing.assert_close(out, (x.double() @ w.double().t() + b.double()).float(), atol=1e-4, rtol=1e-5)
 
 
+# every tile shape (16x16, 32x32, 32x64, 64x64), with rows, columns and K past its last whole tile, and rows that are not
+# 16-byte aligned (odd K, odd stride)
+@pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (130, 4100, 65), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
+    torch.manual_seed(61)
+    wide, w, b = torch.randn(M, K + pad), torch.randn(N, K), torch.randn(N)
+    x = wide[:, :K]
+    out = ops.linear(dev(wide)[:, :K], dev(w), dev(b)).cpu().double()
+    want = x.double() @ w.double().t() + b.double()
+    # a float32 sum of 16 products is off by at most 16 roundings of the sum of their sizes; the float64 sum's one rounding at the end
+    bound = 2.0 ** -24 * (16.5 * (x.abs().double() @ w.abs().double().t()) + want.abs()) + 1e-30
+    assert float(((out - want).abs() / bound).max()) <= 1.0
+
+
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 48, 64, 65, 96, 100, 128, 129, 144, 160, 170, 192, 193, 300])
 @pytest.mark.parametrize("N,K", [(40, 24), (100, 176), (257, 96), (384, 96), (4096 + 16, 512), (20000, 64)])
 def test_gemm_bf16(ops, M, N, K):
