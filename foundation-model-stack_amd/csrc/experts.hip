@@ -3,18 +3,24 @@
 //   route:    float32 router logits [T, E] -> the `top` largest per token (ties: the lower index) and their weights:
 //             the softmax over those `top` logits alone, or every chosen logit's sigmoid (as it is, or divided by the
 //             sum of the chosen ones).
-//   group:    the T * top (token, choice) pairs sorted by expert, cut into tiles of 16 rows that belong to one expert
+//   group:    the T * top (token, choice) pairs sorted by expert, cut into tiles of rows that belong to one expert
 //             each.  It runs on the device, in one block, so a step never waits for the host (and can be captured).
 //   gate_up:  for every tile, hidden = clamp-gated activation of (x Wg_e^T, x Wu_e^T)
 //   down:     for every tile, y[pair] = hidden Wd_e^T, float32, at the pair's own place (token * top + choice)
 //   combine:  out[t] = sum_j weight[t, j] y[t * top + j]  (+ sigmoid(shared_gate[t]) * shared[t]), summed in the order
 //             of j: a token's result does not depend on what else is in the batch.
 //
-// The products take their rows through tile_product.h: float32 FMA for the 32-bit path, MFMA 16x16x32 for bfloat16.
+// The products take their rows through tile_product.h (float32 FMA for the 32-bit path and for bfloat16 rows that are not
+// aligned to 16 bytes) and tile_product_lds.h (MFMA 32x32x16 for bfloat16).
 // The grids are sized for the worst case (every expert with a ragged last tile); tiles that do not exist leave at once.
 #include "common.h"
 #include "fmsamd.h"
 #include "tile_product.h"
+#include "tile_product_lds.h"
+
+// rows of the matrix-core kernels' tiles
+#define TILE_SMALL_ROWS 32
+#define TILE_BIG_ROWS 128
 
 #define ROUTE_MAX_EXPERTS 1024
 #define ROUTE_MAX_TOP 64
@@ -200,45 +206,81 @@ extern "C" int fmsamd_moe_route_grouped(const float* logits, long ld, int n_toke
 }
 
 // --------------------------------------------------------------------------
-// group: order[0 .. n) = the pairs sorted by expert; tiles[i] = (expert, first row in order, rows), rows 0: no tile
+// group: order[0 .. n) = the pairs sorted by expert; tiles[i] = (expert, first row in order, rows), rows 0: no tile; behind
+// the max_tiles of them, how many there are
 // --------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024)
+// One block.  Its time is round trips: a thread asks for eight ids at a time, and the experts' places come from a scan over
+// the threads (an expert each).  8192 pairs of 32 experts: 7.6 us (12.6 with ids one by one and one thread adding up); 32 pairs:
+// 4.9 (5.9).
+#define GROUP_THREADS 1024
+__global__ void __launch_bounds__(GROUP_THREADS)
     group_kernel(const int* __restrict__ ids, int n_pairs, int n_experts, int* __restrict__ order, int* __restrict__ tiles,
                  int max_tiles, int tile_rows) {
   __shared__ int counts[ROUTE_MAX_EXPERTS];
   __shared__ int cursor[ROUTE_MAX_EXPERTS];
-  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) counts[e] = 0;
+  __shared__ int wave_pairs[GROUP_THREADS / WAVE], wave_tiles[GROUP_THREADS / WAVE];
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+  for (int e = tid; e < n_experts; e += GROUP_THREADS) counts[e] = 0;
   __syncthreads();
-  for (int a = threadIdx.x; a < n_pairs; a += blockDim.x) {
-    const int e = ids[a];
-    if (e >= 0 && e < n_experts) atomicAdd(&counts[e], 1);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, nt = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      cursor[e] = at;
-      const int c = counts[e];
-      for (int r = 0; r < c && nt < max_tiles; r += tile_rows, ++nt) {
-        tiles[3 * nt] = e;
-        tiles[3 * nt + 1] = at + r;
-        tiles[3 * nt + 2] = c - r < tile_rows ? c - r : tile_rows;
-      }
-      at += c;
+  constexpr int AHEAD = 8;
+  for (int a0 = tid; a0 < n_pairs; a0 += AHEAD * GROUP_THREADS) {
+    int e[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int a = a0 + i * GROUP_THREADS;
+      e[i] = a < n_pairs ? ids[a] : -1;
     }
-    for (; nt < max_tiles; ++nt) tiles[3 * nt] = 0, tiles[3 * nt + 1] = 0, tiles[3 * nt + 2] = 0;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (e[i] >= 0 && e[i] < n_experts) atomicAdd(&counts[e[i]], 1);
   }
   __syncthreads();
-  for (int a = threadIdx.x; a < n_pairs; a += blockDim.x) {
-    const int e = ids[a];
-    if (e >= 0 && e < n_experts) order[atomicAdd(&cursor[e], 1)] = a;
+  // thread e: how many pairs and tiles the experts before e have (there are no more experts than threads)
+  const int c = tid < n_experts ? counts[tid] : 0, t = (c + tile_rows - 1) / tile_rows;
+  int pairs = c, some = t;
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const int p = __shfl_up(pairs, off, WAVE), q = __shfl_up(some, off, WAVE);
+    if (lane >= off) pairs += p, some += q;
+  }
+  if (lane == WAVE - 1) wave_pairs[wave] = pairs, wave_tiles[wave] = some;
+  __syncthreads();
+  int before = pairs - c, nt = some - t, all = 0;
+  for (int w = 0; w < GROUP_THREADS / WAVE; ++w) {
+    if (w < wave) before += wave_pairs[w], nt += wave_tiles[w];
+    all += wave_tiles[w];
+  }
+  all = all < max_tiles ? all : max_tiles;
+  if (tid < n_experts) {
+    cursor[tid] = before;
+    for (int r = 0; r < c && nt < max_tiles; r += tile_rows, ++nt) {
+      tiles[3 * nt] = tid;
+      tiles[3 * nt + 1] = before + r;
+      tiles[3 * nt + 2] = c - r < tile_rows ? c - r : tile_rows;
+    }
+  }
+  if (tid == 0) tiles[3 * max_tiles] = all;
+  for (int i = 3 * all + tid; i < 3 * max_tiles; i += GROUP_THREADS) tiles[i] = 0;
+  __syncthreads();
+  for (int a0 = tid; a0 < n_pairs; a0 += AHEAD * GROUP_THREADS) {
+    int e[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int a = a0 + i * GROUP_THREADS;
+      e[i] = a < n_pairs ? ids[a] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (e[i] >= 0 && e[i] < n_experts) order[atomicAdd(&cursor[e[i]], 1)] = a0 + i * GROUP_THREADS;
   }
 }
 
-// Rows of a tile: 64 where the experts have that many rows on average (prompts) and the matrix-core kernel can run
-// (wide_ok: bfloat16, rows aligned to 16 bytes), else 16.
+// Rows of a tile.  The matrix-core kernels (wide_ok: bfloat16, everything aligned to 16 bytes) take large tiles from 20 rows an
+// expert on, where most experts would need two small ones and read their weights twice (32 experts, 4 a token: 192 tokens 58 +
+// 32 us in small tiles, 50 + 28 in large ones; 128 tokens 44 + 24 against 48 + 26).
 extern "C" int fmsamd_moe_tile_rows(int n_pairs, int n_experts, int wide_ok) {
-  return (wide_ok && n_pairs >= (long)TILE_WIDE_ROWS * n_experts) ? TILE_WIDE_ROWS : TILE_ROWS;
+  if (!wide_ok) return TILE_ROWS;
+  return n_pairs >= 20L * n_experts ? TILE_BIG_ROWS : TILE_SMALL_ROWS;
 }
 
 extern "C" int fmsamd_moe_max_tiles(int n_pairs, int n_experts, int tile_rows) {
@@ -251,10 +293,11 @@ extern "C" int fmsamd_moe_group(const int* ids, int n_pairs, int n_experts, int*
   if (n_pairs == 0) return 0;
   FMS_REQUIRE(n_pairs > 0 && n_experts > 0 && n_experts <= ROUTE_MAX_EXPERTS, "moe_group: %d pairs, %d experts (at most %d)", n_pairs,
               n_experts, ROUTE_MAX_EXPERTS);
-  FMS_REQUIRE(tile_rows == TILE_ROWS || tile_rows == TILE_WIDE_ROWS, "moe_group: tiles of %d rows", tile_rows);
+  FMS_REQUIRE(tile_rows == TILE_ROWS || tile_rows == TILE_SMALL_ROWS || tile_rows == TILE_BIG_ROWS, "moe_group: tiles of %d rows", tile_rows);
   FMS_REQUIRE(max_tiles >= fmsamd_moe_max_tiles(n_pairs, n_experts, tile_rows), "moe_group: room for %d tiles, %d may be needed", max_tiles,
               fmsamd_moe_max_tiles(n_pairs, n_experts, tile_rows));
-  group_kernel<<<1, 1024, 0, stream>>>(ids, n_pairs, n_experts, order, tiles, max_tiles, tile_rows);
+  static_assert(ROUTE_MAX_EXPERTS <= GROUP_THREADS, "an expert a thread");
+  group_kernel<<<1, GROUP_THREADS, 0, stream>>>(ids, n_pairs, n_experts, order, tiles, max_tiles, tile_rows);
   FMS_LAUNCH_CHECK("moe_group");
   return 0;
 }
@@ -335,115 +378,116 @@ __global__ void __launch_bounds__(TILE_THREADS) expert_down_fma_kernel(ExpertArg
   }
 }
 
-__global__ void __launch_bounds__(TILE_THREADS) expert_gate_up_mfma_kernel(ExpertArgs a) {
-  const int e = a.tiles[3 * blockIdx.x], start = a.tiles[3 * blockIdx.x + 1], rows = a.tiles[3 * blockIdx.x + 2];
-  if (rows == 0) return;
-  const int n0 = blockIdx.y * TILE_MFMA_COLS;
+// The same two products in bfloat16: tiles of 32 or 128 rows, through LDS (tile_product_lds.h).  For the gated product half of a
+// wave's tiles are gate columns and the others the up columns of the same elements, so that both meet in one lane.  The
+// column blocks of a tile follow one another on one of the eight dies (blocks are dealt to the dies in turn), the tiles of
+// an expert behind each other, so that rows and weights come from memory once.
+//
+// Few rows an expert (decode) are bound by the weights' bytes: tiles of 32 rows by 128 rows of W, two waves and three stages of
+// 20 KB a block, two blocks a compute unit.  Many rows (prompts) by the matrix unit, the weights' bytes and the start and end of
+// a block together: 128 rows by 256 rows of W.  Measured with 32 experts, 4 a token, width 2048, hidden 1024 (gate and up + down;
+// in brackets tiles of 16 rows, from 2048 on of 64, straight from memory): 8 tokens 28 + 16 us (69 + 29), 32 tokens 42 + 23 (76 +
+// 31; 6.4 TB/s), 128 tokens 44 + 24 (92 + 46), 2048 tokens 136 + 74 (445 + 225), 4096 tokens 217 + 130.
+// Also measured for 2048 tokens: 128 x 256 as waves of 64 x 64 142 + 73, 64 x 256 137 + 68 (4096: 241 + 145), 128 x 128 with two
+// blocks a compute unit 153 + 74, 128 x 512 154 + 77.
+__device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles, int col_blocks, int& tile, int& col) {
+  const int total = a.tiles[3 * max_tiles] * col_blocks;  // the tiles there are
+  const int per_die = (total + 7) / 8;
+  const int at = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
+  tile = at / col_blocks, col = at % col_blocks;
+  return (int)(blockIdx.x >> 3) < per_die && at < total;
+}
+
+template <int WM, int WN, int TM, int TN, int ST, bool GATED>
+__global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_gate_up_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
+  typedef TileLds<WM, WN, TM, TN, ST> S;
+  __shared__ __attribute__((aligned(16))) bf16 lds[S::LDS_ELEMENTS];
+  int tile, col;
+  if (!expert_place(a, max_tiles, col_blocks, tile, col)) return;
+  const int e = a.tiles[3 * tile], start = a.tiles[3 * tile + 1], rows = a.tiles[3 * tile + 2];
   const bf16* x = (const bf16*)a.x;
   const bf16* wg = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
   const bf16* wu = (const bf16*)a.w2 + (size_t)e * a.N * a.K;
-  auto a_row = [&](int m) { return m < rows ? x + (size_t)(a.order[start + m] / a.top) * a.ldx : (const bf16*)nullptr; };
-  const bool gated = a.w2 != nullptr;
-  f32x4 g[TILE_MFMA_WAVE_TILES], u[TILE_MFMA_WAVE_TILES];
-#pragma unroll
-  for (int tl = 0; tl < TILE_MFMA_WAVE_TILES; ++tl) u[tl] = f32x4{0.f, 0.f, 0.f, 0.f};
-  tile_product_mfma(a_row, [&](int n) { return n0 + n < a.N ? wg + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, g);
-  if (gated) tile_product_mfma(a_row, [&](int n) { return n0 + n < a.N ? wu + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, u);
+  // gated: a wave's first TN / 2 tiles are gate columns, the others the up columns of the same elements
+  const int n0 = col * (GATED ? S::BN / 2 : S::BN);
+  f32x16 acc[TM][TN];
+  tile_product_lds<WM, WN, TM, TN, ST>([&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; },
+                                   [&](int n) {
+                                     const int t = n / 32;
+                                     const bool up = GATED && t % TN >= TN / 2;
+                                     const int c = n0 + (GATED ? ((t / TN) * (TN / 2) + t % (TN / 2)) * 32 + n % 32 : n);
+                                     return (up ? wu : wg) + (size_t)(c < a.N ? c : 0) * a.K;
+                                   },
+                                   a.K, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = (lane >> 4) * 4 + i;
-    if (m >= rows) continue;
-    const float sc = pair_scale(a, start + m);
+  for (int i = 0; i < TM; ++i) {
 #pragma unroll
-    for (int tl = 0; tl < TILE_MFMA_WAVE_TILES; ++tl) {
-      const int n = n0 + wave * (16 * TILE_MFMA_WAVE_TILES) + tl * 16 + (lane & 15);
-      if (n < a.N) ((bf16*)a.y)[(size_t)(start + m) * a.N + n] = (bf16)hidden_value(a, gated, g[tl][i] * sc, u[tl][i] * sc);
-    }
-  }
-}
-
-__global__ void __launch_bounds__(TILE_THREADS) expert_down_mfma_kernel(ExpertArgs a) {
-  const int e = a.tiles[3 * blockIdx.x], start = a.tiles[3 * blockIdx.x + 1], rows = a.tiles[3 * blockIdx.x + 2];
-  if (rows == 0) return;
-  const int n0 = blockIdx.y * TILE_MFMA_COLS;
-  const bf16* x = (const bf16*)a.x;
-  const bf16* w = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
-  f32x4 acc[TILE_MFMA_WAVE_TILES];
-  tile_product_mfma([&](int m) { return m < rows ? x + (size_t)(start + m) * a.ldx : (const bf16*)nullptr; },
-                    [&](int n) { return n0 + n < a.N ? w + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, acc);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = (lane >> 4) * 4 + i;
-    if (m >= rows) continue;
-    float* yrow = (float*)a.y + (size_t)a.order[start + m] * a.N;
-#pragma unroll
-    for (int tl = 0; tl < TILE_MFMA_WAVE_TILES; ++tl) {
-      const int n = n0 + wave * (16 * TILE_MFMA_WAVE_TILES) + tl * 16 + (lane & 15);
-      if (n < a.N) yrow[n] = acc[tl][i];
-    }
-  }
-}
-
-// The same two products on tiles of 64 rows (tile_product_mfma_wide).
-__global__ void __launch_bounds__(TILE_THREADS) expert_gate_up_wide_kernel(ExpertArgs a) {
-  const int e = a.tiles[3 * blockIdx.x], start = a.tiles[3 * blockIdx.x + 1], rows = a.tiles[3 * blockIdx.x + 2];
-  if (rows == 0) return;
-  const int n0 = blockIdx.y * TILE_MFMA_COLS;
-  const bf16* x = (const bf16*)a.x;
-  const bf16* wg = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
-  const bf16* wu = (const bf16*)a.w2 + (size_t)e * a.N * a.K;
-  auto a_row = [&](int m) { return m < rows ? x + (size_t)(a.order[start + m] / a.top) * a.ldx : (const bf16*)nullptr; };
-  const bool gated = a.w2 != nullptr;
-  f32x4 g[2][4], u[2][4];
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) u[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  tile_product_mfma_wide(a_row, [&](int n) { return n0 + n < a.N ? wg + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, g);
-  if (gated) tile_product_mfma_wide(a_row, [&](int n) { return n0 + n < a.N ? wu + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, u);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = (wave >> 1) * 32 + mt * 16 + (lane >> 4) * 4 + i;
+    for (int v = 0; v < 16; ++v) {
+      const int m = ((wave / WN) * TM + i) * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
       if (m >= rows) continue;
       const float sc = pair_scale(a, start + m);
+      bf16* to = (bf16*)a.y + (size_t)(start + m) * a.N;
+      if constexpr (GATED) {
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int n = n0 + (wave & 1) * 64 + nt * 16 + (lane & 15);
-        if (n < a.N) ((bf16*)a.y)[(size_t)(start + m) * a.N + n] = (bf16)hidden_value(a, gated, g[mt][nt][i] * sc, u[mt][nt][i] * sc);
+        for (int j = 0; j < TN / 2; ++j) {
+          const int n = n0 + ((wave % WN) * (TN / 2) + j) * 32 + (lane & 31);
+          if (n < a.N) to[n] = (bf16)clamp_gated(acc[i][j][v] * sc, acc[i][TN / 2 + j][v] * sc, a.limit, a.alpha, a.shift);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int n = n0 + ((wave % WN) * TN + j) * 32 + (lane & 31);
+          if (n < a.N) to[n] = (bf16)fms_activate(acc[i][j][v] * sc, a.act);
+        }
       }
     }
   }
 }
 
-__global__ void __launch_bounds__(TILE_THREADS) expert_down_wide_kernel(ExpertArgs a) {
-  const int e = a.tiles[3 * blockIdx.x], start = a.tiles[3 * blockIdx.x + 1], rows = a.tiles[3 * blockIdx.x + 2];
-  if (rows == 0) return;
-  const int n0 = blockIdx.y * TILE_MFMA_COLS;
+template <int WM, int WN, int TM, int TN, int ST>
+__global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_down_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
+  typedef TileLds<WM, WN, TM, TN, ST> S;
+  __shared__ __attribute__((aligned(16))) bf16 lds[S::LDS_ELEMENTS];
+  int tile, col;
+  if (!expert_place(a, max_tiles, col_blocks, tile, col)) return;
+  const int e = a.tiles[3 * tile], start = a.tiles[3 * tile + 1], rows = a.tiles[3 * tile + 2];
+  const int n0 = col * S::BN;
   const bf16* x = (const bf16*)a.x;
   const bf16* w = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
-  f32x4 acc[2][4];
-  tile_product_mfma_wide([&](int m) { return m < rows ? x + (size_t)(start + m) * a.ldx : (const bf16*)nullptr; },
-                         [&](int n) { return n0 + n < a.N ? w + (size_t)(n0 + n) * a.K : (const bf16*)nullptr; }, a.K, acc);
+  f32x16 acc[TM][TN];
+  tile_product_lds<WM, WN, TM, TN, ST>([&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; },
+                                   [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; }, a.K, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
+  for (int i = 0; i < TM; ++i) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = (wave >> 1) * 32 + mt * 16 + (lane >> 4) * 4 + i;
+    for (int v = 0; v < 16; ++v) {
+      const int m = ((wave / WN) * TM + i) * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
       if (m >= rows) continue;
-      float* yrow = (float*)a.y + (size_t)a.order[start + m] * a.N;
+      float* to = (float*)a.y + (size_t)a.order[start + m] * a.N;
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int n = n0 + (wave & 1) * 64 + nt * 16 + (lane & 15);
-        if (n < a.N) yrow[n] = acc[mt][nt][i];
+      for (int j = 0; j < TN; ++j) {
+        const int n = n0 + ((wave % WN) * TN + j) * 32 + (lane & 31);
+        if (n < a.N) to[n] = acc[i][j][v];
       }
     }
   }
+}
+
+template <int WM, int WN, int TM, int TN, int ST>
+static int launch_lds(int stage, const ExpertArgs& a, int max_tiles, hipStream_t stream) {
+  typedef TileLds<WM, WN, TM, TN, ST> S;
+  const int col_blocks = ceil_div(a.N, stage == 0 && a.w2 != nullptr ? S::BN / 2 : S::BN);
+  FMS_REQUIRE((long)max_tiles * col_blocks <= 0x7ffffff0L, "moe_experts: %d tiles of %d columns are too many for one launch", max_tiles, a.N);
+  const int blocks = 8 * ceil_div((long)max_tiles * col_blocks, 8);
+  if (stage == 1)
+    expert_down_lds_kernel<WM, WN, TM, TN, ST><<<blocks, S::THREADS, 0, stream>>>(a, max_tiles, col_blocks);
+  else if (a.w2 != nullptr)
+    expert_gate_up_lds_kernel<WM, WN, TM, TN, ST, true><<<blocks, S::THREADS, 0, stream>>>(a, max_tiles, col_blocks);
+  else
+    expert_gate_up_lds_kernel<WM, WN, TM, TN, ST, false><<<blocks, S::THREADS, 0, stream>>>(a, max_tiles, col_blocks);
+  return 0;
 }
 
 // stage 0: hidden = act(x Wg^T, x Wu^T) for the tiles' rows; stage 1: y = hidden Wd^T
@@ -454,30 +498,26 @@ extern "C" int fmsamd_moe_experts(int stage, const void* x, long ldx, const void
   if (max_tiles == 0) return 0;
   FMS_REQUIRE(act >= 0 && act <= FMS_ACT_LAST, "moe_experts: unknown activation %d", act);
   FMS_REQUIRE(stage == 0 || stage == 1, "moe_experts: stage %d", stage);
-  FMS_REQUIRE(tile_rows == TILE_ROWS || tile_rows == TILE_WIDE_ROWS, "moe_experts: tiles of %d rows", tile_rows);
+  FMS_REQUIRE(tile_rows == TILE_ROWS || tile_rows == TILE_SMALL_ROWS || tile_rows == TILE_BIG_ROWS, "moe_experts: tiles of %d rows", tile_rows);
   FMS_REQUIRE(max_tiles > 0 && top > 0 && N > 0 && K > 0 && ldx >= K, "moe_experts: bad sizes tiles=%d top=%d N=%d K=%d ldx=%ld", max_tiles,
               top, N, K, ldx);
   ExpertArgs a{x, ldx, w1, w2, y, order, tiles, top, N, K, limit, alpha, shift, stage == 0 ? in_scale : nullptr, act};
   const bool mfma = dtype == FMS_BF16 && K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w1 % 16) == 0 &&
                     (w2 == nullptr || ((uintptr_t)w2 % 16) == 0);
-  const dim3 grid(max_tiles, ceil_div(N, mfma ? TILE_MFMA_COLS : TILE_FMA_COLS));
+  const dim3 grid(max_tiles, ceil_div(N, TILE_FMA_COLS));
   FMS_REQUIRE(grid.y <= 65535, "moe_experts: %d columns are too many for one launch", N);
-  if (tile_rows == TILE_WIDE_ROWS) {
-    // tiles of 64 rows are made for the matrix-core kernel only
+  if (tile_rows != TILE_ROWS) {
+    // the larger tiles are made for the matrix-core kernels only
     FMS_REQUIRE(mfma, "moe_experts: tiles of %d rows need bfloat16 rows aligned to 16 bytes", tile_rows);
-    if (stage == 0) expert_gate_up_wide_kernel<<<grid, TILE_THREADS, 0, stream>>>(a);
-    else expert_down_wide_kernel<<<grid, TILE_THREADS, 0, stream>>>(a);
+    const int st = tile_rows == TILE_BIG_ROWS ? launch_lds<4, 2, 1, 4, 3>(stage, a, max_tiles, stream)
+                                              : launch_lds<1, 2, 1, 2, 3>(stage, a, max_tiles, stream);
+    if (st) return st;
   } else if (dtype == FMS_F32) {
     if (stage == 0) expert_gate_up_fma_kernel<float><<<grid, TILE_THREADS, 0, stream>>>(a);
     else expert_down_fma_kernel<float><<<grid, TILE_THREADS, 0, stream>>>(a);
   } else if (dtype == FMS_BF16) {
-    if (mfma) {
-      if (stage == 0) expert_gate_up_mfma_kernel<<<grid, TILE_THREADS, 0, stream>>>(a);
-      else expert_down_mfma_kernel<<<grid, TILE_THREADS, 0, stream>>>(a);
-    } else {
-      if (stage == 0) expert_gate_up_fma_kernel<bf16><<<grid, TILE_THREADS, 0, stream>>>(a);
-      else expert_down_fma_kernel<bf16><<<grid, TILE_THREADS, 0, stream>>>(a);
-    }
+    if (stage == 0) expert_gate_up_fma_kernel<bf16><<<grid, TILE_THREADS, 0, stream>>>(a);
+    else expert_down_fma_kernel<bf16><<<grid, TILE_THREADS, 0, stream>>>(a);
   } else {
     FMS_REQUIRE(false, "moe_experts: unknown dtype %d", dtype);
   }

@@ -1215,12 +1215,13 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, gate_w: Optional[torch.Tenso
             raise TypeError("the experts' weights are contiguous and of the type of x")
     lib = load()
     n_pairs = T * top
-    # tiles of 64 rows where the experts have many rows (prompts) and the matrix-core kernel can load the rows
-    wide_ok = x.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and x.stride(0) % 8 == 0
+    # the matrix-core kernels load 16 bytes at a time
+    wide_ok = x.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and x.stride(0) % 8 == 0 and not any(
+        t.data_ptr() % 16 for t in (x, gate_w, up_w, down_w))
     tile_rows = lib.fmsamd_moe_tile_rows(n_pairs, E, int(wide_ok))
     max_tiles = lib.fmsamd_moe_max_tiles(n_pairs, E, tile_rows)
     order = torch.empty(n_pairs, dtype=torch.int32, device=x.device)
-    tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=x.device)
+    tiles = torch.empty(3 * max_tiles + 1, dtype=torch.int32, device=x.device)  # the tiles, and how many there are
     check(lib.fmsamd_moe_group(ids.data_ptr(), n_pairs, E, order.data_ptr(), tiles.data_ptr(), max_tiles, tile_rows, _stream()))
     hidden = torch.empty(n_pairs, ff, dtype=x.dtype, device=x.device)
     y = torch.empty(n_pairs, width, dtype=torch.float32, device=x.device)

@@ -364,6 +364,40 @@ def test_experts_and_their_sum(lib, dtype, sizes):
     torch.testing.assert_close(out.float().cpu(), want, **tol)
 
 
+# rows an expert around the edges of a tile (32 rows up to 20 rows an expert on average, 128 above), experts without rows,
+# K past a whole step of 64 (72, 200, 136), columns past a block's 128 or 256, and rows that are not aligned to 16 bytes
+@pytest.mark.parametrize("counts", [(1, 31, 0), (32, 2, 33, 0, 1), (127, 0, 129), (128, 1, 256, 20), (21, 20), (700,)])
+@pytest.mark.parametrize("ff,width", [(136, 72), (264, 200), (8, 520)])
+@pytest.mark.parametrize("form", ["gated", "scaled", "plain", "unaligned"])
+def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(ff + len(counts))
+    E, T = len(counts), sum(counts)
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(T, generator=gen)].to(torch.int32)[:, None].contiguous()
+    x = torch.randn(T, width, generator=gen).to(torch.bfloat16)
+    wg, wu = [(torch.randn(E, ff, width, generator=gen) * 2 / math.sqrt(width)).to(torch.bfloat16) for _ in range(2)]
+    wd = (torch.randn(E, width, ff, generator=gen) / math.sqrt(ff)).to(torch.bfloat16)
+    scale = torch.rand(T, 1, generator=gen) + 0.5 if form == "scaled" else None
+    rows = x.to(DEV)
+    if form == "unaligned":
+        rows = torch.zeros(T * width + 4, dtype=torch.bfloat16, device=DEV)[4:].view(T, width).copy_(rows)
+    y = ops.moe_experts(rows, ids.to(DEV), None if form == "plain" else wg.to(DEV), wu.to(DEV), wd.to(DEV), 1.25, 1.702, 1.0,
+                        in_scale=None if scale is None else scale.to(DEV), activation="relu2" if form == "plain" else "identity").cpu().double()
+    for e in range(E):
+        at = torch.where(ids[:, 0] == e)[0]
+        xe = x[at].double() if scale is None else x[at].double() * scale[at].double()
+        u = xe @ wu[e].double().T
+        if form == "plain":
+            h = u.clamp(min=0) ** 2
+        else:
+            g = (xe @ wg[e].double().T).clamp(max=1.25)
+            h = g * torch.sigmoid(1.702 * g) * (u.clamp(-1.25, 1.25) + 1)
+        # hidden is kept in bfloat16 (a rounding of 2^-9, twice that where a 32-bit sum falls on the other side of a tie)
+        bound = 2.0 ** -8 * (h.abs() @ wd[e].double().abs().T) + 1e-4
+        assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
+
+
 # ---- the engine ------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("name", sorted(CONFIGS))
 @pytest.mark.parametrize("dtype", DTYPES)
