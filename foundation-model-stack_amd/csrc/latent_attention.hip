@@ -14,12 +14,14 @@
 //   headwise_linear:      y[t, h, :] = W_h x[t, h, :] (optionally times sigmoid(gate[t, h])), FMA or MFMA
 //   latent_attn_generic:  float32 arithmetic on any storage type; one block per (head, token)
 //   latent_attn_mfma:     bfloat16, MFMA 16x16x32; a wave owns 16 heads of one token (+ merge of partial results)
+//   latent_attn_prompt:   the same for prompts with a latent of 512, keys and latent straight into LDS
 //
 // Cache layout: rows [page][token in page][R + P]; for the MFMA kernel also the latent transposed, [page][R][token in
 // page], so that both products read their contraction index contiguously, straight from global memory.
 #include "common.h"
 #include "fmsamd.h"
 #include "tile_product.h"
+#include "tile_product_lds.h"
 
 // --------------------------------------------------------------------------
 // cache write
@@ -459,6 +461,18 @@ __device__ __forceinline__ void latent_finish(LatentState<RT, WC>& st, bf16* __r
   }
 }
 
+#define LAT_GROUP 4  // tiles of a block of latent_attn_prompt_kernel
+
+// do the tiles of a group belong to one sequence?  (the same answer in every lane)
+__device__ __forceinline__ bool latent_group_together(int group, int n_tiles, int tiles_per_token, const int* seq_of_token) {
+  const int first = group * LAT_GROUP, last = first + LAT_GROUP < n_tiles ? first + LAT_GROUP - 1 : n_tiles - 1;
+  const int t0 = first / tiles_per_token, t1 = last / tiles_per_token;
+  const int seq = uniform_load(seq_of_token + t0);
+  bool same = seq >= 0;
+  for (int t = t0 + 1; t <= t1; ++t) same = same && uniform_load(seq_of_token + t) == seq;
+  return same;
+}
+
 // LDS: the four waves of a block (four consecutive tiles of one sequence: neighbouring tokens, or the head groups of
 // one token) share every tile of keys through LDS, so a tile comes from the caches once a block instead of once a
 // wave; a block whose tiles lie in different sequences, and every block of a decode step, loads straight from
@@ -469,11 +483,13 @@ __global__ void __launch_bounds__(256)
                             const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                             const int* __restrict__ block_table, int table_stride, const bf16* __restrict__ cache,
                             const bf16* __restrict__ vt_cache, const float* __restrict__ sink, int n_tokens, int nheads,
-                            int rank, int width, float scale, int window, int tiles_per_token, int n_parts) {
+                            int rank, int width, float scale, int window, int tiles_per_token, int n_parts, int mixed_groups_only) {
   extern __shared__ __attribute__((aligned(16))) bf16 lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int n_tiles = n_tokens * tiles_per_token;
+  // what latent_attn_prompt_kernel has left: groups of tiles of several sequences
+  if (LDS && mixed_groups_only && latent_group_together(blockIdx.x, n_tiles, tiles_per_token, seq_of_token)) return;
   int tile, part;
   if (n_parts == 1) {
     tile = blockIdx.x * 4 + wave;
@@ -644,6 +660,215 @@ __global__ void __launch_bounds__(256)
   latent_finish<RT, WC, EXACT>(st, out, ldo, ws, t, head, nheads, rank, n_parts, part, grp);
 }
 
+// --------------------------------------------------------------------------
+// bfloat16 prompts with a latent of RT * 16 elements in rows of WC * 32, the arithmetic of the kernel above.  A
+// wave owns one tile (a token and 16 of its heads), its queries and results in registers, a SIMD to itself; the four
+// tiles of a block share every 32 keys (rows and transposed latent) through LDS, in two buffers filled straight from memory
+// while the other one is worked on, and operands are read from LDS some products ahead.
+//
+// Bound by the LDS reads of the operands (68 KB a wave and 32 keys for a latent of 512) and the chain through a tile's products and
+// softmax, which a wave alone on its SIMD cannot hide.  One prompt of 2048 tokens, 16 heads, latent 512 + 64: 138 us; with the keys
+// through registers and the shortest contexts first (the kernel above) 355, with results scaled whenever a maximum moved 212,
+// with that inside the loop over the keys 182.
+// Blocks whose tiles belong to several sequences are left to latent_attn_mfma_kernel.
+// --------------------------------------------------------------------------
+#define LAT_SLACK 8.f
+
+template <int RT, int WC>
+__global__ void __launch_bounds__(256, 1)
+    latent_attn_prompt_kernel(const bf16* __restrict__ qa, long ldq, bf16* __restrict__ out, long ldo, const int* __restrict__ positions,
+                              const int* __restrict__ seq_of_token, const int* __restrict__ block_table, int table_stride,
+                              const bf16* __restrict__ cache, const bf16* __restrict__ vt_cache, const float* __restrict__ sink,
+                              int n_tokens, int nheads, float scale, int window, int tiles_per_token) {
+  constexpr int RANK = RT * 16, WIDTH = WC * 32;
+  constexpr int K_BYTES = 32 * WIDTH * 2, V_BYTES = RANK * 64, STAGE = K_BYTES + V_BYTES;
+  constexpr int K_LOADS = K_BYTES / 4096, V_LOADS = V_BYTES / 4096;  // of 1 KB, a wave
+  constexpr int PIECES = WIDTH / 8;                                  // of 16 bytes in a key's row
+  static_assert(K_BYTES % 4096 == 0 && V_BYTES % 4096 == 0 && PIECES % 8 == 0, "whole loads, whole groups of pieces");
+  extern __shared__ __attribute__((aligned(16))) bf16 lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int n_tiles = n_tokens * tiles_per_token;
+  const int group = gridDim.x - 1 - blockIdx.x;  // the longest contexts first
+  if (!latent_group_together(group, n_tiles, tiles_per_token, seq_of_token)) return;
+  const int first_tile = group * LAT_GROUP, last_tile = first_tile + LAT_GROUP < n_tiles ? first_tile + LAT_GROUP - 1 : n_tiles - 1;
+  const int tile = first_tile + wave;
+  const bool works = tile <= last_tile;
+  const int t = (works ? tile : last_tile) / tiles_per_token, head = (tile % tiles_per_token) * 16 + col;
+  const bool valid = works && head < nheads;
+  const int seq = uniform_load(seq_of_token + t);
+  const int* bt = block_table + (size_t)seq * table_stride;
+  int first_pos = 0x7fffffff, last_pos = -1;  // of the block's tokens
+  for (int u = first_tile / tiles_per_token; u <= last_tile / tiles_per_token; ++u) {
+    const int p = uniform_load(positions + u);
+    first_pos = p < first_pos ? p : first_pos, last_pos = p > last_pos ? p : last_pos;
+  }
+  const int pos = uniform_load(positions + t);
+  const int first_lo = window > 0 && first_pos - window + 1 > 0 ? first_pos - window + 1 : 0;
+  const int lo = window > 0 && pos - window + 1 > 0 ? pos - window + 1 : 0;
+
+  bf16x8 q[WC];
+  {
+    const bf16* qrow = qa + (size_t)t * ldq + (size_t)(head < nheads ? head : 0) * WIDTH + grp * 8;
+#pragma unroll
+    for (int c = 0; c < WC; ++c) q[c] = *reinterpret_cast<const bf16x8*>(qrow + c * 32);
+  }
+
+  // what this lane loads: LDS holds a tile's pieces in the order of the rows; which piece of its group of eight (of a latent
+  // element's four) a lane asks for is swizzled with the key (the element), so that operand reads cover all banks
+  auto key_swizzle = [](int key) { return (key & 3) | ((key >> 1) & 4); };
+  unsigned k_from[K_LOADS];
+#pragma unroll
+  for (int n = 0; n < K_LOADS; ++n) {
+    const int at = (wave * K_LOADS + n) * 64 + lane, key = at / PIECES, p = at % PIECES;
+    k_from[n] = (key * PIECES + (p ^ key_swizzle(key))) * 16;
+  }
+  const int v_row = wave * V_LOADS * 16 + (lane >> 2);
+  const unsigned v_from = v_row * (PAGE_TOKENS * 2) + ((lane & 3) ^ ((lane >> 3) & 3)) * 16;  // rows 16 apart swizzle alike
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)lds;
+  auto fetch = [&](int base, int buffer) {
+    const size_t page = readable_page(uniform_load(bt + base / PAGE_TOKENS));
+    const int in_page = base % PAGE_TOKENS;
+    const char* kp = (const char*)(cache + (page * PAGE_TOKENS + in_page) * WIDTH);
+    const char* vp = (const char*)(vt_cache + page * RANK * PAGE_TOKENS + in_page);
+    const unsigned to = lds0 + buffer * STAGE;
+#pragma unroll
+    for (int n = 0; n < K_LOADS; ++n) load_to_lds(kp, k_from[n], to + (wave * K_LOADS + n) * 1024);
+#pragma unroll
+    for (int n = 0; n < V_LOADS; ++n) load_to_lds(vp + n * 16 * PAGE_TOKENS * 2, v_from, to + K_BYTES + (wave * V_LOADS + n) * 1024);
+  };
+
+  // operand reads: this lane's key in score tile a (tile b: + 4), its latent element of every 16.  Steps of K two apart differ
+  // by 128 bytes, which leaves the swizzle as it is.
+  const int key_a = 8 * (col >> 2) + (col & 3);
+  int k_at[2][2], v_at;  // [tile][step of K % 2]
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) k_at[w][c] = (key_a + 4 * w) * WIDTH * 2 + ((4 * c + grp) ^ key_swizzle(key_a + 4 * w)) * 16;
+  v_at = K_BYTES + col * 64 + (grp ^ ((col >> 1) & 3)) * 16;
+
+  f32x4 acc[RT];
+#pragma unroll
+  for (int d = 0; d < RT; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the sink is where the softmax starts
+  float m = sink && valid ? sink[head] : LAT_EMPTY, l = sink && valid && grp == 0 ? 1.f : 0.f;
+
+  constexpr int KG = 3, VG = 4;  // steps of K, and tiles of the latent, that are read before the ones in front are multiplied
+  bf16x8 ka[2][KG], kb[2][KG], v[2][VG];
+  float s[8];
+  // the scores of the buffer's 32 keys: s[i] is key base + 8 grp + i of this lane's column
+  auto scores = [&](const char* kv, int base) {
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    auto read_k = [&](int set, int c0) {
+#pragma unroll
+      for (int c = 0; c < KG; ++c)
+        if (c0 + c < WC) {
+          ka[set][c] = *reinterpret_cast<const bf16x8*>(kv + k_at[0][(c0 + c) & 1] + ((c0 + c) >> 1) * 128);
+          kb[set][c] = *reinterpret_cast<const bf16x8*>(kv + k_at[1][(c0 + c) & 1] + ((c0 + c) >> 1) * 128);
+        }
+    };
+    read_k(0, 0);
+#pragma unroll
+    for (int c0 = 0; c0 < WC; c0 += KG) {
+      const int set = (c0 / KG) & 1;
+      if (c0 + KG < WC) read_k(set ^ 1, c0 + KG);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < KG; ++c)
+        if (c0 + c < WC) {
+          sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[set][c], q[c0 + c], sa, 0, 0, 0);
+          sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[set][c], q[c0 + c], sb, 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = sa[i] * scale, s[4 + i] = sb[i] * scale;
+    if (base + 31 > pos || base < lo) {  // the same in all lanes
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = base + 8 * grp + i;
+        s[i] = key >= lo && key <= pos ? s[i] : -INFINITY;
+      }
+    }
+    float top = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+    top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+    return fmaxf(top, __shfl_xor(top, 32, WAVE));
+  };
+  // their probabilities and values into the sums
+  auto values = [&](const char* kv) {
+    auto read_v = [&](int set, int d0) {
+#pragma unroll
+      for (int d = 0; d < VG; ++d) v[set][d] = *reinterpret_cast<const bf16x8*>(kv + v_at + (d0 + d) * 16 * 64);
+    };
+    read_v(0, 0);
+    float psum = 0.f;
+    bf16x8 pmat;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float p = __expf(s[i] - m);  // exp(-inf) = 0 for the keys that are not seen
+      psum += p;
+      pmat[i] = (bf16)p;
+    }
+    l += psum;
+#pragma unroll
+    for (int d0 = 0; d0 < RT; d0 += VG) {
+      const int set = (d0 / VG) & 1;
+      if (d0 + VG < RT) read_v(set ^ 1, d0 + VG);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < VG; ++d) acc[d0 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[set][d], pmat, acc[d0 + d], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // The reference m that probabilities are taken against follows the maximum only where that has left it LAT_SLACK behind: sums
+  // and results are float32, and a bfloat16 probability is as exact at e^LAT_SLACK as at 1.  The results live in the matrix
+  // unit's registers and have to be moved out and back to be scaled: that stands outside the loop over the keys, or the
+  // compiler moves them for every tile (the waves of a block meet at the same barriers wherever they stand in the code).
+  const int first_base = first_lo / 32 * 32;
+  fetch(first_base, 0);
+  int base = first_base, buffer = 0;
+  float top = LAT_EMPTY;
+  for (;;) {
+    bool behind = false;
+    for (; base <= last_pos; base += 32, buffer ^= 1) {
+      if (base + 32 <= last_pos) {
+        fetch(base + 32, buffer ^ 1);
+        tile_wait<K_LOADS + V_LOADS>();
+      } else {
+        tile_wait<0>();
+      }
+      if (works && base <= pos) {  // the same in all lanes of the wave
+        const char* kv = (const char*)lds + buffer * STAGE;
+        top = scores(kv, base);
+        behind = __any(top > m + LAT_SLACK);
+        if (behind) break;
+        values(kv);
+      }
+      block_sync_lds();  // everybody has read the buffer
+    }
+    if (!behind) break;
+    const float m_new = top > m + LAT_SLACK ? top : m;
+    const float alpha = __expf(m - m_new);
+    l *= alpha;
+    m = m_new;
+#pragma unroll
+    for (int d = 0; d < RT; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[d][i] *= alpha;
+    values((const char*)lds + buffer * STAGE);
+    block_sync_lds();
+    base += 32, buffer ^= 1;
+  }
+  if (!works) return;
+  LatentState<RT, WC> st;
+#pragma unroll
+  for (int d = 0; d < RT; ++d) st.acc[d] = acc[d];
+  st.m = m, st.l = l;
+  latent_finish<RT, WC, true>(st, out, ldo, nullptr, t, head, nheads, RANK, 1, 0, grp);
+}
+
 // out[t, h, :] = sum_i acc_i exp(m_i - M) / sum_i l_i exp(m_i - M) over the parts i.  The parts' maxima and sums are
 // loaded side by side (a thread a part) and their weights left in LDS: no chain of dependent loads.
 #define LAT_MAX_PARTS 256
@@ -732,11 +957,37 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
   if (n_splits == 0)                                                                                                               \
     latent_attn_mfma_kernel<RT, WC, true, EXACT><<<grid, 256, lds, stream>>>(                                                      \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
-        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts);  \
+        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts,   \
+        prompt_kernel);                                                                                                            \
   else                                                                                                                             \
     latent_attn_mfma_kernel<RT, WC, false, EXACT><<<grid, 256, q_lds, stream>>>(                                                   \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
-        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts)
+        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts, 0)
+  // prompts with a latent of 512: the groups of tiles that belong to one sequence first, what is left with the other kernel
+  const int prompt_kernel = n_splits == 0 && rank == 512 && (width == 576 || width == 512);
+  if (prompt_kernel) {
+    const int groups = ceil_div(tiles, LAT_GROUP);
+#define LAUNCH_PROMPT(RT, WC)                                                                                                      \
+  const size_t bytes = 2 * (size_t)(32 * WC * 32 * 2 + RT * 16 * 64); /* two buffers of keys and latent */                         \
+  static bool allowed = false;                                                                                                     \
+  if (!allowed) {                                                                                                                  \
+    const hipError_t e = hipFuncSetAttribute((const void*)latent_attn_prompt_kernel<RT, WC>,                                       \
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                              \
+    FMS_REQUIRE(e == hipSuccess, "latent_attn_mfma: the kernel's LDS could not be sized: %s", hipGetErrorString(e));               \
+    allowed = true;                                                                                                                \
+  }                                                                                                                                \
+  latent_attn_prompt_kernel<RT, WC><<<groups, 256, bytes, stream>>>((const bf16*)qa, ldq, (bf16*)out, ldo, positions, seq_of_token, \
+                                                                    block_table, table_stride, (const bf16*)cache,                 \
+                                                                    (const bf16*)vt_cache, sink, n_tokens, nheads, scale, window,   \
+                                                                    tiles_per_token)
+    if (width == 576) {
+      LAUNCH_PROMPT(32, 18);
+    } else {
+      LAUNCH_PROMPT(32, 16);
+    }
+#undef LAUNCH_PROMPT
+    FMS_LAUNCH_CHECK("latent_attn_prompt");
+  }
   // the sizes of the largest configuration exactly (a latent of 512 with a rotated part of 64, or with none) and the
   // smaller latents without a rotated part run without a question around any product; everything else in the smallest
   // configuration that holds it

@@ -33,6 +33,11 @@ __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_at) : "memory", "m0");
 }
 
+// The same from `offset` bytes behind an address that all lanes share.
+__device__ __forceinline__ void load_to_lds(const void* base, unsigned offset, unsigned lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_at) : "memory", "m0");
+}
+
 // All but the last OUTSTANDING loads of this wave have arrived and its reads from LDS are done; then the block's barrier.
 template <int OUTSTANDING>
 __device__ __forceinline__ void tile_wait() {

@@ -364,6 +364,37 @@ def test_experts_and_their_sum(lib, dtype, sizes):
     torch.testing.assert_close(out.float().cpu(), want, **tol)
 
 
+# prompts with a latent of 512: blocks of one sequence (the kernel that shares keys through LDS), blocks that straddle two (left
+# to the other one), a last block that is not full, positions that start inside a sequence, windows, one to three tiles a token
+@pytest.mark.parametrize("heads", [5, 16, 20, 40])
+@pytest.mark.parametrize("rot", [64, 0])
+@pytest.mark.parametrize("runs,window", [([(0, 70)], 0), ([(0, 1), (0, 5), (60, 9)], 0), ([(130, 34), (0, 33)], 40), ([(31, 2), (95, 66)], 7)])
+def test_latent_attention_of_prompts(lib, heads, rot, runs, window):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(heads + rot)
+    R, W = 512, 512 + rot
+    pages_of = [-(-(s + n) // 64) for s, n in runs]
+    order = torch.randperm(sum(pages_of), generator=gen).tolist()
+    table = torch.full((len(runs), max(pages_of)), -1, dtype=torch.int32)
+    for i, n in enumerate(pages_of):
+        table[i, :n] = torch.tensor([order.pop() for _ in range(n)])
+    cache = torch.randn(sum(pages_of), 1, 64, W, generator=gen).to(torch.bfloat16).to(DEV)
+    values = cache[..., :R].transpose(2, 3).contiguous()
+    T = sum(n for _, n in runs)
+    seq = torch.cat([torch.full((n,), i) for i, (_, n) in enumerate(runs)]).to(torch.int32).to(DEV)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in runs]).to(torch.int32).to(DEV)
+    qa = torch.randn(T, heads * W, generator=gen).to(torch.bfloat16).to(DEV)
+    sink = torch.randn(heads, generator=gen).to(DEV)
+    args = (qa, pos, seq, table.to(DEV), cache, sink, heads, R, rot, 0.05, window)
+    got = ops.latent_attention(*args, vt_cache=values).float()
+    want = ops.latent_attention(*args, force_generic=True).float()  # float32 arithmetic, result rounded to bfloat16
+    # probabilities and results are rounded to bfloat16 (by at most 2^-8 each, once more for the other kernel's result); results
+    # are at most the largest latent in size, and most are far below
+    assert float((got - want).abs().max()) <= 3 * 2.0 ** -8 * float(cache.float().abs().max())
+    assert float((got - want).norm() / want.norm()) < 0.01
+
+
 # rows an expert around the edges of a tile (32 rows up to 20 rows an expert on average, 128 above), experts without rows,
 # K past a whole step of 64 (72, 200, 136), columns past a block's 128 or 256, and rows that are not aligned to 16 bytes
 @pytest.mark.parametrize("counts", [(1, 31, 0), (32, 2, 33, 0, 1), (127, 0, 129), (128, 1, 256, 20), (21, 20), (700,)])
@@ -393,7 +424,7 @@ def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
         else:
             g = (xe @ wg[e].double().T).clamp(max=1.25)
             h = g * torch.sigmoid(1.702 * g) * (u.clamp(-1.25, 1.25) + 1)
-        # hidden is kept in bfloat16 (a rounding of 2^-9, twice that where a 32-bit sum falls on the other side of a tie)
+        # hidden is kept in bfloat16: rounded by at most 2^-8 of itself
         bound = 2.0 ** -8 * (h.abs() @ wd[e].double().abs().T) + 1e-4
         assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
 
