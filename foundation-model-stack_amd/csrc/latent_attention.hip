@@ -971,7 +971,9 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
         (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts, 0)
   // prompts with a latent of 512: the groups of tiles that belong to one sequence first, what is left with the other kernel
-  const int prompt_kernel = n_splits == 0 && rank == 512 && (width == 576 || width == 512);
+  // (its rows go straight to LDS, which wants 16-byte addresses)
+  const int prompt_kernel =
+      n_splits == 0 && rank == 512 && (width == 576 || width == 512) && (uintptr_t)cache % 16 == 0 && (uintptr_t)vt_cache % 16 == 0;
   if (prompt_kernel) {
     const int groups = ceil_div(tiles, LAT_GROUP);
 #define LAUNCH_PROMPT(RT, WC)                                                                                                      \

@@ -393,6 +393,10 @@ def test_latent_attention_of_prompts(lib, heads, rot, runs, window):
     # are at most the largest latent in size, and most are far below
     assert float((got - want).abs().max()) <= 3 * 2.0 ** -8 * float(cache.float().abs().max())
     assert float((got - want).norm() / want.norm()) < 0.01
+    # a cache that starts at no 16-byte address goes to the other kernel
+    moved = [torch.zeros(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t) for t in (cache, values)]
+    got = ops.latent_attention(*args[:4], moved[0], *args[5:], vt_cache=moved[1]).float()
+    assert float((got - want).norm() / want.norm()) < 0.01
 
 
 # rows an expert around the edges of a tile (32 rows up to 20 rows an expert on average, 128 above), experts without rows,
