@@ -548,11 +548,13 @@ static void launch_skinny(const void* x, long ldx, const void* w, const void* bi
 #define SK_COMPUTE_UNITS 256
 static int skinny_x_rows(int M) { return ceil_div(M, 4) * 4; }
 
-// 17 to 32 rows of x and a short K: the kernel above with two tiles of x a wave beats the kernels of
-// gemm_wide.hip, which have to cut so short a K into slices that meet in memory and need a second kernel
-// (measured at K = 4096: 13.5 against 17.2 us for 6144 weight rows, 11.3 against 14.5 for 4096; at K = 14336, and
-// from 33 rows on, where every block reads more of x than of W, the wide kernels win).
-static bool skinny_takes_many_rows(int M, int N, int K) { return M > 16 && M <= 32 && K <= 8192; }
+// 17 to 32 rows of x, a short K and weight rows that are too few to give every compute unit a block of gemm_wide.hip: the
+// kernel above with two tiles of x a wave beats the kernels there, which have to cut K into slices that meet in memory and
+// need a second kernel (measured with 24 rows at K = 4096: 12.7 against 16.2 us for 4096 weight rows, 15.6 against 17.2 for
+// 6144, 26 against 29 for 12288, but 40.0 against 29.8 for 16384 and 72 against 44 for 32768; at K = 2048 the lines cross
+// between 12288 and 16384 as well; at K = 14336, and from 33 rows on, where every block reads more of x than of W, the wide
+// kernels win).
+static bool skinny_takes_many_rows(int M, int N, int K) { return M > 16 && M <= 32 && K <= 8192 && N < 16384; }
 
 static int skinny_rows_per_block(int N, int M) {
   int best = 0;

@@ -33,7 +33,12 @@ __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_at) : "memory", "m0");
 }
 
-// The same from `offset` bytes behind an address that all lanes share.
+// The same for bytes that nobody else reads soon: they pass the caches by.
+__device__ __forceinline__ void load_once_to_lds(const void* from, unsigned lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(from), "s"(lds_at) : "memory", "m0");
+}
+
+// The same as load_to_lds from `offset` bytes behind an address that all lanes share.
 __device__ __forceinline__ void load_to_lds(const void* base, unsigned offset, unsigned lds_at) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_at) : "memory", "m0");
 }

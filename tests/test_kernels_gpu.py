@@ -490,6 +490,23 @@ def test_gemm_bf16(ops, M, N, K):
     torch.testing.assert_close(out.double(), want, atol=3e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 97, 129, 161, 192])
+@pytest.mark.parametrize("N,K,skip", [(33004, 72, 0), (512, 4104, 0), (16384, 520, 0), (20, 8200, 0), (300, 1032, 3)])
+def test_gemm_bf16_cuts_of_the_wide_product(ops, M, N, K, skip):
+    """Two rounds of blocks, slices of K with a short last step, blocks that own fewer rows than they have places for, rows
+    that start at no 16-byte address.
+
+    A product of two bfloat16 is exact in float32; a sum of K of them in any order is off by at most K 2^-24 sum |x w|."""
+    torch.manual_seed(9)
+    rows = torch.randn(M, K + 8).to(torch.bfloat16)
+    x = rows[:, skip : skip + K]
+    w = (torch.randn(N, K) * 0.1).to(torch.bfloat16)
+    out = ops.linear(dev(rows)[:, skip : skip + K], dev(w), None, out_dtype=torch.float32, allow_library=False).cpu().double()
+    want = (x.float() @ w.float().t()).double() if N * K > 4e6 else x.double() @ w.double().t()
+    bound = 2 * K * 2.0**-24 * (x.float().abs() @ w.float().abs().t()).double()  # (twice: the reference may be float32 too)
+    assert bool(((out - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M", [1, 5, 17, 64, 70, 200])
 @pytest.mark.parametrize("N,K", [(37, 12), (100, 44), (60, 50), (301, 1000 + 4)])
 def test_gemm_bf16_of_widths_that_are_no_multiple_of_8(ops, M, N, K):
