@@ -1045,7 +1045,7 @@ __device__ __forceinline__ void decode_keys(WaveState<MAXDT, 1>& st, const bf16x
 __device__ __forceinline__ void staged_load(bf16x8 (&raw)[16], const bf16* __restrict__ p) {
   const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) raw[i] = load_bf16x8(p + i * 512 + lane * 8);
+  for (int i = 0; i < 16; ++i) raw[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p + i * 512 + lane * 8));
 }
 
 // One page: its keys are on their way into raw; vp points at its values, kn (PREFETCH) at the next page's
