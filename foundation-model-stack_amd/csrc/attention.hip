@@ -1042,6 +1042,8 @@ __device__ __forceinline__ void decode_keys(WaveState<MAXDT, 1>& st, const bf16x
 // A compute unit's loads queue up behind one another (16 KB asked for when the unit's other waves have just
 // asked for theirs take some microseconds); a wave that asks again the moment its registers are free keeps
 // that queue full instead of waiting at its end once a page.
+// The loads are marked as bytes that are not read again: 64 sequences of 128 to 2048 tokens (8 kv heads) take 52.2 us instead
+// of 58.3, 8 of 6950 tokens 38.8 instead of 44.
 __device__ __forceinline__ void staged_load(bf16x8 (&raw)[16], const bf16* __restrict__ p) {
   const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll

@@ -411,7 +411,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
   // gated: a wave's first TN / 2 tiles are gate columns, the others the up columns of the same elements
   const int n0 = col * (GATED ? S::BN / 2 : S::BN);
   f32x16 acc[TM][TN];
-  tile_product_lds<WM, WN, TM, TN, ST>([&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; },
+  tile_product_lds<WM, WN, TM, TN, ST, S::BM == TILE_SMALL_ROWS>([&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; },
                                    [&](int n) {
                                      const int t = n / 32;
                                      const bool up = GATED && t % TN >= TN / 2;
@@ -456,7 +456,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
   const bf16* x = (const bf16*)a.x;
   const bf16* w = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
   f32x16 acc[TM][TN];
-  tile_product_lds<WM, WN, TM, TN, ST>([&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; },
+  tile_product_lds<WM, WN, TM, TN, ST, S::BM == TILE_SMALL_ROWS>([&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; },
                                    [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; }, a.K, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll

@@ -52,7 +52,8 @@ __device__ __forceinline__ void tile_wait() {
 // a_row(m), m < BM, and w_row(n), n < BN, return the first element of a row that can be read; a row that is not there is any
 // row that is (its results are not stored).  After the call, lane l of wave w holds
 //   acc[i][j][e] = C[row ((w / WN) * TM + i) * 32 + 8 (e / 4) + 4 (l / 32) + e % 4][column ((w % WN) * TN + j) * 32 + l % 32].
-template <int WM, int WN, int TM, int TN, int STAGES, typename ARow, typename WRow>
+// W_ONCE: nobody else reads these rows of W soon.
+template <int WM, int WN, int TM, int TN, int STAGES, bool W_ONCE = false, typename ARow, typename WRow>
 __device__ __forceinline__ void tile_product_lds(ARow a_row, WRow w_row, int K, bf16* lds, f32x16 (&acc)[TM][TN]) {
   typedef TileLds<WM, WN, TM, TN, STAGES> S;
   // load instructions of a step, 8 rows each: RA for rows of A and RB for rows of W a wave (where there are fewer rows of A
@@ -86,6 +87,12 @@ __device__ __forceinline__ void tile_product_lds(ARow a_row, WRow w_row, int K, 
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
+  auto load = [&](int i, const void* from, unsigned to) {
+    if (W_ONCE && i >= RA)
+      load_once_to_lds(from, to);
+    else
+      load_to_lds(from, to);
+  };
   const int steps = (K + TL_BK - 1) / TL_BK;
   const void* from[R];
   // where step s comes from; past the end: zeros, so that every step has the same number of loads under way
@@ -112,7 +119,7 @@ __device__ __forceinline__ void tile_product_lds(ARow a_row, WRow w_row, int K, 
   for (int s = 0; s < STAGES; ++s) {
     find(s);
 #pragma unroll
-    for (int i = 0; i < R; ++i) load_to_lds(from[i], put[i] + s * (STAGE * 2));
+    for (int i = 0; i < R; ++i) load(i, from[i], put[i] + s * (STAGE * 2));
   }
   tile_wait<(STAGES - 1) * R>();
   read(0, lds, 0);
@@ -142,7 +149,7 @@ __device__ __forceinline__ void tile_product_lds(ARow a_row, WRow w_row, int K, 
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[set][i], wv[set][j], acc[i][j], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int l = q * PER; l < (q + 1) * PER && l < R; ++l) load_to_lds(from[l], put[l] + stage * (STAGE * 2));
+          for (int l = q * PER; l < (q + 1) * PER && l < R; ++l) load(l, from[l], put[l] + stage * (STAGE * 2));
           __builtin_amdgcn_sched_barrier(0);
         }
       }
