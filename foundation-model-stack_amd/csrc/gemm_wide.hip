@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(512)
   // bytes of their rows at the same time (rows lie a multiple of kilobytes apart) crowd into few memory
   // channels.  The start depends on the block's place only, so the order of the sum does too.
   const int n_steps = g_end - g_begin;
-  const int rot = (blockIdx.x * 5) % n_steps;
+  const int rot = WD_GROUP / BK * ((blockIdx.x * 5) % ((n_steps + WD_GROUP / BK - 1) / (WD_GROUP / BK)));  // (whole groups)
   auto fetch = [&](int t, int stage) {  // past the end: zeros, so that every step has the same number of loads under way
     const int u = t + rot;
     const int k0 = (g_begin + (u >= n_steps ? u - n_steps : u)) * BK;
@@ -417,6 +417,9 @@ static bool wide_finishes_itself(int epi) { return epi == EPI_PLAIN || epi == EP
 static WidePlan wide_plan(int epi, int M, int rows, int K) {
   const int ngroups = ceil_div(K, WD_GROUP), mt = ceil_div(M, 32);
   const double busy = 0.1 + 0.3 * ((mt + 1) / 2);
+  // A short K: a slice a group, as the waves of the kernel for fewer rows (gemm.hip) take it, so that a batch that shrinks below
+  // 33 rows, or is one of fewer rows for some steps, goes on with the same bits.
+  if (ngroups <= 8 && ceil_div(rows, WD_ROWS) * ngroups <= WD_COMPUTE_UNITS) return {WD_ROWS, ngroups};
   WidePlan best{WD_ROWS, 1};
   double best_cost = -1;
   for (int slices = 1; slices <= ngroups && slices <= 64; ++slices) {
