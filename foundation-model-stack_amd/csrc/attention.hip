@@ -1042,17 +1042,20 @@ __device__ __forceinline__ void decode_keys(WaveState<MAXDT, 1>& st, const bf16x
 // A compute unit's loads queue up behind one another (16 KB asked for when the unit's other waves have just
 // asked for theirs take some microseconds); a wave that asks again the moment its registers are free keeps
 // that queue full instead of waiting at its end once a page.
-// The loads are marked as bytes that are not read again: 64 sequences of 128 to 2048 tokens (8 kv heads) take 52.2 us instead
-// of 58.3, 8 of 6950 tokens 38.8 instead of 44.
+// ONCE: the pages are marked as bytes that are not read again.
+template <bool ONCE>
 __device__ __forceinline__ void staged_load(bf16x8 (&raw)[16], const bf16* __restrict__ p) {
   const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) raw[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p + i * 512 + lane * 8));
+  for (int i = 0; i < 16; ++i) {
+    const bf16* at = p + i * 512 + lane * 8;
+    raw[i] = ONCE ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(at)) : load_bf16x8(at);
+  }
 }
 
 // One page: its keys are on their way into raw; vp points at its values, kn (PREFETCH) at the next page's
 // keys.  The softmax takes the page's 64 keys at once.
-template <bool PREFETCH>
+template <bool PREFETCH, bool ONCE>
 __device__ __forceinline__ void staged_page_step(WaveState<8, 1>& st, const bf16x8 (&qreg)[4], int qpos, int qlo,
                                                  int key0, bf16x8 (&raw)[16], const bf16* __restrict__ vp,
                                                  const bf16* __restrict__ kn, bf16* __restrict__ buf, Scale2 scale2,
@@ -1071,7 +1074,7 @@ __device__ __forceinline__ void staged_page_step(WaveState<8, 1>& st, const bf16
     }
   }
   __builtin_amdgcn_wave_barrier();
-  staged_load(raw, vp);
+  staged_load<ONCE>(raw, vp);
   // Which key sits in which row of the two score tiles: see decode_keys.  The swizzle key of row key_a is r,
   // and so is that of key_a + 4.
   const int key_a = (r >> 2) * 8 + (r & 3);
@@ -1157,7 +1160,7 @@ __device__ __forceinline__ void staged_page_step(WaveState<8, 1>& st, const bf16
     }
   }
   __builtin_amdgcn_wave_barrier();
-  if (PREFETCH) staged_load(raw, kn);
+  if (PREFETCH) staged_load<ONCE>(raw, kn);
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf) {
     bf16x8 vreg[8];
@@ -1181,6 +1184,7 @@ struct PageWalk {
 };
 
 // The pages of the counts first, first + stride, ... <= last of a sequence's walk, for kv head kh.
+template <bool ONCE>
 __device__ __forceinline__ void decode_pages_staged(WaveState<8, 1>& st, const bf16x8 (&qreg)[4], int qpos, int qlo,
                                                     int first, int stride, int last, PageWalk walk, const int* __restrict__ bt,
                                                     const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
@@ -1190,15 +1194,15 @@ __device__ __forceinline__ void decode_pages_staged(WaveState<8, 1>& st, const b
   const size_t head_off = (size_t)kh * PAGE_TOKENS * 128;
   bf16x8 raw[16];
   size_t phys = readable_page(uniform_load(bt + walk.page(first)));
-  staged_load(raw, k_cache + phys * page_elems + head_off);
+  staged_load<ONCE>(raw, k_cache + phys * page_elems + head_off);
   int pi = first;
   for (; pi + stride <= last; pi += stride) {
     const size_t next = readable_page(uniform_load(bt + walk.page(pi + stride)));
-    staged_page_step<true>(st, qreg, qpos, qlo, walk.page(pi) * PAGE_TOKENS, raw, v_cache + phys * page_elems + head_off,
+    staged_page_step<true, ONCE>(st, qreg, qpos, qlo, walk.page(pi) * PAGE_TOKENS, raw, v_cache + phys * page_elems + head_off,
                            k_cache + next * page_elems + head_off, buf, scale2, ex);
     phys = next;
   }
-  staged_page_step<false>(st, qreg, qpos, qlo, walk.page(pi) * PAGE_TOKENS, raw, v_cache + phys * page_elems + head_off, nullptr,
+  staged_page_step<false, ONCE>(st, qreg, qpos, qlo, walk.page(pi) * PAGE_TOKENS, raw, v_cache + phys * page_elems + head_off, nullptr,
                           buf, scale2, ex);
 }
 
@@ -1224,8 +1228,8 @@ __device__ __forceinline__ int split_pages(int lo, int pos, int keep, int n_spli
 // meet in LDS; the splits of a token meet in the merge kernel.  (Merging in the block that finishes last,
 // behind a device-wide fence and a counter, was measured four times slower: the fence writes back and
 // invalidates the whole L2 of the block's XCD while the other blocks stream through it.)
-// STAGED (head size 128 only): pages go through LDS (decode_page_staged), 16 KB a wave.
-template <int MAXDT, int MAXW, bool STAGED>
+// STAGED (head size 128 only): pages go through LDS (decode_page_staged), 16 KB a wave.  ONCE goes with STAGED.
+template <int MAXDT, int MAXW, bool STAGED, bool ONCE = false>
 __global__ void __launch_bounds__(MAXW* WAVE) __attribute__((amdgpu_waves_per_eu(MAXDT <= 8 ? 2 : 1)))
     attn_decode_bf16_kernel(const bf16* __restrict__ q, long q_stride, bf16* __restrict__ out, long out_stride,
                             float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits,
@@ -1295,7 +1299,7 @@ __global__ void __launch_bounds__(MAXW* WAVE) __attribute__((amdgpu_waves_per_eu
                           dist_len, 1.f / scale};
   if (STAGED) {
     if constexpr (MAXDT == 8)
-      decode_pages_staged(st, qreg, pos, lo, page_lo + wave, n_waves, page_hi, walk, bt, k_cache, v_cache, page_elems, kh,
+      decode_pages_staged<ONCE>(st, qreg, pos, lo, page_lo + wave, n_waves, page_hi, walk, bt, k_cache, v_cache, page_elems, kh,
                           stage + wave * 8192, make_scale2(scale, soft_cap), ex);
   } else {
     for (int wi = page_lo + wave; wi <= page_hi; wi += n_waves) {
@@ -1585,8 +1589,8 @@ extern "C" int fmsamd_attn_decode_bf16(const void* q, long q_stride, void* out, 
   float* part_o = (float*)workspace;
   float* part_ml = part_o ? part_o + (size_t)n_tokens * nheads * n_splits * head_dim : nullptr;
   dim3 grid(n_splits, kvheads * tiles_per_kv, n_tokens);
-#define FMS_DC(M, MAXW, STAGED, LDS)                                                                                 \
-  attn_decode_bf16_kernel<M, MAXW, STAGED><<<grid, dim3(waves * WAVE), LDS, stream>>>(                               \
+#define FMS_DC(M, MAXW, STAGED, LDS, ...)                                                                            \
+  attn_decode_bf16_kernel<M, MAXW, STAGED, ##__VA_ARGS__><<<grid, dim3(waves * WAVE), LDS, stream>>>(                               \
       (const bf16*)q, q_stride, (bf16*)out, out_stride, part_o, part_ml, n_splits, positions, seq_of_token,          \
       block_table, table_stride, (const bf16*)k_cache, (const bf16*)v_cache, nheads, kvheads, head_dim, scale,       \
       window, tile_cols, row_order, soft_cap, chunk, sink, keep_first, dist_bias, dist_len)
@@ -1594,8 +1598,16 @@ extern "C" int fmsamd_attn_decode_bf16(const void* q, long q_stride, void* out, 
   FMS_REQUIRE(staged == 0 || (keep_first == 0 && dist_bias == nullptr), "attn_decode_bf16: kept first keys and a distance table go with pages loaded straight into registers (staged = 0)");
   if (staged != 0) {
     // the waves' results meet in the page buffers: 16 KB a wave hold 16 columns of 130 floats
-    if (waves <= 4)
+    // More pages than the chip's L2 caches hold (32 MB) pass them by: 64 sequences of 128 to 2048 tokens (8 kv heads) take 52.2 us
+    // instead of 58.3, 8 of 6950 tokens 38.8 instead of 44; one sequence of 2048 tokens, whose pages the caches still hold, takes
+    // half a microsecond longer that way.
+    const bool once = (double)n_tokens * (window > 0 && window < max_context ? window : max_context) * kvheads * 128 * 4 > 32e6;
+    if (waves <= 4 && once)
+      FMS_DC(8, 4, true, 0, true);
+    else if (waves <= 4)
       FMS_DC(8, 4, true, 0);
+    else if (once)
+      FMS_DC(8, 8, true, 0, true);
     else
       FMS_DC(8, 8, true, 0);
   } else if (head_dim <= 64)

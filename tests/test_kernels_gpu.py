@@ -349,6 +349,13 @@ def test_attention_decode_bf16(ops, H, K, D):
                            pages_per_block=pages, waves=waves, staged=True)
 
 
+@pytest.mark.parametrize("waves", [3, 8])
+@pytest.mark.parametrize("longest", [1300, 1500])
+def test_attention_decode_on_both_sides_of_what_the_caches_hold(ops, waves, longest):
+    """Six sequences of 8 kv heads: up to 1302 tokens their pages are loaded as ones that stay in the caches, from there on not."""
+    attention_case(ops, torch.bfloat16, 16, 8, 128, starts=[longest, 2, 600, 63, 64, 190], lens=[1] * 6, decode=True, pages_per_block=8, waves=waves)
+
+
 @pytest.mark.parametrize("dtype,decode", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_attention_far_key_and_window(ops, dtype, decode):
     lens = [1, 1] if decode else [40, 3]
