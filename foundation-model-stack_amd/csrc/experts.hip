@@ -206,8 +206,9 @@ extern "C" int fmsamd_moe_route_grouped(const float* logits, long ld, int n_toke
 }
 
 // --------------------------------------------------------------------------
-// group: order[0 .. n) = the pairs sorted by expert; tiles[i] = (expert, first row in order, rows), rows 0: no tile; behind
-// the max_tiles of them, how many there are
+// group: order[0 .. n) = the pairs sorted by expert; tiles[i] = (expert, first row in order, rows), rows 0: no tile.  The last
+// of the max_tiles places never holds one (fmsamd_moe_max_tiles asks for more than there can be): its second number says
+// how many tiles there are.
 // --------------------------------------------------------------------------
 // One block.  Its time is round trips: a thread asks for eight ids at a time, and the experts' places come from a scan over
 // the threads (an expert each).  8192 pairs of 32 experts: 7.6 us (12.6 with ids one by one and one thread adding up); 32 pairs:
@@ -259,8 +260,7 @@ __global__ void __launch_bounds__(GROUP_THREADS)
       tiles[3 * nt + 2] = c - r < tile_rows ? c - r : tile_rows;
     }
   }
-  if (tid == 0) tiles[3 * max_tiles] = all;
-  for (int i = 3 * all + tid; i < 3 * max_tiles; i += GROUP_THREADS) tiles[i] = 0;
+  for (int i = 3 * all + tid; i < 3 * max_tiles; i += GROUP_THREADS) tiles[i] = i == 3 * max_tiles - 2 ? all : 0;
   __syncthreads();
   for (int a0 = tid; a0 < n_pairs; a0 += AHEAD * GROUP_THREADS) {
     int e[AHEAD];
@@ -283,6 +283,7 @@ extern "C" int fmsamd_moe_tile_rows(int n_pairs, int n_experts, int wide_ok) {
   return n_pairs >= 20L * n_experts ? TILE_BIG_ROWS : TILE_SMALL_ROWS;
 }
 
+// More than there can be: an expert with c pairs has at most (c + tile_rows - 1) / tile_rows tiles, less than c / tile_rows + 1.
 extern "C" int fmsamd_moe_max_tiles(int n_pairs, int n_experts, int tile_rows) {
   if (tile_rows <= 0) return 0;
   return (n_pairs + tile_rows - 1) / tile_rows + (n_experts < n_pairs ? n_experts : n_pairs);
@@ -391,7 +392,7 @@ __global__ void __launch_bounds__(TILE_THREADS) expert_down_fma_kernel(ExpertArg
 // Also measured for 2048 tokens: 128 x 256 as waves of 64 x 64 142 + 73, 64 x 256 137 + 68 (4096: 241 + 145), 128 x 128 with two
 // blocks a compute unit 153 + 74, 128 x 512 154 + 77.
 __device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles, int col_blocks, int& tile, int& col) {
-  const int total = a.tiles[3 * max_tiles] * col_blocks;  // the tiles there are
+  const int total = a.tiles[3 * max_tiles - 2] * col_blocks;  // the tiles there are (group_kernel)
   const int per_die = (total + 7) / 8;
   const int at = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
   tile = at / col_blocks, col = at % col_blocks;

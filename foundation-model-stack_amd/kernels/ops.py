@@ -1221,7 +1221,7 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, gate_w: Optional[torch.Tenso
     tile_rows = lib.fmsamd_moe_tile_rows(n_pairs, E, int(wide_ok))
     max_tiles = lib.fmsamd_moe_max_tiles(n_pairs, E, tile_rows)
     order = torch.empty(n_pairs, dtype=torch.int32, device=x.device)
-    tiles = torch.empty(3 * max_tiles + 1, dtype=torch.int32, device=x.device)  # the tiles, and how many there are
+    tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=x.device)
     check(lib.fmsamd_moe_group(ids.data_ptr(), n_pairs, E, order.data_ptr(), tiles.data_ptr(), max_tiles, tile_rows, _stream()))
     hidden = torch.empty(n_pairs, ff, dtype=x.dtype, device=x.device)
     y = torch.empty(n_pairs, width, dtype=torch.float32, device=x.device)

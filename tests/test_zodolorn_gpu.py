@@ -433,6 +433,29 @@ def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
         assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
 
 
+# the C interface with buffers of the sizes that its header states, between numbers that nobody may touch: few pairs an expert
+# (tiles of 32 rows), many (128), rows that are not aligned (16), and as many tiles as pairs
+@pytest.mark.parametrize("T,E,wide_ok", [(40, 5, 1), (300, 3, 1), (40, 5, 0), (7, 7, 1), (1, 1, 1)])
+def test_group_writes_its_tiles_and_nothing_else(lib, T, E, wide_ok):
+    from fms_amd.kernels import load
+    from fms_amd.kernels.library import check
+
+    native = load()
+    ids = (torch.arange(T) * 5 % E).to(torch.int32).to(DEV)
+    rows = native.fmsamd_moe_tile_rows(T, E, wide_ok)
+    room = native.fmsamd_moe_max_tiles(T, E, rows)
+    order, tiles = torch.full((T + 16,), -7, dtype=torch.int32, device=DEV), torch.full((3 * room + 16,), -7, dtype=torch.int32, device=DEV)
+    check(native.fmsamd_moe_group(ids.data_ptr(), T, E, order[8:].data_ptr(), tiles[8:].data_ptr(), room, rows, torch.cuda.current_stream().cuda_stream))
+    assert bool((order[:8] == -7).all()) and bool((order[8 + T :] == -7).all())
+    assert bool((tiles[:8] == -7).all()) and bool((tiles[8 + 3 * room :] == -7).all())
+    want = [(e, r) for e in range(E) for c in [int((ids == e).sum())] for r in [min(rows, c - at) for at in range(0, c, rows)]]
+    got = tiles[8 : 8 + 3 * room].view(room, 3).tolist()
+    assert [(e, r) for e, _, r in got if r] == want and len(want) < room and got[-1] == [0, len(want), 0]
+    for e, first, r in got[: len(want)]:
+        assert all(int(ids[p]) == e for p in order[8 + first : 8 + first + r].tolist())
+    assert sorted(order[8 : 8 + T].tolist()) == list(range(T))
+
+
 # ---- the engine ------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("name", sorted(CONFIGS))
 @pytest.mark.parametrize("dtype", DTYPES)
