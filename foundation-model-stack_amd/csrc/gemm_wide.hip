@@ -53,8 +53,9 @@ __device__ __forceinline__ void store4(bf16* p, f32x4 v) {
 }
 
 // MT: tiles of 32 rows of x.  The waves form four rows of two: a pair shares 32 weight rows and deals the tiles of x between
-// its two waves.  STAGES steps of rows in LDS, as many as fit.
-template <int MT, int MODE, typename OutT>
+// its two waves.  STAGES steps of rows in LDS, as many as fit.  FOLD: every group of WD_GROUP k-values is a sum of its own, and
+// the groups are added up in their order (wide_plan says when).
+template <int MT, int MODE, typename OutT, bool FOLD>
 __global__ void __launch_bounds__(512)
     wide_kernel(const bf16* __restrict__ x, long ldx, const bf16* __restrict__ w, float* __restrict__ part, int M,
                 int rows, int K, int groups_per_slice, WideOut o) {
@@ -107,7 +108,8 @@ __global__ void __launch_bounds__(512)
   // bytes of their rows at the same time (rows lie a multiple of kilobytes apart) crowd into few memory
   // channels.  The start depends on the block's place only, so the order of the sum does too.
   const int n_steps = g_end - g_begin;
-  const int rot = WD_GROUP / BK * ((blockIdx.x * 5) % ((n_steps + WD_GROUP / BK - 1) / (WD_GROUP / BK)));  // (whole groups)
+  // (by whole groups; the groups that are folded keep their order)
+  const int rot = FOLD ? 0 : WD_GROUP / BK * ((blockIdx.x * 5) % ((n_steps + WD_GROUP / BK - 1) / (WD_GROUP / BK)));
   auto fetch = [&](int t, int stage) {  // past the end: zeros, so that every step has the same number of loads under way
     const int u = t + rot;
     const int k0 = (g_begin + (u >= n_steps ? u - n_steps : u)) * BK;
@@ -137,6 +139,9 @@ __global__ void __launch_bounds__(512)
   for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[j][v] = 0.f;
+  f32x16 folded[FOLD ? NT : 1];  // the groups before this one
+#pragma unroll
+  for (int j = 0; j < (FOLD ? NT : 1); ++j) folded[j] = acc[0];
 
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
@@ -189,6 +194,16 @@ __global__ void __launch_bounds__(512)
       }
     }
     stage = stage == STAGES - 1 ? 0 : stage + 1;
+    if (FOLD && ((t + 1) % (WD_GROUP / BK) == 0 || t + 1 == n_steps)) {  // uniform
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) folded[j][v] += acc[j][v], acc[j][v] = 0.f;
+    }
+  }
+  if (FOLD) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = folded[j];
   }
   tile_wait<0>();  // nothing is on its way to LDS any more, and everybody has read the last step
 
@@ -409,6 +424,16 @@ struct WidePlan {
 
 static bool wide_finishes_itself(int epi) { return epi == EPI_PLAIN || epi == EPI_GATED; }
 
+// A K of up to four groups of WD_GROUP is summed as the kernel for 17 to 32 rows sums it (gemm.hip, a group to each of its
+// waves): every group by itself, then the groups in their order.  One slice does that in registers (FOLD), one slice a group
+// leaves it to the second kernel, and no other cut is taken.  So the products' sums are the same bits for any 17 to 192 rows, and a
+// batch that shrinks below 33 rows goes on with them.  (From WD_MANY weight rows on that kernel takes no product of 17 rows or more,
+// and one cut for any number of rows does it.)  With a longer K the cut, and with it the order, goes with the number of rows.
+// Four groups: up to there one of those two cuts is the fastest or within a tenth of it; from six on those in between are a
+// fifth faster.
+#define WD_MANY 16384
+static bool wide_keeps_groups(int K) { return ceil_div(K, WD_GROUP) <= 4; }
+
 // The cut with the least estimated time.  The blocks run in rounds over the compute units; a round's time is its steps and a
 // start; the partial sums of slices are written and read once, by a kernel of its own unless the product kernel finishes its
 // one slice itself.  A step takes what its rows take to arrive (measured with all units at work: 28 bytes a nanosecond of
@@ -417,9 +442,19 @@ static bool wide_finishes_itself(int epi) { return epi == EPI_PLAIN || epi == EP
 static WidePlan wide_plan(int epi, int M, int rows, int K) {
   const int ngroups = ceil_div(K, WD_GROUP), mt = ceil_div(M, 32);
   const double busy = 0.1 + 0.3 * ((mt + 1) / 2);
-  // A short K: a slice a group, as the waves of the kernel for fewer rows (gemm.hip) take it, so that a batch that shrinks below
-  // 33 rows, or is one of fewer rows for some steps, goes on with the same bits.
-  if (ngroups <= 8 && ceil_div(rows, WD_ROWS) * ngroups <= WD_COMPUTE_UNITS) return {WD_ROWS, ngroups};
+  // A short K and blocks of 64 weight rows that make one round: as many slices as the round holds.  Measured at 33, 64, 128 and
+  // 192 rows, in microseconds (blocks of 128 rows and a slice a group in brackets): 2048 weight rows of K = 512 6.2, 6.5, 8.1, 9.8
+  // (6.7, 7.5, 9.8, 12.2), 3072 of 768 7.2, 7.7, 9.8, 12.2 (7.6, 9.3, 13.1, 17.1), 2048 of 1024 6.5, 6.9, 8.8, 11.0 (7.4, 9.0, 12.3,
+  // 15.9), 16384 of 256 6.2, 6.7, 8.8, 10.9 (10.1, 13.5, 20.7, 25.9).  Blocks of 32 rows take up to a tenth longer.
+  static_assert(WD_MANY <= WD_COMPUTE_UNITS * WD_ROWS / 2, "blocks of 64 rows make one round");
+  const int most = WD_COMPUTE_UNITS / ceil_div(rows, WD_ROWS / 2);
+  if (ngroups <= 8 && rows <= WD_MANY && (most > 1 || wide_keeps_groups(K))) {
+    return {WD_ROWS / 2, most >= ngroups ? ngroups : wide_keeps_groups(K) ? 1 : most};
+  }
+  if (wide_keeps_groups(K)) {  // one slice, and the fewest rows a block that do not add a round
+    const int rounds = ceil_div(ceil_div(rows, WD_ROWS), WD_COMPUTE_UNITS);
+    return {ceil_div(ceil_div(rows, WD_COMPUTE_UNITS * rounds), 4) * 4, 1};
+  }
   WidePlan best{WD_ROWS, 1};
   double best_cost = -1;
   for (int slices = 1; slices <= ngroups && slices <= 64; ++slices) {
@@ -471,8 +506,12 @@ static void launch_finish(const float* part, int slices, int rows, const void* b
 template <int MODE, typename OutT>
 static void launch_wide(dim3 grid, const void* x, long ldx, const void* w, float* part, int M, int rows, int K,
                         int per_slice, const WideOut& o, hipStream_t stream) {
-#define FMS_WK(MT) \
-  wide_kernel<MT, MODE, OutT><<<grid, 512, 0, stream>>>((const bf16*)x, ldx, (const bf16*)w, part, M, rows, K, per_slice, o)
+  const bool fold = per_slice > 1 && rows <= WD_MANY && wide_keeps_groups(K);
+#define FMS_WK(MT)                                                                                                          \
+  if (fold)                                                                                                                 \
+    wide_kernel<MT, MODE, OutT, true><<<grid, 512, 0, stream>>>((const bf16*)x, ldx, (const bf16*)w, part, M, rows, K, per_slice, o); \
+  else                                                                                                                      \
+    wide_kernel<MT, MODE, OutT, false><<<grid, 512, 0, stream>>>((const bf16*)x, ldx, (const bf16*)w, part, M, rows, K, per_slice, o)
   switch (ceil_div(M, 32)) {
     case 1: FMS_WK(1); break;
     case 2: FMS_WK(2); break;

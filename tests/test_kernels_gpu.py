@@ -498,7 +498,7 @@ def test_gemm_bf16(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 97, 129, 161, 192])
-@pytest.mark.parametrize("N,K,skip", [(33004, 72, 0), (512, 4104, 0), (16384, 520, 0), (20, 8200, 0), (300, 1032, 3)])
+@pytest.mark.parametrize("N,K,skip", [(33004, 72, 0), (512, 4104, 0), (16384, 520, 0), (3080, 776, 0), (20, 8200, 0), (300, 1032, 3)])
 def test_gemm_bf16_cuts_of_the_wide_product(ops, M, N, K, skip):
     """Two rounds of blocks, slices of K with a short last step, blocks that own fewer rows than they have places for, rows
     that start at no 16-byte address.
@@ -512,6 +512,25 @@ def test_gemm_bf16_cuts_of_the_wide_product(ops, M, N, K, skip):
     want = (x.float() @ w.float().t()).double() if N * K > 4e6 else x.double() @ w.double().t()
     bound = 2 * K * 2.0**-24 * (x.float().abs() @ w.float().abs().t()).double()  # (twice: the reference may be float32 too)
     assert bool(((out - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("N,K", [(40, 24), (304, 136), (768, 512), (8200, 512), (16384, 256), (16400, 504), (33000, 264)])
+def test_short_products_keep_their_bits(ops, N, K):
+    """17 to 192 rows and a K of up to 512: a row has the same bits in every product, whatever the number of rows, the
+    kernel that takes them (gemm.hip up to 32 rows and below 16384 weight rows, else gemm_wide.hip) and its cut.  (Not so the
+    scale of a norm that was left to the product: the partial sums it comes from are of runs of other lengths.)"""
+    torch.manual_seed(10)
+    x, w, b = dev(torch.randn(192, K).to(torch.bfloat16)), dev((torch.randn(N, K) * 0.1).to(torch.bfloat16)), dev(torch.randn(N).to(torch.bfloat16))
+    stream, nw = dev(torch.randn(192, N)), dev(torch.randn(N))
+
+    def products(M):
+        resid = stream[:M].clone()
+        scaled, _ = ops.linear_into_stream(x[:M], w, b, resid, nw, 1e-5)
+        return [ops.linear(x[:M], w, None), ops.linear(x[:M], w, b, out_dtype=torch.float32), resid, scaled, ops.gated_linear(x[:M], w, b, "swish")]
+
+    whole = products(192)
+    for M in (17, 31, 32, 33, 64, 65, 100, 130, 160, 191):
+        assert all(torch.equal(got, want[:M]) for got, want in zip(products(M), whole))
 
 
 @pytest.mark.parametrize("M", [1, 5, 17, 64, 70, 200])
