@@ -459,9 +459,10 @@ def test_gemm_f32(ops, M, N, K):
     torch.testing.assert_close(out, (x.double() @ w.double().t() + b.double()).float(), atol=1e-4, rtol=1e-5)
 
 
-# every tile shape (16x16, 32x32, 32x64, 64x64), with rows, columns and K past its last whole tile, and rows that are not
-# 16-byte aligned (odd K, odd stride)
-@pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (130, 4100, 65), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7)])
+# every tile shape with rows, columns and K past its last whole tile.  Aligned: 16x16 (17 by 300, 48 by 4100), 32x32 (130 by 4100,
+# 64 by 8190, 301 by 8200), 32x64 (513 by 16390).  Rows that are not 16-byte aligned (odd K, odd stride): 16x16, 32x32 in long
+# steps (130 by 3000: two rounds of blocks) and in short ones (301 by 8200)
+@pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     torch.manual_seed(61)
@@ -472,6 +473,23 @@ def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     # a float32 sum of 16 products is off by at most 16 roundings of the sum of their sizes; the float64 sum's one rounding at the end
     bound = 2.0 ** -24 * (16.5 * (x.abs().double() @ w.abs().double().t()) + want.abs()) + 1e-30
     assert float(((out - want).abs() / bound).max()) <= 1.0
+
+
+@pytest.mark.parametrize("K", [7, 36, 1000, 1028])
+def test_gemm_f32_rows_keep_their_bits(ops, K):
+    """A row has the same bits whatever else is in the product: tiles of 16x16 (1, 8 and 33 rows, and 301 by 100), 32x32 (17) and
+    32x64 (61, 130 and 301), rows that are not 16-byte aligned (an odd stride, an odd K) in tiles of 16x16 (1 and 8), 32x32 in
+    long steps (17) and in short ones (from 33 on)."""
+    torch.manual_seed(62)
+    N = 12790
+    x, w, b = dev(torch.randn(301, K)), dev(torch.randn(N, K)), dev(torch.randn(N))
+    odd = torch.zeros(301, K + 1, device="cuda")[:, :K].copy_(x)
+    whole = ops.linear(x, w, b)
+    for M in (1, 8, 17, 33, 61, 130):
+        assert torch.equal(ops.linear(x[:M], w, b), whole[:M]), M
+        assert torch.equal(ops.linear(odd[:M], w, b), whole[:M]), M
+    assert torch.equal(ops.linear(odd, w, b), whole)
+    assert torch.equal(ops.linear(x, w[:100], b[:100]), whole[:, :100])
 
 
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 48, 64, 65, 96, 100, 128, 129, 144, 160, 170, 192, 193, 300])
