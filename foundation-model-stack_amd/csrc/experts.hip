@@ -21,6 +21,7 @@
 // rows of the matrix-core kernels' tiles
 #define TILE_SMALL_ROWS 32
 #define TILE_BIG_ROWS 128
+#define EXPERT_COMPUTE_UNITS 256
 
 #define ROUTE_MAX_EXPERTS 1024
 #define ROUTE_MAX_TOP 64
@@ -399,6 +400,19 @@ __device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles,
   return (int)(blockIdx.x >> 3) < per_die && at < total;
 }
 
+// Are the weight rows of this tile loaded as bytes that are not read again?  Where a tile of 32 rows is the only one of its expert,
+// nobody else reads them; the other tiles of a popular expert do.  And with fewer blocks than compute units such loads take
+// longer.  Gate, up and down of 32 experts, 4 a token, width 2048, hidden 1024: 32 tokens 80 us (88 without the mark), one token 28
+// (33 with it), 128 tokens of which most go to a few experts 104 (118 with every load marked, 113 with none); 64 experts, 8 a token,
+// hidden 768, 128 such tokens 134 (163, 157).
+template <int BM>
+__device__ __forceinline__ bool expert_reads_once(const ExpertArgs& a, int max_tiles, int col_blocks, int tile, int e) {
+  if (BM != TILE_SMALL_ROWS) return false;
+  const int* const t = a.tiles + 3 * tile;  // (the place behind the last tile is there: fmsamd_moe_max_tiles)
+  const bool alone = !(tile > 0 && t[-3] == e) && !(t[3] == e && t[5] > 0);
+  return alone && a.tiles[3 * max_tiles - 2] * col_blocks >= EXPERT_COMPUTE_UNITS;
+}
+
 template <int WM, int WN, int TM, int TN, int ST, bool GATED>
 __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_gate_up_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
   typedef TileLds<WM, WN, TM, TN, ST> S;
@@ -412,14 +426,17 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
   // gated: a wave's first TN / 2 tiles are gate columns, the others the up columns of the same elements
   const int n0 = col * (GATED ? S::BN / 2 : S::BN);
   f32x16 acc[TM][TN];
-  tile_product_lds<WM, WN, TM, TN, ST, S::BM == TILE_SMALL_ROWS>([&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; },
-                                   [&](int n) {
-                                     const int t = n / 32;
-                                     const bool up = GATED && t % TN >= TN / 2;
-                                     const int c = n0 + (GATED ? ((t / TN) * (TN / 2) + t % (TN / 2)) * 32 + n % 32 : n);
-                                     return (up ? wu : wg) + (size_t)(c < a.N ? c : 0) * a.K;
-                                   },
-                                   a.K, lds, acc);
+  auto a_row = [&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; };
+  auto w_row = [&](int n) {
+    const int t = n / 32;
+    const bool up = GATED && t % TN >= TN / 2;
+    const int c = n0 + (GATED ? ((t / TN) * (TN / 2) + t % (TN / 2)) * 32 + n % 32 : n);
+    return (up ? wu : wg) + (size_t)(c < a.N ? c : 0) * a.K;
+  };
+  if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
+    tile_product_lds<WM, WN, TM, TN, ST, true>(a_row, w_row, a.K, lds, acc);
+  else
+    tile_product_lds<WM, WN, TM, TN, ST>(a_row, w_row, a.K, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -457,8 +474,12 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
   const bf16* x = (const bf16*)a.x;
   const bf16* w = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
   f32x16 acc[TM][TN];
-  tile_product_lds<WM, WN, TM, TN, ST, S::BM == TILE_SMALL_ROWS>([&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; },
-                                   [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; }, a.K, lds, acc);
+  auto a_row = [&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; };
+  auto w_row = [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; };
+  if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
+    tile_product_lds<WM, WN, TM, TN, ST, true>(a_row, w_row, a.K, lds, acc);
+  else
+    tile_product_lds<WM, WN, TM, TN, ST>(a_row, w_row, a.K, lds, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {

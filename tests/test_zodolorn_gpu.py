@@ -433,6 +433,28 @@ def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
         assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
 
 
+# tiles of 32 rows in more blocks than there are compute units, where an expert's only tile loads its weights with a mark and the tiles of
+# a popular expert (experts 0 and 5 here, the last one in the second case) without
+@pytest.mark.parametrize("counts", [(33, 1, 2, 0, 7, 65, 1, 4, 1, 1, 2, 1, 3, 1, 1, 5, 1, 1), (1,) * 17 + (40,)])
+def test_experts_whose_weights_are_read_once_and_more_than_once(lib, counts):
+    from fms_amd.kernels import ops
+
+    E, T, ff, width = len(counts), sum(counts), 1032, 2056
+    gen = torch.Generator(device=DEV).manual_seed(E + T)
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(T)].to(torch.int32)[:, None].contiguous().to(DEV)
+    x = torch.randn(T, width, generator=gen, device=DEV).to(torch.bfloat16)
+    wg, wu = [(torch.randn(E, ff, width, generator=gen, device=DEV) * 2 / math.sqrt(width)).to(torch.bfloat16) for _ in range(2)]
+    wd = (torch.randn(E, width, ff, generator=gen, device=DEV) / math.sqrt(ff)).to(torch.bfloat16)
+    y = ops.moe_experts(x, ids, wg, wu, wd, 1.25, 1.702, 1.0).double()
+    for e in range(E):
+        at = torch.where(ids[:, 0] == e)[0]
+        g, u = [x[at].double() @ w[e].double().T for w in (wg, wu)]
+        g = g.clamp(max=1.25)
+        h = g * torch.sigmoid(1.702 * g) * (u.clamp(-1.25, 1.25) + 1)
+        # hidden is kept in bfloat16: rounded by at most 2^-8 of itself
+        assert bool(((y[at] - h @ wd[e].double().T).abs() <= 2.0 ** -8 * (h.abs() @ wd[e].double().abs().T) + 1e-4).all())
+
+
 # the C interface with buffers of the sizes that its header states, between numbers that nobody may touch: few pairs an expert
 # (tiles of 32 rows), many (128), rows that are not aligned (16), and as many tiles as pairs
 @pytest.mark.parametrize("T,E,wide_ok", [(40, 5, 1), (300, 3, 1), (40, 5, 0), (7, 7, 1), (1, 1, 1)])
