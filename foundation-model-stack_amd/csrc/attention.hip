@@ -1598,10 +1598,15 @@ extern "C" int fmsamd_attn_decode_bf16(const void* q, long q_stride, void* out, 
   FMS_REQUIRE(staged == 0 || (keep_first == 0 && dist_bias == nullptr), "attn_decode_bf16: kept first keys and a distance table go with pages loaded straight into registers (staged = 0)");
   if (staged != 0) {
     // the waves' results meet in the page buffers: 16 KB a wave hold 16 columns of 130 floats
-    // More pages than the chip's L2 caches hold (32 MB) pass them by: 64 sequences of 128 to 2048 tokens (8 kv heads) take 52.2 us
-    // instead of 58.3, 8 of 6950 tokens 38.8 instead of 44; one sequence of 2048 tokens, whose pages the caches still hold, takes
-    // half a microsecond longer that way.
-    const bool once = (double)n_tokens * (window > 0 && window < max_context ? window : max_context) * kvheads * 128 * 4 > 32e6;
+    // The pages are marked as bytes that are not read again (they pass the caches by) where a step may read more of them than the
+    // chip's L2 caches hold (32 MB: what the contexts' bound allows; the contexts themselves are known on the device only) and one
+    // block reads a page: with more query heads a kv head than a tile holds, several do.  Measured with the weights of a layer
+    // read in between, microseconds without and with the mark, 8 kv heads of 4 query heads: 8 sequences of 2000 tokens 17.7, 15.6,
+    // of 7000 46.5, 41.1, 64 of 2000 97, 86; short contexts under the same bound lose nothing (8 of 100 tokens 8.1, 8.1, of 500 9.4,
+    // 9.4; 32 of 100 6.9, 6.8).  Below the line a context near its bound is slower with it: one sequence of 2000 tokens 9.7,
+    // 10.7, two 10.2, 11.4.  32 query heads a kv head (two tiles): 8 sequences of 7000 tokens 87, 115.
+    const double pages = (double)n_tokens * (window > 0 && window < max_context ? window : max_context) * kvheads * 128 * 4;
+    const bool once = tiles_per_kv == 1 && pages > 32e6;
     if (waves <= 4 && once)
       FMS_DC(8, 4, true, 0, true);
     else if (waves <= 4)

@@ -356,6 +356,12 @@ def test_attention_decode_on_both_sides_of_what_the_caches_hold(ops, waves, long
     attention_case(ops, torch.bfloat16, 16, 8, 128, starts=[longest, 2, 600, 63, 64, 190], lens=[1] * 6, decode=True, pages_per_block=8, waves=waves)
 
 
+@pytest.mark.parametrize("waves", [3, 8])
+def test_attention_decode_of_pages_that_several_blocks_read(ops, waves):
+    """More query heads a kv head than a tile holds, and more pages than the caches: every page is read by two blocks or three."""
+    attention_case(ops, torch.bfloat16, 160, 8, 128, starts=[1500, 2, 600, 63, 64, 190], lens=[1] * 6, decode=True, pages_per_block=8, waves=waves)
+
+
 @pytest.mark.parametrize("dtype,decode", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_attention_far_key_and_window(ops, dtype, decode):
     lens = [1, 1] if decode else [40, 3]
