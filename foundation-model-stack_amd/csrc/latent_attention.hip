@@ -225,11 +225,9 @@ extern "C" int fmsamd_headwise_linear(const void* x, long ldx, long x_head_strid
     headwise_fma_kernel<float><<<dim3(row_tiles, nheads, ceil_div(N, TILE_FMA_COLS)), TILE_THREADS, 0, stream>>>(a);
   } else if (dtype == FMS_BF16) {
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && x_head_stride % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
-    if (aligned && n_tokens >= 128) {  // a tile of tokens that is full
-      const dim3 grid(ceil_div(N, 128), nheads, ceil_div(n_tokens, 128));
-      FMS_REQUIRE(grid.z <= 65535, "headwise_linear: %d tokens are too many for one launch", n_tokens);
+    const dim3 grid(ceil_div(N, 128), nheads, ceil_div(n_tokens, 128));
+    if (aligned && n_tokens >= 128 && grid.z <= 65535)  // a tile of tokens that is full, and tiles that fit a launch
       headwise_lds_kernel<<<grid, 256, 0, stream>>>(a);
-    }
     else if (aligned)
       headwise_mfma_kernel<<<dim3(row_tiles, nheads, ceil_div(N, TILE_MFMA_COLS)), TILE_THREADS, 0, stream>>>(a);
     else

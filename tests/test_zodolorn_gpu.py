@@ -433,6 +433,21 @@ def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
         assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
 
 
+def test_headwise_linear_of_more_tokens_than_a_launch_has_tiles(lib):
+    """The C interface takes any number of tokens; the kernel with tiles of 128 has room for 65535 of them in a launch."""
+    from fms_amd.kernels import load
+    from fms_amd.kernels.library import check
+
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    T, N, K = 65535 * 128 + 1, 8, 8
+    x, w = torch.randn(T, K, generator=gen, device=DEV).to(torch.bfloat16), torch.randn(1, N, K, generator=gen, device=DEV).to(torch.bfloat16)
+    y = torch.empty(T, N, dtype=torch.bfloat16, device=DEV)
+    check(load().fmsamd_headwise_linear(x.data_ptr(), K, K, w.data_ptr(), y.data_ptr(), N, N, None, 0, 1, T, 1, N, K, torch.cuda.current_stream().cuda_stream))
+    want = x.float() @ w[0].float().T
+    # eight exact products, a float32 sum, one rounding to bfloat16 (by at most 2^-8 of the value)
+    assert bool(((y.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
+
+
 # tiles of 32 rows in more blocks than there are compute units, where an expert's only tile loads its weights with a mark and the tiles of
 # a popular expert (experts 0 and 5 here, the last one in the second case) without
 @pytest.mark.parametrize("counts", [(33, 1, 2, 0, 7, 65, 1, 4, 1, 1, 2, 1, 3, 1, 1, 5, 1, 1), (1,) * 17 + (40,)])
