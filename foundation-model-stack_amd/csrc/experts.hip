@@ -501,7 +501,8 @@ template <int WM, int WN, int TM, int TN, int ST>
 static int launch_lds(int stage, const ExpertArgs& a, int max_tiles, hipStream_t stream) {
   typedef TileLds<WM, WN, TM, TN, ST> S;
   const int col_blocks = ceil_div(a.N, stage == 0 && a.w2 != nullptr ? S::BN / 2 : S::BN);
-  FMS_REQUIRE((long)max_tiles * col_blocks <= 0x7ffffff0L, "moe_experts: %d tiles of %d columns are too many for one launch", max_tiles, a.N);
+  // (a launch's threads are counted in 32 bits)
+  FMS_REQUIRE((long)max_tiles * col_blocks <= 0xffffffffL / S::THREADS - 8, "moe_experts: %d tiles of %d columns are too many for one launch", max_tiles, a.N);
   const int blocks = 8 * ceil_div((long)max_tiles * col_blocks, 8);
   if (stage == 1)
     expert_down_lds_kernel<WM, WN, TM, TN, ST><<<blocks, S::THREADS, 0, stream>>>(a, max_tiles, col_blocks);

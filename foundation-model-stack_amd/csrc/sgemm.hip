@@ -301,17 +301,9 @@ static int sgemm_shape(const SgemmShape (&shapes)[SHAPES], int M, int N) {
   return best;
 }
 
-// Bound by the matrix unit's float32 rate (154 TFLOP/s for the vendor's product of 8192^3, 100 here; without the conversions and
-// additions in float64 the same); with few rows by the weights' bytes.  301 rows, K 4096: 610 us for 22016 rows of W (89
-// TFLOP/s; 2450 with one float32 product a thread and instruction), 126 for 4096 (140 in blocks of 32 x 64); 160 rows: 315 for
-// 22016, 81 for 4096 (92 in tiles of 16 x 16); 8 rows: 40 us for 12288 rows of W (5.0 TB/s), 27 for 4096.
-extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
-                               int N, int K, hipStream_t stream) {
-  if (M == 0 || N == 0) return 0;
-  FMS_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
-  FMS_REQUIRE(lda >= K && ldc >= N, "gemm_f32: leading dimensions too small");
-  FMS_REQUIRE((long)ceil_div(M, 16) * ceil_div(N, 16) <= 0x7ffffff0L, "gemm_f32: M=%d N=%d exceed one launch", M, N);
-  if (K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0) {
+static void sgemm(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K, bool aligned,
+                  hipStream_t stream) {
+  if (aligned) {
     switch (sgemm_shape(SGEMM_SHAPES, M, N)) {
       case 0: sgemm_launch<16, 8, 1, true>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
       case 1: sgemm_lds_launch<16, 2, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
@@ -326,6 +318,27 @@ extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const f
   } else {
     sgemm_launch<32, 2, 1, false>(a, lda, w, bias, c, ldc, M, N, K, stream);
   }
+}
+
+// What one launch takes: its threads are counted in 32 bits (and wrap round silently), at most two for a result.
+#define SGEMM_LAUNCH_TILES (1 << 22)  // of 16 x 16 results
+
+// Bound by the matrix unit's float32 rate (154 TFLOP/s for the vendor's product of 8192^3, 100 here; without the conversions and
+// additions in float64 the same); with few rows by the weights' bytes.  301 rows, K 4096: 610 us for 22016 rows of W (89
+// TFLOP/s; 2450 with one float32 product a thread and instruction), 126 for 4096 (140 in blocks of 32 x 64); 160 rows: 315 for
+// 22016, 81 for 4096 (92 in tiles of 16 x 16); 8 rows: 40 us for 12288 rows of W (5.0 TB/s), 27 for 4096.
+extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
+                               int N, int K, hipStream_t stream) {
+  if (M == 0 || N == 0) return 0;
+  FMS_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
+  FMS_REQUIRE(lda >= K && ldc >= N, "gemm_f32: leading dimensions too small");
+  const bool aligned = K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0;
+  const long cols = N < 16L * SGEMM_LAUNCH_TILES ? N : 16L * SGEMM_LAUNCH_TILES;
+  const long rows = SGEMM_LAUNCH_TILES / ceil_div(cols, 16) * 16;
+  for (long n = 0; n < N; n += cols)
+    for (long m = 0; m < M; m += rows)
+      sgemm(a + m * lda, lda, w + n * K, bias ? bias + n : nullptr, c + m * ldc + n, ldc, (int)(M - m < rows ? M - m : rows),
+            (int)(N - n < cols ? N - n : cols), K, aligned, stream);
   FMS_LAUNCH_CHECK("gemm_f32");
   return 0;
 }

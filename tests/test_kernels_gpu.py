@@ -498,6 +498,20 @@ def test_gemm_f32_rows_keep_their_bits(ops, K):
     assert torch.equal(ops.linear(x, w[:100], b[:100]), whole[:, :100])
 
 
+def test_gemm_f32_of_more_results_than_a_launch_has_threads(ops):
+    """1.7e10 results (69 GB): the threads of one launch are counted in 32 bits."""
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 80e9:
+        pytest.skip("needs 80 GB of memory")
+    torch.manual_seed(63)
+    x, w = torch.randn(131072, 1, device="cuda"), torch.randn(131136, 1, device="cuda")
+    out = ops.linear(x, w, None)
+    for at in list(range(0, 131072, 8192)) + [131071]:
+        assert torch.equal(out[at : at + 40], x[at : at + 40] * w.t())
+    del out
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 48, 64, 65, 96, 100, 128, 129, 144, 160, 170, 192, 193, 300])
 @pytest.mark.parametrize("N,K", [(40, 24), (100, 176), (257, 96), (384, 96), (4096 + 16, 512), (20000, 64)])
 def test_gemm_bf16(ops, M, N, K):
