@@ -832,7 +832,7 @@ __global__ void __launch_bounds__(256, 1)
   // unit's registers and have to be moved out and back to be scaled: that stands outside the loop over the keys, or the
   // compiler moves them for every tile (the waves of a block meet at the same barriers wherever they stand in the code).
   const int first_base = first_lo / 32 * 32;
-  fetch(first_base, 0);
+  if (first_base <= last_pos) fetch(first_base, 0);  // (no load may be on its way to LDS when the block ends)
   int base = first_base, buffer = 0;
   float top = LAT_EMPTY;
   for (;;) {

@@ -433,6 +433,21 @@ def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
         assert bool(((y[at] - h @ wd[e].double().T).abs() <= bound).all())
 
 
+def test_latent_attention_of_tokens_that_see_no_key(lib):
+    """Positions before the sequence's start: nothing is read, and the sink alone leaves zeros."""
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(3)
+    cache = torch.randn(1, 1, 64, 576, generator=gen).to(torch.bfloat16).to(DEV)
+    T, heads = 9, 16
+    qa = torch.randn(T, heads * 576, generator=gen).to(torch.bfloat16).to(DEV)
+    pos = torch.full((T,), -1, dtype=torch.int32, device=DEV)
+    pos[8] = 3  # a block of its own
+    out = ops.latent_attention(qa, pos, torch.zeros(T, dtype=torch.int32, device=DEV), torch.zeros(1, 1, dtype=torch.int32, device=DEV), cache,
+                               torch.zeros(heads, device=DEV), heads, 512, 64, 0.05, vt_cache=cache[..., :512].transpose(2, 3).contiguous())
+    assert float(out[:8].float().abs().max()) == 0.0 and bool((out[8].float() != 0).any())
+
+
 def test_headwise_linear_of_more_tokens_than_a_launch_has_tiles(lib):
     """The C interface takes any number of tokens; the kernel with tiles of 128 has room for 65535 of them in a launch."""
     from fms_amd.kernels import load
