@@ -258,9 +258,10 @@ int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long ldo, void*
 #define FMS_ROUTE_SIGMOID_NORMED 2
 int fmsamd_moe_route(const float* logits, long ld, int n_tokens, int n_experts, int top, int score, int* ids, float* weights,
                      hipStream_t stream);
-// Rows of a tile of (token, choice) pairs of one expert: 32, or 128 where experts have many rows, where the matrix-core
-// kernels can run (wide_ok: bfloat16, widths and row strides multiples of 8, x and all weights at 16-byte addresses), else
-// 16; how many tiles to make room for (more than there can be); the pairs sorted by expert and cut into tiles:
+// Rows of a tile of (token, choice) pairs of one expert: 32, or 128 where experts have many rows, for a product that the
+// matrix-core kernels can take (wide_ok: bfloat16, K and row strides multiples of 8, rows and weights at 16-byte addresses), else
+// 16 (where only one of a step's two products can, the pairs are grouped for each, and both go by the first call's order);
+// how many tiles to make room for (more than there can be); the pairs sorted by expert and cut into tiles:
 // order [n_pairs], tiles [max_tiles][3] = (expert, first row in order, rows), rows 0: no tile.  The last place is never a
 // tile, its second number is how many there are.
 int fmsamd_moe_tile_rows(int n_pairs, int n_experts, int wide_ok);

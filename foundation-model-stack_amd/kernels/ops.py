@@ -1215,20 +1215,28 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, gate_w: Optional[torch.Tenso
             raise TypeError("the experts' weights are contiguous and of the type of x")
     lib = load()
     n_pairs = T * top
-    # the matrix-core kernels load 16 bytes at a time
-    wide_ok = x.dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0 and x.stride(0) % 8 == 0 and not any(
-        t.data_ptr() % 16 for t in (x, gate_w, up_w, down_w))
-    tile_rows = lib.fmsamd_moe_tile_rows(n_pairs, E, int(wide_ok))
-    max_tiles = lib.fmsamd_moe_max_tiles(n_pairs, E, tile_rows)
+    # The matrix-core kernels load 16 bytes at a time; each of the two products takes them where its own rows allow.  (32 experts, 4 a
+    # token, width 2048, a hidden size of 1028: 512 tokens take 608 us, 1774 with neither product on them; 16 tokens 204, 739.)
+    fits = [x.dtype == torch.bfloat16 and k % 8 == 0 and stride % 8 == 0 and not any(t.data_ptr() % 16 for t in tensors)
+            for k, stride, tensors in ((width, x.stride(0), (x, gate_w, up_w)), (ff, ff, (down_w,)))]
     order = torch.empty(n_pairs, dtype=torch.int32, device=x.device)
-    tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=x.device)
-    check(lib.fmsamd_moe_group(ids.data_ptr(), n_pairs, E, order.data_ptr(), tiles.data_ptr(), max_tiles, tile_rows, _stream()))
+    groups = []  # a product's tiles, how many there is room for, and rows of a tile
+    for fit in fits if fits[0] != fits[1] else fits[:1]:
+        tile_rows = lib.fmsamd_moe_tile_rows(n_pairs, E, int(fit))
+        max_tiles = lib.fmsamd_moe_max_tiles(n_pairs, E, tile_rows)
+        tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=x.device)
+        # (the places of an expert's pairs are the same in every grouping, their order within them is the first one's)
+        check(lib.fmsamd_moe_group(ids.data_ptr(), n_pairs, E, (torch.empty_like(order) if groups else order).data_ptr(), tiles.data_ptr(), max_tiles,
+                                   tile_rows, _stream()))
+        groups.append((tiles, max_tiles, tile_rows))
     hidden = torch.empty(n_pairs, ff, dtype=x.dtype, device=x.device)
     y = torch.empty(n_pairs, width, dtype=torch.float32, device=x.device)
     code = _code(x.dtype)
+    tiles, max_tiles, tile_rows = groups[0]
     check(lib.fmsamd_moe_experts(0, x.data_ptr(), x.stride(0), gate_w.data_ptr(), up_w.data_ptr() if gated else None, hidden.data_ptr(), code,
                                  order.data_ptr(), tiles.data_ptr(), max_tiles, tile_rows, top, ff, width, float(limit), float(alpha), float(shift),
                                  _ptr(in_scale), ACTIVATIONS[activation], _stream()))
+    tiles, max_tiles, tile_rows = groups[-1]
     check(lib.fmsamd_moe_experts(1, hidden.data_ptr(), hidden.stride(0), down_w.data_ptr(), None, y.data_ptr(), code,
                                  order.data_ptr(), tiles.data_ptr(), max_tiles, tile_rows, top, width, ff, float(limit), float(alpha), float(shift),
                                  None, 0, _stream()))
