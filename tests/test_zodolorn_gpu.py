@@ -463,6 +463,39 @@ def test_headwise_linear_of_more_tokens_than_a_launch_has_tiles(lib):
     assert bool(((y.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
 
 
+# a width or a hidden size that is no multiple of 8: the rows of one product are aligned to 16 bytes, those of the other are not
+@pytest.mark.parametrize("counts", [(1, 31, 0), (17, 33, 2, 0, 1), (129, 0, 16), (700,)])
+@pytest.mark.parametrize("ff,width,aligned", [(132, 72, 0), (1, 64, 0), (136, 68, 1), (40, 9, 1)])
+def test_experts_with_one_aligned_product(lib, monkeypatch, counts, ff, width, aligned):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(ff + len(counts))
+    E, T = len(counts), sum(counts)
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(T, generator=gen)].to(torch.int32)[:, None].contiguous().to(DEV)
+    x = torch.randn(T, width, generator=gen).to(torch.bfloat16).to(DEV)
+    wg, wu = [(torch.randn(E, ff, width, generator=gen) * 2 / math.sqrt(width)).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    wd = (torch.randn(E, width, ff, generator=gen) / math.sqrt(ff)).to(torch.bfloat16).to(DEV)
+    native, rows = ops.load(), []
+
+    class Listening:
+        def __getattr__(self, name):
+            if name != "fmsamd_moe_experts":
+                return getattr(native, name)
+            return lambda stage, *args: (rows.append(args[9]), native.fmsamd_moe_experts(stage, *args))[1]
+
+    monkeypatch.setattr(ops, "load", lambda: Listening())
+    y = ops.moe_experts(x, ids, wg, wu, wd, 1.25, 1.702, 1.0).double()
+    # the matrix-core kernels' tiles for the aligned product, the other kernel's for the other one
+    assert rows[aligned] == (128 if T >= 20 * E else 32) and rows[1 - aligned] == 16
+    for e in range(E):
+        at = torch.where(ids[:, 0] == e)[0]
+        g, u = [x[at].double() @ w[e].double().T for w in (wg, wu)]
+        g = g.clamp(max=1.25)
+        h = g * torch.sigmoid(1.702 * g) * (u.clamp(-1.25, 1.25) + 1)
+        # hidden is kept in bfloat16: rounded by at most 2^-8 of itself
+        assert bool(((y[at] - h @ wd[e].double().T).abs() <= 2.0 ** -8 * (h.abs() @ wd[e].double().abs().T) + 1e-4).all())
+
+
 # tiles of 32 rows in more blocks than there are compute units, where an expert's only tile loads its weights with a mark and the tiles of
 # a popular expert (experts 0 and 5 here, the last one in the second case) without
 @pytest.mark.parametrize("counts", [(33, 1, 2, 0, 7, 65, 1, 4, 1, 1, 2, 1, 3, 1, 1, 5, 1, 1), (1,) * 17 + (40,)])
@@ -518,39 +551,6 @@ def test_whole_sequence_and_every_layer(lib, folders, name, dtype):
     model = get(lib, folders, name, dtype)
     engine = Engine(model, max_tokens=256, max_slots=2)
     slot = engine.new_sequence()
-# a width or a hidden size that is no multiple of 8: the rows of one product are aligned to 16 bytes, those of the other are not
-@pytest.mark.parametrize("counts", [(1, 31, 0), (17, 33, 2, 0, 1), (129, 0, 16), (700,)])
-@pytest.mark.parametrize("ff,width,aligned", [(132, 72, 0), (1, 64, 0), (136, 68, 1), (40, 9, 1)])
-def test_experts_with_one_aligned_product(lib, monkeypatch, counts, ff, width, aligned):
-    from fms_amd.kernels import ops
-
-    gen = torch.Generator().manual_seed(ff + len(counts))
-    E, T = len(counts), sum(counts)
-    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(T, generator=gen)].to(torch.int32)[:, None].contiguous().to(DEV)
-    x = torch.randn(T, width, generator=gen).to(torch.bfloat16).to(DEV)
-    wg, wu = [(torch.randn(E, ff, width, generator=gen) * 2 / math.sqrt(width)).to(torch.bfloat16).to(DEV) for _ in range(2)]
-    wd = (torch.randn(E, width, ff, generator=gen) / math.sqrt(ff)).to(torch.bfloat16).to(DEV)
-    native, rows = ops.load(), []
-
-    class Listening:
-        def __getattr__(self, name):
-            if name != "fmsamd_moe_experts":
-                return getattr(native, name)
-            return lambda stage, *args: (rows.append(args[9]), native.fmsamd_moe_experts(stage, *args))[1]
-
-    monkeypatch.setattr(ops, "load", lambda: Listening())
-    y = ops.moe_experts(x, ids, wg, wu, wd, 1.25, 1.702, 1.0).double()
-    # the matrix-core kernels' tiles for the aligned product, the other kernel's for the other one
-    assert rows[aligned] == (128 if T >= 20 * E else 32) and rows[1 - aligned] == 16
-    for e in range(E):
-        at = torch.where(ids[:, 0] == e)[0]
-        g, u = [x[at].double() @ w[e].double().T for w in (wg, wu)]
-        g = g.clamp(max=1.25)
-        h = g * torch.sigmoid(1.702 * g) * (u.clamp(-1.25, 1.25) + 1)
-        # hidden is kept in bfloat16: rounded by at most 2^-8 of itself
-        assert bool(((y[at] - h @ wd[e].double().T).abs() <= 2.0 ** -8 * (h.abs() @ wd[e].double().abs().T) + 1e-4).all())
-
-
     judge(engine.step([slot], [ids], "all"), want, dtype)
     engine.end_sequence(slot)
     engine.cache.check()
