@@ -466,18 +466,6 @@ __device__ __forceinline__ void latent_finish(LatentState<RT, WC>& st, bf16* __r
   }
 }
 
-#define LAT_GROUP 4  // tiles of a block of latent_attn_prompt_kernel
-
-// do the tiles of a group belong to one sequence?  (the same answer in every lane)
-__device__ __forceinline__ bool latent_group_together(int group, int n_tiles, int tiles_per_token, const int* seq_of_token) {
-  const int first = group * LAT_GROUP, last = first + LAT_GROUP < n_tiles ? first + LAT_GROUP - 1 : n_tiles - 1;
-  const int t0 = first / tiles_per_token, t1 = last / tiles_per_token;
-  const int seq = uniform_load(seq_of_token + t0);
-  bool same = seq >= 0;
-  for (int t = t0 + 1; t <= t1; ++t) same = same && uniform_load(seq_of_token + t) == seq;
-  return same;
-}
-
 // LDS: the four waves of a block (four consecutive tiles of one sequence: neighbouring tokens, or the head groups of
 // one token) share every tile of keys through LDS, so a tile comes from the caches once a block instead of once a
 // wave; a block whose tiles lie in different sequences, and every block of a decode step, loads straight from
@@ -488,13 +476,11 @@ __global__ void __launch_bounds__(256)
                             const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                             const int* __restrict__ block_table, int table_stride, const bf16* __restrict__ cache,
                             const bf16* __restrict__ vt_cache, const float* __restrict__ sink, int n_tokens, int nheads,
-                            int rank, int width, float scale, int window, int tiles_per_token, int n_parts, int mixed_groups_only) {
+                            int rank, int width, float scale, int window, int tiles_per_token, int n_parts) {
   extern __shared__ __attribute__((aligned(16))) bf16 lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int n_tiles = n_tokens * tiles_per_token;
-  // what latent_attn_prompt_kernel has left: groups of tiles of several sequences
-  if (LDS && mixed_groups_only && latent_group_together(blockIdx.x, n_tiles, tiles_per_token, seq_of_token)) return;
   int tile, part;
   if (n_parts == 1) {
     tile = blockIdx.x * 4 + wave;
@@ -675,9 +661,13 @@ __global__ void __launch_bounds__(256)
 // softmax, which a wave alone on its SIMD cannot hide.  One prompt of 2048 tokens, 16 heads, latent 512 + 64: 138 us; with the keys
 // through registers and the shortest contexts first (the kernel above) 355, with results scaled whenever a maximum moved 212,
 // with that inside the loop over the keys 182.
-// Blocks whose tiles belong to several sequences are left to latent_attn_mfma_kernel.
+// A block whose tiles belong to several sequences takes the sequences one after the other: each wave works while its own
+// tile's is there.  So a token has the same bits whatever else is in the step.  16 heads: 333, 1 and 90 tokens behind 1000 cached
+// ones 172 us, nine prompts of 17 tokens 12.3 (355 and 27 with such blocks left to a second launch, of the kernel above; that
+// kernel alone 277 and 17.2); 16 sequences of one token behind 500, four to a block, 110 (131).
 // --------------------------------------------------------------------------
 #define LAT_SLACK 8.f
+#define LAT_GROUP 4  // tiles of a block
 
 template <int RT, int WC>
 __global__ void __launch_bounds__(256, 1)
@@ -695,21 +685,22 @@ __global__ void __launch_bounds__(256, 1)
   const int col = lane & 15, grp = lane >> 4;
   const int n_tiles = n_tokens * tiles_per_token;
   const int group = gridDim.x - 1 - blockIdx.x;  // the longest contexts first
-  if (!latent_group_together(group, n_tiles, tiles_per_token, seq_of_token)) return;
   const int first_tile = group * LAT_GROUP, last_tile = first_tile + LAT_GROUP < n_tiles ? first_tile + LAT_GROUP - 1 : n_tiles - 1;
-  const int tile = first_tile + wave;
-  const bool works = tile <= last_tile;
-  const int t = (works ? tile : last_tile) / tiles_per_token, head = (tile % tiles_per_token) * 16 + col;
-  const bool valid = works && head < nheads;
-  const int seq = uniform_load(seq_of_token + t);
-  const int* bt = block_table + (size_t)seq * table_stride;
-  int first_pos = 0x7fffffff, last_pos = -1;  // of the block's tokens
-  for (int u = first_tile / tiles_per_token; u <= last_tile / tiles_per_token; ++u) {
-    const int p = uniform_load(positions + u);
-    first_pos = p < first_pos ? p : first_pos, last_pos = p > last_pos ? p : last_pos;
+  int seqs[LAT_GROUP], places[LAT_GROUP];  // of the tiles; seqs -1: a padding row, or no tile
+#pragma unroll
+  for (int i = 0; i < LAT_GROUP; ++i) {
+    const int u = (first_tile + i <= last_tile ? first_tile + i : last_tile) / tiles_per_token;
+    seqs[i] = uniform_load(seq_of_token + u), places[i] = uniform_load(positions + u);
+    if (first_tile + i > last_tile) seqs[i] = -1;
   }
-  const int pos = uniform_load(positions + t);
-  const int first_lo = window > 0 && first_pos - window + 1 > 0 ? first_pos - window + 1 : 0;
+  const int tile = first_tile + wave;
+  const bool there = tile <= last_tile;
+  const int t = (there ? tile : last_tile) / tiles_per_token, head = (tile % tiles_per_token) * 16 + col;
+  const bool valid = there && head < nheads;
+  int own_seq = -1, pos = -1;
+#pragma unroll
+  for (int i = 0; i < LAT_GROUP; ++i)
+    if (i == wave) own_seq = seqs[i], pos = places[i];
   const int lo = window > 0 && pos - window + 1 > 0 ? pos - window + 1 : 0;
 
   bf16x8 q[WC];
@@ -731,7 +722,7 @@ __global__ void __launch_bounds__(256, 1)
   const int v_row = wave * V_LOADS * 16 + (lane >> 2);
   const unsigned v_from = v_row * (PAGE_TOKENS * 2) + ((lane & 3) ^ ((lane >> 3) & 3)) * 16;  // rows 16 apart swizzle alike
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)lds;
-  auto fetch = [&](int base, int buffer) {
+  auto fetch = [&](const int* bt, int base, int buffer) {
     const size_t page = readable_page(uniform_load(bt + base / PAGE_TOKENS));
     const int in_page = base % PAGE_TOKENS;
     const char* kp = (const char*)(cache + (page * PAGE_TOKENS + in_page) * WIDTH);
@@ -831,42 +822,61 @@ __global__ void __launch_bounds__(256, 1)
   // and results are float32, and a bfloat16 probability is as exact at e^LAT_SLACK as at 1.  The results live in the matrix
   // unit's registers and have to be moved out and back to be scaled: that stands outside the loop over the keys, or the
   // compiler moves them for every tile (the waves of a block meet at the same barriers wherever they stand in the code).
-  const int first_base = first_lo / 32 * 32;
-  if (first_base <= last_pos) fetch(first_base, 0);  // (no load may be on its way to LDS when the block ends)
-  int base = first_base, buffer = 0;
   float top = LAT_EMPTY;
-  for (;;) {
-    bool behind = false;
-    for (; base <= last_pos; base += 32, buffer ^= 1) {
-      if (base + 32 <= last_pos) {
-        fetch(base + 32, buffer ^ 1);
-        tile_wait<K_LOADS + V_LOADS>();
-      } else {
-        tile_wait<0>();
+#pragma unroll 1
+  for (int turn = 0; turn < LAT_GROUP; ++turn) {
+    int seq = -1;  // of tile `turn`; its turn if no tile before it has the same
+    bool again = false;
+    int first_pos = 0x7fffffff, last_pos = -1;  // of the sequence's tokens in the block
+#pragma unroll
+    for (int i = 0; i < LAT_GROUP; ++i)
+      if (i == turn) seq = seqs[i];
+#pragma unroll
+    for (int i = 0; i < LAT_GROUP; ++i)
+      if (seqs[i] == seq) {
+        again = again || i < turn;
+        first_pos = places[i] < first_pos ? places[i] : first_pos, last_pos = places[i] > last_pos ? places[i] : last_pos;
       }
-      if (works && base <= pos) {  // the same in all lanes of the wave
-        const char* kv = (const char*)lds + buffer * STAGE;
-        top = scores(kv, base);
-        behind = __any(top > m + LAT_SLACK);
-        if (behind) break;
-        values(kv);
+    if (seq < 0 || again) continue;
+    const bool works = own_seq == seq;
+    const int* bt = block_table + (size_t)seq * table_stride;
+    const int first_lo = window > 0 && first_pos - window + 1 > 0 ? first_pos - window + 1 : 0;
+    const int first_base = first_lo / 32 * 32;
+    if (first_base <= last_pos) fetch(bt, first_base, 0);  // (no load may be on its way to LDS when the block ends)
+    int base = first_base, buffer = 0;
+    for (;;) {
+      bool behind = false;
+      for (; base <= last_pos; base += 32, buffer ^= 1) {
+        if (base + 32 <= last_pos) {
+          fetch(bt, base + 32, buffer ^ 1);
+          tile_wait<K_LOADS + V_LOADS>();
+        } else {
+          tile_wait<0>();
+        }
+        if (works && base <= pos) {  // the same in all lanes of the wave
+          const char* kv = (const char*)lds + buffer * STAGE;
+          top = scores(kv, base);
+          behind = __any(top > m + LAT_SLACK);
+          if (behind) break;
+          values(kv);
+        }
+        block_sync_lds();  // everybody has read the buffer
       }
-      block_sync_lds();  // everybody has read the buffer
+      if (!behind) break;
+      const float m_new = top > m + LAT_SLACK ? top : m;
+      const float alpha = __expf(m - m_new);
+      l *= alpha;
+      m = m_new;
+#pragma unroll
+      for (int d = 0; d < RT; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[d][i] *= alpha;
+      values((const char*)lds + buffer * STAGE);
+      block_sync_lds();
+      base += 32, buffer ^= 1;
     }
-    if (!behind) break;
-    const float m_new = top > m + LAT_SLACK ? top : m;
-    const float alpha = __expf(m - m_new);
-    l *= alpha;
-    m = m_new;
-#pragma unroll
-    for (int d = 0; d < RT; ++d)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[d][i] *= alpha;
-    values((const char*)lds + buffer * STAGE);
-    block_sync_lds();
-    base += 32, buffer ^= 1;
   }
-  if (!works) return;
+  if (!there) return;
   LatentState<RT, WC> st;
 #pragma unroll
   for (int d = 0; d < RT; ++d) st.acc[d] = acc[d];
@@ -962,15 +972,13 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
   if (n_splits == 0)                                                                                                               \
     latent_attn_mfma_kernel<RT, WC, true, EXACT><<<grid, 256, lds, stream>>>(                                                      \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
-        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts,   \
-        prompt_kernel);                                                                                                            \
+        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts);  \
   else                                                                                                                             \
     latent_attn_mfma_kernel<RT, WC, false, EXACT><<<grid, 256, q_lds, stream>>>(                                                   \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
-        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts, 0)
-  // prompts with a latent of 512: the groups of tiles that belong to one sequence first, what is left with the other kernel
-  // (its rows go straight to LDS, which wants 16-byte addresses)
-  const int prompt_kernel =
+        (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts)
+  // prompts with a latent of 512 (the rows go straight to LDS, which wants 16-byte addresses)
+  const bool prompt_kernel =
       n_splits == 0 && rank == 512 && (width == 576 || width == 512) && (uintptr_t)cache % 16 == 0 && (uintptr_t)vt_cache % 16 == 0;
   if (prompt_kernel) {
     const int groups = ceil_div(tiles, LAT_GROUP);
@@ -994,6 +1002,7 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
     }
 #undef LAUNCH_PROMPT
     FMS_LAUNCH_CHECK("latent_attn_prompt");
+    return 0;
   }
   // the sizes of the largest configuration exactly (a latent of 512 with a rotated part of 64, or with none) and the
   // smaller latents without a rotated part run without a question around any product; everything else in the smallest

@@ -364,8 +364,7 @@ def test_experts_and_their_sum(lib, dtype, sizes):
     torch.testing.assert_close(out.float().cpu(), want, **tol)
 
 
-# prompts with a latent of 512: blocks of one sequence (the kernel that shares keys through LDS), blocks that straddle two (left
-# to the other one), a last block that is not full, positions that start inside a sequence, windows, one to three tiles a token
+# prompts with a latent of 512: blocks of one sequence, blocks that straddle two or three, a last block that is not full, positions that start inside a sequence, windows, one to three tiles a token
 @pytest.mark.parametrize("heads", [5, 16, 20, 40])
 @pytest.mark.parametrize("rot", [64, 0])
 @pytest.mark.parametrize("runs,window", [([(0, 70)], 0), ([(0, 1), (0, 5), (60, 9)], 0), ([(130, 34), (0, 33)], 40), ([(31, 2), (95, 66)], 7)])
@@ -397,6 +396,40 @@ def test_latent_attention_of_prompts(lib, heads, rot, runs, window):
     moved = [torch.zeros(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t) for t in (cache, values)]
     got = ops.latent_attention(*args[:4], moved[0], *args[5:], vt_cache=moved[1]).float()
     assert float((got - want).norm() / want.norm()) < 0.01
+
+
+# blocks of one to four sequences in any order, one of them twice, with padding rows between them; windows; one tile a token to three
+@pytest.mark.parametrize("heads", [5, 16, 40])
+@pytest.mark.parametrize("rot,window", [(64, 0), (0, 0), (64, 33)])
+@pytest.mark.parametrize("sink", [True, False])
+def test_latent_attention_rows_keep_their_bits(lib, heads, rot, window, sink):
+    """A token of a prompt has the same bits whatever else is in the step."""
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(heads + rot)
+    R, W = 512, 512 + rot
+    order = [0, 1, 2, 3, 1, 1, -1, 0, 3, 3, 3, 3, 2, -1, -1, -1, -1, 2] + [1] * 37 + [0, 3]  # a token's sequence
+    at = [699, 0, 62, 190]  # where the sequences start
+    pos = []
+    for b in order:
+        pos.append(at[b] if b >= 0 else 0)
+        at = [n + (i == b) for i, n in enumerate(at)]
+    seq, pos = torch.tensor(order, dtype=torch.int32, device=DEV), torch.tensor(pos, dtype=torch.int32, device=DEV)
+    table = torch.randperm(4 * 12, generator=gen).to(torch.int32).view(4, 12).to(DEV)
+    cache = torch.randn(48, 1, 64, W, generator=gen).to(torch.bfloat16).to(DEV)
+    values = cache[..., :R].transpose(2, 3).contiguous()
+    qa = torch.randn(len(order), heads * W, generator=gen).to(torch.bfloat16).to(DEV)
+    logit = torch.randn(heads, generator=gen).to(DEV) if sink else None
+
+    def rows(which):
+        return ops.latent_attention(qa[which].contiguous(), pos[which].contiguous(), seq[which].contiguous(), table, cache, logit, heads, R, rot, 0.05, window, vt_cache=values)
+
+    whole = rows(torch.arange(len(order), device=DEV))
+    assert float(whole[seq < 0].float().abs().max()) == 0.0
+    for b in range(4):
+        which = torch.where(seq == b)[0]
+        assert torch.equal(rows(which), whole[which]), b
+        assert torch.equal(rows(which[-1:]), whole[which[-1:]]), b
 
 
 # rows an expert around the edges of a tile (32 rows up to 20 rows an expert on average, 128 above), experts without rows,
