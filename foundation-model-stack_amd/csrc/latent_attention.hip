@@ -211,6 +211,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) h
   }
 }
 
+#define HEADWISE_COMPUTE_UNITS 256
+
 extern "C" int fmsamd_headwise_linear(const void* x, long ldx, long x_head_stride, const void* w, void* y, long ldy,
                                       long y_head_stride, const float* gate, long ldg, int dtype, int n_tokens, int nheads,
                                       int N, int K, hipStream_t stream) {
@@ -226,7 +228,13 @@ extern "C" int fmsamd_headwise_linear(const void* x, long ldx, long x_head_strid
   } else if (dtype == FMS_BF16) {
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && x_head_stride % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
     const dim3 grid(ceil_div(N, 128), nheads, ceil_div(n_tokens, 128));
-    if (aligned && n_tokens >= 128 && grid.z <= 65535)  // a tile of tokens that is full, and tiles that fit a launch
+    // The kernel through LDS takes 7 to 10 us however little it has to do: it is for at least a full tile of tokens, more blocks of
+    // the other kernel than there are compute units, and enough products.  Measured for both, us (16 tokens a block first): 16 heads of
+    // 128 into 512, 128 tokens 6.4, 8.0, 200 (2.1e8 products) 9.0, 8.2; 32 of 128 into 128, 256 tokens 6.1, 7.9, 512 9.1, 8.2; 4 of 64
+    // into 2048, 256 tokens 6.6, 7.6, 384 (2.0e8) 8.7, 8.1; 16 of 512 into 128, 256 tokens (256 blocks) 8.7, 10.4, 384 13.9, 10.6.
+    const bool full = n_tokens >= 128 && (long)row_tiles * nheads * ceil_div(N, TILE_MFMA_COLS) > HEADWISE_COMPUTE_UNITS &&
+                      (double)n_tokens * nheads * N * K >= 2e8;
+    if (aligned && K >= TL_BK && full && grid.z <= 65535)  // (and tiles that fit a launch)
       headwise_lds_kernel<<<grid, 256, 0, stream>>>(a);
     else if (aligned)
       headwise_mfma_kernel<<<dim3(row_tiles, nheads, ceil_div(N, TILE_MFMA_COLS)), TILE_THREADS, 0, stream>>>(a);

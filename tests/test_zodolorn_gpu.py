@@ -250,6 +250,28 @@ def test_a_product_per_head(lib, dtype, shape):
     assert float(y[:, H * N :].float().abs().max()) == 0.0  # nothing written past the heads
 
 
+# many products (T, H, K, N): the kernel through LDS, with tokens, elements and K past its last whole tile and step
+@pytest.mark.parametrize("shape", [(300, 8, 136, 648), (129, 40, 72, 600), (128, 40, 512, 96), (1000, 3, 264, 257)])
+def test_a_product_per_head_of_many_products(lib, shape):
+    from fms_amd.kernels import ops
+
+    T, H, K, N = shape
+    assert T * H * K * N >= 2e8  # where that kernel begins
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, H * (K + 8), generator=gen, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(H, N, K, generator=gen, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    gate = torch.randn(T, H + 3, generator=gen, device=DEV)
+    y = torch.zeros(T, H * N + 16, dtype=torch.bfloat16, device=DEV)
+    ops.headwise_linear(x, K + 8, w, y, N, gate=gate[:, 2 : 2 + H])
+    factor = torch.sigmoid(gate[:, 2 : 2 + H].double())
+    for h in range(H):
+        xs = x[:, h * (K + 8) : h * (K + 8) + K].double()
+        want, size = (xs @ w[h].double().T) * factor[:, h : h + 1], (xs.abs() @ w[h].double().abs().T) * factor[:, h : h + 1]
+        # one rounding to bfloat16 (by at most 2^-8 of the value), float32 sums of K exact products, the gate in float32
+        assert bool(((y[:, h * N : (h + 1) * N].double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + 8) * 2.0 ** -23 * size).all())
+    assert float(y[:, H * N :].float().abs().max()) == 0.0  # nothing written past the heads
+
+
 def _latent_cache(lib, n_pages, width, dtype):
     return torch.zeros(n_pages, 1, 64, width, dtype=dtype, device=DEV)
 
@@ -487,13 +509,13 @@ def test_headwise_linear_of_more_tokens_than_a_launch_has_tiles(lib):
     from fms_amd.kernels.library import check
 
     gen = torch.Generator(device=DEV).manual_seed(5)
-    T, N, K = 65535 * 128 + 1, 8, 8
+    T, N, K = 65535 * 128 + 1, 8, 64
     x, w = torch.randn(T, K, generator=gen, device=DEV).to(torch.bfloat16), torch.randn(1, N, K, generator=gen, device=DEV).to(torch.bfloat16)
     y = torch.empty(T, N, dtype=torch.bfloat16, device=DEV)
     check(load().fmsamd_headwise_linear(x.data_ptr(), K, K, w.data_ptr(), y.data_ptr(), N, N, None, 0, 1, T, 1, N, K, torch.cuda.current_stream().cuda_stream))
     want = x.float() @ w[0].float().T
-    # eight exact products, a float32 sum, one rounding to bfloat16 (by at most 2^-8 of the value)
-    assert bool(((y.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
+    # float32 sums of 64 exact products of at most 30 each, on both sides, and one rounding to bfloat16 (by at most 2^-8 of the value)
+    assert bool(((y.float() - want).abs() <= 2.0 ** -8 * want.abs() + 2 * 64 * 2.0 ** -24 * 64 * 30).all())
 
 
 # a width or a hidden size that is no multiple of 8: the rows of one product are aligned to 16 bytes, those of the other are not
