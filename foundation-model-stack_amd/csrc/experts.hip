@@ -276,12 +276,16 @@ __global__ void __launch_bounds__(GROUP_THREADS)
   }
 }
 
-// Rows of a tile.  The matrix-core kernels (wide_ok: bfloat16, everything aligned to 16 bytes) take large tiles from 20 rows an
-// expert on, where most experts would need two small ones and read their weights twice (32 experts, 4 a token: 192 tokens 58 +
-// 32 us in small tiles, 50 + 28 in large ones; 128 tokens 44 + 24 against 48 + 26).
+// Rows of a tile.  The matrix-core kernels (wide_ok: bfloat16, everything aligned to 16 bytes) take large tiles where experts fill
+// more than one small one on average and read their weights twice, and there are pairs enough to give the compute units work in
+// large tiles.  Both products and the grouping, us, small tiles and large ones: 32 experts, 4 a token, width 2048, hidden 1024, 200
+// tokens (25 rows an expert) 94, 112, 300 tokens (38) 123, 112; 64 experts, 8 a token, hidden 768, 200 tokens (25) 143, 163, 300 (38)
+// 174, 170; 8 experts, 2 a token, width 768, hidden 2048, 256 tokens (512 pairs) 50, 60, 512 (1024 pairs) 63, 64; width 1024, hidden
+// 512, 512 tokens 31, 43, 1024 tokens 46, 44.
+#define TILE_BIG_PAIRS 1024
 extern "C" int fmsamd_moe_tile_rows(int n_pairs, int n_experts, int wide_ok) {
   if (!wide_ok) return TILE_ROWS;
-  return n_pairs >= 20L * n_experts ? TILE_BIG_ROWS : TILE_SMALL_ROWS;
+  return n_pairs >= TILE_BIG_PAIRS && n_pairs >= (long)TILE_SMALL_ROWS * n_experts ? TILE_BIG_ROWS : TILE_SMALL_ROWS;
 }
 
 // More than there can be: an expert with c pairs has at most (c + tile_rows - 1) / tile_rows tiles, less than c / tile_rows + 1.

@@ -454,9 +454,9 @@ def test_latent_attention_rows_keep_their_bits(lib, heads, rot, window, sink):
         assert torch.equal(rows(which[-1:]), whole[which[-1:]]), b
 
 
-# rows an expert around the edges of a tile (32 rows up to 20 rows an expert on average, 128 above), experts without rows,
+# rows an expert around the edges of a tile (128 rows from 1024 pairs and 32 rows an expert on average on, else 32), experts without rows,
 # K past a whole step of 64 (72, 200, 136), columns past a block's 128 or 256, and rows that are not aligned to 16 bytes
-@pytest.mark.parametrize("counts", [(1, 31, 0), (32, 2, 33, 0, 1), (127, 0, 129), (128, 1, 256, 20), (21, 20), (700,)])
+@pytest.mark.parametrize("counts", [(1, 31, 0), (32, 2, 33, 0, 1), (127, 0, 129), (128, 1, 256, 20), (21, 20), (700,), (127, 0, 129, 769), (128, 1, 256, 20, 700), (1024,), (1153, 3)])
 @pytest.mark.parametrize("ff,width", [(136, 72), (264, 200), (8, 520)])
 @pytest.mark.parametrize("form", ["gated", "scaled", "plain", "unaligned"])
 def test_experts_at_the_edges_of_their_tiles(lib, counts, ff, width, form):
@@ -519,7 +519,7 @@ def test_headwise_linear_of_more_tokens_than_a_launch_has_tiles(lib):
 
 
 # a width or a hidden size that is no multiple of 8: the rows of one product are aligned to 16 bytes, those of the other are not
-@pytest.mark.parametrize("counts", [(1, 31, 0), (17, 33, 2, 0, 1), (129, 0, 16), (700,)])
+@pytest.mark.parametrize("counts", [(1, 31, 0), (17, 33, 2, 0, 1), (129, 0, 16), (1024,)])
 @pytest.mark.parametrize("ff,width,aligned", [(132, 72, 0), (1, 64, 0), (136, 68, 1), (40, 9, 1)])
 def test_experts_with_one_aligned_product(lib, monkeypatch, counts, ff, width, aligned):
     from fms_amd.kernels import ops
@@ -541,7 +541,7 @@ def test_experts_with_one_aligned_product(lib, monkeypatch, counts, ff, width, a
     monkeypatch.setattr(ops, "load", lambda: Listening())
     y = ops.moe_experts(x, ids, wg, wu, wd, 1.25, 1.702, 1.0).double()
     # the matrix-core kernels' tiles for the aligned product, the other kernel's for the other one
-    assert rows[aligned] == (128 if T >= 20 * E else 32) and rows[1 - aligned] == 16
+    assert rows[aligned] == (128 if T >= 1024 else 32) and rows[1 - aligned] == 16
     for e in range(E):
         at = torch.where(ids[:, 0] == e)[0]
         g, u = [x[at].double() @ w[e].double().T for w in (wg, wu)]
@@ -575,7 +575,7 @@ def test_experts_whose_weights_are_read_once_and_more_than_once(lib, counts):
 
 # the C interface with buffers of the sizes that its header states, between numbers that nobody may touch: few pairs an expert
 # (tiles of 32 rows), many (128), rows that are not aligned (16), and as many tiles as pairs
-@pytest.mark.parametrize("T,E,wide_ok", [(40, 5, 1), (300, 3, 1), (40, 5, 0), (7, 7, 1), (1, 1, 1)])
+@pytest.mark.parametrize("T,E,wide_ok", [(40, 5, 1), (1100, 3, 1), (40, 5, 0), (7, 7, 1), (1, 1, 1)])
 def test_group_writes_its_tiles_and_nothing_else(lib, T, E, wide_ok):
     from fms_amd.kernels import load
     from fms_amd.kernels.library import check
