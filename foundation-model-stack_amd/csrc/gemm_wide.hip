@@ -436,7 +436,9 @@ static bool wide_keeps_groups(int K) { return ceil_div(K, WD_GROUP) <= 4; }
 
 // The cut with the least estimated time.  The blocks run in rounds over the compute units; a round's time is its steps and a
 // start; the partial sums of slices are written and read once, by a kernel of its own unless the product kernel finishes its
-// one slice itself.  A step takes what its rows take to arrive (measured with all units at work: 28 bytes a nanosecond of
+// one slice itself (with two tiles of x its blocks then take some 3 us longer than their steps say: 14336 weight rows of
+// K = 4096 in one slice and in two at 33, 48 and 64 rows 34.2, 32.1, 32.3 us against 25.8, 27.2, 29.1, 7168 of K = 2048 at 64 rows 18.3
+// against 15.6).  A step takes what its rows take to arrive (measured with all units at work: 28 bytes a nanosecond of
 // weights for each; rows of x come out of the caches at about three times that) but never less than the operands' way from LDS
 // to the matrix units (measured 0.4, 0.7 and 1.0 us for a step of one or two, three or four, five or six tiles of x).
 static WidePlan wide_plan(int epi, int M, int rows, int K) {
@@ -468,7 +470,10 @@ static WidePlan wide_plan(int epi, int M, int rows, int K) {
       if (own > WD_ROWS) continue;
       const double step = (own + 0.35 * 32 * mt) * (TL_BK * 2 / 28000.);
       double cost = rounds * (ceil_div(ngroups, slices) * (WD_GROUP / TL_BK) * (step > busy ? step : busy) + 3.);
-      if (slices > 1 || !wide_finishes_itself(epi)) cost += 5. + (double)slices * M * rows * 8 / 4e6;
+      if (slices > 1 || !wide_finishes_itself(epi))
+        cost += 5. + (double)slices * M * rows * 8 / 4e6;
+      else if (mt == 2)
+        cost += 3.;
       if (best_cost < 0 || cost < best_cost) best = {own, slices}, best_cost = cost;
     }
   }
