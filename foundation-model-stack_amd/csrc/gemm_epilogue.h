@@ -75,8 +75,9 @@ struct RopeEpilogue {
 #define FMS_SKINNY_MAX_ROWS 192
 
 // ---- 17 to 192 rows (gemm_wide.hip) ------------------------------------------
-// The product runs as two kernels: blocks of 128 weight rows times a slice of K leave float32 partial sums
-// in a workspace [slices][M][rows]; a second kernel adds the slices in a fixed order and applies the epilogue.
+// Blocks of up to 128 weight rows times a slice of K.  With several slices they leave float32 partial sums in a workspace
+// [slices][M][rows], and a second kernel adds the slices in a fixed order and applies the epilogue; a plain or gated product
+// with one slice is finished by the first kernel.
 // `rows` counts all rows of W (for the gated product both halves).
 long wide_workspace_bytes(int M, int rows, int K);
 int wide_product(int epi, const void* x, long ldx, const void* w, const void* bias, int bias_dtype, void* out,
