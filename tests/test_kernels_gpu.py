@@ -362,6 +362,13 @@ def test_attention_decode_of_pages_that_several_blocks_read(ops, waves):
     attention_case(ops, torch.bfloat16, 160, 8, 128, starts=[1500, 2, 600, 63, 64, 190], lens=[1] * 6, decode=True, pages_per_block=8, waves=waves)
 
 
+# windows whose first key is the first, second, third and last of four, windows shorter than four keys and longer than a block's 256
+@pytest.mark.parametrize("window", [1, 2, 3, 6, 65, 259, 300])
+@pytest.mark.parametrize("H,K,D", [(4, 2, 40), (2, 1, 50), (3, 3, 128)])
+def test_attention_generic_f32_window(ops, window, H, K, D):
+    attention_case(ops, torch.float32, H, K, D, starts=[0, 301, 62], lens=[9, 6, 7], window=window)
+
+
 @pytest.mark.parametrize("dtype,decode", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_attention_far_key_and_window(ops, dtype, decode):
     lens = [1, 1] if decode else [40, 3]
