@@ -114,14 +114,7 @@ __global__ void __launch_bounds__(512)
     const int u = t + rot;
     const int k0 = (g_begin + (u >= n_steps ? u - n_steps : u)) * BK;
     const unsigned to = stage * (STAGE * 2);
-    if (!o.aligned) {  // uniform: the way to LDS wants 16-byte addresses, registers do not
-      const bool in = t < n_steps && k0 + piece * 8 < K;
-#pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(in ? src[i] + k0 : (const bf16*)tile_zeros);
-        *reinterpret_cast<bf16x8*>(smem + (put[i] - lds0) + to + lane * 16) = v;
-      }
-    } else if (t < n_steps && k0 + BK <= K) {  // uniform
+    if (t < n_steps && k0 + BK <= K) {  // uniform
 #pragma unroll
       for (int i = 0; i < RX; ++i) load_to_lds(src[i] + k0, put[i] + to);
 #pragma unroll
@@ -131,6 +124,26 @@ __global__ void __launch_bounds__(512)
 #pragma unroll
       for (int i = 0; i < R; ++i) load_to_lds(in ? (const void*)(src[i] + k0) : (const void*)tile_zeros, put[i] + to);
     }
+  };
+
+  // The way straight to LDS wants 16-byte addresses.  Where x or w starts at another one the rows go through registers, AHEAD steps
+  // before they are put into LDS: 33 rows of such x by 4096 and 28672 weight rows of K = 4096 17 and 49 us (24 and 79 with every step's
+  // loads waited for; 14 for the first where both are aligned).
+  constexpr int AHEAD = 3;
+  bf16x8 held[AHEAD][R];
+  auto ask = [&](int t, bf16x8 (&to)[R]) {
+    const int u = t + rot;
+    const int k0 = (g_begin + (u >= n_steps ? u - n_steps : u)) * BK;
+    const bool in = t < n_steps && k0 + piece * 8 < K;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const bf16x8* const from = reinterpret_cast<const bf16x8*>(in ? src[i] + k0 : (const bf16*)tile_zeros);
+      to[i] = i < RX ? *from : __builtin_nontemporal_load(from);
+    }
+  };
+  auto put_held = [&](int stage, const bf16x8 (&of)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) *reinterpret_cast<bf16x8*>(smem + (put[i] - lds0) + stage * (STAGE * 2) + lane * 16) = of[i];
   };
 
   constexpr int NT = (MT + 1) / 2;  // tiles of x a wave takes at most (tiles side, side + 2, ...)
@@ -143,8 +156,13 @@ __global__ void __launch_bounds__(512)
 #pragma unroll
   for (int j = 0; j < (FOLD ? NT : 1); ++j) folded[j] = acc[0];
 
+  if (o.aligned) {  // uniform
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
+    for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
+  } else {
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) ask(d, held[d]);
+  }
   constexpr int RPW = MT * 4;  // rows a wave works out the scale of
   if (MODE != WD_PARTIAL) {
     // 1 / rms of the rows of x, if their norm was left to this product.  The partial sums are asked for behind the
@@ -171,10 +189,7 @@ __global__ void __launch_bounds__(512)
       }
     }
   }
-  int stage = 0;
-  for (int t = 0; t < n_steps; ++t) {
-    tile_wait<(STAGES - 2) * R>();  // step t is there, and everybody is done with step t - 1
-    fetch(t + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
+  auto multiply = [&](int t, int stage) {
     const bf16* const xs = reinterpret_cast<const bf16*>(smem) + stage * STAGE;
     const bf16* const ws = xs + (XROWS + pair * 32) * BK;
     auto operand = [&](const bf16* rows32, int st) {
@@ -193,12 +208,36 @@ __global__ void __launch_bounds__(512)
         for (int st = 0; st < 4; ++st) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b[st], acc[j], 0, 0, 0);
       }
     }
-    stage = stage == STAGES - 1 ? 0 : stage + 1;
     if (FOLD && ((t + 1) % (WD_GROUP / BK) == 0 || t + 1 == n_steps)) {  // uniform
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) folded[j][v] += acc[j][v], acc[j][v] = 0.f;
+    }
+  };
+  if (o.aligned) {  // uniform
+    int stage = 0;
+    for (int t = 0; t < n_steps; ++t) {
+      tile_wait<(STAGES - 2) * R>();  // step t is there, and everybody is done with step t - 1
+      fetch(t + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
+      multiply(t, stage);
+      stage = stage == STAGES - 1 ? 0 : stage + 1;
+    }
+  } else {
+    put_held(0, held[0]);
+    ask(AHEAD, held[0]);
+    block_sync_lds();
+    for (int t0 = 0; t0 < n_steps; t0 += AHEAD) {
+#pragma unroll
+      for (int d = 0; d < AHEAD; ++d) {
+        // step t + 1 into the buffer that step t - 1 was in; loads and stores stand behind no branch, so that the compiler can wait
+        // for the oldest loads alone (steps past the end are zeros)
+        const int t = t0 + d;
+        put_held((t + 1) & 1, held[(d + 1) % AHEAD]);
+        ask(t + 1 + AHEAD, held[(d + 1) % AHEAD]);
+        if (t < n_steps) multiply(t, t & 1);  // uniform
+        block_sync_lds();
+      }
     }
   }
   if (FOLD) {
