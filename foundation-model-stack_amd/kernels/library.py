@@ -75,6 +75,7 @@ _SIGNATURES = {
     "fmsamd_scale_f32": [P, L, F, P],
     "fmsamd_cast_cols": [P, L, P, I, L, I, I, P],
     "fmsamd_delta_prepare": [P, L, I, P, L, I, P, I, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, P, I, P],
+    "fmsamd_delta_runs": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, L, P],
     "fmsamd_delta_rule": [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
     "fmsamd_gated_head_norm": [P, P, L, P, I, F, I, F, P, I, L, P, I, I, I, P],
     "fmsamd_moe_combine": [P, P, I, P, P, L, P, I, I, I, P, I, P, L, P],
@@ -138,6 +139,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
         lib.fmsamd_ssd_chunk_workspace.argtypes = [I, I, I]
         lib.fmsamd_linear_recurrence_workspace.restype = c_long
         lib.fmsamd_linear_recurrence_workspace.argtypes = [I, I, I, I, I]
+        lib.fmsamd_delta_runs_workspace.restype = c_long
+        lib.fmsamd_delta_runs_workspace.argtypes = [I, I, I, I, I]
         lib.fmsamd_talking_attn_workspace.restype = c_long
         lib.fmsamd_talking_attn_workspace.argtypes = [I, I, I, I]
         lib.fmsamd_moe_max_tiles.restype = c_int

@@ -1470,6 +1470,10 @@ def soft_cap_(x: torch.Tensor, cap: float) -> torch.Tensor:
 # --------------------------------------------------------------------------
 DELTA_MAX_TAPS = 8
 DELTA_MAX_DIM = 256
+# Tokens a sequence, on average, from which a step's recurrence goes in runs of 16 tokens on the matrix unit: two kernels and a
+# workspace instead of one (16 heads of 128 by 128, one sequence of 64 tokens 17 us against 15, eight of 64 38 against 37,
+# four heads of a sequence of 300 and one of 77 29 against 54; with a decay per key channel eight of 64 38 against 53).
+DELTA_RUN_TOKENS = 96
 
 
 def delta_prepare(proj: torch.Tensor, col_b: int, a: torch.Tensor, col_a: int, conv_w: torch.Tensor, a_log: torch.Tensor,
@@ -1544,7 +1548,15 @@ def delta_rule(qkv: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, kq: t
     if seq_starts.numel() < n_seqs + 1 or slot_ids.numel() < n_seqs or seq_of_token.numel() < T:
         raise ValueError("the step's index arrays are shorter than its sequences or tokens")
     out = torch.empty(T, heads * vdim, dtype=torch.float32, device=qkv.device)
-    check(load().fmsamd_delta_rule(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), kq.data_ptr(), state.data_ptr(), out.data_ptr(),
+    lib = load()
+    if not single_tokens and dim % 64 == 0 and vdim % 16 == 0 and T >= DELTA_RUN_TOKENS * n_seqs and state.data_ptr() % 16 == 0:
+        ws_bytes = lib.fmsamd_delta_runs_workspace(T, n_seqs, heads, dim, vdim)
+        workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=qkv.device)
+        check(lib.fmsamd_delta_runs(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), state.data_ptr(), out.data_ptr(), seq_starts.data_ptr(),
+                                    seq_of_token.data_ptr(), slot_ids.data_ptr(), T, n_seqs, heads, kv_heads, dim, vdim,
+                                    int(bool(per_channel)), workspace.data_ptr(), ws_bytes, _stream()))
+        return out
+    check(lib.fmsamd_delta_rule(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), kq.data_ptr(), state.data_ptr(), out.data_ptr(),
                                    seq_starts.data_ptr(), seq_of_token.data_ptr(), slot_ids.data_ptr(), n_seqs, heads, kv_heads, dim,
                                    vdim, int(bool(per_channel)), int(bool(single_tokens)), _stream()))
     return out

@@ -323,6 +323,61 @@ def test_delta_rule_whole_in_portions_and_in_a_batch(lib, sizes):
     assert bool((S == before).all())
 
 
+@pytest.mark.parametrize("sizes", [(4, 2, 128, 16, False), (1, 1, 64, 48, True), (3, 1, 192, 32, False), (2, 2, 256, 80, True), (2, 1, 256, 272, False)])
+def test_delta_rule_in_runs(lib, sizes):
+    """Steps long enough for runs of 16 tokens: sequences that end at, one before and one behind a run's end, states that
+    earlier steps left, decays that are nothing and underflow within a run, beside the recurrence in 64 bits; and a value that
+    is no number, which no earlier token and no other value channel may see."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, per_channel = sizes
+    lens = [1, 255, 16, 160, 97]
+    T, per = sum(lens), D if per_channel else 1
+    assert T >= ops.DELTA_RUN_TOKENS * len(lens)
+    gen = torch.Generator().manual_seed(D + V)
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    q, k, v = unit(torch.randn(T, G, D, generator=gen)), unit(torch.randn(T, G, D, generator=gen) + 0.1), torch.randn(T, H, V, generator=gen)
+    beta = torch.sigmoid(2 * torch.randn(T, H, generator=gen))
+    decay = torch.exp(-torch.exp(3 * torch.randn(T, H, per, generator=gen) - 2))
+    decay[torch.rand(T, H, per, generator=gen) < 0.05] = 0.0
+    decay[torch.rand(T, H, per, generator=gen) < 0.05] = 1e-30
+    state = 0.3 * torch.randn(len(lens) + 1, H, V, D, generator=gen)
+    slots = torch.tensor([3, 0, 5, 2, 1], dtype=torch.int32)
+    starts = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32)
+
+    def run(values):
+        S = state.to(DEV)
+        qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1), values.reshape(T, -1)], dim=1).to(DEV)
+        out = ops.delta_rule(qkv, beta.to(DEV), decay.reshape(T, -1).to(DEV), (q * k).sum(-1).to(DEV), S, starts.to(DEV), seq.to(DEV),
+                             slots.to(DEV), len(lens), H, G, D, V, per_channel)
+        return out.cpu().view(T, H, V), S.cpu()
+
+    got, left = run(v)
+    heads = lambda t: t.double().repeat_interleave(H // G, dim=1)
+    for b, n in enumerate(lens):
+        S, at = state[slots[b]].double().transpose(1, 2), int(starts[b])  # [H, D, V]
+        want = []
+        for t in range(at, at + n):
+            S = S * decay[t].double()[:, :, None]
+            kt, qt = heads(k[t][None])[0], heads(q[t][None])[0]
+            u = beta[t].double()[:, None] * (v[t].double() - torch.matmul(kt[:, None], S)[:, 0])
+            S = S + kt[:, :, None] * u[:, None, :]
+            want.append(torch.matmul(qt[:, None], S)[:, 0])
+        # sums of up to 256 and 16 terms of a state of size 0.3, rounded to 24 bits a few times a run: some 1e-6 of the largest
+        torch.testing.assert_close(got[at : at + n], torch.stack(want).float(), atol=5e-6, rtol=1e-5)
+        torch.testing.assert_close(left[slots[b]], S.transpose(1, 2).float(), atol=5e-6, rtol=1e-5)
+    assert torch.equal(left[4], state[4])  # nobody's slot
+
+    t = int(starts[1]) + 37  # the sixth token of a run
+    broken = v.clone()
+    broken[t, 0, 3] = float("inf")
+    got2, _ = run(broken)
+    mine = torch.zeros(T, H, V, dtype=torch.bool)
+    mine[t : int(starts[2]), 0, 3] = True
+    assert not bool(torch.isfinite(got2[t, 0, 3])) and torch.equal(got2[~mine], got[~mine])
+
+
 def test_a_lost_state_shows(lib):
     """The recurrence's memory matters: a value written long ago, read by a matching query much later, with decays near one."""
     from fms_amd.kernels import ops
