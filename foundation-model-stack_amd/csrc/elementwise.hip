@@ -259,6 +259,69 @@ extern "C" int fmsamd_add_norm(float* resid, const void* branch, int act_dtype, 
   return 0;
 }
 
+// The embedding and the first norm as one kernel: x = table[id] * scale, left as float32 in resid; out = x / rms(x) * weight.
+// The arithmetic of embed and add_norm (the rows' sums in the same order), without a launch and a pass over the stream between
+// (a decode step loses a kernel of some 4 us; it is bound by the round trips to the token, its row and the sum).
+template <typename TableT, typename WeightT, typename OutT>
+__global__ void __launch_bounds__(1024)
+    embed_norm_kernel(const int* __restrict__ ids, const TableT* __restrict__ table, float* __restrict__ resid,
+                      const WeightT* __restrict__ weight, OutT* __restrict__ out, int width, int vocab, float scale, float eps) {
+  __shared__ float scratch[17];
+  int id = ids[blockIdx.x];
+  id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);  // the host has checked the range; never read outside
+  const TableT* row = table + (size_t)id * width;
+  float* x = resid + (size_t)blockIdx.x * width;
+  const int stride = blockDim.x * 4;
+  float keep[4][4], wkeep[4][4], sq = 0.f;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int i = threadIdx.x * 4 + n * stride;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) keep[n][e] = 0.f, wkeep[n][e] = 1.f;
+    if (i < width) {
+      load_vec<4>(row + i, keep[n]);
+      if (weight) load_vec<4>(weight + i, wkeep[n]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) keep[n][e] *= scale;
+      store_vec<4>(x + i, keep[n]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sq += keep[n][e] * keep[n][e];
+  }
+  const float inv = rsqrtf(block_sum(sq, scratch) / (float)width + eps);
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int i = threadIdx.x * 4 + n * stride;
+    if (i < width) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = keep[n][e] * inv * wkeep[n][e];
+      store_vec<4>(out + (size_t)blockIdx.x * width + i, v);
+    }
+  }
+}
+
+extern "C" int fmsamd_embed_norm(const int* ids, const void* table, int act_dtype, float* resid, const void* weight, int weight_dtype,
+                                 void* out, int n_tokens, int width, int vocab, float scale, float eps, hipStream_t stream) {
+  if (n_tokens == 0) return 0;
+  FMS_REQUIRE(n_tokens > 0 && width > 0 && vocab > 0 && eps >= 0.f, "embed_norm: bad sizes T=%d width=%d vocab=%d", n_tokens, width, vocab);
+  FMS_REQUIRE(width % 4 == 0 && width <= 16384 && (((size_t)table | (size_t)resid | (size_t)weight | (size_t)out) & 15) == 0,
+              "embed_norm: a width of %d (multiples of 4 up to 16384, at 16-byte addresses)", width);
+  int threads = (width / 16 + 63) / 64 * 64;  // as add_norm has them
+  threads = threads < 64 ? 64 : (threads > 1024 ? 1024 : threads);
+  if (n_tokens <= 256 && width <= 4096) threads = (width / 4 + 63) / 64 * 64;
+#define FMS_EN(A, W) \
+  embed_norm_kernel<A, W, A><<<n_tokens, threads, 0, stream>>>(ids, (const A*)table, resid, (const W*)weight, (A*)out, width, vocab, scale, eps)
+  if (act_dtype == FMS_F32 && weight_dtype == FMS_F32) FMS_EN(float, float);
+  else if (act_dtype == FMS_F32 && weight_dtype == FMS_BF16) FMS_EN(float, bf16);
+  else if (act_dtype == FMS_BF16 && weight_dtype == FMS_F32) FMS_EN(bf16, float);
+  else if (act_dtype == FMS_BF16 && weight_dtype == FMS_BF16) FMS_EN(bf16, bf16);
+  else FMS_REQUIRE(false, "embed_norm: unknown dtypes act=%d weight=%d", act_dtype, weight_dtype);
+#undef FMS_EN
+  FMS_LAUNCH_CHECK("embed_norm");
+  return 0;
+}
+
 // --------------------------------------------------------------------------
 // the stream with what is still to be added, as rows of the activation type (the stream itself stays as it is)
 // --------------------------------------------------------------------------

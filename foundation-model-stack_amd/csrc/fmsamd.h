@@ -35,6 +35,10 @@ int fmsamd_abi_version();
 // resid[t, :] = float(table[ids[t], :]) * scale
 int fmsamd_embed(const int* ids, const void* table, int table_dtype, float* out, int n_tokens, int width, int vocab,
                  float scale, hipStream_t stream);
+// The embedding and the RMS norm that reads it first (weight may be null): resid = table[ids] * scale in float32, out = the
+// normed rows in act_dtype, which is the table's.  width a multiple of 4 up to 16384, everything at 16-byte addresses.
+int fmsamd_embed_norm(const int* ids, const void* table, int act_dtype, float* resid, const void* weight, int weight_dtype,
+                      void* out, int n_tokens, int width, int vocab, float scale, float eps, hipStream_t stream);
 
 // resid += branch (float32 sum, written back unless `rows` is given); out = norm(resid) * weight + bias.
 // branch, weight, bias and rows may be null.  act_dtype is the type of branch and out.  branch_scale (float32 [width] or
@@ -172,6 +176,11 @@ long fmsamd_argmax_workspace(int rows, int vocab);
 int fmsamd_argmax(const float* logits, long ld, int rows, int vocab, void* workspace, long workspace_bytes,
                   int* out_tokens, hipStream_t stream);
 
+// The same choices with the step behind them: positions[r] += 1 for every row whose seq_of_token is not negative.
+int fmsamd_sample_advance(const float* logits, long ld, int rows, int vocab, int do_sample, float temperature, int top_k,
+                          void* rng_state, int* out_tokens, int* positions, const int* seq_of_token, hipStream_t stream);
+int fmsamd_argmax_advance(const float* logits, long ld, int rows, int vocab, void* workspace, long workspace_bytes,
+                          int* out_tokens, int* positions, const int* seq_of_token, hipStream_t stream);
 // The greedy choice of fmsamd_argmax without a workspace, for callers that cannot allocate device memory:
 // code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart
 // in the reference.  The partial results of the first stage go to an array of FMSAMD_ARGMAX_STATIC_BYTES

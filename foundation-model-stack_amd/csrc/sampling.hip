@@ -112,6 +112,11 @@ __device__ __forceinline__ void for_each_value(const float* __restrict__ x, int 
   }
 }
 
+// The step behind the choice in a captured decode step: the row's next position (positions may be null; padding rows stay).
+__device__ __forceinline__ void advance_position(int* __restrict__ positions, const int* __restrict__ seq_of_token, int row) {
+  if (positions != nullptr && seq_of_token[row] >= 0) positions[row] += 1;
+}
+
 // One block per row.  The row is read in passes whose loads are coalesced.
 //   Always: the largest value.
 //   top_k up to 512: each thread's largest value as well.  At least k values are as large as the k-th largest
@@ -126,7 +131,9 @@ __device__ __forceinline__ void for_each_value(const float* __restrict__ x, int 
 // the logits as they are, and only values that pass a bound lowered by a little are divided and compared exactly.
 __global__ void __launch_bounds__(SMP_THREADS)
     sample_kernel(const float* __restrict__ logits, long ld, int vocab, int do_sample, float temperature, int top_k,
-                  unsigned long long* __restrict__ rng, int* __restrict__ out_tokens) {
+                  unsigned long long* __restrict__ rng, int* __restrict__ out_tokens, int* __restrict__ positions,
+                  const int* __restrict__ seq_of_token) {
+  if (threadIdx.x == 0) advance_position(positions, seq_of_token, blockIdx.x);
   __shared__ float scratch[17];
   __shared__ unsigned int hist[256];
   __shared__ unsigned int wave_total[4];
@@ -365,7 +372,8 @@ __global__ void __launch_bounds__(ARG_THREADS)
 
 __global__ void __launch_bounds__(ARG_THREADS)
     argmax_final_kernel(const float* __restrict__ part_val, const int* __restrict__ part_idx, int chunks,
-                        int* __restrict__ out_tokens) {
+                        int* __restrict__ out_tokens, int* __restrict__ positions, const int* __restrict__ seq_of_token) {
+  if (threadIdx.x == 0) advance_position(positions, seq_of_token, blockIdx.x);
   __shared__ float scratch[17];
   __shared__ int sh_arg;
   const int row = blockIdx.x;
@@ -389,8 +397,9 @@ extern "C" long fmsamd_argmax_workspace(int rows, int vocab) {
 }
 
 // greedy choice with a workspace of fmsamd_argmax_workspace(rows, vocab) bytes
-extern "C" int fmsamd_argmax(const float* logits, long ld, int rows, int vocab, void* workspace, long workspace_bytes,
-                             int* out_tokens, hipStream_t stream) {
+extern "C" int fmsamd_argmax_advance(const float* logits, long ld, int rows, int vocab, void* workspace, long workspace_bytes,
+                                     int* out_tokens, int* positions, const int* seq_of_token, hipStream_t stream) {
+  FMS_REQUIRE(positions == nullptr || seq_of_token != nullptr, "argmax: positions advance by the rows' sequences");
   if (rows == 0) return 0;
   FMS_REQUIRE(rows > 0 && vocab > 0 && ld >= vocab, "argmax: bad sizes rows=%d vocab=%d ld=%ld", rows, vocab, ld);
   FMS_REQUIRE(rows <= 65535, "argmax: %d rows exceed one launch", rows);
@@ -401,9 +410,14 @@ extern "C" int fmsamd_argmax(const float* logits, long ld, int rows, int vocab, 
   int* part_idx = (int*)(part_val + (size_t)rows * chunks);
   argmax_partial_kernel<<<dim3(chunks, rows), ARG_THREADS, 0, stream>>>(logits, ld, vocab, part_val, part_idx, chunks);
   FMS_LAUNCH_CHECK("argmax_partial");
-  argmax_final_kernel<<<rows, ARG_THREADS, 0, stream>>>(part_val, part_idx, chunks, out_tokens);
+  argmax_final_kernel<<<rows, ARG_THREADS, 0, stream>>>(part_val, part_idx, chunks, out_tokens, positions, seq_of_token);
   FMS_LAUNCH_CHECK("argmax_final");
   return 0;
+}
+
+extern "C" int fmsamd_argmax(const float* logits, long ld, int rows, int vocab, void* workspace, long workspace_bytes,
+                             int* out_tokens, hipStream_t stream) {
+  return fmsamd_argmax_advance(logits, ld, rows, vocab, workspace, workspace_bytes, out_tokens, nullptr, nullptr, stream);
 }
 
 // ---- the same greedy choice for callers that cannot allocate ---------------------------------
@@ -453,13 +467,15 @@ extern "C" int fmsamd_argmax_static(const float* logits, long ld, int rows, int 
   int* part_idx = (int*)(part_val + (size_t)rows * chunks);
   argmax_partial_kernel<<<dim3(chunks, rows), ARG_THREADS, 0, stream>>>(logits, ld, vocab, part_val, part_idx, chunks);
   FMS_LAUNCH_CHECK("argmax_static (first stage)");
-  argmax_final_kernel<<<rows, ARG_THREADS, 0, stream>>>(part_val, part_idx, chunks, out_tokens);
+  argmax_final_kernel<<<rows, ARG_THREADS, 0, stream>>>(part_val, part_idx, chunks, out_tokens, nullptr, nullptr);
   FMS_LAUNCH_CHECK("argmax_static (second stage)");
   return 0;
 }
 
-extern "C" int fmsamd_sample(const float* logits, long ld, int rows, int vocab, int do_sample, float temperature,
-                             int top_k, void* rng_state, int* out_tokens, hipStream_t stream) {
+extern "C" int fmsamd_sample_advance(const float* logits, long ld, int rows, int vocab, int do_sample, float temperature,
+                                     int top_k, void* rng_state, int* out_tokens, int* positions, const int* seq_of_token,
+                                     hipStream_t stream) {
+  FMS_REQUIRE(positions == nullptr || seq_of_token != nullptr, "sample: positions advance by the rows' sequences");
   if (rows == 0) return 0;
   FMS_REQUIRE(rows > 0 && vocab > 0 && ld >= vocab, "sample: bad sizes rows=%d vocab=%d ld=%ld", rows, vocab, ld);
   if (do_sample) {
@@ -468,7 +484,12 @@ extern "C" int fmsamd_sample(const float* logits, long ld, int rows, int vocab, 
     FMS_REQUIRE(rng_state != nullptr, "sample: sampling needs generator state");
   }
   sample_kernel<<<rows, SMP_THREADS, 0, stream>>>(logits, ld, vocab, do_sample, temperature, top_k,
-                                                  (unsigned long long*)rng_state, out_tokens);
+                                                  (unsigned long long*)rng_state, out_tokens, positions, seq_of_token);
   FMS_LAUNCH_CHECK("sample");
   return 0;
+}
+
+extern "C" int fmsamd_sample(const float* logits, long ld, int rows, int vocab, int do_sample, float temperature,
+                             int top_k, void* rng_state, int* out_tokens, hipStream_t stream) {
+  return fmsamd_sample_advance(logits, ld, rows, vocab, do_sample, temperature, top_k, rng_state, out_tokens, nullptr, nullptr, stream);
 }

@@ -81,8 +81,8 @@ class DecodeGraph:
         logits = self.engine.model.forward(self.batch, self.engine.cache)
         self.logits = logits  # [rows, vocab]; after a replay, that step's logits (padding rows: anything)
         s = self.sampling
-        ops.sample(logits, s.do_sample, s.temperature, s.top_k or 0, self.rng if s.do_sample else None, out=self.tokens)
-        ops.advance_positions_(self.positions, self.seq_of_token)
+        ops.sample(logits, s.do_sample, s.temperature, s.top_k or 0, self.rng if s.do_sample else None, out=self.tokens,
+                   positions=self.positions, seq_of_token=self.seq_of_token)
 
     def capture(self) -> None:
         # Padding rows only (sequence -1): nothing is written to the cache while warming up and capturing.

@@ -138,7 +138,7 @@ class DecoderModel(Part):
         """float32 logits [n wanted rows, vocab] of the tokens in `batch`; the cache is extended in place."""
         max_position = batch.max_context - 1
         batch.shared.clear()
-        stream = ResidualStream(self.embedding.forward(batch.token_ids, batch))
+        stream = self._embedded(batch)
         for part in self.entrances.values():
             part.begin(stream, batch, self.dtype)
         for n, entry in enumerate(self.schedule):
@@ -162,3 +162,16 @@ class DecoderModel(Part):
                 block.forward(stream, batch, view, self.dtype)
         normed = stream.normed(self.final_norm, self.dtype, rows=batch.logit_rows)
         return self.head.forward(normed)
+
+    def _embedded(self, batch) -> ResidualStream:
+        """The stream as the embedding leaves it, with the first block's norm of it where one kernel makes both."""
+        first = self.schedule[0] if self.schedule else None
+        fused = getattr(self.embedding, "forward_normed", None)
+        if first is not None and first.enter is None and fused is not None and ResidualStream.fuse_products:
+            norm = getattr(self.layers[first.layer], "first_norm", lambda: None)()
+            made = fused(batch.token_ids, norm, self.dtype) if norm is not None else None
+            if made is not None:
+                stream = ResidualStream(made[0])
+                stream.prepared = (norm, made[1])
+                return stream
+        return ResidualStream(self.embedding.forward(batch.token_ids, batch))

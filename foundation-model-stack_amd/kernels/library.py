@@ -26,6 +26,7 @@ P, I, L, F = c_void_p, c_int, c_long, c_float
 
 _SIGNATURES = {
     "fmsamd_embed": [P, P, I, P, I, I, I, F, P],
+    "fmsamd_embed_norm": [P, P, I, P, P, I, P, I, I, I, F, F, P],
     "fmsamd_add_norm": [P, P, I, P, P, I, P, P, I, I, F, I, P, P],
     "fmsamd_stream_rows": [P, P, P, P, I, L, I, I, P],
     "fmsamd_gated_act": [P, P, I, P, I, L, I, I, I, P, P],
@@ -47,6 +48,8 @@ _SIGNATURES = {
     "fmsamd_gemm_skinny_residual_partials": [I, I, I],
     "fmsamd_gemm_skinny_residual_bf16": [P, L, P, P, I, P, L, P, I, P, L, P, I, I, I, I, P, P, L, P],
     "fmsamd_sample": [P, L, I, I, I, F, I, P, P, P],
+    "fmsamd_sample_advance": [P, L, I, I, I, F, I, P, P, P, P, P],
+    "fmsamd_argmax_advance": [P, L, I, I, P, L, P, P, P, P],
     "fmsamd_argmax": [P, L, I, I, P, L, P, P],
     "fmsamd_norm_add_norm": [P, P, I, P, F, P, I, F, P, P, I, I, P],
     "fmsamd_norm_add_norm_affine": [P, P, I, P, P, F, I, P, P, I, F, I, P, P, I, I, P],

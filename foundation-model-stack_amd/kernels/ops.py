@@ -69,6 +69,26 @@ def embed(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0) -> torch.T
     return out
 
 
+def embed_norm(ids: torch.Tensor, table: torch.Tensor, scale: float, weight: Optional[torch.Tensor], eps: float):
+    """(embed(ids, table, scale), its RMS norm times weight in the table's type) as one kernel; None for widths and addresses
+    that it does not take (embed and add_norm do)."""
+    _need_cuda(ids, table, weight)
+    _need_i32("ids", ids)
+    if table.dim() != 2 or not table.is_contiguous():
+        raise ValueError("embedding table must be a contiguous [vocab, width] tensor")
+    width = table.shape[1]
+    if weight is not None and (weight.shape != (width,) or not weight.is_contiguous()):
+        raise ValueError(f"norm weight must be a contiguous [{width}] tensor, got {tuple(weight.shape)}")
+    if width % 4 or width > 16384 or table.data_ptr() % 16 or (weight is not None and weight.data_ptr() % 16):
+        return None
+    resid = torch.empty(ids.numel(), width, dtype=torch.float32, device=table.device)
+    out = torch.empty(ids.numel(), width, dtype=table.dtype, device=table.device)
+    check(load().fmsamd_embed_norm(ids.data_ptr(), table.data_ptr(), _code(table.dtype), resid.data_ptr(), _ptr(weight),
+                                   _code(weight.dtype) if weight is not None else 0, out.data_ptr(), ids.numel(), width, table.shape[0],
+                                   float(scale), float(eps), _stream()))
+    return resid, out
+
+
 def add_norm(
     resid: torch.Tensor,
     branch: Optional[torch.Tensor],
@@ -529,7 +549,11 @@ def decode_split(rows: int, n_pages: int):
     deals its own pages out evenly over the splits; the waves of a block run their pages as a pipeline,
     so a block of many pages is cheaper than many blocks).  The waves of a block share its pages and merge in LDS, the blocks of a row
     merge in a second kernel."""
-    by_rows = min(-(-256 // max(rows, 1)), max(1, n_pages // 8))  # but no splits of under 8 pages: one for each wave
+    # But no splits of under 8 pages, one for each wave, and one split up to 16 pages.  Microseconds with two splits and their
+    # merge, and with one, under a bound of 1024 tokens: a sequence of 4 kv heads of 64, 64 tokens 6.7 and 4.7, 300 7.5 and 6.6,
+    # 512 8.1 and 7.7, 700 8.7 and 9.0, 1024 9.7 and 11.1; 64 sequences of 8 kv heads of 128, 300 tokens 27.7 and 18.3, 1024 53
+    # and 47.7.
+    by_rows = min(-(-256 // max(rows, 1)), max(1, n_pages // 8)) if n_pages > 16 else 1
     splits = max(1, min(max(by_rows, -(-n_pages // 128)), n_pages))
     pages = -(-n_pages // splits)
     waves = max(1, min(8 if rows * splits <= 512 else 4, pages))
@@ -1807,9 +1831,17 @@ def sample(
     top_k: int = 0,
     rng_state: Optional[torch.Tensor] = None,
     out: Optional[torch.Tensor] = None,
+    positions: Optional[torch.Tensor] = None,
+    seq_of_token: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    """One token per row of float32 logits.  rng_state: int64 [rows, 2] (seed, counter), advanced in place."""
-    _need_cuda(logits, rng_state, out)
+    """One token per row of float32 logits.  rng_state: int64 [rows, 2] (seed, counter), advanced in place.  positions, with
+    seq_of_token: advanced as advance_positions_ does, by the same kernel."""
+    _need_cuda(logits, rng_state, out, positions, seq_of_token)
+    if positions is not None:
+        _need_i32("positions", positions)
+        _need_i32("seq_of_token", seq_of_token)
+        if positions.numel() != logits.shape[0] or seq_of_token.numel() != logits.shape[0]:
+            raise ValueError("positions and seq_of_token must have one entry per row")
     _rows2d("logits", logits)
     if logits.dtype != torch.float32:
         raise TypeError("logits are float32")
@@ -1827,10 +1859,11 @@ def sample(
         lib = load()
         nbytes = lib.fmsamd_argmax_workspace(rows, vocab)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=logits.device)
-        check(lib.fmsamd_argmax(logits.data_ptr(), logits.stride(0), rows, vocab, ws.data_ptr(), nbytes, out.data_ptr(), _stream()))
+        check(lib.fmsamd_argmax_advance(logits.data_ptr(), logits.stride(0), rows, vocab, ws.data_ptr(), nbytes, out.data_ptr(),
+                                        _ptr(positions), _ptr(seq_of_token), _stream()))
         return out
-    check(load().fmsamd_sample(logits.data_ptr(), logits.stride(0), rows, vocab, int(bool(do_sample)), float(temperature),
-                               int(top_k or 0), _ptr(rng_state), out.data_ptr(), _stream()))
+    check(load().fmsamd_sample_advance(logits.data_ptr(), logits.stride(0), rows, vocab, int(bool(do_sample)), float(temperature),
+                                       int(top_k or 0), _ptr(rng_state), out.data_ptr(), _ptr(positions), _ptr(seq_of_token), _stream()))
     return out
 
 

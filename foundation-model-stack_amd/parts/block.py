@@ -34,12 +34,13 @@ class ResidualStream:
         self.pending: Optional[torch.Tensor] = None
         self.pending_norm: Optional[Part] = None  # the norm that the pending branch passes before it is added
         self.pending_scale: Optional[torch.Tensor] = None  # a factor per channel on the pending branch
-        self.prepared: Optional[tuple] = None  # (norm, NormedRows) of the stream as it is now
+        self.prepared: Optional[tuple] = None  # (norm, NormedRows or normed tensor) of the stream as it is now
 
     def normed(self, norm: Part, act_dtype: torch.dtype, deferred_ok: bool = False, rows: Optional[torch.Tensor] = None):
         """The stream (with what is pending added) through `norm`: a tensor, or a NormedRows if allowed and at hand."""
         prepared, self.prepared = self.prepared, None
-        if prepared is not None and prepared[0] is norm and deferred_ok and rows is None and self.fuse_products:
+        if (prepared is not None and prepared[0] is norm and rows is None and self.fuse_products
+                and (deferred_ok or not isinstance(prepared[1], NormedRows))):
             return prepared[1]
         pending, self.pending = self.pending, None
         pending_norm, self.pending_norm = self.pending_norm, None

@@ -23,6 +23,14 @@ class TokenEmbedding(Part):
         every token): an embedding that adds a learned vector per position reads it, this one does not."""
         return ops.embed(token_ids, self.w["weight"], self.scale)
 
+    def forward_normed(self, token_ids: torch.Tensor, norm: Part, act_dtype: torch.dtype):
+        """(the stream, the stream through `norm`) as one kernel, or None where there is none for this norm and these types."""
+        if getattr(self.forward, "__func__", None) is not TokenEmbedding.forward:  # somebody else's forward
+            return None
+        if act_dtype != self.w["weight"].dtype or not getattr(norm, "deferrable", lambda: False)():
+            return None
+        return ops.embed_norm(token_ids, self.w["weight"], self.scale, norm.scale_weight(), norm.eps)
+
 
 class LinearHead(Part):
     def __init__(self, width: int, vocab: int, scale: float = 1.0, soft_cap: float = 0.0):

@@ -66,6 +66,25 @@ def test_add_norm(ops, width, dtype):
     torch.testing.assert_close(out3.cpu().float(), P.rms_norm(resid, weight.float(), eps), **tol(dtype))
 
 
+@pytest.mark.parametrize("rows, width, act, weight_type", [(1, 4, torch.bfloat16, torch.bfloat16), (3, 260, torch.float32, torch.float32),
+                                                           (257, 2048, torch.bfloat16, torch.float32), (2, 16384, torch.float32, torch.bfloat16),
+                                                           (5, 4096, torch.bfloat16, None)])
+def test_embed_norm_is_embed_and_add_norm(ops, rows, width, act, weight_type):
+    """The same bits as the two kernels it stands for; sizes that it leaves to them; and a choice that advances positions."""
+    gen = torch.Generator().manual_seed(width)
+    table = dev(torch.randn(50, width, generator=gen).to(act))
+    ids = dev(torch.randint(0, 50, (rows,), generator=gen, dtype=torch.int32))
+    weight = None if weight_type is None else dev(torch.randn(width, generator=gen).to(weight_type))
+    want = ops.embed(ids, table, 1.5)
+    resid, normed = ops.embed_norm(ids, table, 1.5, weight, 1e-5)
+    assert torch.equal(resid, want) and torch.equal(normed, ops.add_norm(want, None, weight, None, 1e-5, act))
+    assert ops.embed_norm(ids, dev(torch.randn(50, width + 2, generator=gen)), 1.0, None, 1e-5) is None
+    positions, seq = dev(torch.arange(rows, dtype=torch.int32)), dev((torch.arange(rows, dtype=torch.int32) % 3) - 1)
+    logits = dev(torch.randn(rows, 50 * width, generator=gen)) if rows * width < 10000 else dev(torch.randn(rows, 60, generator=gen))
+    assert torch.equal(ops.sample(logits, False, positions=positions, seq_of_token=seq), ops.sample(logits, False))
+    assert torch.equal(positions, torch.arange(rows, device=seq.device, dtype=torch.int32) + (seq >= 0))
+
+
 def test_add_norm_with_mean_and_shift(ops):
     torch.manual_seed(2)
     x = torch.randn(3, 48) + 1.5
