@@ -359,9 +359,8 @@ extern "C" int fmsamd_latent_attn_generic(const void* qa, long ldq, void* out, l
 // Two ways to share the work of a block's four waves:
 //   * prompts: each wave another (token, head group); every wave walks all keys of its token (the waves of a block
 //     read the same rows, which the caches serve);
-//   * single tokens: all waves of a block, and the blocks of several splits, share one (token, head group) and deal
-//     its key tiles out in turn; every part leaves (maximum, sum, unnormalised result) in a workspace and a second
-//     kernel merges them.
+//   * single tokens: a block's waves deal out a run of key tiles of one (token, head group) in turn and meet in LDS; the
+//     blocks that share it leave (maximum, sum, unnormalised result) each in a workspace, and a second kernel merges them.
 // The sink starts the maximum of every part and is counted in the sum of part 0 only.
 // --------------------------------------------------------------------------
 #define LAT_EMPTY -1e30f
@@ -379,16 +378,29 @@ struct LatentState {
 
 // EXACT: the latent has exactly RT * 16 elements and a row exactly WC * 32, so no product of the loops below has
 // to be asked whether it exists (each such question is a branch around a matrix instruction).
-template <int RT, int WC, int KG, int VG, bool EXACT, typename LoadQ, typename LoadK, typename LoadV>
+// AHEAD: the tile's keys and the first VG tiles of its latent are asked for at once, the next VG once the keys have been
+// multiplied, and so on VG at a time behind the products: not a round trip to memory for every group (KG is the whole of K).
+template <int RT, int WC, int KG, int VG, bool EXACT, bool AHEAD = false, typename LoadQ, typename LoadK, typename LoadV>
 __device__ __forceinline__ void latent_tile(LatentState<RT, WC>& st, LoadQ load_q, LoadK load_k, LoadV load_v, int base,
                                             int lo, int pos, int rank, int width, float scale, int grp) {
   f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+  bf16x8 ahead[2][AHEAD ? VG : 1];
+  auto ask = [&](int set, int d0) {
+#pragma unroll
+    for (int dt = 0; dt < VG; ++dt)
+      if (d0 + dt < RT && (EXACT || (d0 + dt) * 16 < rank)) ahead[set][AHEAD ? dt : 0] = load_v(d0 + dt);
+  };
 #pragma unroll
   for (int c0 = 0; c0 < WC; c0 += KG) {
     bf16x8 ka[KG], kb[KG];
 #pragma unroll
     for (int c = 0; c < KG; ++c) {
       if (c0 + c < WC && (EXACT || (c0 + c) * 32 < width)) ka[c] = load_k(0, c0 + c), kb[c] = load_k(1, c0 + c);
+    }
+    if constexpr (AHEAD) {
+      static_assert(KG >= WC, "one group of keys");
+      ask(0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int c = 0; c < KG; ++c) {
@@ -398,6 +410,11 @@ __device__ __forceinline__ void latent_tile(LatentState<RT, WC>& st, LoadQ load_
         sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[c], q, sb, 0, 0, 0);
       }
     }
+  }
+  if constexpr (AHEAD && VG < RT) {
+    __builtin_amdgcn_sched_barrier(0);
+    ask(1, VG);
+    __builtin_amdgcn_sched_barrier(0);
   }
   // this lane's scores: keys base + 8 grp + i (sa) and base + 8 grp + 4 + i (sb) of its column
   float s[8];
@@ -431,7 +448,10 @@ __device__ __forceinline__ void latent_tile(LatentState<RT, WC>& st, LoadQ load_
     bf16x8 v[VG];
 #pragma unroll
     for (int dt = 0; dt < VG; ++dt) {
-      if (d0 + dt < RT && (EXACT || (d0 + dt) * 16 < rank)) v[dt] = load_v(d0 + dt);
+      if (d0 + dt < RT && (EXACT || (d0 + dt) * 16 < rank)) {
+        if constexpr (AHEAD) v[dt] = ahead[d0 / VG & 1][dt];
+        else v[dt] = load_v(d0 + dt);
+      }
     }
 #pragma unroll
     for (int dt = 0; dt < VG; ++dt) {
@@ -443,35 +463,129 @@ __device__ __forceinline__ void latent_tile(LatentState<RT, WC>& st, LoadQ load_
         st.acc[d0 + dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[dt], pmat, st.acc[d0 + dt], 0, 0, 0);
       }
     }
+    if constexpr (AHEAD) {
+      if (d0 + 2 * VG < RT) ask(d0 / VG & 1, d0 + 2 * VG);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
-// What a wave leaves: the normalised result (one part) or its part's maximum, sum and unnormalised result.
+// What a wave that has all keys of its tile leaves: the normalised result.
 template <int RT, int WC, bool EXACT>
-__device__ __forceinline__ void latent_finish(LatentState<RT, WC>& st, bf16* __restrict__ out, long ldo, float* __restrict__ ws, int t,
-                                              int head, int nheads, int rank, int n_parts, int part, int grp) {
+__device__ __forceinline__ void latent_finish(LatentState<RT, WC>& st, bf16* __restrict__ out, long ldo, int t, int head, int nheads,
+                                              int rank, int grp) {
   st.l += __shfl_xor(st.l, 16, WAVE);
   st.l += __shfl_xor(st.l, 32, WAVE);
   if (head >= nheads) return;
   // acc[dt][i] is element d = dt * 16 + grp * 4 + i of this lane's column
-  if (n_parts == 1) {
-    const float inv = st.l > 0.f ? 1.f / st.l : 0.f;
-    bf16* o = out + (size_t)t * ldo + (size_t)head * rank;
+  const float inv = st.l > 0.f ? 1.f / st.l : 0.f;
+  bf16* o = out + (size_t)t * ldo + (size_t)head * rank;
 #pragma unroll
-    for (int dt = 0; dt < RT; ++dt) {
-      if (EXACT || dt * 16 < rank) {
-        bf16x4 r = {(bf16)(st.acc[dt][0] * inv), (bf16)(st.acc[dt][1] * inv), (bf16)(st.acc[dt][2] * inv), (bf16)(st.acc[dt][3] * inv)};
-        *reinterpret_cast<bf16x4*>(o + dt * 16 + grp * 4) = r;
-      }
-    }
-  } else {
-    float* w = ws + (((size_t)t * nheads + head) * n_parts + part) * (rank + 4);
-    if (grp == 0) w[0] = st.m, w[1] = st.l;
-#pragma unroll
-    for (int dt = 0; dt < RT; ++dt) {
-      if (EXACT || dt * 16 < rank) *reinterpret_cast<f32x4*>(w + 4 + dt * 16 + grp * 4) = st.acc[dt];
+  for (int dt = 0; dt < RT; ++dt) {
+    if (EXACT || dt * 16 < rank) {
+      bf16x4 r = {(bf16)(st.acc[dt][0] * inv), (bf16)(st.acc[dt][1] * inv), (bf16)(st.acc[dt][2] * inv), (bf16)(st.acc[dt][3] * inv)};
+      *reinterpret_cast<bf16x4*>(o + dt * 16 + grp * 4) = r;
     }
   }
+}
+
+// What a block of single tokens leaves, whose four waves had a share of the keys each: they meet in LDS (`lds`: 4 x 16 rows of
+// RT * 16 + 4 floats, in the place of the queries), and the block leaves one part: maximum, sum and unnormalised result, or with
+// no other part the result itself.  (A part a wave was 34 MB to write and to read again for 32 tokens of 16 heads.)  `used`: the
+// waves that had any keys, the first ones.
+template <int RT, int WC, bool EXACT>
+__device__ __forceinline__ void latent_meet(LatentState<RT, WC>& st, float* __restrict__ lds, bf16* __restrict__ out, long ldo,
+                                            float* __restrict__ ws, int t, int head0, int nheads, int rank, int n_parts, int part,
+                                            int used) {
+  constexpr int ROW = RT * 16 + 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+  st.l += __shfl_xor(st.l, 16, WAVE);
+  st.l += __shfl_xor(st.l, 32, WAVE);
+  __syncthreads();  // the queries have been read
+  float* row = lds + (wave * 16 + col) * ROW;
+  if (wave < used) {
+#pragma unroll
+    for (int dt = 0; dt < RT; ++dt)
+      if (EXACT || dt * 16 < rank) *reinterpret_cast<f32x4*>(row + dt * 16 + grp * 4) = st.acc[dt];
+    if (grp == 0) row[RT * 16] = st.m, row[RT * 16 + 1] = st.l;
+  }
+  __syncthreads();
+  // a wave takes the same quarter of every column
+#pragma unroll
+  for (int n = 0; n < RT / 4; ++n) {
+    const int at = n * 64 + lane, c = at / RT, d = (wave * RT + at % RT) * 4;
+    if (head0 + c >= nheads || (!EXACT && d >= rank)) continue;
+    float m[4], top = LAT_EMPTY, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m[w] = w < used ? lds[(w * 16 + c) * ROW + RT * 16] : LAT_EMPTY, top = fmaxf(top, m[w]);
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (w >= used) break;
+      const float e = __expf(m[w] - top);
+      l = fmaf(lds[(w * 16 + c) * ROW + RT * 16 + 1], e, l);
+      sum += *reinterpret_cast<const f32x4*>(lds + (w * 16 + c) * ROW + d) * e;
+    }
+    if (n_parts == 1) {
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+      const bf16x4 r = {(bf16)(sum[0] * inv), (bf16)(sum[1] * inv), (bf16)(sum[2] * inv), (bf16)(sum[3] * inv)};
+      *reinterpret_cast<bf16x4*>(out + (size_t)t * ldo + (size_t)(head0 + c) * rank + d) = r;
+    } else {
+      float* o = ws + (((size_t)t * nheads + head0 + c) * n_parts + part) * (rank + 4);
+      *reinterpret_cast<f32x4*>(o + 4 + d) = sum;
+      if (d == 0) o[0] = top, o[1] = l;
+    }
+  }
+}
+
+// The (token, 16 heads) and the part of its keys that a block of a decode step works on, where the parts of all tokens at the
+// context bound would be more blocks than the chip holds at once.  What bounds these blocks is what a compute unit takes in (27
+// to 38 GB/s, 68 KB for 32 keys of a latent of 512 + 64), beside some ten microseconds a block for its queries and its result; so
+// every block gets the same share of tiles of 32 keys, and the share is what spreads all tiles of the step, by the contexts as
+// they are, over one round of blocks: long contexts over many of them, short ones over few.  64 sequences of 128 to 2048 tokens
+// 41 us, with four blocks for each of them 47 (52 with as many and a part a wave); 32 sequences 31 either way (36); up to 16,
+// where a block for every four tiles at the bound fits, 26 with shares and 24 without (32).
+// Returns the tile of 16 heads (-1: a block too many), its part and the share; a padding row gets one block.  At most 256
+// (token, 16 heads); scratch: 12 numbers.
+#define LAT_DEAL_TOKENS 256
+__device__ __forceinline__ int deal_tiles(const int* __restrict__ positions, const int* __restrict__ seq_of_token, int n_tokens,
+                                          int tiles_per_token, int window, int n_parts, int* scratch, int* part, int* share) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = threadIdx.x;
+  const int n_tiles = n_tokens * tiles_per_token;
+  int keys = 0;
+  if (i < n_tiles) {
+    const int t = i / tiles_per_token, p = positions[t];
+    if (seq_of_token[t] >= 0) keys = p / 32 + 1 - (window > 0 && p - window + 1 > 0 ? (p - window + 1) / 32 : 0);
+  }
+  int sum = keys, most = keys;
+#pragma unroll
+  for (int off = WAVE / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, WAVE), most = max(most, __shfl_xor(most, off, WAVE));
+  if (lane == 0) scratch[wave] = sum, scratch[4 + wave] = most;
+  __syncthreads();
+  sum = scratch[0] + scratch[1] + scratch[2] + scratch[3];
+  most = max(max(scratch[4], scratch[5]), max(scratch[6], scratch[7]));
+  const int blocks = 256 - n_tiles / 2;  // every one's last block is half empty
+  int s = (sum + blocks - 1) / blocks;
+  s = max(max(s, 4), (most + n_parts - 1) / n_parts);
+  const int mine = i < n_tiles ? max((keys + s - 1) / s, 1) : 0;  // blocks
+  int upto = mine;                                               // and those of the tiles before it
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const int other = __shfl_up(upto, off, WAVE);
+    if (lane >= off) upto += other;
+  }
+  __syncthreads();  // the sums have been read
+  if (lane == 63) scratch[wave] = upto;
+  if (i == 0) scratch[8] = -1, scratch[9] = 0;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) upto += scratch[w];
+  const int k = blockIdx.x;
+  if (mine > 0 && upto - mine <= k && k < upto) scratch[8] = i, scratch[9] = k - (upto - mine);
+  __syncthreads();
+  const int tile = __builtin_amdgcn_readfirstlane(scratch[8]);
+  *part = __builtin_amdgcn_readfirstlane(scratch[9]), *share = __builtin_amdgcn_readfirstlane(s);
+  __syncthreads();  // the scratch is the caller's again
+  return tile;
 }
 
 // LDS: the four waves of a block (four consecutive tiles of one sequence: neighbouring tokens, or the head groups of
@@ -489,13 +603,15 @@ __global__ void __launch_bounds__(256)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int n_tiles = n_tokens * tiles_per_token;
-  int tile, part;
-  if (n_parts == 1) {
-    tile = blockIdx.x * 4 + wave;
-    part = 0;
-  } else {
-    tile = blockIdx.x;
-    part = blockIdx.y * 4 + wave;
+  // prompts: four tiles a block; single tokens (!LDS): one, whose keys up to n_parts blocks share, and their waves
+  int tile = LDS ? blockIdx.x * 4 + wave : blockIdx.x, block_part = 0, share = 0x10000000;
+  if constexpr (!LDS) {
+    if (n_parts > 1 && gridDim.y == n_parts) {
+      block_part = blockIdx.y, share = 4;
+    } else if (n_parts > 1) {
+      tile = deal_tiles(positions, seq_of_token, n_tokens, tiles_per_token, window, n_parts, reinterpret_cast<int*>(lds), &block_part, &share);
+      if (tile < 0) return;
+    }
   }
   // do the block's four tiles share their keys?  (every wave works that out for itself, and all agree)
   bool together = false;
@@ -536,24 +652,45 @@ __global__ void __launch_bounds__(256)
   }
   const int lo = window > 0 ? (pos - window + 1 > 0 ? pos - window + 1 : 0) : 0;
 
-  // The wave's queries wait in LDS, each lane's eight elements of every step of K in a slot of its own (written and
-  // read by the same lane: no barrier): in registers they would crowd out the loads that have to be in flight.
+  // single tokens: the block's keys are tiles first .. end - 1, `share` of them as far as there are
+  int first = lo / 32, end = pos / 32 + 1, used = 4;  // used: the waves that have keys to work on, the first ones
+  if constexpr (!LDS) {
+    const int least = (end - first + n_parts - 1) / n_parts;
+    share = share > least ? share : least;
+    const int parts = (end - first + share - 1) / share;
+    if (n_parts > 1 && block_part == 0) {  // what the merge passes by
+      for (int i = parts + wave * 4 + grp; i < n_parts; i += 16)
+        if (head < nheads) {
+          float* w = ws + (((size_t)t * nheads + head) * n_parts + i) * (rank + 4);
+          w[0] = LAT_EMPTY, w[1] = 0.f;
+        }
+    }
+    first += block_part * share;
+    end = end < first + share ? end : first + share;
+    used = end - first < 4 ? end - first : 4;
+    if (used <= 0) return;
+  }
+  // The queries wait in LDS, each lane's eight elements of every step of K in a slot: in registers they would crowd out
+  // the loads that have to be in flight.  A prompt's wave has its own (written and read by the same lane: no barrier), the
+  // waves of a single token share them.
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  bf16* q_lds = lds + ((size_t)wave * WC * 64 + lane) * 8;
+  bf16* q_lds = lds + ((size_t)(LDS ? wave * WC * 64 : 0) + lane) * 8;
   {
     const bf16* qrow = qa + (size_t)t * ldq + (size_t)(valid ? head : 0) * width;
 #pragma unroll
     for (int c = 0; c < WC; ++c) {
+      if (!LDS && (c & 3) != wave) continue;
       const int k = c * 32 + grp * 8;
       *reinterpret_cast<bf16x8*>(q_lds + c * 64 * 8) = (valid && (EXACT || k < width)) ? *reinterpret_cast<const bf16x8*>(qrow + k) : zero8;
     }
   }
+  if constexpr (!LDS) __syncthreads();
   auto load_q = [&](int c) { return *reinterpret_cast<const bf16x8*>(q_lds + c * 64 * 8); };
   LatentState<RT, WC> st;
 #pragma unroll
   for (int dt = 0; dt < RT; ++dt) st.acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   st.m = (sink && valid) ? sink[head] : LAT_EMPTY;
-  st.l = (sink && valid && part == 0 && grp == 0) ? 1.f : 0.f;
+  st.l = (sink && valid && (LDS || (block_part == 0 && wave == 0)) && grp == 0) ? 1.f : 0.f;
   const int key_a = 8 * (col >> 2) + (col & 3);  // the key of this lane's row in score tile a; tile b: + 4
 
   if (LDS && together) {
@@ -640,14 +777,16 @@ __global__ void __launch_bounds__(256)
     }
   } else {
     const int* bt = block_table + (size_t)seq * table_stride;
-    for (int kt = lo / 32 + part; kt * 32 <= pos; kt += n_parts) {
+    for (int kt = first + (LDS ? 0 : wave); kt < end; kt += LDS ? 1 : 4) {
       const int base = kt * 32;
       const size_t page = readable_page(uniform_load(bt + base / PAGE_TOKENS));
       const int in_page = base % PAGE_TOKENS;
       const bf16* ka = cache + (page * PAGE_TOKENS + in_page + key_a) * width + grp * 8;
       const bf16* vt = vt_cache + (page * rank + col) * PAGE_TOKENS + in_page + grp * 8;
-      // straight from global memory: half a tile of key loads, then half its latent loads, in flight at once (all of them up to medium sizes)
-      latent_tile<RT, WC, (WC <= 10 ? WC : (WC % 8 == 0 ? 8 : 9)), (RT <= 16 ? RT : 16), EXACT>(
+      // straight from global memory (guarded products of the largest sizes, and blocks of a prompt whose tiles lie in several
+      // sequences, have no registers for loads that far ahead)
+      constexpr bool AHEAD = !LDS && (EXACT || RT <= 16);
+      latent_tile<RT, WC, (!AHEAD && WC > 10 ? (WC % 8 == 0 ? 8 : 9) : WC), (AHEAD && RT > 8 ? 8 : RT <= 16 ? RT : 16), EXACT, AHEAD>(
           st, load_q,
           [&](int which, int c) {
             return (EXACT || c * 32 + grp * 8 < width) ? *reinterpret_cast<const bf16x8*>(ka + which * 4 * (size_t)width + c * 32) : zero8;
@@ -656,7 +795,8 @@ __global__ void __launch_bounds__(256)
           grp);
     }
   }
-  latent_finish<RT, WC, EXACT>(st, out, ldo, ws, t, head, nheads, rank, n_parts, part, grp);
+  if constexpr (LDS) latent_finish<RT, WC, EXACT>(st, out, ldo, t, head, nheads, rank, grp);
+  else latent_meet<RT, WC, EXACT>(st, reinterpret_cast<float*>(lds), out, ldo, ws, t, tile % tiles_per_token * 16, nheads, rank, n_parts, block_part, used);
 }
 
 // --------------------------------------------------------------------------
@@ -889,17 +1029,18 @@ __global__ void __launch_bounds__(256, 1)
 #pragma unroll
   for (int d = 0; d < RT; ++d) st.acc[d] = acc[d];
   st.m = m, st.l = l;
-  latent_finish<RT, WC, true>(st, out, ldo, nullptr, t, head, nheads, RANK, 1, 0, grp);
+  latent_finish<RT, WC, true>(st, out, ldo, t, head, nheads, RANK, grp);
 }
 
 // out[t, h, :] = sum_i acc_i exp(m_i - M) / sum_i l_i exp(m_i - M) over the parts i.  The parts' maxima and sums are
 // loaded side by side (a thread a part) and their weights left in LDS: no chain of dependent loads.
-#define LAT_MAX_PARTS 256
+#define LAT_MAX_PARTS 64
 __global__ void __launch_bounds__(256)
     latent_attn_merge_kernel(const float* __restrict__ ws, bf16* __restrict__ out, long ldo, const int* __restrict__ seq_of_token,
                              int nheads, int rank, int n_parts) {
   __shared__ float weight[LAT_MAX_PARTS];
   __shared__ float inv_total;
+  __shared__ int n_used;  // the parts that have keys: the first ones
   const int h = blockIdx.x, t = blockIdx.y;
   bf16* o = out + (size_t)t * ldo + (size_t)h * rank;
   if (seq_of_token[t] < 0) {
@@ -908,31 +1049,31 @@ __global__ void __launch_bounds__(256)
   }
   const float* w = ws + ((size_t)t * nheads + h) * n_parts * (rank + 4);
   if (threadIdx.x < WAVE) {  // the first wave weighs the parts
-    float top = LAT_EMPTY;
-    for (int i = threadIdx.x; i < n_parts; i += WAVE) top = fmaxf(top, w[(size_t)i * (rank + 4)]);
-    top = wave_max(top);
-    float total = 0.f;
-    for (int i = threadIdx.x; i < n_parts; i += WAVE) {
-      const float e = __expf(w[(size_t)i * (rank + 4)] - top);
-      weight[i] = e;
-      total += w[(size_t)i * (rank + 4) + 1] * e;
-    }
-    total = wave_sum(total);
-    if (threadIdx.x == 0) inv_total = total > 0.f ? 1.f / total : 0.f;
+    float top;
+    const int i = threadIdx.x;  // n_parts <= 64: a part a lane
+    const float m = i < n_parts ? w[(size_t)i * (rank + 4)] : LAT_EMPTY, l = i < n_parts ? w[(size_t)i * (rank + 4) + 1] : 0.f;
+    const bool counts = m > 0.5f * LAT_EMPTY || m != m;
+    top = wave_max(m);
+    const float e = __expf(m - top);
+    if (i < n_parts) weight[i] = e;
+    const float total = wave_sum(counts ? l * e : 0.f);
+    const unsigned long long mask = __ballot(counts);
+    if (i == 0) inv_total = total > 0.f ? 1.f / total : 0.f, n_used = mask == 0 ? 0 : 64 - __clzll(mask);
   }
   __syncthreads();
   const float inv = inv_total;
+  const int used = n_used;
   for (int d = threadIdx.x; d < rank; d += blockDim.x) {
     float v = 0.f;
 #pragma unroll 8
-    for (int i = 0; i < n_parts; ++i) v = fmaf(w[(size_t)i * (rank + 4) + 4 + d], weight[i], v);
+    for (int i = 0; i < used; ++i) v = fmaf(w[(size_t)i * (rank + 4) + 4 + d], weight[i], v);
     o[d] = (bf16)(v * inv);
   }
 }
 
-// bytes of the workspace for n_splits blocks of four parts each (0: one block per four tiles, no workspace)
+// bytes of the workspace for n_splits blocks, a part each (0: one block per four tiles; neither that nor one block need any)
 extern "C" long fmsamd_latent_attn_workspace(int n_tokens, int nheads, int rank, int n_splits) {
-  return n_splits <= 0 ? 0 : (long)n_tokens * nheads * n_splits * 4 * (rank + 4) * (long)sizeof(float);
+  return n_splits <= 1 ? 0 : (long)n_tokens * nheads * n_splits * (rank + 4) * (long)sizeof(float);
 }
 
 // 1 if the MFMA kernel takes these sizes
@@ -953,18 +1094,21 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
               n_tokens, nheads, rank, rot);
   FMS_REQUIRE(ldq >= (long)nheads * width && ldq % 8 == 0 && ldo >= (long)nheads * rank && ldo % 4 == 0 && ((uintptr_t)qa % 16) == 0,
               "latent_attn_mfma: rows too short or not aligned");
-  FMS_REQUIRE(cache != nullptr && vt_cache != nullptr && window >= 0 && n_splits >= 0 && n_splits * 4 <= LAT_MAX_PARTS, "latent_attn_mfma: bad arguments (at most 64 splits)");
+  FMS_REQUIRE(cache != nullptr && vt_cache != nullptr && window >= 0 && n_splits >= 0 && n_splits <= LAT_MAX_PARTS, "latent_attn_mfma: bad arguments (at most 64 splits)");
   const int tiles_per_token = ceil_div(nheads, 16);
   const long tiles = (long)n_tokens * tiles_per_token;
-  const int n_parts = n_splits == 0 ? 1 : n_splits * 4;
-  FMS_REQUIRE(n_splits == 0 || (workspace != nullptr && workspace_bytes >= fmsamd_latent_attn_workspace(n_tokens, nheads, rank, n_splits)),
+  if (tiles > LAT_DEAL_TOKENS && n_splits > 1) n_splits = 1;  // a block each fills the chip
+  const int n_parts = n_splits == 0 ? 1 : n_splits;
+  FMS_REQUIRE(n_splits <= 1 || (workspace != nullptr && workspace_bytes >= fmsamd_latent_attn_workspace(n_tokens, nheads, rank, n_splits)),
               "latent_attn_mfma: the workspace is too small");
-  const dim3 grid(n_splits == 0 ? ceil_div(tiles, 4) : (unsigned)tiles, n_splits == 0 ? 1 : n_splits);
-  FMS_REQUIRE(tiles <= 0x7fffffffL && grid.y <= 65535, "latent_attn_mfma: too many tiles for one launch");
+  // with splits, a block for every share of at most 256 - tiles / 2 and for every tile's last one
+  const bool deal = n_splits > 1 && tiles * n_splits > 256;
+  const dim3 grid(n_splits == 0 ? ceil_div(tiles, 4) : deal ? min(256 + (tiles + 1) / 2, tiles * n_splits) : tiles, deal || n_splits == 0 ? 1 : n_splits);
+  FMS_REQUIRE(tiles <= 0x7fffffffL, "latent_attn_mfma: too many tiles for one launch");
   // LDS: every wave's queries; for prompts also a tile of 32 key rows and the same keys' latent, transposed, which the
   // waves of a block share
 #define LAUNCH_LATENT(RT, WC, EXACT)                                                                                               \
-  const size_t q_lds = (size_t)4 * WC * 64 * 8 * sizeof(bf16); /* the four waves' queries */                                       \
+  const size_t q_lds = (size_t)4 * WC * 64 * 8 * sizeof(bf16); /* the four waves' queries of a prompt */                           \
   const size_t lds = q_lds + (size_t)(32 * (width + 8) + rank * 40) * sizeof(bf16);                                                \
   static bool allowed = false; /* more than 64 KB of LDS a block has to be asked for, once a kernel */                             \
   if (!allowed) {                                                                                                                  \
@@ -976,13 +1120,14 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
                 hipGetErrorString(e1 != hipSuccess ? e1 : e2));                                                                    \
     allowed = true;                                                                                                                \
   }                                                                                                                                \
-  FMS_REQUIRE(lds <= 160 * 1024, "latent_attn_mfma: %zu bytes of LDS", lds);                                                       \
+  const size_t meet = (size_t)4 * 16 * (RT * 16 + 4) * sizeof(float); /* where the waves of a single token meet */                 \
+  FMS_REQUIRE(lds <= 160 * 1024 && meet <= 160 * 1024, "latent_attn_mfma: %zu bytes of LDS", lds);                                 \
   if (n_splits == 0)                                                                                                               \
     latent_attn_mfma_kernel<RT, WC, true, EXACT><<<grid, 256, lds, stream>>>(                                                      \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
         (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts);  \
   else                                                                                                                             \
-    latent_attn_mfma_kernel<RT, WC, false, EXACT><<<grid, 256, q_lds, stream>>>(                                                   \
+    latent_attn_mfma_kernel<RT, WC, false, EXACT><<<grid, 256, meet > q_lds / 4 ? meet : q_lds / 4, stream>>>(                                                   \
         (const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, seq_of_token, block_table, table_stride,              \
         (const bf16*)cache, (const bf16*)vt_cache, sink, n_tokens, nheads, rank, width, scale, window, tiles_per_token, n_parts)
   // prompts with a latent of 512 (the rows go straight to LDS, which wants 16-byte addresses)

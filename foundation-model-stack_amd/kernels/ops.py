@@ -1051,11 +1051,12 @@ def latent_attention_fits_mfma(rank: int, rot: int) -> bool:
 
 
 def latent_attention_splits(n_tokens: int, nheads: int, max_context: int) -> int:
-    """How many blocks share one (token, 16 heads) of the decode step of the MFMA kernel: enough for some 256 blocks in
-    all (one a compute unit), no wave with fewer than two tiles of 32 keys at the context bound, at most 32 (every
-    part's result goes through the workspace and is merged)."""
+    """Into how many parts at most the keys of a (token, 16 heads) of a decode step are cut: no block of four waves with fewer
+    than four tiles of 32 keys at the context bound, and one round of 256 blocks in all.  From 17 (token, 16 heads) on, twice as
+    many parts: the kernel then spreads the tiles by the contexts as they are."""
     tiles = n_tokens * -(-nheads // 16)
-    return max(1, min(-(-256 // tiles), -(-max_context // 32) // 8, 32))
+    most = 256 // tiles if tiles <= 16 else -(-512 // tiles)
+    return max(1, min(most, -(-max_context // 128), 64)) if tiles <= 256 else 1
 
 
 def _check_tables(cos, sin, rot: int) -> int:

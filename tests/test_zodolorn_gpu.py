@@ -901,3 +901,37 @@ def test_a_model_from_the_registry_alone(lib):
     alone = Engine(model, max_tokens=256, max_slots=1)
     s = alone.new_sequence()
     torch.testing.assert_close(alone.step([s], [[5, 6, 7]], "last"), logits[1:], atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("tokens, heads, sizes, window", [(1, 16, (512, 64), 0), (16, 16, (512, 64), 0), (17, 16, (512, 64), 700), (9, 33, (64, 16), 0),
+                                                          (40, 16, (256, 64), 0), (129, 16, (128, 0), 90), (300, 16, (64, 16), 0)])
+def test_latent_attention_of_unequal_contexts(lib, tokens, heads, sizes, window):
+    """Decode steps around the numbers of tokens where the kernel's blocks are dealt out another way: contexts of one token, of
+    whole tiles and one beside, and of the bound, a padding row in their middle; beside the same in 64 bits."""
+    from fms_amd.kernels import ops
+
+    rank, rot = sizes
+    bound, pool = 2304, 40
+    gen = torch.Generator().manual_seed(tokens)
+    contexts = torch.randint(1, bound, (tokens,), generator=gen)
+    for i, n in enumerate((bound, 1, 32, 33, 128, 129, 0, 64)):
+        if i < tokens:
+            contexts[i] = n  # 0: a padding row
+    cache = (torch.randn(pool, 1, 64, rank + rot, generator=gen)).bfloat16()
+    table = torch.stack([torch.randperm(pool, generator=gen)[: bound // 64] for _ in range(tokens)]).to(torch.int32)
+    qa = (0.3 * torch.randn(tokens, heads * (rank + rot), generator=gen)).bfloat16()
+    sink = torch.randn(heads, generator=gen)
+    seq = torch.where(contexts > 0, torch.arange(tokens), torch.full((tokens,), -1)).to(torch.int32)
+    got = ops.latent_attention(qa.to(DEV), (contexts - 1).clamp(min=0).to(torch.int32).to(DEV), seq.to(DEV), table.to(DEV), cache.to(DEV), sink.to(DEV),
+                               heads, rank, rot, 0.05, window, decode=True, max_context=bound,
+                               vt_cache=cache[..., :rank].transpose(2, 3).contiguous().to(DEV)).float().cpu().view(tokens, heads, rank)
+    for t in range(tokens):
+        n = int(contexts[t])
+        if n == 0:
+            assert not bool(got[t].any())
+            continue
+        rows = cache[table[t].long(), 0].reshape(-1, rank + rot)[max(0, n - window) if window else 0 : n].double()
+        scores = torch.cat([torch.matmul(qa[t].view(heads, -1).double(), rows.T) * 0.05, sink[:, None].double()], dim=1)
+        want = torch.matmul(torch.softmax(scores, dim=1)[:, :-1], rows[:, :rank])
+        # probabilities and results rounded to 8 bits: 2^-9 each, of the sum and of its largest terms
+        assert float((got[t].double() - want).norm() / want.norm()) < 6e-3, (t, n)
