@@ -66,6 +66,51 @@ def test_add_norm(ops, width, dtype):
     torch.testing.assert_close(out3.cpu().float(), P.rms_norm(resid, weight.float(), eps), **tol(dtype))
 
 
+@pytest.mark.parametrize("heads, kvheads, dim, lens, contexts, window", [
+    (4, 4, 16, [64], [64], 0), (2, 1, 128, [97], [97], 0), (6, 3, 112, [33], [200], 50), (32, 8, 64, [15, 1, 130, 31], [15, 300, 130, 95], 0),
+    (32, 32, 48, [16, 40, 3], [16, 161, 257], 33)])
+def test_float32_prompt_attention(ops, heads, kvheads, dim, lens, contexts, window):
+    """The float32 prompt kernel beside 64 bits: rows of several sequences in a block, portions behind a cached context, windows,
+    a context that ends inside a tile; behind the contexts the cache holds what is no number.  Then a value that is no number
+    inside: only the queries that see it may show it."""
+    gen = torch.Generator().manual_seed(dim)
+    B, T, pages = len(lens), sum(lens), max(contexts) // 64 + 1
+    assert ops.f32_prompt_pays(T, heads, max(contexts), B)
+    k, v = torch.randn(B * pages, kvheads, 64, dim, generator=gen), torch.randn(B * pages, kvheads, dim, 64, generator=gen)
+    table = torch.randperm(B * pages, generator=gen).to(torch.int32).view(B, pages)
+    for b, n in enumerate(contexts):
+        page = int(table[b, n // 64])
+        k[page, :, n % 64 :], v[page, :, :, n % 64 :] = float("nan"), float("nan")
+    q = torch.randn(T, (heads + 2 * kvheads) * dim, generator=gen)
+    seq = torch.repeat_interleave(torch.arange(B), torch.tensor(lens)).to(torch.int32)
+    pos = torch.cat([torch.arange(c - n, c) for n, c in zip(lens, contexts)]).to(torch.int32)
+
+    def run(values):
+        return ops.attention(dev(q), dev(pos), dev(seq), dev(table), dev(k), dev(values), heads, kvheads, dim, dim ** -0.5, window,
+                             max_context=max(contexts)).cpu().view(T, heads, dim)
+
+    got = run(v)
+    for i in range(T):
+        b, hi = int(seq[i]), int(pos[i]) + 1
+        lo = max(0, hi - window) if window else 0
+        keys = k[table[b].long()].permute(0, 2, 1, 3).reshape(-1, kvheads, dim)[lo:hi].double().repeat_interleave(heads // kvheads, dim=1)
+        values = v[table[b].long()].permute(0, 3, 1, 2).reshape(-1, kvheads, dim)[lo:hi].double().repeat_interleave(heads // kvheads, dim=1)
+        p = torch.softmax((keys * q[i, : heads * dim].view(heads, dim).double()).sum(-1) * dim ** -0.5, dim=0)
+        # 24-bit sums of up to 300 terms of size one
+        torch.testing.assert_close(got[i].double(), (p[:, :, None] * values).sum(0), atol=3e-6, rtol=1e-5)
+    b = B - 1
+    j = contexts[b] - lens[b] // 2 - 1  # a token of the last sequence's own
+    broken = v.clone()
+    broken[int(table[b, j // 64]), 0, 3, j % 64] = float("inf")
+    got2 = run(broken)
+    sees = (seq == b) & (pos >= j) & ((pos - j < window) if window else torch.ones(T, dtype=torch.bool))
+    assert 0 < int(sees.sum()) < T
+    shown = torch.zeros(T, heads, dim, dtype=torch.bool)
+    shown[sees, : heads // kvheads, 3] = True
+    assert not bool(torch.isfinite(got2[shown]).any()) and bool(torch.isfinite(got2[~shown]).all())
+    torch.testing.assert_close(got2[~shown], got[~shown], atol=3e-6, rtol=1e-5)
+
+
 @pytest.mark.parametrize("rows, width, act, weight_type", [(1, 4, torch.bfloat16, torch.bfloat16), (3, 260, torch.float32, torch.float32),
                                                            (257, 2048, torch.bfloat16, torch.float32), (2, 16384, torch.float32, torch.bfloat16),
                                                            (5, 4096, torch.bfloat16, None)])
