@@ -98,6 +98,123 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
+// The same for prompts: a block takes 16 tokens and the channels of a q head and its k head, 256 value channels, or 256 decays (and
+// the betas).  A thread has a channel of all 16 tokens and asks for its inputs at once, each of them once (the kernel above
+// reads an input once for every tap, in eight passes of a block that has one token and all channels, and is bound by their
+// round trips: 2277 tokens of 4096 channels 63 us, 41 here; with a decay per channel 78 and 47).
+#define PREP_TOKENS 16
+template <typename W>
+__global__ void __launch_bounds__(256)
+    delta_prepare_tokens_kernel(const float* __restrict__ proj, long ld, int col_b, const float* __restrict__ a, long lda, int col_a,
+                                const W* __restrict__ conv_w, int taps, const float* __restrict__ a_log,
+                                const float* __restrict__ dt_bias, const float* __restrict__ conv_state,
+                                const int* __restrict__ seq_of_token, const int* __restrict__ slot_ids, float* __restrict__ qkv,
+                                float* __restrict__ beta, float* __restrict__ decay, float* __restrict__ kq, int n_tokens, int H, int G,
+                                int D, int Dv, int per_channel, float q_scale) {
+  extern __shared__ float y[];  // q and k of the block's tokens: [16][2 D + 4]
+  __shared__ int sq[PREP_TOKENS + DELTA_MAX_TAPS - 1];  // sequences, from the first token's earliest predecessor on
+  __shared__ float inv[2][PREP_TOKENS];
+  const int tb = blockIdx.x * PREP_TOKENS, tid = threadIdx.x, n = n_tokens - tb < PREP_TOKENS ? n_tokens - tb : PREP_TOKENS;
+  const int C = 2 * G * D + H * Dv, v_units = (H * Dv + 255) / 256;
+  int unit = blockIdx.y;
+  if (tid < PREP_TOKENS + DELTA_MAX_TAPS - 1) {
+    const int t = tb + tid - (DELTA_MAX_TAPS - 1);
+    sq[tid] = t >= 0 && t < n_tokens ? seq_of_token[t] : -2;
+  }
+  __syncthreads();
+  const int* own = sq + DELTA_MAX_TAPS - 1;  // own[i]: of token tb + i
+
+  if (unit >= G + v_units) {  // decays and betas
+    const int per = per_channel ? D : 1, c = (unit - G - v_units) * 256 + tid;
+    for (int i = 0; i < n; ++i) {
+      if (own[i] < 0) continue;
+      const size_t t = tb + i;
+      if (unit == G + v_units)
+        for (int h = tid; h < H; h += 256) beta[t * H + h] = sigmoid_f32(proj[t * ld + col_b + h]);
+      if (c < H * per) decay[t * H * per + c] = expf(-expf(a_log[c / per]) * softplus_f32(a[t * lda + col_a + c] + dt_bias[c]));
+    }
+    return;
+  }
+
+  bool one = true;  // all tokens and their predecessors are of one sequence
+  for (int i = 1 - taps; i < PREP_TOKENS; ++i) one = one && own[i] == own[0];
+  one = one && own[0] >= 0;
+  auto convolve = [&](int c, float (&out)[PREP_TOKENS]) {
+    float w[DELTA_MAX_TAPS];
+#pragma unroll
+    for (int j = 0; j < DELTA_MAX_TAPS; ++j) w[j] = j < taps ? to_f32(conv_w[(size_t)c * taps + j]) : 0.f;
+    if (one) {
+      float x[PREP_TOKENS + DELTA_MAX_TAPS - 1];  // x[r]: token tb + r - (taps - 1)
+      const float* row = proj + (size_t)(tb - (taps - 1)) * ld + c;
+#pragma unroll
+      for (int r = 0; r < PREP_TOKENS + DELTA_MAX_TAPS - 1; ++r) x[r] = r < PREP_TOKENS + taps - 1 ? row[(size_t)r * ld] : 0.f;
+#pragma unroll
+      for (int i = 0; i < PREP_TOKENS; ++i) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < DELTA_MAX_TAPS; ++j) acc = j < taps ? fmaf(w[j], x[i + j], acc) : acc;
+        out[i] = acc;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < PREP_TOKENS; ++i) {
+        out[i] = 0.f;
+        const int seq = own[i];
+        if (seq < 0) continue;  // uniform
+        int have = 0;           // predecessors in the step
+        while (have < taps - 1 && own[i - have - 1] == seq) ++have;
+        const float* state = conv_state + (size_t)slot_ids[seq] * (taps - 1) * C;
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < DELTA_MAX_TAPS; ++j) {
+          const int d = taps - 1 - j;
+          if (j < taps) acc = fmaf(w[j], d <= have ? proj[(size_t)(tb + i - d) * ld + c] : state[(size_t)(taps - 1 + have - d) * C + c], acc);
+        }
+        out[i] = acc;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PREP_TOKENS; ++i) out[i] = out[i] / (1.f + expf(-out[i]));
+  };
+
+  float out[PREP_TOKENS];
+  if (unit >= G) {  // values
+    const int c = (unit - G) * 256 + tid;
+    if (c >= H * Dv) return;
+    convolve(2 * G * D + c, out);
+#pragma unroll
+    for (int i = 0; i < PREP_TOKENS; ++i)
+      if (own[i] >= 0) qkv[(size_t)(tb + i) * C + 2 * G * D + c] = out[i];
+    return;
+  }
+  const int stride = 2 * D + 4;
+  for (int c = tid; c < 2 * D; c += 256) {
+    convolve((c < D ? 0 : G * D - D) + unit * D + c, out);
+#pragma unroll
+    for (int i = 0; i < PREP_TOKENS; ++i) y[i * stride + c] = out[i];
+  }
+  __syncthreads();
+  {
+    const int i = tid / 16, part = tid % 16;  // 16 lanes a token
+    const float *q = y + i * stride, *k = q + D;
+    float qq = 0.f, kk = 0.f, dot = 0.f;
+    for (int d = part; d < D; d += 16) qq = fmaf(q[d], q[d], qq), kk = fmaf(k[d], k[d], kk);
+    const float iq = q_scale / sqrtf(row16_sum(qq) + 1e-6f), ik = 1.f / sqrtf(row16_sum(kk) + 1e-6f);
+    for (int d = part; d < D; d += 16) dot = fmaf(q[d] * iq, k[d] * ik, dot);  // k . q of the finished vectors
+    dot = row16_sum(dot);
+    if (part == 0) {
+      inv[0][i] = iq, inv[1][i] = ik;
+      if (own[i] >= 0) kq[(size_t)(tb + i) * G + unit] = dot;
+    }
+  }
+  __syncthreads();
+  for (int c = tid; c < 2 * D; c += 256) {
+    const int col = (c < D ? 0 : G * D - D) + unit * D + c;
+    for (int i = 0; i < n; ++i)
+      if (own[i] >= 0) qkv[(size_t)(tb + i) * C + col] = y[i * stride + c] * inv[c < D ? 0 : 1][i];
+  }
+}
+
 // --------------------------------------------------------------------------
 // the recurrence
 // --------------------------------------------------------------------------
@@ -326,10 +443,24 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
   FMS_REQUIRE(seq_starts == nullptr || n_seqs > 0, "delta_prepare: no sequences");
   const size_t lds = (size_t)C * sizeof(float);
   const int threads = n_tokens <= 64 ? 1024 : 256;
+  // 16 tokens a block where there are more of them than a decode step has, and enough channels (C >= 4096: 65 tokens 19 us instead of
+  // 22, 40 sequences of 17 28 instead of 31; with 384 channels a block's chain of loads, sums and gates is longer than the other
+  // kernel's single pass, 20 us instead of 13)
+  const long units = kv_heads + (heads * (long)vdim + 255) / 256 + (heads * (long)(per_channel ? dim : 1) + 255) / 256;
+  const bool by_tokens = n_tokens > 64 && C >= 4096 && dim <= 256 && units <= 65535;
+  const dim3 grid(ceil_div(n_tokens, PREP_TOKENS), (unsigned)units);
+  const size_t token_lds = (size_t)PREP_TOKENS * (2 * dim + 4) * sizeof(float);
 #define FMS_PREP(W)                                                                                                   \
-  delta_prepare_kernel<W><<<n_tokens, threads, lds, stream>>>(proj, ld, col_b, a, lda, col_a, (const W*)conv_w, taps, a_log, \
-                                                          dt_bias, conv_state, seq_of_token, slot_ids, qkv, beta, decay, \
-                                                          kq, heads, kv_heads, dim, vdim, per_channel, q_scale)
+  do {                                                                                                                \
+    if (by_tokens)                                                                                                    \
+      delta_prepare_tokens_kernel<W><<<grid, 256, token_lds, stream>>>(proj, ld, col_b, a, lda, col_a, (const W*)conv_w, taps, a_log, \
+                                                                       dt_bias, conv_state, seq_of_token, slot_ids, qkv, beta, decay, \
+                                                                       kq, n_tokens, heads, kv_heads, dim, vdim, per_channel, q_scale); \
+    else                                                                                                              \
+      delta_prepare_kernel<W><<<n_tokens, threads, lds, stream>>>(proj, ld, col_b, a, lda, col_a, (const W*)conv_w, taps, a_log, \
+                                                                  dt_bias, conv_state, seq_of_token, slot_ids, qkv, beta, decay, \
+                                                                  kq, heads, kv_heads, dim, vdim, per_channel, q_scale); \
+  } while (0)
   if (conv_dtype == FMS_F32) FMS_PREP(float);
   else if (conv_dtype == FMS_BF16) FMS_PREP(bf16);
   else FMS_REQUIRE(false, "delta_prepare: unknown dtype %d", conv_dtype);

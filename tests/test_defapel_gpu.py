@@ -378,6 +378,47 @@ def test_delta_rule_in_runs(lib, sizes):
     assert not bool(torch.isfinite(got2[t, 0, 3])) and torch.equal(got2[~mine], got[~mine])
 
 
+@pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (16, 4, 256, 130, 8, True), (20, 20, 40, 130, 1, False), (33, 3, 24, 121, 3, True)])
+def test_delta_prepare_of_many_channels(lib, sizes):
+    """Blocks of 16 tokens: sequences that begin and end inside them, shorter than the convolution's reach and behind a state,
+    padding rows, the last block's remainder; beside the kernel that takes a token a block (which few tokens run)."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, taps, per_channel = sizes
+    C, per = 2 * G * D + H * V, D if per_channel else 1
+    assert C >= 4096
+    lens = [1, 30, 2, 17, 3, 33]
+    T = sum(lens)
+    gen = torch.Generator().manual_seed(T + D)
+    proj, a = torch.randn(T, C + H + 3, generator=gen).to(DEV), torch.randn(T, H * per + 2, generator=gen).to(DEV)
+    conv_w = (0.5 * torch.randn(C, taps, generator=gen)).to(DEV)
+    a_log, dt_bias = (torch.randn(H, generator=gen) - 1).to(DEV), torch.randn(H * per, generator=gen).to(DEV)
+    state = torch.randn(len(lens) + 1, max(taps - 1, 1), C, generator=gen).to(DEV)
+    slots = [5, 3, 0, 6, 1, 2]
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32)
+    seq[40:42] = -1  # padding
+    kept = seq >= 0
+
+    def run(rows, slot_ids, seqs, conv_state):
+        return ops.delta_prepare(proj[rows], C, a[rows], 1, conv_w, a_log, dt_bias, conv_state, seqs.to(DEV),
+                                 torch.tensor(slot_ids, dtype=torch.int32, device=DEV), H, G, D, V, per_channel, D ** -0.5)
+
+    whole_state = state.clone()
+    got = run(slice(0, T), slots, seq, whole_state)
+    want_state, at = state.clone(), 0
+    for b, n in enumerate(lens):  # a sequence alone: at most 33 tokens, a block each
+        rows = slice(at, at + n)
+        want = run(rows, [slots[b]], torch.where(kept[rows], 0, -1).to(torch.int32), want_state)
+        live = kept[rows].to(DEV)
+        if b != 3:  # the sequence with the padding rows inside is cut in two: its convolution starts anew behind them
+            for x, y in zip(got, want):
+                # 24-bit sums of up to 8 and 256 terms in two orders, through silu and a root
+                torch.testing.assert_close(x[rows][live], y[live], atol=2e-6, rtol=2e-6)
+        at += n
+    alone = [slots[b] for b in range(len(lens)) if b != 3]
+    assert torch.equal(whole_state[alone], want_state[alone])
+
+
 def test_a_lost_state_shows(lib):
     """The recurrence's memory matters: a value written long ago, read by a matching query much later, with decays near one."""
     from fms_amd.kernels import ops
