@@ -1,14 +1,19 @@
-// Attention of prompts in float32 on the matrix unit's float32 products (16x16x4): a block per 16 query rows of a head, whose
+// Attention in float32 on the matrix unit's float32 products (16x16x4): a block per 16 query rows of a head and sequence, whose
 // four waves take tiles of 32 keys in turn and meet in LDS.  S^T = K Q^T leaves keys 4 (lane / 16) + r
 // of a lane's query in register r, which is the operand layout of O^T = V^T P for a product that takes these four keys as its
 // four: nothing goes through LDS, and a lane's keys and values are 16 consecutive bytes (the steps of K are dealt the same way).
 //
-// A query's result has the same bits whatever rows stand beside it: keys are cut at absolute places, a tile that it does not
-// see changes nothing, and rows of several sequences take the sequences one after the other.
+// A query's result has the same bits whatever rows stand beside it, in a prompt, a portion or a decode step: keys are cut at
+// absolute places, and a tile that it does not see changes nothing.  So single tokens run here too, with one row of 16 in use:
+// the products they waste hide behind the keys and values.
 //
-// Bound by what a compute unit takes in: a head's keys and values once for every 16 queries.  301 tokens of 32 heads of 128:
-// 26 us, where the kernel with a block per token and head takes 175 (1000 tokens 152 and 1756).  The scores are sums of four
-// accumulators and the results of four waves: errors against 64 bits of 1.35e-7 and 2.6e-7.
+// Bound by what a compute unit takes in: a head's keys and values once for every 16 queries.  Microseconds, in brackets with a
+// block of FMAs per token and head: 301 tokens of 32 heads of 128 25 (175), 1000 tokens 151 (1752); one token behind 8, 64, 300,
+// 1000 and 4000 tokens 6.6, 6.8, 16, 41 and 161 (4.8, 6.5, 16, 47, 193); 64 single tokens behind 1000 each 388 (504).  (A branch
+// that leaves out a tile's second half where it has no key is 0.6 us faster for contexts up to 16 and a quarter slower beyond.)
+// 15 single tokens behind 2000 and a prompt of 64 197 (212), where a block that takes the sequences of its rows one after the other
+// needs a chain of 16 contexts.  The scores are sums of four
+// accumulators and the results of four waves: errors against 64 bits of 1.35e-7 and 2.6e-7 (301 tokens).
 #include "common.h"
 #include "fmsamd.h"
 
@@ -31,6 +36,7 @@ template <int NT>
 __global__ void __launch_bounds__(256, 2) attn_f32_kernel(AttnF32Args a) {
   constexpr int D = NT * 16, ROW = D + 4;
   __shared__ __attribute__((aligned(16))) float meet[4][16][ROW];
+  __shared__ bool theirs[16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, quad = lane >> 4;
   const int h = blockIdx.x, kh = h / (a.nheads / a.kvheads);
@@ -38,7 +44,18 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(AttnF32Args a) {
   const int n_rows = a.n_tokens - t0 < 16 ? a.n_tokens - t0 : 16;
   const bool there = col < n_rows;
   const int t = t0 + (there ? col : 0);
-  const int seq = there ? a.seq_of_token[t] : -1, pos = seq >= 0 ? a.positions[t] : -1;
+  const int seq = there ? a.seq_of_token[t] : -1;
+  // The block's sequence: the blockIdx.z-th of those of the 16 rows (rows without one go with the first block).  Contexts of
+  // several sequences side by side, not one behind the other; a block too many leaves after one round trip.
+  unsigned long long left = __ballot(seq >= 0 && lane < 16);
+  if (blockIdx.z > 0) {
+    for (int z = 0; z < (int)blockIdx.z && left != 0; ++z)
+      left &= ~__ballot(seq == __builtin_amdgcn_readlane(seq, __builtin_ctzll(left)));
+    if (left == 0) return;
+  }
+  const int turn = left != 0 ? __builtin_amdgcn_readlane(seq, __builtin_ctzll(left)) : 0;
+  const bool writes = there && (seq == turn || (seq < 0 && blockIdx.z == 0));
+  const int pos = seq >= 0 ? a.positions[t] : -1;
   const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
 
   f32x4 q[NT];
@@ -49,12 +66,9 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(AttnF32Args a) {
   for (int d = 0; d < NT; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = F32_ATTN_EMPTY, l = 0.f;
 
-  // one sequence after the other: of the rows whose sequence is `turn`, the keys from the first to the last that any sees
-  unsigned long long left = __ballot(seq >= 0);
-  while (left != 0) {
-    const int turn = __builtin_amdgcn_readlane(seq, __builtin_ctzll(left));
+  // of the rows whose sequence is `turn`, the keys from the first to the last that any sees
+  if (left != 0) {
     const bool mine = seq == turn;
-    left &= ~__ballot(mine);
     int last = mine ? pos : -1, first = mine ? lo : 0x7fffffff;
     int all_lo = mine ? lo : 0, all_pos = mine ? pos : -1;  // what every column sees (nothing, beside a row of another sequence)
 #pragma unroll
@@ -159,9 +173,11 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(AttnF32Args a) {
 #pragma unroll
   for (int d = 0; d < NT; ++d) *(f32x4*)&meet[wave][col][16 * d + 4 * quad] = acc[d];
   if (quad == 0) meet[wave][col][D] = m, meet[wave][col][D + 1] = l;
+  if (wave == 0 && quad == 0) theirs[col] = writes;
   __syncthreads();
   for (int x = threadIdx.x; x < n_rows * (D / 4); x += 256) {
     const int c = x / (D / 4), d = x % (D / 4) * 4;
+    if (!theirs[c]) continue;
     float top = F32_ATTN_EMPTY, sum = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) top = fmaxf(top, meet[w][c][D]);
@@ -180,9 +196,9 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(AttnF32Args a) {
 
 extern "C" int fmsamd_attn_f32(const float* q, long q_stride, float* out, long out_stride, const int* positions, const int* seq_of_token,
                                const int* block_table, int table_stride, const float* k_cache, const float* v_cache, int n_tokens,
-                               int nheads, int kvheads, int head_dim, float scale, int window, hipStream_t stream) {
+                               int n_seqs, int nheads, int kvheads, int head_dim, float scale, int window, hipStream_t stream) {
   if (n_tokens == 0) return 0;
-  FMS_REQUIRE(n_tokens > 0 && nheads > 0 && kvheads > 0 && nheads % kvheads == 0 && window >= 0, "attn_f32: bad sizes");
+  FMS_REQUIRE(n_tokens > 0 && n_seqs >= 0 && nheads > 0 && kvheads > 0 && nheads % kvheads == 0 && window >= 0, "attn_f32: bad sizes");
   FMS_REQUIRE(head_dim > 0 && head_dim % 16 == 0 && head_dim <= 128, "attn_f32: head size %d is no multiple of 16 up to 128", head_dim);
   FMS_REQUIRE(q_stride >= (long)nheads * head_dim && out_stride >= (long)nheads * head_dim && q_stride % 4 == 0 && out_stride % 4 == 0,
               "attn_f32: rows too short or not of whole 16 bytes");
@@ -190,7 +206,7 @@ extern "C" int fmsamd_attn_f32(const float* q, long q_stride, float* out, long o
   FMS_REQUIRE(ceil_div(n_tokens, 16) <= 65535, "attn_f32: %d tokens exceed one launch", n_tokens);
   AttnF32Args a{q, q_stride, out, out_stride, positions, seq_of_token, block_table, table_stride, k_cache, v_cache,
                 n_tokens, nheads, kvheads, window, scale};
-  const dim3 grid(nheads, ceil_div(n_tokens, 16));
+  const dim3 grid(nheads, ceil_div(n_tokens, 16), n_seqs < 1 ? 1 : n_seqs < 16 ? n_seqs : 16);
   switch (head_dim / 16) {
 #define FMS_AF(NT) case NT: attn_f32_kernel<NT><<<grid, 256, 0, stream>>>(a); break
     FMS_AF(1); FMS_AF(2); FMS_AF(3); FMS_AF(4); FMS_AF(5); FMS_AF(6); FMS_AF(7); FMS_AF(8);

@@ -91,11 +91,11 @@ int fmsamd_attn_generic(const void* q, long q_stride, void* out, long out_stride
                         const void* v_cache, int n_tokens, int nheads, int kvheads, int head_dim, float scale,
                         int window, const float* slopes, float soft_cap, int value_dim, int chunk, int keep_first,
                         const float* sink, const float* dist_bias, int dist_len, hipStream_t stream);
-// float32 attention without further terms on the matrix unit, for prompts (attention_f32.hip): head_dim a multiple of 16 up to
-// 128, rows and caches of whole 16 bytes at 16-byte addresses.
+// float32 attention without further terms on the matrix unit (attention_f32.hip): head_dim a multiple of 16 up to
+// 128, rows and caches of whole 16 bytes at 16-byte addresses.  n_seqs: rows of the block table.
 int fmsamd_attn_f32(const float* q, long q_stride, float* out, long out_stride, const int* positions, const int* seq_of_token,
-                    const int* block_table, int table_stride, const float* k_cache, const float* v_cache, int n_tokens, int nheads,
-                    int kvheads, int head_dim, float scale, int window, hipStream_t stream);
+                    const int* block_table, int table_stride, const float* k_cache, const float* v_cache, int n_tokens, int n_seqs,
+                    int nheads, int kvheads, int head_dim, float scale, int window, hipStream_t stream);
 
 // soft_cap (0: none) of the two bfloat16 kernels: scores become soft_cap * tanh(score / soft_cap); chunk and sink as in
 // fmsamd_attn_generic; so are keep_first and dist_bias (the prefill kernel has them for head sizes up to 64, and for 128).

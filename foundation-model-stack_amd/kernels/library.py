@@ -35,7 +35,7 @@ _SIGNATURES = {
     "fmsamd_bias_add": [P, I, P, I, I, I, P],
     "fmsamd_rope_table": [P, P, P, I, I, F, P],
     "fmsamd_rope_kv_write": [P, I, L, P, P, P, I, P, P, I, I, P, P, I, I, I, I, I, P],
-    "fmsamd_attn_f32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, F, I, P],
+    "fmsamd_attn_f32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P],
     "fmsamd_attn_generic": [P, L, P, L, I, P, P, P, I, P, P, I, I, I, I, F, I, P, F, I, I, I, P, P, I, P],
     "fmsamd_attn_prefill_bf16": [P, L, P, L, P, P, P, P, I, I, P, I, P, P, I, I, I, I, F, I, F, I, P, I, P, I, P],
     "fmsamd_attn_decode_bf16": [P, L, P, L, P, L, P, P, P, I, P, P, I, I, I, I, F, I, I, I, I, I, P, F, I, P, I, P, I, P],

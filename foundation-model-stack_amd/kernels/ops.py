@@ -450,9 +450,9 @@ def attention(
     c * tanh(s / c) first.  With slopes both types run the generic kernel (the MFMA kernels have no such term); the
     cap they have.
 
-    q is a [T, >= nheads*head_dim] view (the query columns of the qkv rows).  float32 runs the
-    generic kernel, and prompts of some size without further terms the float32 products of the matrix unit; bfloat16 runs the MFMA kernels (prefill needs the query blocks, decode the
-    largest context).  row_order (decode, optional): int32 [T], the token rows in the order in which the
+    q is a [T, >= nheads*head_dim] view (the query columns of the qkv rows).  float32 runs the float32 products of the
+    matrix unit, with further terms or head sizes that these do not take the generic kernel; bfloat16 runs the MFMA kernels
+    (prefill needs the query blocks, decode the largest context).  row_order (decode, optional): int32 [T], the token rows in the order in which the
     kernel's blocks are to take them, longest context first; the result does not depend on it.
     """
     _need_cuda(q, positions, seq_of_token, block_table, k_cache, v_cache)
@@ -484,14 +484,17 @@ def attention(
             raise ValueError(f"distance_bias must be a contiguous float32 [{nheads}, L] tensor")
         dist_len = distance_bias.shape[1]
     plain_scores = not keep_first and not chunk and not soft_cap and score_slopes is None and sink is None and distance_bias is None
-    if (q.dtype == torch.float32 and not decode and not force_generic and plain_scores and head_dim % 16 == 0 and head_dim <= 128
-            and not value_dim and q.stride(0) % 4 == 0 and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
-            and f32_prompt_pays(T, nheads, max_context or block_table.shape[1] * PAGE_TOKENS, block_table.shape[0])):
+    # The rule names nothing that differs between two steps of a model: a float32 row's result then has the same bits in a prompt,
+    # in portions, in a decode step and beside any other rows.  (Contexts of under some 30 tokens are 1 to 2 us slower than in the
+    # generic kernel, 64 rows of grouped heads behind 300 tokens 7 per cent; everything longer is as fast or faster, prompts up to ten times.)
+    if (q.dtype == torch.float32 and not force_generic and plain_scores and head_dim % 16 == 0 and head_dim <= 128
+            and not value_dim and q.stride(0) % 4 == 0 and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0):
         for t0 in range(0, T, 65520):
             n = min(65520, T - t0)
             check(lib.fmsamd_attn_f32(q[t0:].data_ptr(), q.stride(0), out[t0:].data_ptr(), out.stride(0), positions[t0:].data_ptr(),
                                       seq_of_token[t0:].data_ptr(), block_table.data_ptr(), block_table.stride(0), k_cache.data_ptr(),
-                                      v_cache.data_ptr(), n, nheads, kvheads, head_dim, float(scale), int(window), _stream()))
+                                      v_cache.data_ptr(), n, block_table.shape[0], nheads, kvheads, head_dim, float(scale), int(window),
+                                      _stream()))
         return out
     prefill_extras = bool(keep_first) or distance_bias is not None  # kept keys or a table: not every matrix-core kernel has them
     if (q.dtype == torch.float32 or force_generic or head_dim % 16 or score_slopes is not None or value_dim
@@ -548,17 +551,6 @@ def attention(
                                        k_cache.data_ptr(), v_cache.data_ptr(), *common_tail[:-1], float(soft_cap), chunk, _ptr(sink),
                                        keep_first, _ptr(distance_bias), dist_len, common_tail[-1]))
     return out
-
-
-def f32_prompt_pays(n_tokens: int, nheads: int, max_context: int, n_seqs: int) -> bool:
-    """Whether a float32 prompt runs on the matrix unit (a block per 16 rows and head, the sequences in it one after the other)
-    or with a block per token and head.  Microseconds of the two kernels, the second first: a prompt of 301 tokens and 32 heads
-    of 128 176 and 27, of 64 14.5 and 9, of 8 5.2 and 7.9, of 64 and 8 heads of 64 6.5 and 5.9; four prompts of 133 tokens
-    together 24.7 and 24 with 32 heads, 7 and 15 with 8; rows of 500 and 301 tokens of context 56 and 42 with 32 heads, 20 and 24
-    with 8."""
-    if n_seqs == 1:
-        return max_context >= 64
-    return n_tokens * nheads * max_context >= 400_000
 
 
 def decode_split(rows: int, n_pages: int):

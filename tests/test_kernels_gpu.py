@@ -75,7 +75,6 @@ def test_float32_prompt_attention(ops, heads, kvheads, dim, lens, contexts, wind
     inside: only the queries that see it may show it."""
     gen = torch.Generator().manual_seed(dim)
     B, T, pages = len(lens), sum(lens), max(contexts) // 64 + 1
-    assert ops.f32_prompt_pays(T, heads, max(contexts), B)
     k, v = torch.randn(B * pages, kvheads, 64, dim, generator=gen), torch.randn(B * pages, kvheads, dim, 64, generator=gen)
     table = torch.randperm(B * pages, generator=gen).to(torch.int32).view(B, pages)
     for b, n in enumerate(contexts):
@@ -109,6 +108,37 @@ def test_float32_prompt_attention(ops, heads, kvheads, dim, lens, contexts, wind
     shown[sees, : heads // kvheads, 3] = True
     assert not bool(torch.isfinite(got2[shown]).any()) and bool(torch.isfinite(got2[~shown]).all())
     torch.testing.assert_close(got2[~shown], got[~shown], atol=3e-6, rtol=1e-5)
+
+
+@pytest.mark.parametrize("heads, kvheads, dim, window", [(4, 4, 16, 0), (6, 2, 128, 0), (3, 1, 48, 37)])
+def test_float32_attention_has_the_same_bits_in_any_step(ops, heads, kvheads, dim, window):
+    """A float32 row's attention alone, in its whole prompt, in portions, in decode steps (with padding rows, beside more sequences
+    than a block has rows) and beside a long context: the same bits."""
+    gen = torch.Generator().manual_seed(dim)
+    contexts = [1, 7, 16, 17, 33, 70, 131] + [5 + 3 * i for i in range(12)] + [900]
+    B, pages = len(contexts), 15
+    k, v = dev(torch.randn(B * pages, kvheads, 64, dim, generator=gen)), dev(torch.randn(B * pages, kvheads, dim, 64, generator=gen))
+    table = dev(torch.randperm(B * pages, generator=gen).to(torch.int32).view(B, pages))
+    q = [dev(torch.randn(n, (heads + 2 * kvheads) * dim, generator=gen)) for n in contexts]
+
+    def run(pieces, decode=False):  # [(sequence or -1, first position, tokens)] -> the rows' results
+        ids = dev(torch.cat([torch.full((n,), b) for b, _, n in pieces]).to(torch.int32))
+        pos = dev(torch.cat([torch.arange(at, at + n) for _, at, n in pieces]).to(torch.int32))
+        rows = torch.cat([q[max(b, 0)][at : at + n] for b, at, n in pieces])
+        return ops.attention(rows, pos, ids, table, k, v, heads, kvheads, dim, dim ** -0.5, window, decode=decode, max_context=max(contexts)).cpu()
+
+    whole = [run([(b, 0, n)]) for b, n in enumerate(contexts)]
+    together = run([(b, 0, n) for b, n in enumerate(contexts)]).split(contexts)
+    for b, n in enumerate(contexts):
+        assert torch.equal(together[b], whole[b])
+        for cut in {1, n // 2, n - 1} - {0, n}:
+            assert torch.equal(run([(b, 0, cut)]), whole[b][:cut]) and torch.equal(run([(b, cut, n - cut)]), whole[b][cut:])
+    last = [(b, n - 1, 1) for b, n in enumerate(contexts)]
+    single = run(last[:9] + [(-1, 0, 1)] + last[9:], decode=True)
+    want = torch.cat([w[-1:] for w in whole])
+    assert torch.equal(torch.cat([single[:9], single[10:]]), want) and not bool(single[9].any())
+    mixed = run(last[7:] + [(5, 3, 60)])  # running sequences and a portion, in one step that is no decode step
+    assert torch.equal(mixed, torch.cat([want[7:], whole[5][3:63]]))
 
 
 @pytest.mark.parametrize("rows, width, act, weight_type", [(1, 4, torch.bfloat16, torch.bfloat16), (3, 260, torch.float32, torch.float32),
