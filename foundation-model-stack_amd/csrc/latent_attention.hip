@@ -364,6 +364,7 @@ extern "C" int fmsamd_latent_attn_generic(const void* qa, long ldq, void* out, l
 // The sink starts the maximum of every part and is counted in the sum of part 0 only.
 // --------------------------------------------------------------------------
 #define LAT_EMPTY -1e30f
+#define LAT_NO_KEYS -1.f  // the sum of a part without keys: a real one is no negative number
 
 // The state of a wave's 16 columns, and one tile of 32 keys worked into it.  load_k(which, c) gives this lane's eight
 // elements c * 32 + grp * 8 .. of its row of score tile a (which 0) or b (1); load_v(dt) its eight keys grp * 8 .. of
@@ -662,7 +663,7 @@ __global__ void __launch_bounds__(256)
       for (int i = parts + wave * 4 + grp; i < n_parts; i += 16)
         if (head < nheads) {
           float* w = ws + (((size_t)t * nheads + head) * n_parts + i) * (rank + 4);
-          w[0] = LAT_EMPTY, w[1] = 0.f;
+          w[0] = LAT_EMPTY, w[1] = LAT_NO_KEYS;
         }
     }
     first += block_part * share;
@@ -1052,7 +1053,7 @@ __global__ void __launch_bounds__(256)
     float top;
     const int i = threadIdx.x;  // n_parts <= 64: a part a lane
     const float m = i < n_parts ? w[(size_t)i * (rank + 4)] : LAT_EMPTY, l = i < n_parts ? w[(size_t)i * (rank + 4) + 1] : 0.f;
-    const bool counts = m > 0.5f * LAT_EMPTY || m != m;
+    const bool counts = i < n_parts && l != LAT_NO_KEYS;  // also where every score is no number: the maximum passes those by
     top = wave_max(m);
     const float e = __expf(m - top);
     if (i < n_parts) weight[i] = e;

@@ -935,3 +935,36 @@ def test_latent_attention_of_unequal_contexts(lib, tokens, heads, sizes, window)
         want = torch.matmul(torch.softmax(scores, dim=1)[:, :-1], rows[:, :rank])
         # probabilities and results rounded to 8 bits: 2^-9 each, of the sum and of its largest terms
         assert float((got[t].double() - want).norm() / want.norm()) < 6e-3, (t, n)
+
+
+@pytest.mark.parametrize("tokens, bound", [(1, 128), (1, 2048), (20, 2048), (300, 256)])
+def test_latent_attention_of_queries_that_are_no_number(lib, tokens, bound):
+    """A query that is no number shows in its own head and row and nowhere else, into however many parts the keys are cut (one,
+    sixteen, what a step of 20 tokens has, and one again); no sink, whose logit would be the maximum.  Padding rows stay zero."""
+    from fms_amd.kernels import ops
+
+    heads, rank, rot, pages = 16, 64, 16, bound // 64
+    gen = torch.Generator().manual_seed(bound + tokens)
+    cache = torch.randn(pages, 1, 64, rank + rot, generator=gen).bfloat16()
+    values = cache[..., :rank].transpose(2, 3).contiguous().to(DEV)
+    table = torch.arange(pages, dtype=torch.int32).repeat(tokens, 1)
+    qa = (0.3 * torch.randn(tokens, heads, rank + rot, generator=gen)).bfloat16()
+    positions = torch.randint(0, bound, (tokens,), generator=gen, dtype=torch.int32)
+    positions[0] = bound - 1
+    seq = torch.arange(tokens, dtype=torch.int32)
+    if tokens > 1:
+        seq[1] = -1
+
+    def run(q):
+        return ops.latent_attention(q.reshape(tokens, -1).to(DEV), positions.to(DEV), seq.to(DEV), table.to(DEV), cache.to(DEV), None, heads, rank,
+                                    rot, 0.05, decode=True, max_context=bound, vt_cache=values).cpu().view(tokens, heads, rank)
+
+    want = run(qa)
+    assert bool(torch.isfinite(want).all()) and not bool(want[seq < 0].any())
+    broken = qa.clone()
+    broken[0, 3, 5] = float("nan")
+    got = run(broken)
+    assert bool(torch.isnan(got[0, 3]).all())
+    mine = torch.zeros(tokens, heads, dtype=torch.bool)
+    mine[0, 3] = True
+    assert torch.equal(got[~mine], want[~mine])
