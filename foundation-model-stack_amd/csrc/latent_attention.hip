@@ -539,56 +539,6 @@ __device__ __forceinline__ void latent_meet(LatentState<RT, WC>& st, float* __re
   }
 }
 
-// The (token, 16 heads) and the part of its keys that a block of a decode step works on, where the parts of all tokens at the
-// context bound would be more blocks than the chip holds at once.  What bounds these blocks is what a compute unit takes in (27
-// to 38 GB/s, 68 KB for 32 keys of a latent of 512 + 64), beside some ten microseconds a block for its queries and its result; so
-// every block gets the same share of tiles of 32 keys, and the share is what spreads all tiles of the step, by the contexts as
-// they are, over one round of blocks: long contexts over many of them, short ones over few.  64 sequences of 128 to 2048 tokens
-// 41 us, with four blocks for each of them 47 (52 with as many and a part a wave); 32 sequences 31 either way (36); up to 16,
-// where a block for every four tiles at the bound fits, 26 with shares and 24 without (32).
-// Returns the tile of 16 heads (-1: a block too many), its part and the share; a padding row gets one block.  At most 256
-// (token, 16 heads); scratch: 12 numbers.
-#define LAT_DEAL_TOKENS 256
-__device__ __forceinline__ int deal_tiles(const int* __restrict__ positions, const int* __restrict__ seq_of_token, int n_tokens,
-                                          int tiles_per_token, int window, int n_parts, int* scratch, int* part, int* share) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = threadIdx.x;
-  const int n_tiles = n_tokens * tiles_per_token;
-  int keys = 0;
-  if (i < n_tiles) {
-    const int t = i / tiles_per_token, p = positions[t];
-    if (seq_of_token[t] >= 0) keys = p / 32 + 1 - (window > 0 && p - window + 1 > 0 ? (p - window + 1) / 32 : 0);
-  }
-  int sum = keys, most = keys;
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, WAVE), most = max(most, __shfl_xor(most, off, WAVE));
-  if (lane == 0) scratch[wave] = sum, scratch[4 + wave] = most;
-  __syncthreads();
-  sum = scratch[0] + scratch[1] + scratch[2] + scratch[3];
-  most = max(max(scratch[4], scratch[5]), max(scratch[6], scratch[7]));
-  const int blocks = 256 - n_tiles / 2;  // every one's last block is half empty
-  int s = (sum + blocks - 1) / blocks;
-  s = max(max(s, 4), (most + n_parts - 1) / n_parts);
-  const int mine = i < n_tiles ? max((keys + s - 1) / s, 1) : 0;  // blocks
-  int upto = mine;                                               // and those of the tiles before it
-#pragma unroll
-  for (int off = 1; off < WAVE; off <<= 1) {
-    const int other = __shfl_up(upto, off, WAVE);
-    if (lane >= off) upto += other;
-  }
-  __syncthreads();  // the sums have been read
-  if (lane == 63) scratch[wave] = upto;
-  if (i == 0) scratch[8] = -1, scratch[9] = 0;
-  __syncthreads();
-  for (int w = 0; w < wave; ++w) upto += scratch[w];
-  const int k = blockIdx.x;
-  if (mine > 0 && upto - mine <= k && k < upto) scratch[8] = i, scratch[9] = k - (upto - mine);
-  __syncthreads();
-  const int tile = __builtin_amdgcn_readfirstlane(scratch[8]);
-  *part = __builtin_amdgcn_readfirstlane(scratch[9]), *share = __builtin_amdgcn_readfirstlane(s);
-  __syncthreads();  // the scratch is the caller's again
-  return tile;
-}
-
 // LDS: the four waves of a block (four consecutive tiles of one sequence: neighbouring tokens, or the head groups of
 // one token) share every tile of keys through LDS, so a tile comes from the caches once a block instead of once a
 // wave; a block whose tiles lie in different sequences, and every block of a decode step, loads straight from
@@ -605,15 +555,7 @@ __global__ void __launch_bounds__(256)
   const int col = lane & 15, grp = lane >> 4;
   const int n_tiles = n_tokens * tiles_per_token;
   // prompts: four tiles a block; single tokens (!LDS): one, whose keys up to n_parts blocks share, and their waves
-  int tile = LDS ? blockIdx.x * 4 + wave : blockIdx.x, block_part = 0, share = 0x10000000;
-  if constexpr (!LDS) {
-    if (n_parts > 1 && gridDim.y == n_parts) {
-      block_part = blockIdx.y, share = 4;
-    } else if (n_parts > 1) {
-      tile = deal_tiles(positions, seq_of_token, n_tokens, tiles_per_token, window, n_parts, reinterpret_cast<int*>(lds), &block_part, &share);
-      if (tile < 0) return;
-    }
-  }
+  const int tile = LDS ? blockIdx.x * 4 + wave : blockIdx.x, block_part = LDS ? 0 : blockIdx.y;
   // do the block's four tiles share their keys?  (every wave works that out for itself, and all agree)
   bool together = false;
   int seq = -1, pos = -1, t = 0;
@@ -653,11 +595,13 @@ __global__ void __launch_bounds__(256)
   }
   const int lo = window > 0 ? (pos - window + 1 > 0 ? pos - window + 1 : 0) : 0;
 
-  // single tokens: the block's keys are tiles first .. end - 1, `share` of them as far as there are
+  // single tokens: the block's keys are tiles first .. end - 1, `share` of them as far as there are.  The cut goes by this token's
+  // own context and the number of parts, so that what the other rows of the step hold changes no bit.  (Shares that spread the
+  // tiles of all rows over one round of blocks by the contexts as they are take 31.5 us instead of 32.2 for 32 sequences of 128 to
+  // 2048 tokens, 16 heads, latent 512 + 64, and 41 instead of 47.5 for 64; where all have 2000, 40.5 instead of 34 and 63 instead of 58.)
   int first = lo / 32, end = pos / 32 + 1, used = 4;  // used: the waves that have keys to work on, the first ones
   if constexpr (!LDS) {
-    const int least = (end - first + n_parts - 1) / n_parts;
-    share = share > least ? share : least;
+    const int least = (end - first + n_parts - 1) / n_parts, share = n_parts > 1 && least < 4 ? 4 : least;  // a tile a wave
     const int parts = (end - first + share - 1) / share;
     if (n_parts > 1 && block_part == 0) {  // what the merge passes by
       for (int i = parts + wave * 4 + grp; i < n_parts; i += 16)
@@ -1098,13 +1042,10 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
   FMS_REQUIRE(cache != nullptr && vt_cache != nullptr && window >= 0 && n_splits >= 0 && n_splits <= LAT_MAX_PARTS, "latent_attn_mfma: bad arguments (at most 64 splits)");
   const int tiles_per_token = ceil_div(nheads, 16);
   const long tiles = (long)n_tokens * tiles_per_token;
-  if (tiles > LAT_DEAL_TOKENS && n_splits > 1) n_splits = 1;  // a block each fills the chip
   const int n_parts = n_splits == 0 ? 1 : n_splits;
   FMS_REQUIRE(n_splits <= 1 || (workspace != nullptr && workspace_bytes >= fmsamd_latent_attn_workspace(n_tokens, nheads, rank, n_splits)),
               "latent_attn_mfma: the workspace is too small");
-  // with splits, a block for every share of at most 256 - tiles / 2 and for every tile's last one
-  const bool deal = n_splits > 1 && tiles * n_splits > 256;
-  const dim3 grid(n_splits == 0 ? ceil_div(tiles, 4) : deal ? min(256 + (tiles + 1) / 2, tiles * n_splits) : tiles, deal || n_splits == 0 ? 1 : n_splits);
+  const dim3 grid(n_splits == 0 ? ceil_div(tiles, 4) : (unsigned)tiles, n_splits == 0 ? 1 : n_splits);
   FMS_REQUIRE(tiles <= 0x7fffffffL, "latent_attn_mfma: too many tiles for one launch");
   // LDS: every wave's queries; for prompts also a tile of 32 key rows and the same keys' latent, transposed, which the
   // waves of a block share

@@ -906,7 +906,7 @@ def test_a_model_from_the_registry_alone(lib):
 @pytest.mark.parametrize("tokens, heads, sizes, window", [(1, 16, (512, 64), 0), (16, 16, (512, 64), 0), (17, 16, (512, 64), 700), (9, 33, (64, 16), 0),
                                                           (40, 16, (256, 64), 0), (129, 16, (128, 0), 90), (300, 16, (64, 16), 0)])
 def test_latent_attention_of_unequal_contexts(lib, tokens, heads, sizes, window):
-    """Decode steps around the numbers of tokens where the kernel's blocks are dealt out another way: contexts of one token, of
+    """Decode steps of many, few and one part a token: contexts of one token, of
     whole tiles and one beside, and of the bound, a padding row in their middle; beside the same in 64 bits."""
     from fms_amd.kernels import ops
 
@@ -968,3 +968,27 @@ def test_latent_attention_of_queries_that_are_no_number(lib, tokens, bound):
     mine = torch.zeros(tokens, heads, dtype=torch.bool)
     mine[0, 3] = True
     assert torch.equal(got[~mine], want[~mine])
+
+
+@pytest.mark.parametrize("tokens", [3, 17, 40, 130])
+def test_latent_attention_of_a_row_does_not_depend_on_the_others(lib, tokens):
+    """As many rows, another context beside every second one: the rows that stayed have the same bits."""
+    from fms_amd.kernels import ops
+
+    heads, rank, rot, bound = 16, 128, 32, 2048
+    gen = torch.Generator().manual_seed(tokens)
+    cache = torch.randn(bound // 64, 1, 64, rank + rot, generator=gen).bfloat16()
+    values = cache[..., :rank].transpose(2, 3).contiguous().to(DEV)
+    table = torch.arange(bound // 64, dtype=torch.int32).repeat(tokens, 1).to(DEV)
+    qa = (0.3 * torch.randn(tokens, heads * (rank + rot), generator=gen)).bfloat16().to(DEV)
+    seq = torch.arange(tokens, dtype=torch.int32, device=DEV)
+    positions = torch.randint(0, 600, (tokens,), generator=gen, dtype=torch.int32)
+    positions[0] = 1900
+
+    def run(pos):
+        return ops.latent_attention(qa, pos.to(DEV), seq, table, cache.to(DEV), None, heads, rank, rot, 0.05, decode=True, max_context=bound, vt_cache=values)
+
+    want, others = run(positions), positions.clone()
+    for longer in (bound - 1, 0):
+        others[1::2] = longer
+        assert torch.equal(run(others)[::2], want[::2])
