@@ -12,32 +12,38 @@
 //
 // Two kernels.  delta_runs_prepare: everything that does not need the state (Y, W, G * Q, P, R_15 * K), a block per run and
 // head, so all runs at once; sums, decays and the triangular solve in 64 bits, every result rounded once to float32.
-// delta_runs: the chain over a sequence's runs, a block per (sequence, head, 16 value channels), in float32: a wave keeps a
-// quarter of S's rows in the accumulators of 16x16x4 products, which are the operand layout of the next product as they are
-// (register e of a lane is row 4 (lane / 16) + e: product e of a tile takes exactly these rows as its four).  What it
+// delta_runs: the chain over a sequence's runs, a block per (sequence, head, 16 value channels): W S0, (G * Q) S0 and P U in
+// float32, u and the update of S in 64 bits, S itself rounded to float32 once a run.  A wave keeps a
+// quarter of S's rows in registers as 16x16x4 products take and leave them (register e of a lane is row 4 (lane / 16) + e: product
+// e of a tile takes exactly these rows as its four; the 64-bit product leaves row 4 e + lane / 16 there, so that R_15 * K has its
+// rows in that order).  What it
 // multiplies is asked for two runs ahead, straight into registers, in the order in which the first kernel left it (the loads
 // stand among the products: all of them at a run's start cost 0.16 us a run).
 // Row r of a run's 16-row tiles is token 4 (r % 4) + r / 4: product e of a sum over the tokens then takes tokens 4 e to 4 e + 3,
 // so that sums grow from the oldest token (the one that the decays have made smallest) to the newest.
 //
-// Sequences of 777 and 1500 tokens, 16 heads of 128 by 128: 39 + 82 us (44 + 82 with a decay per key channel), where the kernel
-// that goes token by token takes 305 (350), bound by some 45 vector instructions a token.  The first kernel is near what its
-// 77 MB of results and 40 MB of inputs take; a run of the chain is 0.87 us, of which its 25 products a wave are 0.34 and the
-// rest is the way of the partial sums through LDS and what a compute unit takes in (without loads 0.76).
-// Errors against 64 bits (300 tokens, heads of 128 by 128), this kernel and the other one: outputs 5.6e-8 and 6.7e-8 for decays
-// around 0.5, 7.3e-8 and 9.9e-8 around 0.86, 1.4e-7 and 3.1e-7 around 0.999; the state 5.5e-8 and 5.2e-8, 7.2e-8 and 7.7e-8,
-// 1.4e-7 and 3.7e-7.
+// Sequences of 777 and 1500 tokens, 16 heads of 128 by 128: 132 us (138 with a decay per key channel), of which the first kernel
+// takes 39 (44), where the kernel that goes token by token takes 305 (350), bound by some 45 vector instructions a token.  The first
+// kernel is near what its 77 MB of results and 40 MB of inputs take; a run of the chain is 1 us, of which its 25 products a wave are
+// 0.45 and the rest is the way of the partial sums through LDS and what a compute unit takes in.
+// Errors against 64 bits (300 tokens, heads of 128 by 128), this kernel and the other one: outputs 5.5e-8 and 6.6e-8 for decays
+// around 0.5, 6.9e-8 and 9.8e-8 around 0.86, 1.2e-7 and 3.2e-7 around 0.999; the state 3.8e-8 and 5.1e-8, 4.2e-8 and 7.5e-8,
+// 1.0e-7 and 3.7e-7; where keys are alike, outputs 5.8e-8 and 6.7e-8, 8.9e-8 and 1.0e-7, 1.3e-7 and 3.9e-7, the state 4.0e-8 and
+// 5.1e-8, 6.2e-8 and 8.0e-8, 1.2e-7 and 4.9e-7.  (With the update in float32 a run is 0.16 us shorter, and the state is up to a fifth
+// further off than token by token where decays are fast: a sum of 16 products then rounds more often than the decays forget.)
 #include "common.h"
 #include "fmsamd.h"
 
 #include <type_traits>
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 #define RUN 16               // tokens of a run
 #define RUNS_THREADS 256     // threads of a block of either kernel
 
 // What delta_runs_prepare leaves of one run of one head, in floats:
 //   W, G * Q, R_15 * K: [D / 16 tiles][64 lanes][4], lane l of tile t holding for e < 4
-//       (G * Q)[row l % 16][16 t + 4 (l / 16) + e] and W likewise, (R_15 * K)[token 4 e + l / 16][16 t + l % 16]
+//       (G * Q)[row l % 16][16 t + 4 (l / 16) + e] and W likewise, (R_15 * K)[token 4 e + l / 16][16 t + row_token(l % 16)]
 //   Y: [Dv / 16 tiles][64][4], lane l holding Y[token 4 e + l / 16][16 t + l % 16]
 //   P without its diagonal: [4][64], P[row l % 16][token 4 e + l / 16] at e, l; then the diagonal, by tokens
 //   G_15: [D]
@@ -169,7 +175,7 @@ __global__ void __launch_bounds__(RUNS_THREADS, PER_CHANNEL ? 3 : 4) delta_runs_
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      *(f32x4*)(oK + (d / 16) * 256 + (j * 16 + d % 16) * 4) = f32x4{back[j], back[4 + j], back[8 + j], back[12 + j]};
+      *(f32x4*)(oK + (d / 16) * 256 + (j * 16 + row_token(d % 16)) * 4) = f32x4{back[j], back[4 + j], back[8 + j], back[12 + j]};
   }
   __syncthreads();
   {
@@ -238,7 +244,7 @@ __global__ void __launch_bounds__(RUNS_THREADS, PER_CHANNEL ? 3 : 4) delta_runs_
 // share of W S0 and (G * Q) S0, 4 ROWS for the update, one for its quarter of P U; partial sums meet in LDS, one barrier
 // a run (what a run leaves there, the run after the next overwrites).
 template <int ROWS>
-__global__ void __launch_bounds__(RUNS_THREADS, ROWS < 4 ? 2 : 1) delta_runs_kernel(RunsArgs a) {
+__global__ void __launch_bounds__(RUNS_THREADS, ROWS < 3 ? 2 : 1) delta_runs_kernel(RunsArgs a) {
   __shared__ f32x4 parts_u[2][4][WAVE], parts_o[2][4][WAVE];
   const int D = a.D, Dv = a.Dv, H = a.H;
   // The blocks of one sequence and head read the same W, G * Q and R_15 * K: blocks go round the XCDs, so with a multiple
@@ -327,6 +333,11 @@ __global__ void __launch_bounds__(RUNS_THREADS, ROWS < 4 ? 2 : 1) delta_runs_ker
     load_w(next, ahead);
     __builtin_amdgcn_sched_barrier(0);
     parts_u[c & 1][wave][lane] = u0 + u1;
+    f64x4 s[ROWS], k[ROWS];
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[t][e] = (double)x.g[t][e] * (double)S[t][e], k[t][e] = (double)x.k[t][e];
     block_sync_lds();
     const f32x4 s0 = parts_u[c & 1][0][lane], s1 = parts_u[c & 1][1][lane], s2 = parts_u[c & 1][2][lane], s3 = parts_u[c & 1][3][lane];
     float part[4];
@@ -342,26 +353,28 @@ __global__ void __launch_bounds__(RUNS_THREADS, ROWS < 4 ? 2 : 1) delta_runs_ker
         o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[t][e], S[t][e], o, 0, 0, 0);
       }
     load_q(next, ahead);
-    const f32x4 u = x.y - ((s0 + s1) + (s2 + s3));
+    const f32x4 ws = (s0 + s1) + (s2 + s3);
+    double u[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = (double)x.y[e] - (double)ws[e];
     __builtin_amdgcn_sched_barrier(0);
-    // the update's sums start from nothing, so that S is rounded once a run
-    f32x4 s[ROWS] = {};
+    // the update in 64 bits, from S as the decays leave it: S is rounded once a run
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int t = 0; t < ROWS; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[t][e], u[e], s[t], 0, 0, 0);
+      for (int t = 0; t < ROWS; ++t) s[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(k[t][e], u[e], s[t], 0, 0, 0);
     load_k(next, ahead);
     parts_o[(c + 1) & 1][wave][lane] = o;
     leave(part);
     mine2 = mine1, diag2 = diag1;
     p1 = x.p, diag1 = x.diag;
-    mine1 = wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3];
+    mine1 = (float)(wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3]);
     o = o0 + o1;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < ROWS; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[t][e] = fmaf(x.g[t][e], S[t][e], s[t][e]);
+      for (int e = 0; e < 4; ++e) S[t][e] = (float)s[t][e];
   };
   Operands x0, x1, x2;
   const float *ahead = run0, *last = run0 + (size_t)(n_runs - 1) * step;

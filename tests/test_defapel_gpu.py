@@ -378,6 +378,45 @@ def test_delta_rule_in_runs(lib, sizes):
     assert not bool(torch.isfinite(got2[t, 0, 3])) and torch.equal(got2[~mine], got[~mine])
 
 
+@pytest.mark.parametrize("decay", [0.2, 0.5, 0.7, 0.86, 0.95, 0.999])
+@pytest.mark.parametrize("alike", [0.0, 3.0])
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_delta_rule_in_runs_is_as_exact_as_token_by_token(lib, monkeypatch, decay, alike, per_channel):
+    """Outputs and state of runs of 16 tokens are no further from 64 bits than those of the kernel that goes token by token, from
+    decays that forget at once to decays that keep everything, for keys that are independent and keys that are alike."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, T = 4, 2, 128, 64, 300
+    gen = torch.Generator().manual_seed(7)
+    draw = lambda *size: torch.randn(*size, generator=gen)
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    q, k, v = unit(draw(T, G, D)) * D ** -0.5, unit(draw(T, G, D) + alike * draw(1, G, D)), draw(T, H, V)
+    beta = torch.sigmoid(1.5 * draw(T, H))
+    g = (1 - (1 - decay) * torch.exp(0.3 * draw(T, H, D if per_channel else 1))).clamp(0, 1)
+    state = 0.3 * draw(1, H, V, D)
+    S, want = state[0].double().transpose(1, 2), []
+    heads = lambda t: t.double().repeat_interleave(H // G, dim=0)
+    for t in range(T):
+        S = S * g[t].double()[:, :, None]
+        u = beta[t].double()[:, None] * (v[t].double() - torch.matmul(heads(k[t])[:, None], S)[:, 0])
+        S = S + heads(k[t])[:, :, None] * u[:, None, :]
+        want.append(torch.matmul(heads(q[t])[:, None], S)[:, 0])
+    want = torch.stack(want)
+
+    def errors(tokens):
+        monkeypatch.setattr(ops, "DELTA_RUN_TOKENS", tokens)
+        left = state.to(DEV)
+        qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], dim=1).to(DEV)
+        out = ops.delta_rule(qkv, beta.to(DEV), g.reshape(T, -1).to(DEV), (q.double() * k.double()).sum(-1).float().to(DEV), left,
+                             torch.tensor([0, T], dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV),
+                             torch.zeros(1, dtype=torch.int32, device=DEV), 1, H, G, D, V, per_channel)
+        return (float((out.cpu().double().view(T, H, V) - want).norm() / want.norm()),
+                float((left[0].cpu().double().transpose(1, 2) - S).norm() / S.norm()))
+
+    (out_runs, state_runs), (out_tokens, state_tokens) = errors(1), errors(T + 1)
+    assert out_runs <= out_tokens and state_runs <= state_tokens, (out_runs, out_tokens, state_runs, state_tokens)
+
+
 @pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (16, 4, 256, 130, 8, True), (20, 20, 40, 130, 1, False), (33, 3, 24, 121, 3, True)])
 def test_delta_prepare_of_many_channels(lib, sizes):
     """Blocks of 16 tokens: sequences that begin and end inside them, shorter than the convolution's reach and behind a state,
