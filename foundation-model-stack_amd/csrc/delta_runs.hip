@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(RUNS_THREADS, PER_CHANNEL ? 3 : 4) delta_runs_
 #pragma unroll
       for (int i = 0; i < RUN; ++i) {
         p *= (double)g[i];
-        least *= fmax((double)g[i], LEAST_DECAY);
+        least *= (double)g[i] < LEAST_DECAY ? LEAST_DECAY : (double)g[i];  // what is no number stays so
         kr[i * KS + d] = (double)k[i] * least;
         qr[i * KS + d] = (double)q[i] * least;
         kc[i * KS + d] = (double)k[i] / least;

@@ -378,6 +378,39 @@ def test_delta_rule_in_runs(lib, sizes):
     assert not bool(torch.isfinite(got2[t, 0, 3])) and torch.equal(got2[~mine], got[~mine])
 
 
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("what", ["decay", "beta", "k", "q"])
+def test_delta_rule_in_runs_shows_what_is_no_number_at_its_token(lib, per_channel, what):
+    """An input of one token that is no number: the outputs of its head (its heads) show it from that token on (q: there alone), as
+    token by token; nothing before it and no other head or sequence does."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, lens = 4, 2, 64, 32, [150, 143]
+    T, at = sum(lens), 150 + 16 * 3 + 6  # the seventh token of a run of the second sequence
+    assert T >= ops.DELTA_RUN_TOKENS * len(lens)
+    gen = torch.Generator().manual_seed(3)
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    x = {"q": unit(torch.randn(T, G, D, generator=gen)), "k": unit(torch.randn(T, G, D, generator=gen)), "v": torch.randn(T, H, V, generator=gen),
+         "beta": torch.sigmoid(torch.randn(T, H, generator=gen)), "decay": torch.rand(T, H, D if per_channel else 1, generator=gen)}
+    starts = torch.tensor([0, lens[0], T], dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(2), torch.tensor(lens)).to(torch.int32).to(DEV)
+
+    def run(x):
+        S = torch.zeros(2, H, V, D, device=DEV)
+        qkv = torch.cat([x[n].reshape(T, -1) for n in ("q", "k", "v")], dim=1).to(DEV)
+        return ops.delta_rule(qkv, x["beta"].to(DEV), x["decay"].reshape(T, -1).to(DEV), (x["q"] * x["k"]).sum(-1).to(DEV), S, starts, seq,
+                              torch.arange(2, dtype=torch.int32, device=DEV), 2, H, G, D, V, per_channel).cpu().view(T, H, V)
+
+    want = run(x)
+    broken = dict(x, **{what: x[what].clone()})
+    broken[what].view(T, x[what].shape[1], -1)[at, 1, 0] = float("nan")
+    got = run(broken)
+    shown = torch.zeros(T, H, V, dtype=torch.bool)
+    hit = slice(2, 4) if what in "qk" else slice(1, 2)  # heads 2 and 3 read the second q and k
+    shown[at : at + 1 if what == "q" else T, hit] = True
+    assert bool(torch.isnan(got[shown]).all()) and torch.equal(got[~shown], want[~shown])
+
+
 @pytest.mark.parametrize("decay", [0.2, 0.5, 0.7, 0.86, 0.95, 0.999])
 @pytest.mark.parametrize("alike", [0.0, 3.0])
 @pytest.mark.parametrize("per_channel", [False, True])
