@@ -433,6 +433,11 @@ extern "C" int fmsamd_delta_runs(const float* qkv, const float* beta, const floa
   const size_t lds = (size_t)(RUN * RUN + RUN) * sizeof(double) + 2 * RUN * sizeof(float) +
                      (size_t)RUN * (dim + 4) * 3 * (per_channel ? sizeof(double) : sizeof(float));
   const dim3 grid(places, heads);
+  if (lds > 64 * 1024) {  // a decay per key channel from 192 channels on: more has to be asked for, once a kernel
+    static const hipError_t sized = hipFuncSetAttribute(reinterpret_cast<const void*>(delta_runs_prepare_kernel<true>),
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    FMS_REQUIRE(sized == hipSuccess && per_channel && lds <= 160 * 1024, "delta_runs: %zu bytes of LDS refused: %s", lds, hipGetErrorString(sized));
+  }
   if (per_channel) delta_runs_prepare_kernel<true><<<grid, RUNS_THREADS, lds, stream>>>(a);
   else delta_runs_prepare_kernel<false><<<grid, RUNS_THREADS, lds, stream>>>(a);
   FMS_LAUNCH_CHECK("delta_runs_prepare");
