@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -1509,9 +1509,14 @@ def soft_cap_(x: torch.Tensor, cap: float) -> torch.Tensor:
 DELTA_MAX_TAPS = 8
 DELTA_MAX_DIM = 256
 # Tokens a sequence, on average, from which a step's recurrence goes in runs of 16 tokens on the matrix unit: two kernels and a
-# workspace instead of one (16 heads of 128 by 128, one sequence of 64 tokens 17 us against 15, eight of 64 38 against 37,
-# four heads of a sequence of 300 and one of 77 29 against 54; with a decay per key channel eight of 64 38 against 53).
+# workspace instead of one, 16 heads of 128 by 128, microseconds token by token and in runs (with a decay per key channel): one sequence
+# of 64 tokens 13.9 and 16.4 (15.8, 16.8), of 96 19.4 and 18.8 (22.1, 19.4), of 128 25 and 21 (28.7, 21.7); eight of 64 39 and 40 (52, 40),
+# of 96 49 and 47 (72, 48).
 DELTA_RUN_TOKENS = 96
+# Whatever the average, a long sequence is a chain that its neighbours wait for: with longest >= 128 + n_seqs / 2 the step goes in runs
+# as well.  2000 tokens beside 8, 32 and 64 single ones 440 and 235, 587 and 244, 634 and 287 (687 and 242, 712 and 249, 740 and 296);
+# 300 beside 32 116 and 75; 130 beside 32 66 and 62; but 96 beside 64 85 and 96.
+DELTA_RUN_LONGEST = 128
 
 
 def delta_prepare(proj: torch.Tensor, col_b: int, a: torch.Tensor, col_a: int, conv_w: torch.Tensor, a_log: torch.Tensor,
@@ -1565,11 +1570,12 @@ def delta_prepare(proj: torch.Tensor, col_b: int, a: torch.Tensor, col_a: int, c
 
 def delta_rule(qkv: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, kq: torch.Tensor, state: torch.Tensor, seq_starts: torch.Tensor,
                seq_of_token: torch.Tensor, slot_ids: torch.Tensor, n_seqs: int, heads: int, kv_heads: int, dim: int, vdim: int,
-               per_channel: bool, single_tokens: bool = False) -> torch.Tensor:
+               per_channel: bool, single_tokens: bool = False, lengths: Optional[Sequence[int]] = None) -> torch.Tensor:
     """The recurrence S = g S; u = beta (v - S^T k); S += k u^T; o = S^T q over the tokens of every sequence of the
     step (kq [T, kv_heads] holds k . q of every token, as delta_prepare leaves it), from and into state [slots, heads, vdim, dim] (float32, S transposed) -> o float32 [T, heads*vdim].
     Sequence b of the step owns the token rows seq_starts[b] .. seq_starts[b + 1] and the state of slot_ids[b].
-    single_tokens: every sequence brings one token (a decode step); the kernel then stages for that."""
+    single_tokens: every sequence brings one token (a decode step); the kernel then stages for that.  lengths: the sequences' tokens
+    as host numbers, for the choice between the kernels (without them it goes by the average)."""
     _need_cuda(qkv, beta, decay, kq, state, seq_starts, seq_of_token, slot_ids)
     for name, t in (("seq_starts", seq_starts), ("seq_of_token", seq_of_token), ("slot_ids", slot_ids)):
         _need_i32(name, t)
@@ -1587,7 +1593,11 @@ def delta_rule(qkv: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, kq: t
         raise ValueError("the step's index arrays are shorter than its sequences or tokens")
     out = torch.empty(T, heads * vdim, dtype=torch.float32, device=qkv.device)
     lib = load()
-    if not single_tokens and dim % 64 == 0 and vdim % 16 == 0 and T >= DELTA_RUN_TOKENS * n_seqs and state.data_ptr() % 16 == 0:
+    if lengths is not None and (len(lengths) != n_seqs or sum(lengths) != T):
+        raise ValueError(f"the lengths are those of {n_seqs} sequences of {T} tokens in all")
+    longest = max(lengths, default=0) if lengths is not None else 0
+    pays = T >= DELTA_RUN_TOKENS * n_seqs or longest >= DELTA_RUN_LONGEST + n_seqs // 2
+    if not single_tokens and dim % 64 == 0 and vdim % 16 == 0 and pays and state.data_ptr() % 16 == 0:
         ws_bytes = lib.fmsamd_delta_runs_workspace(T, n_seqs, heads, dim, vdim)
         workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=qkv.device)
         check(lib.fmsamd_delta_runs(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), state.data_ptr(), out.data_ptr(), seq_starts.data_ptr(),
@@ -1595,8 +1605,8 @@ def delta_rule(qkv: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, kq: t
                                     int(bool(per_channel)), workspace.data_ptr(), ws_bytes, _stream()))
         return out
     check(lib.fmsamd_delta_rule(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), kq.data_ptr(), state.data_ptr(), out.data_ptr(),
-                                   seq_starts.data_ptr(), seq_of_token.data_ptr(), slot_ids.data_ptr(), n_seqs, heads, kv_heads, dim,
-                                   vdim, int(bool(per_channel)), int(bool(single_tokens)), _stream()))
+                                seq_starts.data_ptr(), seq_of_token.data_ptr(), slot_ids.data_ptr(), n_seqs, heads, kv_heads, dim,
+                                vdim, int(bool(per_channel)), int(bool(single_tokens)), _stream()))
     return out
 
 

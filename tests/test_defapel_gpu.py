@@ -379,6 +379,49 @@ def test_delta_rule_in_runs(lib, sizes):
 
 
 @pytest.mark.parametrize("per_channel", [False, True])
+def test_a_long_sequence_beside_many_running_ones_goes_in_runs(lib, per_channel):
+    """A prompt beside so many single tokens that the average is short: the prompt's rows are those of the prompt alone (in runs), the
+    single tokens' those of a decode step to rounding; the line of the rule; lengths that do not fit are refused."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, per = 4, 2, 128, 48, 128 if per_channel else 1
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+
+    def step(lens, only=None, **hints):  # the step of these sequences, or the one of `only` of them alone
+        T, starts = sum(lens), [0] + list(np.cumsum(lens))
+        g = torch.Generator().manual_seed(11)
+        q, k, v = unit(torch.randn(T, G, D, generator=g)), unit(torch.randn(T, G, D, generator=g)), torch.randn(T, H, V, generator=g)
+        beta, decay = torch.sigmoid(torch.randn(T, H, generator=g)), torch.rand(T, H * per, generator=g) ** 0.1
+        state = 0.3 * torch.randn(len(lens), H, V, D, generator=g)
+        which = list(range(len(lens))) if only is None else only
+        rows = torch.cat([torch.arange(starts[b], starts[b + 1]) for b in which])
+        mine, S = [lens[b] for b in which], state[which].to(DEV)
+        qkv, kq = torch.cat([t.reshape(T, -1) for t in (q, k, v)], dim=1), (q * k).sum(-1)
+        out = ops.delta_rule(qkv[rows].to(DEV), beta[rows].to(DEV), decay[rows].to(DEV), kq[rows].to(DEV), S,
+                             torch.tensor([0] + list(np.cumsum(mine)), dtype=torch.int32, device=DEV),
+                             torch.repeat_interleave(torch.arange(len(mine)), torch.tensor(mine)).to(torch.int32).to(DEV),
+                             torch.arange(len(mine), dtype=torch.int32, device=DEV), len(mine), H, G, D, V, per_channel,
+                             **dict({"lengths": mine}, **hints))
+        return out.cpu(), S.cpu()
+
+    lens = [1] * 9 + [301] + [1] * 20 + [17]
+    out, left = step(lens)
+    got, S = step(lens, [9])
+    assert torch.equal(out[9:310], got) and torch.equal(left[9:10], S)
+    singles = [b for b, n in enumerate(lens) if n == 1]
+    got, S = step(lens, singles, single_tokens=True)
+    # one token: sums of 128 products of size 1 / 128 at most a few times, 24 bits
+    torch.testing.assert_close(torch.cat([out[:9], out[310:330]]), got, atol=2e-6, rtol=1e-5)
+    torch.testing.assert_close(left[singles], S, atol=2e-6, rtol=1e-5)
+    line = ops.DELTA_RUN_LONGEST + 3  # seven sequences
+    for n, in_runs in ((line, True), (line - 1, False)):
+        mixed, alone = step([1] * 6 + [n])[0][6:], step([1] * 6 + [n], [6])[0]
+        assert torch.equal(mixed, alone) == in_runs
+    with pytest.raises(ValueError):
+        step(lens, lengths=lens[1:])
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
 @pytest.mark.parametrize("what", ["decay", "beta", "k", "q"])
 def test_delta_rule_in_runs_shows_what_is_no_number_at_its_token(lib, per_channel, what):
     """An input of one token that is no number: the outputs of its head (its heads) show it from that token on (q: there alone), as
