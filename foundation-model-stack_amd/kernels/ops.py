@@ -33,7 +33,8 @@ def _code(dtype: torch.dtype) -> int:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without the object around the number: 0.2 us instead of 3 in every call of a kernel
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -66,6 +66,29 @@ def test_add_norm(ops, width, dtype):
     torch.testing.assert_close(out3.cpu().float(), P.rms_norm(resid, weight.float(), eps), **tol(dtype))
 
 
+def test_kernels_run_on_the_current_stream(ops):
+    """The number that the kernels are launched with is that of torch's current stream: by itself, inside stream contexts and while a
+    graph is captured (whose replays then hold the kernel)."""
+    here = lambda: ops._stream() == torch.cuda.current_stream().cuda_stream
+    assert here()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        assert here() and ops._stream() == a.cuda_stream
+        with torch.cuda.stream(b):
+            assert here() and ops._stream() == b.cuda_stream
+        assert ops._stream() == a.cuda_stream
+    x = dev(torch.ones(300))
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        assert here()
+        ops.scale_(x, 2.0)
+    for n in range(1, 4):
+        graph.replay()
+        assert bool((x == 2.0 ** n).all())
+    assert here()
+
+
 @pytest.mark.parametrize("heads, kvheads, dim, lens, contexts, window", [
     (4, 4, 16, [64], [64], 0), (2, 1, 128, [97], [97], 0), (6, 3, 112, [33], [200], 50), (32, 8, 64, [15, 1, 130, 31], [15, 300, 130, 95], 0),
     (32, 32, 48, [16, 40, 3], [16, 161, 257], 33)])
