@@ -52,6 +52,12 @@ __device__ __forceinline__ int row_token(int r) { return 4 * (r % 4) + r / 4; } 
 
 // Run c of sequence b is place starts[b] / 16 + b + c: sequences of any length never meet, and n tokens in s sequences
 // take at most n / 16 + s places.
+// Long steps go in pieces, so that the workspace stays bounded: a piece is the runs whose first token is one of p0 .. p1 (multiples
+// of 16), which are places from p0 / 16 on, (p1 - p0) / 16 + s at most.  The state passes from piece to piece through memory, as it
+// is: the pieces change no bit.  A piece should hold as many sequences as the chip has blocks for (four with 16 heads of 128 by 128):
+// in pieces of 128, 256, 384 and 512 MB and as one, 8 sequences of 1000 tokens take 417, 368 and 322 us (266 MB is one), 4 of 4000 1713,
+// 1065, 1001, 667 and 616, 16 of 2000 2255, 1629, 1540, 1504 and 1970, one of 16000 1209, 1221, 1200, 1209 and 1197.
+#define RUNS_WORKSPACE (512L << 20)  // bytes: 15600 tokens of 16 heads of 128 by 128
 
 struct RunsArgs {
   const float* qkv;    // [T, C]: q [G*D] | k [G*D] | v [H*Dv]
@@ -64,6 +70,7 @@ struct RunsArgs {
   const int* seq_of_token;
   const int* slot_ids;
   int n_seqs, H, G, D, Dv;
+  int p0, p1;          // the piece
 };
 
 // Products of decays may underflow to nothing; a quotient of two of them is formed from decays of at least this (16 of
@@ -88,7 +95,7 @@ __global__ void __launch_bounds__(RUNS_THREADS, PER_CHANNEL ? 3 : 4) delta_runs_
   KEY* kc = PER_CHANNEL ? qr + RUN * KS : kr;   // [16][KS] k of the column's token (PER_CHANNEL: k / G)
   float* w = (float*)(qr + RUN * KS);           // [16][KS], takes the place of kc
 
-  const int place = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int place = a.p0 / RUN + blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   // the sequence whose places this one is among: the last with first_run <= place
   int b = 0;
   for (int lo = 0, hi = a.n_seqs; lo + 1 < hi;) {
@@ -98,10 +105,10 @@ __global__ void __launch_bounds__(RUNS_THREADS, PER_CHANNEL ? 3 : 4) delta_runs_
   }
   const int t0 = uniform_load(a.seq_starts + b), t1 = uniform_load(a.seq_starts + b + 1);
   const int tb = t0 + (place - t0 / RUN - b) * RUN;
-  if (tb >= t1 || uniform_load(a.seq_of_token + t0) < 0) return;
+  if (tb >= t1 || tb < a.p0 || tb >= a.p1 || uniform_load(a.seq_of_token + t0) < 0) return;
   const int n = t1 - tb < RUN ? t1 - tb : RUN;
   const int C = 2 * G * D + H * Dv, kh = h / (H / G);
-  float* run = a.runs + ((size_t)place * H + h) * run_floats(D, Dv);
+  float* run = a.runs + ((size_t)blockIdx.x * H + h) * run_floats(D, Dv);
   float *oW = run, *oQ = oW + RUN * D, *oK = oQ + RUN * D, *oY = oK + RUN * D, *oP = oY + RUN * Dv, *oG = oP + RUN * (RUN + 1);
 
   // Tokens past the run's end: k = q = v = 0, beta = 0, g = 1.
@@ -253,13 +260,18 @@ __global__ void __launch_bounds__(RUNS_THREADS, ROWS < 3 ? 2 : 1) delta_runs_ker
   const int pair = blockIdx.x % stride, ct = blockIdx.x / stride;
   if (pair >= pairs) return;
   const int b = pair / H, h = pair % H;
-  const int t0 = uniform_load(a.seq_starts + b), t1 = uniform_load(a.seq_starts + b + 1);
+  int t0 = uniform_load(a.seq_starts + b), t1 = uniform_load(a.seq_starts + b + 1);
   if (t0 >= t1 || uniform_load(a.seq_of_token + t0) < 0) return;
+  // the sequence's runs in this piece
+  if (t0 >= a.p1) return;
+  t1 = min(t1, t0 + (a.p1 - t0 + RUN - 1) / RUN * RUN);
+  if (t0 < a.p0) t0 += (a.p0 - t0 + RUN - 1) / RUN * RUN;
+  if (t0 >= t1) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, quad = lane >> 4;
   const int n_runs = (t1 - t0 + RUN - 1) / RUN;
   const size_t step = (size_t)H * run_floats(D, Dv);
-  const float* run0 = a.runs + ((size_t)(t0 / RUN + b) * H + h) * run_floats(D, Dv);
+  const float* run0 = a.runs + ((size_t)(t0 / RUN + b - a.p0 / RUN) * H + h) * run_floats(D, Dv);
   float* state = a.state + (((size_t)a.slot_ids[b] * H + h) * Dv + 16 * ct + col) * D + 16 * ROWS * wave + 4 * quad;
 
   f32x4 S[ROWS];
@@ -412,9 +424,13 @@ __global__ void __launch_bounds__(RUNS_THREADS, ROWS < 3 ? 2 : 1) delta_runs_ker
 }
 
 // --------------------------------------------------------------------------
+// The places of the whole step, or as many as RUNS_WORKSPACE holds, and then at least two a sequence and 64 (a sequence's state is
+// as large as two): a piece is 1000 tokens or more.
 extern "C" long fmsamd_delta_runs_workspace(int n_tokens, int n_seqs, int heads, int dim, int vdim) {
   if (n_tokens < 0 || n_seqs < 0 || heads <= 0 || dim <= 0 || vdim <= 0 || dim % 64 || dim > 256 || vdim % 16) return -1;
-  return (long)(n_tokens / RUN + n_seqs) * heads * (long)run_floats(dim, vdim) * (long)sizeof(float);
+  const long place = heads * (long)run_floats(dim, vdim) * (long)sizeof(float), all = n_tokens / RUN + (long)n_seqs;
+  const long bound = RUNS_WORKSPACE / place > 2L * n_seqs + 64 ? RUNS_WORKSPACE / place : 2L * n_seqs + 64;
+  return (all < bound ? all : bound) * place;
 }
 
 extern "C" int fmsamd_delta_runs(const float* qkv, const float* beta, const float* decay, float* state, float* out, const int* seq_starts,
@@ -425,26 +441,33 @@ extern "C" int fmsamd_delta_runs(const float* qkv, const float* beta, const floa
               "delta_runs: bad sizes heads=%d kv_heads=%d dim=%d vdim=%d", heads, kv_heads, dim, vdim);
   FMS_REQUIRE(dim % 64 == 0 && dim <= 256 && vdim % 16 == 0, "delta_runs: %d key and %d value channels (multiples of 64 up to 256, and of 16)",
               dim, vdim);
-  const long places = n_tokens / RUN + n_seqs, blocks = (((long)n_seqs * heads + 7) & ~7L) * (vdim / 16);
-  FMS_REQUIRE(heads <= 65535 && blocks <= 0x7fffffffL, "delta_runs: too many heads or value channels for one launch");
-  FMS_REQUIRE(workspace_bytes >= fmsamd_delta_runs_workspace(n_tokens, n_seqs, heads, dim, vdim), "delta_runs: the workspace is too small");
+  FMS_REQUIRE(n_tokens <= 0x7fffffff - 4 * RUN, "delta_runs: too many tokens");
+  const long room = workspace_bytes / (heads * (long)run_floats(dim, vdim) * (long)sizeof(float)), all = n_tokens / RUN + (long)n_seqs;
+  const long blocks = (((long)n_seqs * heads + 7) & ~7L) * (vdim / 16);
+  FMS_REQUIRE(heads <= 65535 && blocks <= 0x7fffffffL && all <= 0x7fffffffL, "delta_runs: too many heads or value channels for one launch");
+  FMS_REQUIRE(room >= all || room > n_seqs, "delta_runs: the workspace is too small");
   FMS_REQUIRE(((uintptr_t)state | (uintptr_t)workspace) % 16 == 0, "delta_runs: the state and the workspace start at 16-byte addresses");
-  RunsArgs a{qkv, beta, decay, state, out, (float*)workspace, seq_starts, seq_of_token, slot_ids, n_seqs, heads, kv_heads, dim, vdim};
+  RunsArgs a{qkv, beta, decay, state, out, (float*)workspace, seq_starts, seq_of_token, slot_ids, n_seqs, heads, kv_heads, dim, vdim, 0, 0};
   const size_t lds = (size_t)(RUN * RUN + RUN) * sizeof(double) + 2 * RUN * sizeof(float) +
                      (size_t)RUN * (dim + 4) * 3 * (per_channel ? sizeof(double) : sizeof(float));
-  const dim3 grid(places, heads);
   if (lds > 64 * 1024) {  // a decay per key channel from 192 channels on: more has to be asked for, once a kernel
     static const hipError_t sized = hipFuncSetAttribute(reinterpret_cast<const void*>(delta_runs_prepare_kernel<true>),
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     FMS_REQUIRE(sized == hipSuccess && per_channel && lds <= 160 * 1024, "delta_runs: %zu bytes of LDS refused: %s", lds, hipGetErrorString(sized));
   }
-  if (per_channel) delta_runs_prepare_kernel<true><<<grid, RUNS_THREADS, lds, stream>>>(a);
-  else delta_runs_prepare_kernel<false><<<grid, RUNS_THREADS, lds, stream>>>(a);
-  FMS_LAUNCH_CHECK("delta_runs_prepare");
-  if (dim == 64) delta_runs_kernel<1><<<blocks, RUNS_THREADS, 0, stream>>>(a);
-  else if (dim == 128) delta_runs_kernel<2><<<blocks, RUNS_THREADS, 0, stream>>>(a);
-  else if (dim == 192) delta_runs_kernel<3><<<blocks, RUNS_THREADS, 0, stream>>>(a);
-  else delta_runs_kernel<4><<<blocks, RUNS_THREADS, 0, stream>>>(a);
-  FMS_LAUNCH_CHECK("delta_runs");
+  const int end = (n_tokens + RUN - 1) / RUN * RUN;
+  const long piece = room >= all ? end : (room - n_seqs) * RUN;  // tokens of a piece
+  for (long p0 = 0; p0 < end; p0 += piece) {
+    a.p0 = (int)p0, a.p1 = (int)(p0 + piece < end ? p0 + piece : end);
+    const dim3 grid((unsigned)(room >= all ? all : (a.p1 - a.p0) / RUN + n_seqs), heads);
+    if (per_channel) delta_runs_prepare_kernel<true><<<grid, RUNS_THREADS, lds, stream>>>(a);
+    else delta_runs_prepare_kernel<false><<<grid, RUNS_THREADS, lds, stream>>>(a);
+    FMS_LAUNCH_CHECK("delta_runs_prepare");
+    if (dim == 64) delta_runs_kernel<1><<<blocks, RUNS_THREADS, 0, stream>>>(a);
+    else if (dim == 128) delta_runs_kernel<2><<<blocks, RUNS_THREADS, 0, stream>>>(a);
+    else if (dim == 192) delta_runs_kernel<3><<<blocks, RUNS_THREADS, 0, stream>>>(a);
+    else delta_runs_kernel<4><<<blocks, RUNS_THREADS, 0, stream>>>(a);
+    FMS_LAUNCH_CHECK("delta_runs");
+  }
   return 0;
 }

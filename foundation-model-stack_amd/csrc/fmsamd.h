@@ -340,7 +340,8 @@ int fmsamd_delta_rule(const float* qkv, const float* beta, const float* decay, c
                       const int* seq_starts, const int* seq_of_token, const int* slot_ids, int n_seqs, int heads,
                       int kv_heads, int dim, int vdim, int per_channel, int single_tokens, hipStream_t stream);
 // The same in runs of 16 tokens on the matrix unit (delta_runs.hip): dim a multiple of 64 up to 256, vdim one of 16, state and
-// workspace at 16-byte addresses.  The workspace is that of fmsamd_delta_runs_workspace (-1: sizes that are not taken).
+// workspace at 16-byte addresses.  The workspace is that of fmsamd_delta_runs_workspace (-1: sizes that are not taken), which is
+// bounded: long steps go in pieces, with the same bits.  A smaller one, of at least n_seqs + 1 runs of all heads, makes more pieces.
 long fmsamd_delta_runs_workspace(int n_tokens, int n_seqs, int heads, int dim, int vdim);
 int fmsamd_delta_runs(const float* qkv, const float* beta, const float* decay, float* state, float* out, const int* seq_starts,
                       const int* seq_of_token, const int* slot_ids, int n_tokens, int n_seqs, int heads, int kv_heads, int dim,

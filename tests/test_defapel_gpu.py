@@ -421,6 +421,41 @@ def test_a_long_sequence_beside_many_running_ones_goes_in_runs(lib, per_channel)
         step(lens, lengths=lens[1:])
 
 
+@pytest.mark.parametrize("lens", [[1, 255, 16, 160, 97], [777], [33, 1, 1, 300, 2]])
+@pytest.mark.parametrize("spare", [1, 2, 5, 13])
+def test_delta_rule_in_runs_in_pieces(lib, lens, spare):
+    """A workspace of `spare` runs beside one a sequence: pieces of 16 to 208 tokens, which cut sequences anywhere and leave short ones
+    whole, give the bits of the whole step; a smaller one is refused, and the largest that is asked for stays bounded."""
+    from fms_amd.kernels import load
+
+    entry, H, G, D, V, T = load(), 2, 1, 64, 32, sum(lens)
+    gen = torch.Generator().manual_seed(T)
+    qkv = torch.nn.functional.normalize(torch.randn(T, 2 * G * D + H * V, generator=gen), dim=1).to(DEV)
+    beta, decay = torch.rand(T, H, generator=gen).to(DEV), (torch.rand(T, H, generator=gen) ** 0.05).to(DEV)
+    starts = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32).to(DEV)
+    slots = torch.arange(len(lens), dtype=torch.int32, device=DEV).flip(0).contiguous()
+    state = torch.randn(len(lens), H, V, D, generator=gen)
+
+    def run(nbytes):
+        S, out, ws = state.to(DEV), torch.full((T, H * V), float("nan"), device=DEV), torch.full((nbytes // 4,), float("nan"), device=DEV)
+        err = entry.fmsamd_delta_runs(qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(), S.data_ptr(), out.data_ptr(), starts.data_ptr(),
+                                    seq.data_ptr(), slots.data_ptr(), T, len(lens), H, G, D, V, 0, ws.data_ptr(), nbytes,
+                                    torch.cuda.current_stream().cuda_stream)
+        return err, out, S
+
+    whole = entry.fmsamd_delta_runs_workspace(T, len(lens), H, D, V)
+    place = whole // (T // 16 + len(lens))
+    assert whole == place * (T // 16 + len(lens))
+    err, want, left = run(whole)
+    assert err == 0 and bool(torch.isfinite(want).all())
+    err, got, S = run(place * (len(lens) + spare))
+    assert err == 0 and torch.equal(got, want) and torch.equal(S, left)
+    assert run(place * len(lens))[0] != 0
+    assert entry.fmsamd_delta_runs_workspace(1 << 20, 3, 16, 128, 128) <= 512 << 20
+    assert entry.fmsamd_delta_runs_workspace(1 << 20, 1000, 16, 128, 128) <= 2100 * 560 * 1024
+
+
 @pytest.mark.parametrize("per_channel", [False, True])
 @pytest.mark.parametrize("what", ["decay", "beta", "k", "q"])
 def test_delta_rule_in_runs_shows_what_is_no_number_at_its_token(lib, per_channel, what):
