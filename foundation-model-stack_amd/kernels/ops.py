@@ -522,7 +522,7 @@ def attention(
         if seen:
             max_context = min(int(max_context), seen * PAGE_TOKENS)
         n_pages = -(-max_context // PAGE_TOKENS)
-        auto_pages, auto_waves = decode_split(T * kvheads, n_pages)
+        auto_pages, auto_waves = decode_split(T * kvheads, n_pages, full=bool(seen) and max_context == seen * PAGE_TOKENS)
         if pages_per_block <= 0:
             pages_per_block = auto_pages
         if waves <= 0:
@@ -554,20 +554,22 @@ def attention(
     return out
 
 
-def decode_split(rows: int, n_pages: int):
+def decode_split(rows: int, n_pages: int, full: bool = False):
     """(pages per split, waves per block) of the decode attention kernel.
 
-    rows = tokens x kv heads.  A compute unit pulls only a small share of the memory bandwidth, so
+    rows = tokens x kv heads.  full: the contexts fill the bound (a window's or a chunk's, not the sequences' longest).  A compute unit pulls only a small share of the memory bandwidth, so
     the cache has to be spread over all of them: the context bound is cut into as many splits as give
     a few hundred blocks, and at least so many that a block has no more than 128 pages (every sequence
     deals its own pages out evenly over the splits; the waves of a block run their pages as a pipeline,
     so a block of many pages is cheaper than many blocks).  The waves of a block share its pages and merge in LDS, the blocks of a row
     merge in a second kernel."""
-    # But no splits of under 8 pages, one for each wave, and one split up to 16 pages.  Microseconds with two splits and their
-    # merge, and with one, under a bound of 1024 tokens: a sequence of 4 kv heads of 64, 64 tokens 6.7 and 4.7, 300 7.5 and 6.6,
-    # 512 8.1 and 7.7, 700 8.7 and 9.0, 1024 9.7 and 11.1; 64 sequences of 8 kv heads of 128, 300 tokens 27.7 and 18.3, 1024 53
-    # and 47.7.
-    by_rows = min(-(-256 // max(rows, 1)), max(1, n_pages // 8)) if n_pages > 16 else 1
+    # But no splits of under 8 pages, one for each wave, and one split of 16 pages where the contexts grow to that bound or the rows
+    # fill half the chip.  Microseconds with two splits and their merge, and with one, 16 pages, 4 kv heads of 64: a sequence of 64
+    # tokens 6.6 and 4.7, 300 7.4 and 6.6, 512 8.1 and 7.7, 700 8.8 and 9.1, 860 9.6 and 10.5, 1024 9.8 and 11.1 (a step's merges are
+    # as many launches less, and the whole step is no slower at any of them); 32 sequences 6.9 and 4.9 to 11.2 and 12.1; 48 9.7 and 4.9 to
+    # 18.8 and 14.8.  8 kv heads of 128, 16 sequences 7.3 and 5.1 to 14.8 and 15.3, 24 12 and 5.3 to 23.4 and 17.8.
+    one = n_pages <= 16 and (rows > 128 or not full)
+    by_rows = 1 if one else min(-(-256 // max(rows, 1)), max(1, n_pages // 8))
     splits = max(1, min(max(by_rows, -(-n_pages // 128)), n_pages))
     pages = -(-n_pages // splits)
     waves = max(1, min(8 if rows * splits <= 512 else 4, pages))

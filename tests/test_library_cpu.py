@@ -1094,3 +1094,15 @@ def test_kernels_compile_without_relative_register_indexing(tmp_path):
         assert not re.search(r"s_set_gpr_idx|v_movrel", text), f"{os.path.basename(src)} uses relative register indexing"
         spills = [int(m) for m in re.findall(r"\.vgpr_spill_count:\s+(\d+)", text)]
         assert spills and max(spills) == 0, f"{os.path.basename(src)} spills registers: {spills}"
+
+
+def test_a_full_window_of_sixteen_pages_is_cut_in_two():
+    """The decode attention's split: contexts that grow to a bound of 16 pages go as one, a window that is as long and full as two where
+    the rows leave the chip idle; all other bounds do not ask."""
+    from fms_amd.kernels import ops
+
+    assert ops.decode_split(4, 16) == (16, 8) and ops.decode_split(4, 16, full=True) == (8, 8)
+    assert ops.decode_split(128, 16, full=True)[0] == 8 and ops.decode_split(129, 16, full=True)[0] == 16
+    for rows in (1, 8, 128, 500):
+        for pages in (1, 8, 15, 17, 32, 300):
+            assert ops.decode_split(rows, pages) == ops.decode_split(rows, pages, full=True)
