@@ -10,6 +10,7 @@ import torch
 
 from ..kernels import ops
 from .base import Part, register_part
+from .norm import ParameterizedNorm
 
 
 class TokenEmbedding(Part):
@@ -27,7 +28,9 @@ class TokenEmbedding(Part):
         """(the stream, the stream through `norm`) as one kernel, or None where there is none for this norm and these types."""
         if getattr(self.forward, "__func__", None) is not TokenEmbedding.forward:  # somebody else's forward
             return None
-        if act_dtype != self.w["weight"].dtype or not getattr(norm, "deferrable", lambda: False)():
+        if getattr(getattr(norm, "add_norm", None), "__func__", None) is not ParameterizedNorm.add_norm:  # or norm
+            return None
+        if act_dtype != self.w["weight"].dtype or not norm.deferrable():
             return None
         return ops.embed_norm(token_ids, self.w["weight"], self.scale, norm.scale_weight(), norm.eps)
 

@@ -1106,3 +1106,31 @@ def test_a_full_window_of_sixteen_pages_is_cut_in_two():
     for rows in (1, 8, 128, 500):
         for pages in (1, 8, 15, 17, 32, 300):
             assert ops.decode_split(rows, pages) == ops.decode_split(rows, pages, full=True)
+
+
+def test_embedding_leaves_a_norm_of_somebody_elses_to_that_norm(monkeypatch):
+    """The embedding makes the first norm's rows with its own only for the library's norm as it is: not for a subclass or an object
+    whose add_norm is another, and not for a norm that has no more than the interface asks of one."""
+    from fms_amd.kernels import ops
+    from fms_amd.parts.embedding import TokenEmbedding
+    from fms_amd.parts.norm import ParameterizedNorm
+
+    class Loud(ParameterizedNorm):
+        def add_norm(self, *args, **kwargs):
+            return super().add_norm(*args, **kwargs)
+
+    class Bare:  # add_norm, and what a product needs that applies the norm as a row scale
+        eps, w = 1e-5, {"weight": torch.ones(8)}
+        add_norm = staticmethod(lambda resid, branch, out_dtype, rows=None: resid)
+        deferrable = staticmethod(lambda: True)
+
+    patched = ParameterizedNorm(8)
+    patched.add_norm = lambda *args, **kwargs: None
+    monkeypatch.setattr(ops, "embed_norm", lambda *args: "one kernel")
+    embedding = TokenEmbedding(4, 8)
+    embedding.w["weight"] = torch.zeros(4, 8)
+    ids = torch.zeros(2, dtype=torch.int32)
+    for norm in (Loud(8), Bare(), patched, ParameterizedNorm(8, use_mean=True), ParameterizedNorm(8, groups=2)):
+        assert embedding.forward_normed(ids, norm, torch.float32) is None
+    assert embedding.forward_normed(ids, ParameterizedNorm(8), torch.float32) == "one kernel"
+    assert embedding.forward_normed(ids, ParameterizedNorm(8), torch.bfloat16) is None
