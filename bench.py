@@ -186,7 +186,7 @@ def main() -> int:
         """The share of a decode step's GPU time by kernel class: three eager steps (the same kernels in the same
         shape as the replayed graph) with an event before and after every call into the kernel library."""
         classes = {"qkv_rope_write": "qkv_rope_cache", "attention": "attention", "gated_linear": "gate_up_act",
-                   "sample": "sampling", "embed": "other", "add_norm": "other", "advance_positions_": "other"}
+                   "sample": "sampling", "embed": "other", "embed_norm": "other", "add_norm": "other"}
         spans, originals = [], {}
 
         def timed(name, fn):

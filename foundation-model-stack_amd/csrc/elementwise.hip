@@ -554,20 +554,3 @@ extern "C" int fmsamd_bias_add(void* x, int dtype, const void* bias, int bias_dt
   FMS_LAUNCH_CHECK("bias_add");
   return 0;
 }
-
-// --------------------------------------------------------------------------
-// positions[i] += 1 for the live rows of a fixed-size decode batch, so that a
-// captured step can be replayed without the host touching its index data
-// --------------------------------------------------------------------------
-__global__ void advance_positions_kernel(int* __restrict__ positions, const int* __restrict__ seq_of_token, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && seq_of_token[i] >= 0) positions[i] += 1;
-}
-
-extern "C" int fmsamd_advance_positions(int* positions, const int* seq_of_token, int n, hipStream_t stream) {
-  if (n == 0) return 0;
-  FMS_REQUIRE(n > 0, "advance_positions: negative count");
-  advance_positions_kernel<<<ceil_div(n, 256), 256, 0, stream>>>(positions, seq_of_token, n);
-  FMS_LAUNCH_CHECK("advance_positions");
-  return 0;
-}

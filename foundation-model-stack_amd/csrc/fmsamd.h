@@ -6,7 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
-#define FMSAMD_ABI_VERSION 12
+#define FMSAMD_ABI_VERSION 13
 
 // element types
 #define FMS_F32 0
@@ -60,9 +60,6 @@ typedef struct fmsamd_gate_clamp {
 // null: act is then not used); rows of out ldo apart
 int fmsamd_gated_act(const void* gu, const void* bias, int bias_dtype, void* out, int dtype, long ldo, int n_tokens, int hidden,
                      int act, const fmsamd_gate_clamp* clamp, hipStream_t stream);
-
-// positions[i] += 1 where seq_of_token[i] >= 0
-int fmsamd_advance_positions(int* positions, const int* seq_of_token, int n, hipStream_t stream);
 
 int fmsamd_cast(const void* in, int in_dtype, void* out, int out_dtype, long n, hipStream_t stream);
 int fmsamd_bias_add(void* x, int dtype, const void* bias, int bias_dtype, int rows, int cols, hipStream_t stream);

@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads libamdhip64 before our library asks for it)
 
 from . import build as _build
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
@@ -31,7 +31,6 @@ _SIGNATURES = {
     "fmsamd_stream_rows": [P, P, P, P, I, L, I, I, P],
     "fmsamd_gated_act": [P, P, I, P, I, L, I, I, I, P, P],
     "fmsamd_cast": [P, I, P, I, L, P],
-    "fmsamd_advance_positions": [P, P, I, P],
     "fmsamd_bias_add": [P, I, P, I, I, I, P],
     "fmsamd_rope_table": [P, P, P, I, I, F, P],
     "fmsamd_rope_kv_write": [P, I, L, P, P, P, I, P, P, I, I, P, P, I, I, I, I, I, P],

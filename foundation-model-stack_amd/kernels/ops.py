@@ -222,16 +222,6 @@ def cast(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return out
 
 
-def advance_positions_(positions: torch.Tensor, seq_of_token: torch.Tensor) -> None:
-    """positions += 1 on the live rows (seq_of_token >= 0) of a fixed-size decode batch."""
-    _need_cuda(positions, seq_of_token)
-    _need_i32("positions", positions)
-    _need_i32("seq_of_token", seq_of_token)
-    if positions.numel() != seq_of_token.numel():
-        raise ValueError("positions and seq_of_token must have one entry per row")
-    check(load().fmsamd_advance_positions(positions.data_ptr(), seq_of_token.data_ptr(), positions.numel(), _stream()))
-
-
 def bias_add_(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     _need_cuda(x, bias)
     if x.dim() != 2 or not x.is_contiguous() or bias.shape != (x.shape[1],) or not bias.is_contiguous():
@@ -1862,7 +1852,8 @@ def sample(
     seq_of_token: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """One token per row of float32 logits.  rng_state: int64 [rows, 2] (seed, counter), advanced in place.  positions, with
-    seq_of_token: advanced as advance_positions_ does, by the same kernel."""
+    seq_of_token: += 1 on the rows of a sequence (seq_of_token >= 0) by the same kernel, so that a captured step can be replayed
+    without the host touching its index data."""
     _need_cuda(logits, rng_state, out, positions, seq_of_token)
     if positions is not None:
         _need_i32("positions", positions)
