@@ -101,7 +101,8 @@ __global__ void __launch_bounds__(1024)
 // The same for prompts: a block takes 16 tokens and the channels of a q head and its k head, 256 value channels, or 256 decays (and
 // the betas).  A thread has a channel of all 16 tokens and asks for its inputs at once, each of them once (the kernel above
 // reads an input once for every tap, in eight passes of a block that has one token and all channels, and is bound by their
-// round trips: 2277 tokens of 4096 channels 63 us, 41 here; with a decay per channel 78 and 47).
+// round trips: 2277 tokens of 4096 channels 63 us, 41 here; with a decay per channel 78 and 47; the line between them stands at
+// fmsamd_delta_prepare).
 #define PREP_TOKENS 16
 template <typename W>
 __global__ void __launch_bounds__(256)
@@ -443,11 +444,22 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
   FMS_REQUIRE(seq_starts == nullptr || n_seqs > 0, "delta_prepare: no sequences");
   const size_t lds = (size_t)C * sizeof(float);
   const int threads = n_tokens <= 64 ? 1024 : 256;
-  // 16 tokens a block where there are more of them than a decode step has, and enough channels (C >= 4096: 65 tokens 19 us instead of
-  // 22, 40 sequences of 17 28 instead of 31; with 384 channels a block's chain of loads, sums and gates is longer than the other
-  // kernel's single pass, 20 us instead of 13)
-  const long units = kv_heads + (heads * (long)vdim + 255) / 256 + (heads * (long)(per_channel ? dim : 1) + 255) / 256;
-  const bool by_tokens = n_tokens > 64 && C >= 4096 && dim <= 256 && units <= 65535;
+  // 16 tokens a block where that is less work than it is a longer way: some 21 us for loads, sums and gates one after the other, whatever
+  // the sizes, and then half the time a token.  The other kernel's way is its passes over the columns.  Microseconds of the other kernel
+  // and of this one (with conv_state behind them):
+  //   8192 columns: 65 tokens 32 and 21.7, 2277 121 and 59;  6144 (4096 channels with a decay per channel): 65 22.3 and 21.4, 2277 70 and 48;
+  //   4096: 65 to 256 tokens 19 to 20 and 21 to 22, 512 24.5 and 22.9, 2277 56.3 and 42.6;
+  //   3072: 512 19.6 and 22.5, 2277 46.0 and 39.2;  2048: 2277 35.3 and 33.6, 3000 40.6 and 33.7;  1024: 2277 24.1 and 26.9, 8192 56.5 and 43.9;
+  //   384: 2277 15.2 and 22.4, 8192 40 and 29.8;  heads of 256: 4096 columns, 512 tokens 23.7 and 37.2, 2277 61.5 and 57.8; 1536, 2277 27.9
+  //     and 45.5, 8192 70 and 54.
+  // Blocks of several sequences ask for every tap by itself: 200 sequences of 17 60 and 87 (2304 columns), 86 and 98 (4096), 102 and 109
+  // (6144), 175 and 171 (8192); of 4096 columns 12 of 100 35.4 and 37.6, 8 of 130 35 and 33.4.
+  const long decays = heads * (long)(per_channel ? dim : 1), columns = C + decays, work = n_tokens * columns;
+  const long units = kv_heads + (heads * (long)vdim + 255) / 256 + (decays + 255) / 256;
+  const bool long_seqs = n_tokens >= 128L * n_seqs;
+  const bool pays = dim > 128 ? long_seqs && work >= 8000000
+                              : columns >= 8192 || (long_seqs && (columns >= 6144 || work >= 5000000 || (columns >= 4096 && n_tokens >= 512)));
+  const bool by_tokens = n_tokens > 64 && dim <= 256 && units <= 65535 && pays;
   const dim3 grid(ceil_div(n_tokens, PREP_TOKENS), (unsigned)units);
   const size_t token_lds = (size_t)PREP_TOKENS * (2 * dim + 4) * sizeof(float);
 #define FMS_PREP(W)                                                                                                   \

@@ -528,7 +528,8 @@ def test_delta_rule_in_runs_is_as_exact_as_token_by_token(lib, monkeypatch, deca
     assert out_runs <= out_tokens and state_runs <= state_tokens, (out_runs, out_tokens, state_runs, state_tokens)
 
 
-@pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (16, 4, 256, 130, 8, True), (20, 20, 40, 130, 1, False), (33, 3, 24, 121, 3, True)])
+@pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (16, 4, 256, 130, 8, True), (20, 20, 40, 130, 1, False), (33, 3, 24, 121, 3, True),
+                                   (16, 8, 128, 384, 4, False), (24, 24, 40, 280, 1, False), (33, 3, 24, 221, 3, True)])
 def test_delta_prepare_of_many_channels(lib, sizes):
     """Blocks of 16 tokens: sequences that begin and end inside them, shorter than the convolution's reach and behind a state,
     padding rows, the last block's remainder; beside the kernel that takes a token a block (which few tokens run)."""
@@ -567,6 +568,41 @@ def test_delta_prepare_of_many_channels(lib, sizes):
         at += n
     alone = [slots[b] for b in range(len(lens)) if b != 3]
     assert torch.equal(whole_state[alone], want_state[alone])
+
+
+@pytest.mark.parametrize("sizes", [(16, 4, 256, 130, 8, True), (4, 2, 256, 96, 4, False), (5, 5, 40, 130, 3, False)])
+def test_delta_prepare_of_long_sequences(lib, sizes):
+    """Enough tokens for blocks of 16 of them whatever the columns: sequences that meet inside a block, beside the same in portions of 50
+    tokens, which the kernel with a token a block takes."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, taps, per_channel = sizes
+    C, per = 2 * G * D + H * V, D if per_channel else 1
+    columns = C + H * per
+    n = -(-(8_000_000 if D > 128 else 5_000_000) // columns)  # the line of the rule
+    lens = [n // 2 + 1, 7, n - n // 2, 33]
+    T, starts = sum(lens), [0] + list(np.cumsum(lens))
+    gen = torch.Generator().manual_seed(D)
+    proj, a = torch.randn(T, C + H, generator=gen).to(DEV), torch.randn(T, H * per, generator=gen).to(DEV)
+    conv_w = (0.5 * torch.randn(C, taps, generator=gen)).to(DEV)
+    a_log, dt_bias = (torch.randn(H, generator=gen) - 1).to(DEV), torch.randn(H * per, generator=gen).to(DEV)
+    state = torch.randn(len(lens), taps - 1, C, generator=gen).to(DEV)
+
+    def run(lo, hi, seqs, conv_state):
+        mine = torch.tensor(seqs, dtype=torch.int32)
+        ids = torch.repeat_interleave(torch.arange(len(seqs)), torch.tensor([hi - lo] if len(seqs) == 1 else lens)).to(torch.int32)
+        first = torch.tensor([0, hi - lo] if len(seqs) == 1 else starts, dtype=torch.int32)
+        return ops.delta_prepare(proj[lo:hi], C, a[lo:hi], 0, conv_w, a_log, dt_bias, conv_state, ids.to(DEV), mine.to(DEV), H, G, D, V,
+                                 per_channel, D ** -0.5, seq_starts=first.to(DEV), n_seqs=len(seqs))
+
+    left, want_left = state.clone(), state.clone()
+    got = run(0, T, list(range(len(lens))), left)
+    for b in range(len(lens)):
+        for lo in range(starts[b], starts[b + 1], 50):
+            hi = min(lo + 50, starts[b + 1])
+            for x, y in zip(got, run(lo, hi, [b], want_left)):
+                torch.testing.assert_close(x[lo:hi], y, atol=2e-6, rtol=2e-6)  # 24-bit sums of up to 8 and 256 terms in two orders
+    assert torch.equal(left, want_left)
 
 
 def test_a_lost_state_shows(lib):
