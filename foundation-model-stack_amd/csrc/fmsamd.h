@@ -6,7 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
-#define FMSAMD_ABI_VERSION 13
+#define FMSAMD_ABI_VERSION 14
 
 // element types
 #define FMS_F32 0
@@ -260,6 +260,18 @@ int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long ldo, void*
                             const int* positions, const int* seq_of_token, const int* block_table, int table_stride,
                             const void* cache, const void* vt_cache, const float* sink, int n_tokens, int nheads, int rank,
                             int rot, float scale, int window, int n_splits, hipStream_t stream);
+
+// ---- the same for prompts, with keys and values expanded for the step (latent_expanded.hip) ----------------------------
+// q: rows of every head's dim + rot elements, not yet rotated; uk [nheads * dim, rank], uv [nheads * vdim, rank]; keys and values:
+// room for n_seqs * pages * nheads * 64 * dim and * vdim elements, pages even and at least what the longest sequence holds.
+// qblock_start, qblock_len: the step's tokens in blocks of at most 64 of one sequence.  Bfloat16; gate: float32 logits, a row a token.
+int fmsamd_latent_prompt_fits(int dim, int rot, int vdim, int rank);
+int fmsamd_latent_prompt(const void* q, long ldq, void* out, long ldo, const void* cache, const void* uk, const void* uv,
+                         void* keys, void* values, const int* positions, const int* seq_of_token, const int* seq_starts,
+                         const int* qblock_start, const int* qblock_len, int n_qblocks, const int* block_table,
+                         int table_stride, int pages, const float* cos_t, const float* sin_t, const float* sink,
+                         const float* gate, long ldg, int n_seqs, int nheads, int dim, int rot, int vdim, int rank, float scale,
+                         int window, hipStream_t stream);
 
 // ---- experts (experts.hip) -----------------------------------------------------------------------------------------
 // ids: the `top` largest logits of every token; weights: FMS_ROUTE_SOFTMAX the softmax over the chosen logits,

@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads libamdhip64 before our library asks for it)
 
 from . import build as _build
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
@@ -61,6 +61,8 @@ _SIGNATURES = {
     "fmsamd_latent_q_rotate": [P, L, I, I, I, I, P, L, I, P, P, P, I, I, P],
     "fmsamd_headwise_linear": [P, L, L, P, P, L, L, P, L, I, I, I, I, I, P],
     "fmsamd_latent_attn_generic": [P, L, P, L, I, P, P, P, I, P, P, I, I, I, I, F, I, P],
+    "fmsamd_latent_prompt_fits": [I, I, I, I],
+    "fmsamd_latent_prompt": [P, L, P, L, P, P, P, P, P, P, P, P, P, P, I, P, I, I, P, P, P, P, L, I, I, I, I, I, I, F, I, P],
     "fmsamd_moe_route": [P, L, I, I, I, I, P, P, P],
     "fmsamd_moe_group": [P, I, I, P, P, I, I, P],
     "fmsamd_moe_experts": [I, P, L, P, P, P, I, P, P, I, I, I, I, I, F, F, F, P, I, P],

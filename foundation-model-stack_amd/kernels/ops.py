@@ -1177,6 +1177,93 @@ def latent_attention(qa: torch.Tensor, positions, seq_of_token, block_table, cac
     return out
 
 
+LATENT_PROMPT_QBLOCK = 64  # query tokens of a block of latent_prompt_attention
+LATENT_PROMPT_ROOM = 512 << 20  # bytes of expanded keys and values that a step may take
+
+
+def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int) -> bool:
+    """True if there is a kernel that attends to expanded keys and values of these sizes (the library says)."""
+    return bool(load().fmsamd_latent_prompt_fits(int(dim), int(rot), int(vdim), int(rank)))
+
+
+def latent_prompt_pages(longest: int) -> int:
+    """Pages of every sequence of a step in the room for expanded keys and values: a whole number of pairs."""
+    return -(-longest // (2 * PAGE_TOKENS)) * 2
+
+
+def latent_prompt_pays(starts: Sequence[int], lengths: Sequence[int], nheads: int, dim: int, rot: int, vdim: int, rank: int) -> bool:
+    """True if a step of these sequences (position of the first token, tokens) is faster with expanded keys and values than in the
+    latent space.  Expanding costs what the rows cost, every sequence's as many as the longest one's; measured 5 ns a row for 16 heads
+    of 128 and a latent of 512.  In the latent space the products in and out are launches of their own (10 us more than here for a
+    few tokens), every pair of query and key is a product over the latent twice, and a block of four (token, 16 heads) takes its sequences one after the
+    other, 24 ns a key.  Measured, us, expanded and not: one prompt of 32 tokens 18, 29, of 300 22, 40, of 2048 64, 190; 2 tokens behind
+    8000 180, 427; 100 tokens beside four single ones behind 2000 each 124, 414, beside sixteen of them 403, 426; thirty single
+    tokens behind 100 beside two of 20 tokens 66, 57.
+    """
+    contexts = [s + n for s, n in zip(starts, lengths)]
+    rows = len(contexts) * latent_prompt_pages(max(contexts)) * PAGE_TOKENS
+    if rows * nheads * (dim + vdim) * 2 > LATENT_PROMPT_ROOM:
+        return False
+    expand = rows * nheads * (dim + vdim) * rank / (16 * 256 * 512) * 5e-3
+    chain = max(max(contexts), sum(sorted((c for c, n in zip(contexts, lengths) if n < 4), reverse=True)[:4]))
+    pairs = sum(n * c - n * (n - 1) // 2 for c, n in zip(contexts, lengths))
+    return expand <= 10 + 24e-3 * chain + pairs * nheads * (2 * rank + rot) * 2 / 5.5e8
+
+
+def latent_prompt_aligned(q, uk, uv, cache, cos, sin, out) -> bool:
+    """True if latent_prompt_attention can read and write these tensors (whole pieces of 16 bytes, of 8 for `out`)."""
+    return (all(t is None or t.data_ptr() % 16 == 0 for t in (q, uk, uv, cache, cos, sin)) and q.stride(0) % 8 == 0
+            and (out is None or (out.data_ptr() % 8 == 0 and out.stride(0) % 4 == 0)))
+
+
+def latent_prompt_attention(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor, positions, seq_of_token, seq_starts, qblock_start, qblock_len,
+                            block_table, cache: torch.Tensor, cos, sin, sink: Optional[torch.Tensor], gate: Optional[torch.Tensor],
+                            nheads: int, dim: int, rot: int, vdim: int, rank: int, scale: float, window: int = 0, *, n_seqs: int,
+                            longest: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Causal attention of a prompt step over the latent cache, with the keys [Uk c | shared part] and values Uv c of every cached
+    row of the step's sequences formed first.  q: bfloat16 rows of every head's dim + rot elements, not rotated; uk
+    [nheads * dim, rank], uv [nheads * vdim, rank]; gate: float32 logits [T, >= nheads] whose sigmoid multiplies a head's result, or
+    None; longest: at least what the longest sequence holds with this step.  Returns [T, nheads * vdim] (into `out`, rows of any
+    stride)."""
+    _need_cuda(q, uk, uv, positions, seq_of_token, seq_starts, qblock_start, qblock_len, block_table, cache, cos, sin, sink, gate, out)
+    _rows2d("q", q)
+    T = q.shape[0]
+    if q.dtype != torch.bfloat16 or q.shape[1] != nheads * (dim + rot) or not latent_prompt_fits(dim, rot, vdim, rank):
+        raise ValueError(f"latent_prompt_attention takes bfloat16 rows of {nheads} heads and sizes that it has a kernel for, got {q.dtype} {tuple(q.shape)}")
+    for name, w, rows in (("uk", uk, nheads * dim), ("uv", uv, nheads * vdim)):
+        if w.dtype != q.dtype or tuple(w.shape) != (rows, rank) or not w.is_contiguous():
+            raise ValueError(f"{name} is a contiguous bfloat16 [{rows}, {rank}] tensor")
+    _check_batch_index(positions, seq_of_token, block_table, T)
+    for name, t in (("seq_starts", seq_starts), ("qblock_start", qblock_start), ("qblock_len", qblock_len)):
+        _need_i32(name, t)
+    if seq_starts.numel() < n_seqs + 1 or block_table.shape[0] < n_seqs or qblock_start.numel() != qblock_len.numel():
+        raise ValueError("the step's index arrays are shorter than its sequences")
+    _check_latent_cache(cache, rank + rot, q.dtype)
+    _check_tables(cos, sin, rot)
+    if sink is not None and (sink.dtype != torch.float32 or tuple(sink.shape) != (nheads,) or not sink.is_contiguous()):
+        raise ValueError(f"the sink is a contiguous float32 [{nheads}] tensor")
+    if gate is not None and (gate.dtype != torch.float32 or gate.dim() != 2 or gate.stride(1) != 1 or gate.shape[0] != T or gate.shape[1] < nheads):
+        raise ValueError("the gate is float32 [T, >= heads] with contiguous rows")
+    if out is None:
+        out = torch.empty(T, nheads * vdim, dtype=q.dtype, device=q.device)
+    _rows2d("out", out)
+    if out.dtype != q.dtype or tuple(out.shape) != (T, nheads * vdim):
+        raise ValueError(f"out is bfloat16 [{T}, {nheads * vdim}]")
+    pages = latent_prompt_pages(longest)
+    if longest <= 0 or -(-longest // PAGE_TOKENS) > block_table.shape[1]:
+        raise ValueError(f"sequences of {longest} tokens do not fit a block table of {block_table.shape[1]} pages")
+    keys = torch.empty(n_seqs * pages, nheads, PAGE_TOKENS, dim, dtype=q.dtype, device=q.device)
+    values = torch.empty(n_seqs * pages, nheads, vdim, PAGE_TOKENS, dtype=q.dtype, device=q.device)
+    check(load().fmsamd_latent_prompt(q.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0), cache.data_ptr(), uk.data_ptr(), uv.data_ptr(),
+                                      keys.data_ptr(), values.data_ptr(), positions.data_ptr(), seq_of_token.data_ptr(), seq_starts.data_ptr(),
+                                      qblock_start.data_ptr(), qblock_len.data_ptr(), qblock_start.numel(), block_table.data_ptr(),
+                                      block_table.stride(0), pages, _ptr(cos), _ptr(sin), _ptr(sink), _ptr(gate),
+                                      gate.stride(0) if gate is not None else 0, int(n_seqs), nheads, dim, rot, vdim, rank, float(scale), int(window),
+                                      _stream()))
+    return out
+
+
+
 # --------------------------------------------------------------------------
 # experts
 # --------------------------------------------------------------------------

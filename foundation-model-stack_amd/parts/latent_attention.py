@@ -3,9 +3,11 @@
 Every token leaves two things in the cache: the RMS-normed latent c (kv_rank numbers) and a rotated key part
 that all heads share (rot_dim numbers).  Head h's key is [Uk_h c | shared part], its value Uv_h c.  Because
 (Uk_h c) . q = c . (Uk_h^T q), the mixer never forms keys or values: it takes each head's query into the latent
-space, runs attention as one shared kv head over the cached rows, and takes the result out through Uv_h.  Whole
-prompts, portions of prompts and single tokens run the same kernels over the same cache, so how a sequence is cut
-into steps changes nothing beyond rounding.
+space, runs attention as one shared kv head over the cached rows, and takes the result out through Uv_h.  A prompt step in
+bfloat16 whose head sizes have a kernel for it forms keys and values for the step instead, where that is less work
+(ops.latent_prompt_pays): a pair of query and key is then a product over the head's size and not over the latent twice.
+Whole prompts, portions of prompts and single tokens share the same cache, so how a sequence is cut into steps changes nothing
+beyond rounding.
 
 Options, all constructor arguments: queries through a latent of their own with an RMS norm (q_rank; 0: the queries
 are one projection of the mixer's input), no rotated part at all (rot_dim 0, attention without positions), a sink logit
@@ -75,7 +77,7 @@ class LatentAttention(Mixer):
             self.declare("sink", (nheads,), init="zeros", kind="scale")
         self.o = self.add_child("o", Linear(nheads * vdim, width))
         self._uk_t = self._uv = self._sink = None
-        self._mfma = False  # decided when the model's type is known (finalize)
+        self._mfma = self._expands = False  # decided when the model's type is known (finalize)
 
     def unfused_parameters(self) -> dict:
         """The fused down-projection as the tensors it is made of, in the order of its rows (what the model's
@@ -99,9 +101,13 @@ class LatentAttention(Mixer):
         if self.position_encoder is not None:
             self.position_encoder.check_positions(max_position)
 
+    def prefill_qblock(self, n_tokens: int, dtype) -> int:
+        return ops.LATENT_PROMPT_QBLOCK if self._expands and dtype == torch.bfloat16 else 0
+
     def finalize(self, device, dtype) -> None:
         H, D, R, V = self.nheads, self.dim, self.kv_rank, self.vdim
         self._mfma = dtype == torch.bfloat16 and ops.latent_attention_fits_mfma(R, self.rot_dim) and (H * (R + self.rot_dim)) % 8 == 0
+        self._expands = self._mfma and self.scale > 0 and ops.latent_prompt_fits(D, self.rot_dim, V, R)
         # Uk_h^T as rows of K = dim contiguous elements: the product that takes a query into the latent space
         self._uk_t = self.w["uk.weight"].view(H, D, R).transpose(1, 2).contiguous()
         self._uv = self.w["uv.weight"].view(H, V, R)
@@ -144,6 +150,19 @@ class LatentAttention(Mixer):
             q = self.uq.forward(cq)
         else:
             q = down[:, : self.q_cols] if down.dtype == x.dtype else ops.cast_cols(down, 0, self.q_cols, x.dtype)
+        gate = down[:, self.gate_col : self.gate_col + self.gate_cols] if self.has_gate else None
+        qb_start, qb_len = batch.qblocks.get(ops.LATENT_PROMPT_QBLOCK, (None, None))
+        if (self._expands and not batch.is_decode and qb_start is not None
+                and ops.latent_prompt_aligned(q, self.w["uk.weight"], self.w["uv.weight"], cache.keys, cos, sin, out)
+                and ops.latent_prompt_pays(batch.starts, batch.q_lens, H, D, P, V, R)):
+            by_head = gate if self.gate_cols == H else None
+            into = out if gate is by_head else None
+            mixed = ops.latent_prompt_attention(q, self.w["uk.weight"], self.w["uv.weight"], batch.positions, batch.seq_of_token,
+                                                batch.seq_starts, qb_start, qb_len, table, cache.keys, cos, sin, self._sink, by_head, H, D, P, V, R,
+                                                self.scale, self.window, n_seqs=batch.n_seqs, longest=batch.max_context, out=into)
+            if gate is not by_head:  # a gate per output element
+                mixed = ops.gate_mul(mixed, gate, "sigmoid", out=out)
+            return BranchOutput(mixed, self.o)
         qa = torch.empty(T, H * (R + P), dtype=x.dtype, device=x.device)
         if P:
             ops.latent_q_rotate(q, qa, H, D, P, R, batch.positions, cos, sin)
@@ -152,7 +171,6 @@ class LatentAttention(Mixer):
                                             self.scale, self.window, decode=batch.is_decode, max_context=batch.context_bound,
                                             vt_cache=cache.values)
         mixed = torch.empty(T, H * V, dtype=x.dtype, device=x.device) if out is None else out
-        gate = down[:, self.gate_col : self.gate_col + self.gate_cols] if self.has_gate else None
         if self.gate_cols == H * V:  # a gate per output element: behind the product that leaves the latent space
             ops.headwise_linear(mixed_latent, R, self._uv, mixed, V)
             mixed = ops.gate_mul(mixed, gate, "sigmoid", out=out)

@@ -420,6 +420,68 @@ def test_latent_attention_of_prompts(lib, heads, rot, runs, window):
     assert float((got - want).norm() / want.norm()) < 0.01
 
 
+# keys and values expanded for the step: blocks of 64 queries and steps of 128 keys with one more and one less, portions behind cached
+# tokens, several sequences, windows that leave pages out, one head to three tiles of 128 columns
+@pytest.mark.parametrize("heads", [1, 3])
+@pytest.mark.parametrize("rot,gated", [(64, True), (0, False)])
+@pytest.mark.parametrize("runs,window", [([(0, 1)], 0), ([(0, 63), (0, 65), (0, 64)], 0), ([(0, 129), (127, 3), (128, 1), (200, 70)], 0),
+                                         ([(300, 150), (0, 31)], 40), ([(0, 257)], 100)])
+def test_latent_attention_with_expanded_keys(lib, heads, rot, gated, runs, window):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(17 * heads + rot)
+    D, V, R, scale = 128, 128, 72, 0.06
+    pages_of = [-(-(s + n) // 64) for s, n in runs]
+    order = torch.randperm(sum(pages_of) + 1, generator=gen).tolist()
+    table = torch.full((len(runs), max(pages_of)), -1, dtype=torch.int32)
+    cache = torch.randn(sum(pages_of) + 1, 1, 64, R + rot, generator=gen).to(torch.bfloat16)
+    for i, ((s, n), count) in enumerate(zip(runs, pages_of)):
+        for p in range(count):
+            if not window or (p + 1) * 64 > s - window + 1:  # a window has given the pages in front of it back
+                table[i, p] = order.pop()
+        last = int(table[i, count - 1])
+        cache[last, 0, (s + n - 1) % 64 + 1:] = float("nan")  # rows that no token has written
+    cache[order.pop()] = float("inf")  # nobody's page
+    T = sum(n for _, n in runs)
+    seq = torch.cat([torch.full((n,), i) for i, (_, n) in enumerate(runs)]).to(torch.int32)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in runs]).to(torch.int32)
+    starts = torch.tensor([0] + [sum(n for _, n in runs[: i + 1]) for i in range(len(runs))], dtype=torch.int32)
+    blocks = [(int(starts[i]) + at, min(64, n - at)) for i, (_, n) in enumerate(runs) for at in range(0, n, 64)]
+    q = torch.randn(T, heads * (D + rot), generator=gen).to(torch.bfloat16)
+    uk, uv = ((torch.randn(heads * size, R, generator=gen) * R ** -0.5).to(torch.bfloat16) for size in (D, V))
+    sink = torch.randn(heads, generator=gen) if gated else None
+    gate = torch.randn(T, heads + 2, generator=gen) if gated else None
+    angles = torch.arange(512)[:, None] * 10000.0 ** (-torch.arange(rot // 2) / max(rot // 2, 1))[None]
+    cos, sin = torch.cos(angles).contiguous(), torch.sin(angles).contiguous()
+    dev = lambda t: None if t is None else t.to(DEV)
+    wide = torch.full((T, heads * V + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    got = ops.latent_prompt_attention(dev(q), dev(uk), dev(uv), dev(pos), dev(seq), dev(starts), dev(torch.tensor([b for b, _ in blocks], dtype=torch.int32)),
+                                      dev(torch.tensor([n for _, n in blocks], dtype=torch.int32)), dev(table), dev(cache),
+                                      dev(cos) if rot else None, dev(sin) if rot else None, dev(sink), dev(gate), heads, D, rot, V, R, scale, window,
+                                      n_seqs=len(runs), longest=max(s + n for s, n in runs), out=wide[:, : heads * V]).double().cpu()
+    assert bool((wide[:, heads * V:] == 7.0).all())
+    want = torch.zeros(T, heads * V, dtype=torch.float64)
+    for t in range(T):
+        i, p = int(seq[t]), int(pos[t])
+        lo = max(0, p - window + 1) if window else 0
+        rows = torch.stack([cache[int(table[i, k // 64]), 0, k % 64] for k in range(lo, p + 1)]).double()
+        qt = q[t].double().view(heads, D + rot)
+        if rot:
+            u, w, c, s_ = qt[:, D::2], qt[:, D + 1 :: 2], cos[p].double(), sin[p].double()
+            qt = torch.cat([qt[:, :D], torch.stack([u * c - w * s_, w * c + u * s_], dim=2).flatten(1)], dim=1)
+        for h in range(heads):
+            k = torch.cat([rows[:, :R] @ uk[h * D : (h + 1) * D].double().T, rows[:, R:]], dim=1)
+            score = k @ qt[h] * scale
+            e = torch.exp(score - score.max())
+            total = e.sum() + (torch.exp(sink[h].double() - score.max()) if sink is not None else 0.0)
+            y = (e / total) @ (rows[:, :R] @ uv[h * V : (h + 1) * V].double().T)
+            want[t, h * V : (h + 1) * V] = y * (torch.sigmoid(gate[t, h].double()) if gate is not None else 1.0)
+    # A score is the sum of 192 products of rounded factors times the scale, some 0.06 * 14 * 2^-9 off; keys, the rotated query,
+    # probabilities, values and the result are rounded to bfloat16, 2^-9 of themselves each at most
+    assert float((got - want).abs().max()) <= 8 * 2.0 ** -9 * float(want.abs().max())
+    assert float((got - want).norm() / want.norm()) < 0.01
+
+
 # blocks of one to four sequences in any order, one of them twice, with padding rows between them; windows; one tile a token to three
 @pytest.mark.parametrize("heads", [5, 16, 40])
 @pytest.mark.parametrize("rot,window", [(64, 0), (0, 0), (64, 33)])
