@@ -278,10 +278,10 @@ __global__ void __launch_bounds__(GROUP_THREADS)
 
 // Rows of a tile.  The matrix-core kernels (wide_ok: bfloat16, everything aligned to 16 bytes) take large tiles where experts fill
 // more than one small one on average and read their weights twice, and there are pairs enough to give the compute units work in
-// large tiles.  Both products and the grouping, us, small tiles and large ones: 32 experts, 4 a token, width 2048, hidden 1024, 200
-// tokens (25 rows an expert) 94, 112, 300 tokens (38) 123, 112; 64 experts, 8 a token, hidden 768, 200 tokens (25) 143, 163, 300 (38)
-// 174, 170; 8 experts, 2 a token, width 768, hidden 2048, 256 tokens (512 pairs) 50, 60, 512 (1024 pairs) 63, 64; width 1024, hidden
-// 512, 512 tokens 31, 43, 1024 tokens 46, 44.
+// large tiles.  Both products and the grouping, us, small tiles and large ones, weights out of memory: 32 experts, 4 a token, width 2048,
+// hidden 1024, 150 tokens (18 rows an expert) 78, 85, 200 (25) 96, 88, 256 (32) 116, 89; 64 experts, 8 a token, hidden 768, 200 tokens
+// (25) 136, 144, 256 (32) 158, 147; 8 experts, 2 a token, width 768, hidden 2048, 256 tokens (512 pairs) 50, 57, 512 (1024 pairs) 63,
+// 63; width 1024, hidden 512, 512 tokens 26, 36, 1024 tokens 43, 38.
 #define TILE_BIG_PAIRS 1024
 extern "C" int fmsamd_moe_tile_rows(int n_pairs, int n_experts, int wide_ok) {
   if (!wide_ok) return TILE_ROWS;
@@ -325,6 +325,8 @@ struct ExpertArgs {
   int act;  // gate_up without up weights (w2 null): hidden = act(x W1^T), one of FMS_ACT_*
 };
 
+// (the matrix-core kernels look a tile's pairs and their factors up at the start: at the end, a row after the other, they are a chain of
+// round trips to memory, some 10 us of a large tile)
 __device__ __forceinline__ float pair_scale(const ExpertArgs& a, int sorted_row) {
   return a.in_scale ? a.in_scale[a.order[sorted_row]] : 1.f;
 }
@@ -389,15 +391,17 @@ __global__ void __launch_bounds__(TILE_THREADS) expert_down_fma_kernel(ExpertArg
 // column blocks of a tile follow one another on one of the eight dies (blocks are dealt to the dies in turn), the tiles of
 // an expert behind each other, so that rows and weights come from memory once.
 //
-// Few rows an expert (decode) are bound by the weights' bytes: tiles of 32 rows by 128 rows of W, two waves and three stages of
-// 20 KB a block, two blocks a compute unit.  Many rows (prompts) by the matrix unit, the weights' bytes and the start and end of
-// a block together: 128 rows by 256 rows of W.  Measured with 32 experts, 4 a token, width 2048, hidden 1024 (gate and up + down;
-// in brackets tiles of 16 rows, from 2048 on of 64, straight from memory): 8 tokens 28 + 16 us (69 + 29), 32 tokens 42 + 23 (76 +
-// 31; 6.4 TB/s), 128 tokens 44 + 24 (92 + 46), 2048 tokens 136 + 74 (445 + 225), 4096 tokens 217 + 130.
-// Also measured for 2048 tokens: 128 x 256 as waves of 64 x 64 142 + 73, 64 x 256 137 + 68 (4096: 241 + 145), 128 x 128 with two
-// blocks a compute unit 153 + 74, 128 x 512 154 + 77.
+// Few rows an expert (decode) are bound by the weights' bytes: tiles of 32 rows by 64 rows of W, one wave and three stages of 12 KB a
+// block, four blocks a compute unit.  Many rows (prompts) by the matrix unit, the rounds of blocks over the compute units and the start
+// and end of a block together: 128 rows by 256 rows of W; the waves whose rows a short tile does not have load for the others and
+// multiply nothing.  Blocks start their walk over K at different steps (expert_first_step).
+// Measured with weights out of memory, 32 experts, 4 a token, width 2048, hidden 1024, grouping, gate and up and down together (in
+// brackets the same without that start, with 128 rows of W a small block and the pairs looked up at the end of a block): 8 tokens 52 us
+// (65), 32 tokens 70 (89; 5.8 TB/s), 128 tokens 72 (92), 300 tokens 89 (111), 1000 140 (158), 2048 206 (230), 2277 with scaled inputs
+// 218 (253), 4096 334 (356).  Small tiles with four stages: 85 for 32 tokens; by 128 rows of W: 56 for 8 tokens, the rest as it is.
+// Large ones as waves of 64 x 64: 203 for 2048 tokens, 226 for 2277; 128 x 128 with two blocks a compute unit 224, 238.
 __device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles, int col_blocks, int& tile, int& col) {
-  const int total = a.tiles[3 * max_tiles - 2] * col_blocks;  // the tiles there are (group_kernel)
+  const int total = uniform_load(a.tiles + 3 * max_tiles - 2) * col_blocks;  // the tiles there are (group_kernel)
   const int per_die = (total + 7) / 8;
   const int at = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
   tile = at / col_blocks, col = at % col_blocks;
@@ -406,7 +410,7 @@ __device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles,
 
 // Are the weight rows of this tile loaded as bytes that are not read again?  Where a tile of 32 rows is the only one of its expert,
 // nobody else reads them; the other tiles of a popular expert do.  And with fewer blocks than compute units such loads take
-// longer.  Gate, up and down of 32 experts, 4 a token, width 2048, hidden 1024: 32 tokens 80 us (88 without the mark), one token 28
+// longer.  Gate, up and down of 32 experts, 4 a token, width 2048, hidden 1024 (measured when all blocks walked K from its start): 32 tokens 80 us (88 without the mark), one token 28
 // (33 with it), 128 tokens of which most go to a few experts 104 (118 with every load marked, 113 with none); 64 experts, 8 a token,
 // hidden 768, 128 such tokens 134 (163, 157).
 template <int BM>
@@ -417,30 +421,46 @@ __device__ __forceinline__ bool expert_reads_once(const ExpertArgs& a, int max_t
   return alone && a.tiles[3 * max_tiles - 2] * col_blocks >= EXPERT_COMPUTE_UNITS;
 }
 
+// The step of K that a block starts with: weight rows lie a multiple of kilobytes apart, and blocks that walk them in step crowd into few
+// memory channels (32 tokens of the above: gate and up 42 us instead of 60).  It goes with the expert and the columns alone (in the width of the large tiles' blocks), so
+// that a pair has the same bits in any tile.
+#define TILE_BIG_COLS 256
+__device__ __forceinline__ int expert_first_step(int e, int cols, int K) { return (5 * cols + 3 * e) % ((K + TL_BK - 1) / TL_BK); }
+
 template <int WM, int WN, int TM, int TN, int ST, bool GATED>
 __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_gate_up_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
   typedef TileLds<WM, WN, TM, TN, ST> S;
   __shared__ __attribute__((aligned(16))) bf16 lds[S::LDS_ELEMENTS];
+  __shared__ int pairs[S::BM];  // of the tile's rows
   int tile, col;
   if (!expert_place(a, max_tiles, col_blocks, tile, col)) return;
-  const int e = a.tiles[3 * tile], start = a.tiles[3 * tile + 1], rows = a.tiles[3 * tile + 2];
+  const int e = uniform_load(a.tiles + 3 * tile), start = uniform_load(a.tiles + 3 * tile + 1), rows = uniform_load(a.tiles + 3 * tile + 2);
+  const int own_pair = (int)threadIdx.x < S::BM ? a.order[start + ((int)threadIdx.x < rows ? threadIdx.x : 0)] : 0;
+  const float own_scale = (int)threadIdx.x < S::BM && a.in_scale ? a.in_scale[own_pair] : 1.f;
+  __shared__ float scales[S::BM];
+  if ((int)threadIdx.x < S::BM) pairs[threadIdx.x] = own_pair;
+  __syncthreads();
   const bf16* x = (const bf16*)a.x;
   const bf16* wg = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
   const bf16* wu = (const bf16*)a.w2 + (size_t)e * a.N * a.K;
   // gated: a wave's first TN / 2 tiles are gate columns, the others the up columns of the same elements
   const int n0 = col * (GATED ? S::BN / 2 : S::BN);
   f32x16 acc[TM][TN];
-  auto a_row = [&](int m) { return x + (size_t)(a.order[start + (m < rows ? m : 0)] / a.top) * a.ldx; };
+  const bool works = (int)(threadIdx.x / WAVE) / WN * TM * 32 < rows;
+  auto a_row = [&](int m) { return x + (size_t)(pairs[m] / a.top) * a.ldx; };
   auto w_row = [&](int n) {
     const int t = n / 32;
     const bool up = GATED && t % TN >= TN / 2;
     const int c = n0 + (GATED ? ((t / TN) * (TN / 2) + t % (TN / 2)) * 32 + n % 32 : n);
     return (up ? wu : wg) + (size_t)(c < a.N ? c : 0) * a.K;
   };
+  const int first = expert_first_step(e, n0 / (TILE_BIG_COLS / (GATED ? 2 : 1)), a.K);
   if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
-    tile_product_lds<WM, WN, TM, TN, ST, true>(a_row, w_row, a.K, lds, acc);
+    tile_product_lds<WM, WN, TM, TN, ST, true, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
   else
-    tile_product_lds<WM, WN, TM, TN, ST>(a_row, w_row, a.K, lds, acc);
+    tile_product_lds<WM, WN, TM, TN, ST, false, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
+  if ((int)threadIdx.x < S::BM) scales[threadIdx.x] = own_scale;
+  __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -448,7 +468,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
     for (int v = 0; v < 16; ++v) {
       const int m = ((wave / WN) * TM + i) * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
       if (m >= rows) continue;
-      const float sc = pair_scale(a, start + m);
+      const float sc = scales[m];
       bf16* to = (bf16*)a.y + (size_t)(start + m) * a.N;
       if constexpr (GATED) {
 #pragma unroll
@@ -471,19 +491,25 @@ template <int WM, int WN, int TM, int TN, int ST>
 __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_down_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
   typedef TileLds<WM, WN, TM, TN, ST> S;
   __shared__ __attribute__((aligned(16))) bf16 lds[S::LDS_ELEMENTS];
+  __shared__ int pairs[S::BM];  // of the tile's rows
   int tile, col;
   if (!expert_place(a, max_tiles, col_blocks, tile, col)) return;
-  const int e = a.tiles[3 * tile], start = a.tiles[3 * tile + 1], rows = a.tiles[3 * tile + 2];
+  const int e = uniform_load(a.tiles + 3 * tile), start = uniform_load(a.tiles + 3 * tile + 1), rows = uniform_load(a.tiles + 3 * tile + 2);
+  const int own_pair = (int)threadIdx.x < S::BM ? a.order[start + ((int)threadIdx.x < rows ? threadIdx.x : 0)] : 0;
   const int n0 = col * S::BN;
   const bf16* x = (const bf16*)a.x;
   const bf16* w = (const bf16*)a.w1 + (size_t)e * a.N * a.K;
   f32x16 acc[TM][TN];
+  const bool works = (int)(threadIdx.x / WAVE) / WN * TM * 32 < rows;
   auto a_row = [&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; };
   auto w_row = [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; };
+  const int first = expert_first_step(e, n0 / TILE_BIG_COLS, a.K);
   if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
-    tile_product_lds<WM, WN, TM, TN, ST, true>(a_row, w_row, a.K, lds, acc);
+    tile_product_lds<WM, WN, TM, TN, ST, true, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
   else
-    tile_product_lds<WM, WN, TM, TN, ST>(a_row, w_row, a.K, lds, acc);
+    tile_product_lds<WM, WN, TM, TN, ST, false, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
+  if ((int)threadIdx.x < S::BM) pairs[threadIdx.x] = own_pair;
+  __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -491,7 +517,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
     for (int v = 0; v < 16; ++v) {
       const int m = ((wave / WN) * TM + i) * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
       if (m >= rows) continue;
-      float* to = (float*)a.y + (size_t)a.order[start + m] * a.N;
+      float* to = (float*)a.y + (size_t)pairs[m] * a.N;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int n = n0 + ((wave % WN) * TN + j) * 32 + (lane & 31);
@@ -537,7 +563,7 @@ extern "C" int fmsamd_moe_experts(int stage, const void* x, long ldx, const void
     // the larger tiles are made for the matrix-core kernels only
     FMS_REQUIRE(mfma, "moe_experts: tiles of %d rows need bfloat16 rows aligned to 16 bytes", tile_rows);
     const int st = tile_rows == TILE_BIG_ROWS ? launch_lds<4, 2, 1, 4, 3>(stage, a, max_tiles, stream)
-                                              : launch_lds<1, 2, 1, 2, 3>(stage, a, max_tiles, stream);
+                                              : launch_lds<1, 1, 1, 2, 3>(stage, a, max_tiles, stream);
     if (st) return st;
   } else if (dtype == FMS_F32) {
     if (stage == 0) expert_gate_up_fma_kernel<float><<<grid, TILE_THREADS, 0, stream>>>(a);
