@@ -168,8 +168,12 @@ static void sgemm_launch(const float* a, long lda, const float* w, const float* 
 // k-values ahead, in rows of 128 bytes whose pieces of 16 bytes are XOR-swizzled with the row.  WM x WN places of TILE x TILE results,
 // two waves each: one has the even run of a step, the other the odd one.  The short sums of a step are converted and added
 // while the matrix unit works on the next.
+// A vector instruction costs a float32 product its own time (on this GPU a 64-bit one or a conversion 4.4 clocks, a 32-bit one 2.6, in
+// kernels of nothing else, beside the 64 of a 32x32x2 product), so the loop has little but the two a result and run that the sums in 64 bits
+// need: the steps are unrolled, so that places in LDS are constants and short sums stay where they are, and addresses advance in
+// the scalar unit.
 template <int TILE, int WM, int WN, int STAGES>
-__global__ void __launch_bounds__(2 * WM* WN* WAVE)
+__global__ void __launch_bounds__(2 * WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(TILE == 32 ? 4 : 6)))
     sgemm_lds_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
                      float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
   constexpr int WAVES = 2 * WM * WN, BM = TILE * WM, BN = TILE * WN, BK = 2 * SG_RUN;
@@ -177,7 +181,7 @@ __global__ void __launch_bounds__(2 * WM* WN* WAVE)
   constexpr int STAGE = (BM + BN) * BK;         // floats
   constexpr int ACC = TILE * TILE / WAVE;
   typedef float accv __attribute__((ext_vector_type(ACC)));
-  static_assert((BM + BN) % (8 * WAVES) == 0, "whole rounds of loads");
+  static_assert((BM + BN) % (8 * WAVES) == 0 && BM % 8 == 0, "whole rounds of loads, of x or of W");
   static_assert(BM * BN * 8 <= STAGES * STAGE * 4, "the waves of a place meet in the same LDS");
   __shared__ __attribute__((aligned(16))) float lds[STAGES * STAGE];
   const int per_die = (tiles + 7) / 8;
@@ -188,65 +192,78 @@ __global__ void __launch_bounds__(2 * WM* WN* WAVE)
   const int ks = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
   const int r = lane % TILE, kq = lane / TILE;
 
-  const int piece = (lane & 7) ^ ((lane >> 3) & 7);
-  const float* src[LOADS];
+  auto swizzle = [](int row) { return TILE == 32 ? (row >> 1) & 7 : row & 7; };
+  const char* base[LOADS];  // the same in all lanes: of the block's first row of x or of W
+  unsigned from[LOADS];     // bytes from there to this lane's piece (sgemm asks whether 32 bits hold them)
+  int piece[LOADS];
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    const int row = (wave * LOADS + i) * 8 + (lane >> 3);  // of x, then of W; a row that is not there is the first one
-    const bool of_x = row < BM;
-    const int at = of_x ? m0 + row : n0 + row - BM;
-    src[i] = (of_x ? a + (size_t)(at < M ? at : 0) * lda : w + (size_t)(at < N ? at : 0) * K) + piece * 4;
+    const int first = (wave * LOADS + i) * 8;  // of x, then of W
+    const bool of_x = first < BM;              // uniform
+    const int row = (of_x ? first : first - BM) + (lane >> 3), there = of_x ? M - m0 : N - n0;
+    piece[i] = ((lane & 7) ^ swizzle(row)) * 4;
+    base[i] = (const char*)(of_x ? a + (size_t)m0 * lda : w + (size_t)n0 * K);
+    from[i] = (unsigned)((row < there ? row : 0) * (of_x ? lda : (long)K) + piece[i]) * 4;  // a row that is not there is the first one
   }
   auto fetch = [&](int s, int stage) {  // past the end: zeros, so that every step has the same number of loads under way
     const int k0 = s * BK;
     const unsigned to = lds0 + stage * (STAGE * 4) + wave * LOADS * 1024;
     if (k0 + BK <= K) {  // uniform
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) load_to_lds(src[i] + k0, to + i * 1024);
+      for (int i = 0; i < LOADS; ++i) load_to_lds(base[i] + (size_t)k0 * 4, from[i], to + i * 1024);
     } else {
-      const bool in = k0 + piece * 4 < K;
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) load_to_lds(in ? (const void*)(src[i] + k0) : (const void*)tile_zeros, to + i * 1024);
+      for (int i = 0; i < LOADS; ++i)
+        load_to_lds(k0 + piece[i] < K ? (const void*)(base[i] + (size_t)k0 * 4 + from[i]) : (const void*)tile_zeros, to + i * 1024);
     }
   };
 
   double total[ACC];
-  accv last;  // the short sums of the step before
+  accv sums[2];  // the short sums of this step and of the one before
 #pragma unroll
-  for (int e = 0; e < ACC; ++e) total[e] = 0.0, last[e] = 0.f;
-  auto add = [&]() {
-#pragma unroll
-    for (int e = 0; e < ACC; ++e) total[e] += (double)last[e];
-  };
+  for (int e = 0; e < ACC; ++e) total[e] = 0.0, sums[0][e] = sums[1][e] = 0.f;
   const int steps = (K + BK - 1) / BK;
   for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
-  int stage = 0;
-  for (int s = 0; s < steps; ++s) {
+  constexpr int PARTS = TILE / 16;  // pieces of 16 bytes that a lane has of its row's run
+  int x_at[PARTS], w_at[PARTS];
+#pragma unroll
+  for (int g = 0; g < PARTS; ++g) {
+    const int at = r * BK + ((ks * 4 + g * (WAVE / TILE) + kq) ^ swizzle(r)) * 4;
+    x_at[g] = wm * TILE * BK + at, w_at[g] = (BM + wn * TILE) * BK + at;
+  }
+  auto step = [&](int s, int stage, accv& sum, const accv& last) {
     tile_wait<(STAGES - 2) * LOADS>();  // step s is there, and everybody is done with step s - 1
     fetch(s + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
-    const float* base = lds + stage * STAGE;
-    constexpr int PARTS = TILE / 16;  // pieces of 16 bytes that a lane has of its row's run
     f32x4 xv[PARTS], wv[PARTS];
 #pragma unroll
     for (int g = 0; g < PARTS; ++g) {
-      const int at = r * BK + ((ks * 4 + g * (WAVE / TILE) + kq) ^ (r & 7)) * 4;
-      xv[g] = *reinterpret_cast<const f32x4*>(base + wm * TILE * BK + at);
-      wv[g] = *reinterpret_cast<const f32x4*>(base + (BM + wn * TILE) * BK + at);
+      xv[g] = *reinterpret_cast<const f32x4*>(lds + stage * STAGE + x_at[g]);
+      wv[g] = *reinterpret_cast<const f32x4*>(lds + stage * STAGE + w_at[g]);
     }
     __builtin_amdgcn_sched_barrier(0);  // all pieces are asked for before the first product (5% at 128 rows by 32000)
-    accv sum;
 #pragma unroll
     for (int e = 0; e < ACC; ++e) sum[e] = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int g = 0; g < PARTS; ++g) sum = sgemm_mfma<TILE>(xv[g][e], wv[g][e], sum);
-    add();
-    last = sum;
-    stage = stage == STAGES - 1 ? 0 : stage + 1;
+#pragma unroll
+    for (int e = 0; e < ACC; ++e) total[e] += (double)last[e];
+  };
+  constexpr int ROUND = STAGES % 2 ? 2 * STAGES : STAGES;  // steps after which places and short sums are where they were
+  for (int s0 = 0; s0 < steps; s0 += ROUND) {
+#pragma unroll
+    for (int u = 0; u < ROUND; ++u)
+      if (s0 + u < steps) step(s0 + u, u % STAGES, sums[u & 1], sums[~u & 1]);  // uniform
   }
-  add();
+  if (steps & 1) {
+#pragma unroll
+    for (int e = 0; e < ACC; ++e) total[e] += (double)sums[0][e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < ACC; ++e) total[e] += (double)sums[1][e];
+  }
   tile_wait<0>();
 
   // the odd runs' sums, to the waves that have the even ones'
@@ -275,14 +292,14 @@ static void sgemm_lds_launch(const float* a, long lda, const float* w, const flo
 
 // The tile shape.  What a compute unit needs for its blocks was measured at K = 4096 (8 to 512 rows of x, 4096 to 32000 of W):
 // the first block costs `first` microseconds, every further one `next`, whatever the rows.  Small tiles fill the chip where
-// there are few rows, large ones read less from LDS and the caches per product (60 TFLOP/s of 16 x 16, 95 of 32 x 32, 105 of
-// 32 x 64; blocks of 64 x 64 are within two per cent of the last and were taken out).  Rows that are not 16-byte aligned have
+// there are few rows, large ones read less from LDS and the caches per product (301 rows by 32000: 73 TFLOP/s of 16 x 16, 85 of 32 x 32, 92 of
+// 32 x 64; blocks of 64 x 64 and of 64 x 32 are within two per cent of the last, with four stages it takes a tenth longer).  Rows that are not 16-byte aligned have
 // tiles of their own.
 struct SgemmShape {
   int bm, bn;
   float first, next;
 };
-static const SgemmShape SGEMM_SHAPES[3] = {{16, 16, 22.f, 8.5f}, {32, 32, 40.f, 22.5f}, {32, 64, 67.f, 40.f}};
+static const SgemmShape SGEMM_SHAPES[3] = {{16, 16, 22.f, 8.5f}, {32, 32, 39.f, 24.f}, {32, 64, 58.f, 45.f}};
 static const SgemmShape SGEMM_UNALIGNED[2] = {{16, 16, 34.f, 28.f}, {32, 32, 126.f, 45.f}};
 #define SGEMM_COMPUTE_UNITS 256
 
@@ -301,10 +318,12 @@ static int sgemm_shape(const SgemmShape (&shapes)[SHAPES], int M, int N) {
   return best;
 }
 
+#define SGEMM_NEAR (1 << 23)  // 64 rows of so many floats
 static void sgemm(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K, bool aligned,
                   hipStream_t stream) {
   if (aligned) {
-    switch (sgemm_shape(SGEMM_SHAPES, M, N)) {
+    const bool near = lda < SGEMM_NEAR && K < SGEMM_NEAR;  // a tile's rows lie within 32 bits of bytes
+    switch (near ? sgemm_shape(SGEMM_SHAPES, M, N) : 0) {
       case 0: sgemm_launch<16, 8, 1, true>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
       case 1: sgemm_lds_launch<16, 2, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
       default: sgemm_lds_launch<32, 1, 2, 3>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
@@ -323,10 +342,10 @@ static void sgemm(const float* a, long lda, const float* w, const float* bias, f
 // What one launch takes: its threads are counted in 32 bits (and wrap round silently), at most two for a result.
 #define SGEMM_LAUNCH_TILES (1 << 22)  // of 16 x 16 results
 
-// Bound by the matrix unit's float32 rate (154 TFLOP/s for the vendor's product of 8192^3, 100 here; without the conversions and
-// additions in float64 the same); with few rows by the weights' bytes.  301 rows, K 4096: 610 us for 22016 rows of W (89
-// TFLOP/s; 2450 with one float32 product a thread and instruction), 126 for 4096 (140 in blocks of 32 x 64); 160 rows: 315 for
-// 22016, 81 for 4096 (92 in tiles of 16 x 16); 8 rows: 40 us for 12288 rows of W (5.0 TB/s), 27 for 4096.
+// Bound by the matrix unit's float32 rate (154 TFLOP/s for the vendor's product of 8192^3) and the vector instructions beside it, which
+// take its time: with the 32 that the sums in 64 bits are for a run of 32 x 32 results some 120 would be left, and 110 are reached
+// for 2048 rows (99 with the 57 of a loop that moved short sums and addresses); with few rows by the weights' bytes.  301 rows, K 4096: 630 us for 22016 rows of W (705),
+// 134 for 4096 (144); 160 rows: 326 for 22016 (370), 82 for 4096 (85); 8 rows: 39 us for 12288 rows of W (5.0 TB/s), 23 for 4096.
 extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
                                int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;

@@ -622,6 +622,21 @@ def test_gemm_f32_rows_keep_their_bits(ops, K):
     assert torch.equal(ops.linear(x, w[:100], b[:100]), whole[:, :100])
 
 
+def test_gemm_f32_of_rows_far_apart(ops):
+    """Rows of x 2^23 floats apart and one float less: a tile's rows lie past 32 bits of bytes, and just within them."""
+    if torch.cuda.mem_get_info()[0] < 8e9:
+        pytest.skip("needs 8 GB of memory")
+    torch.manual_seed(64)
+    M, N, K = 130, 4100, 64
+    x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
+    want = ops.linear(x, w, None)
+    for stride in ((1 << 23) + 4, (1 << 23) - 4):
+        far = torch.empty(M * stride, device="cuda").as_strided((M, K), (stride, 1)).copy_(x)
+        assert torch.equal(ops.linear(far, w, None), want)
+        del far
+    torch.cuda.empty_cache()
+
+
 def test_gemm_f32_of_more_results_than_a_launch_has_threads(ops):
     """1.7e10 results (69 GB): the threads of one launch are counted in 32 bits."""
     torch.cuda.empty_cache()
