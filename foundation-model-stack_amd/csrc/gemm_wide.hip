@@ -78,9 +78,11 @@ __global__ void __launch_bounds__(512)
   const int pair = wave >> 1, side = wave & 1;  // the wave's row of waves, and which of its two waves it is
 
   // what the wave loads of a step: RX instructions of 8 rows of x (with few rows some waves load the same ones) and RW of 8
-  // weight rows.  Which piece of its row a lane asks for is swizzled with the row; a row that is not there is one that is.
+  // weight rows.  Which piece of its row a lane asks for is swizzled with half the row's number (tile_product_lds.h; the groups of 8 rows that a
+  // wave loads are all even or all odd ones); a row that is not there is one that is.
   constexpr int GX = XROWS / 8, RX = (GX + 7) / 8, RW = WD_ROWS / 64, R = RX + RW;
-  const int lrow = lane >> 3, piece = (lane & 7) ^ lrow;
+  const int lrow = lane >> 3, piece = (lane & 7) ^ ((wave & 1) * 4 + (lrow >> 1));
+  static_assert(GX % 2 == 0, "even groups of rows of x stay even");
   const bf16* src[R];
   unsigned put[R];
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -193,7 +195,7 @@ __global__ void __launch_bounds__(512)
     const bf16* const xs = reinterpret_cast<const bf16*>(smem) + stage * STAGE;
     const bf16* const ws = xs + (XROWS + pair * 32) * BK;
     auto operand = [&](const bf16* rows32, int st) {
-      return *reinterpret_cast<const bf16x8*>(rows32 + li * BK + ((st * 2 + kb) ^ (li & 7)) * 8);
+      return *reinterpret_cast<const bf16x8*>(rows32 + li * BK + ((st * 2 + kb) ^ ((li >> 1) & 7)) * 8);
     };
     bf16x8 a[4];
 #pragma unroll
