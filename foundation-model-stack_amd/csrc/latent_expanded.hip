@@ -96,15 +96,24 @@ struct PromptArgs {
   float scale2;  // times log2(e)
 };
 
+// In one instruction: fmaxf passes every operand through a maximum with itself first, to quiet a signalling NaN, which the matrix unit
+// does not make.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // Scores S^T = K Q^T of 32 keys by 32 queries, O^T += V^T P^T, both 32x32x16: the lane layout is that of the prompts' attention with
 // head sizes up to 128 (attention.hip).  A block is 64 queries of one head and walks 128 keys a step: two runs of 32 queries by four
-// runs of 32 keys, whose waves meet at the end.  (Blocks of 128 queries by 64 keys take as long a step, but their longest is
-// twice as many steps, and with one sequence of 2048 tokens the longest block is what the kernel takes.)  The longest blocks go
-// first; the heads follow one another on the dies (blocks are dealt to them in turn), so that a head's keys stay in one L2.
-// 16 heads of 128 + 64: 8 us for 32 tokens, 22 for 1000, 48 for 2048, 476 for 8192; in the latent space 10, 62, 134 and 1751, with 17 to
+// runs of 32 keys, whose waves meet at the end.  (Blocks of 128 queries by 64 keys, three pages ahead in LDS: 15 us for 300 tokens, 29 for
+// 1000, 51 for 2048, 385 for 8192: with one sequence the longest block, of twice as many steps, is what the kernel takes.)  The
+// longest blocks go first; the heads follow one another on the dies (blocks are dealt to them in turn), so that a head's keys stay in one L2.
+// 16 heads of 128 + 64: 8 us for 32 tokens, 12 for 300, 22 for 1000, 46 for 2048, 456 for 8192; in the latent space 10, 62, 134 and 1751, with 17 to
 // 55 us more for the products into the latent space and out of it.
 // Keys, shared parts and values go from memory straight into LDS, one step ahead: 80 KB a step for 128 + 64 and 128, twice, is all of a
-// compute unit's LDS.  Their pieces of 16 bytes are XOR-swizzled with the row so that operand reads cover all banks.
+// compute unit's LDS.  Their pieces of 16 bytes are XOR-swizzled with the row, so that the operand reads of 16 neighbouring rows cover
+// all 64 banks (with 8 of them 48 us for 2048 tokens and 476 for 8192).
 // NC, RC: pieces of 16 of a key's own and shared part; DT: tiles of 32 value elements.
 template <int NC, int RC, int DT>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) latent_prompt_kernel(PromptArgs a) {
@@ -113,7 +122,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int KN_LOADS = KN_BYTES / 8192, KR_LOADS = KR_BYTES / 8192, V_LOADS = V_BYTES / 8192;  // of 1 KB, a wave
   constexpr int KN_PIECES = D / 8, KR_PIECES = P > 0 ? P / 8 : 8;
   static_assert(KN_BYTES % 8192 == 0 && KR_BYTES % 8192 == 0 && V_BYTES % 8192 == 0, "whole loads");
-  static_assert(KN_PIECES % 8 == 0 && KR_PIECES % 8 == 0 && 64 % KN_PIECES == 0 && 64 % KR_PIECES == 0, "whole groups of pieces, whole rows a load");
+  static_assert((KN_PIECES == 16 || KN_PIECES == 8) && KR_PIECES == 8 && 64 % KN_PIECES == 0 && 64 % KR_PIECES == 0, "whole groups of pieces, whole rows a load");
   static_assert(2 * STAGE <= 160 * 1024 && 6 * (DT * 16 + 2) * 256 <= 2 * STAGE, "a compute unit's LDS; the waves meet in it");
   extern __shared__ __attribute__((aligned(16))) unsigned char lx_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -155,7 +164,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 
   // what this lane loads: which row of a load's and which piece of it
-  auto key_swizzle = [](int key) { return (key & 3) | ((key >> 1) & 4); };
+  // (rows of 256 bytes by their number, rows of 128 by half of it: sixteen neighbouring rows then cover all 64 banks)
+  auto swizzle = [](int row, int pieces) { return pieces == 16 ? row & 15 : (row >> 1) & 7; };
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lx_lds;
   const size_t page_keys = (size_t)a.H * PAGE_TOKENS * D, page_values = (size_t)a.H * V * PAGE_TOKENS;
   const int half = wave >> 2;  // the page of the two whose keys this wave loads
@@ -163,30 +173,30 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
   for (int n = 0; n < KN_LOADS; ++n) {
     const int key = (wave * KN_LOADS + n) * (64 / KN_PIECES) + lane / KN_PIECES;
-    kn_from[n] = ((key & 63) * D + ((lane % KN_PIECES) ^ key_swizzle(key)) * 8) * 2;
+    kn_from[n] = ((key & 63) * D + ((lane % KN_PIECES) ^ swizzle(key, KN_PIECES)) * 8) * 2;
   }
 #pragma unroll
   for (int n = 0; n < (RC > 0 ? KR_LOADS : 0); ++n) {
     const int key = (wave * KR_LOADS + n) * (64 / KR_PIECES) + lane / KR_PIECES;
-    kr_from[n] = ((key & 63) * (a.rank + P) + a.rank + ((lane % KR_PIECES) ^ key_swizzle(key)) * 8) * 2;
+    kr_from[n] = ((key & 63) * (a.rank + P) + a.rank + ((lane % KR_PIECES) ^ swizzle(key, KR_PIECES)) * 8) * 2;
   }
 #pragma unroll
   for (int n = 0; n < V_LOADS; ++n) {
-    const int d = (wave * V_LOADS + n) * 4 + (lane >> 4), piece = (lane & 15) ^ (d & 7);
+    const int d = (wave * V_LOADS + n) * 4 + (lane >> 4), piece = (lane & 15) ^ swizzle(d, 16);
     v_from[n] = (unsigned)((piece >> 3) * page_values + d * PAGE_TOKENS + (piece & 7) * 8) * 2;
   }
   const char* const own_keys = (const char*)(a.keys + ((size_t)seq * a.pages + half) * page_keys + (size_t)h * PAGE_TOKENS * D);
   const char* const own_values = (const char*)(a.values + (size_t)seq * a.pages * page_values + (size_t)h * V * PAGE_TOKENS);
-  auto fetch = [&](int step, int buffer) {
+  // (the second page of the last step may not be there: nobody sees its keys)
+  auto entry_of = [&](int step) { return RC > 0 ? uniform_load(bt + step * 2 + (step * LX_STEP + half * PAGE_TOKENS <= blk_last ? half : 0)) : 0; };
+  auto fetch = [&](int step, int buffer, int entry) {
     const unsigned to = lds0 + buffer * STAGE;
     const char* const kp = own_keys + (size_t)step * 2 * page_keys * 2;
     const char* const vp = own_values + (size_t)step * 2 * page_values * 2;
 #pragma unroll
     for (int n = 0; n < KN_LOADS; ++n) load_to_lds(kp, kn_from[n], to + (wave * KN_LOADS + n) * 1024);
     if constexpr (RC > 0) {
-      // (the second page of the last step may not be there: nobody sees its keys)
-      const int page = step * 2 + (step * LX_STEP + half * PAGE_TOKENS <= blk_last ? half : 0);
-      const char* const rp = (const char*)(a.cache + readable_page(uniform_load(bt + page)) * PAGE_TOKENS * (size_t)(a.rank + P));
+      const char* const rp = (const char*)(a.cache + readable_page(entry) * PAGE_TOKENS * (size_t)(a.rank + P));
 #pragma unroll
       for (int n = 0; n < KR_LOADS; ++n) load_to_lds(rp, kr_from[n], to + KN_BYTES + (wave * KR_LOADS + n) * 1024);
     }
@@ -197,7 +207,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   // operand reads.  Which key sits in which row of a score tile is free: dealt so that lane half hb holds the probabilities of the
   // keys 8 hb .. 8 hb + 7 and 16 + 8 hb .. of the 32, each eight an operand of the second product as they are
   const int key_row = quarter * 32 + 16 * (j >> 4) + 8 * ((j >> 2) & 1) + 4 * ((j >> 3) & 1) + (j & 3);
-  const int k_swizzle = key_swizzle(key_row);
+  const int n_swizzle = swizzle(key_row, KN_PIECES), r_swizzle = swizzle(key_row, KR_PIECES);
 
   f32x16 acc[DT];
 #pragma unroll
@@ -207,11 +217,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   float m = -1e30f, l = 0.f;
 
   const int step_first = lowest(blk_first) / LX_STEP, step_last = blk_last / LX_STEP;
-  fetch(step_first, 0);
-  int buffer = 0;
+  fetch(step_first, 0, entry_of(step_first));
+  int buffer = 0, entry = step_first < step_last ? entry_of(step_first + 1) : 0;  // a step before it is needed
   for (int step = step_first; step <= step_last; ++step, buffer ^= 1) {
     tile_wait<0>();  // the step is there, and everybody has read the one before
-    if (step < step_last) fetch(step + 1, buffer ^ 1);
+    if (step < step_last) fetch(step + 1, buffer ^ 1, entry);
+    if (step + 1 < step_last) entry = entry_of(step + 2);
     const int key0 = step * LX_STEP + quarter * 32;
     if (!has_work || key0 > wave_hi || key0 + 31 < wave_lo) continue;  // the same in all lanes
     const unsigned char* const kn = lx_lds + buffer * STAGE + key_row * (D * 2);
@@ -223,12 +234,20 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     {
       bf16x8 k[NC + RC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) k[c] = *reinterpret_cast<const bf16x8*>(kn + ((2 * c + hb) ^ k_swizzle) * 16);
+      for (int c = 0; c < NC; ++c) k[c] = *reinterpret_cast<const bf16x8*>(kn + ((2 * c + hb) ^ n_swizzle) * 16);
 #pragma unroll
-      for (int c = 0; c < RC; ++c) k[NC + c] = *reinterpret_cast<const bf16x8*>(kr + ((2 * c + hb) ^ k_swizzle) * 16);
+      for (int c = 0; c < RC; ++c) k[NC + c] = *reinterpret_cast<const bf16x8*>(kr + ((2 * c + hb) ^ r_swizzle) * 16);
+      __builtin_amdgcn_sched_barrier(0);  // all of them are asked for before the first product
 #pragma unroll
       for (int c = 0; c < NC + RC; ++c) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[c], q[c], sc, 0, 0, 0);
     }
+    bf16x8 values[DT][2];  // on their way during the softmax
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        values[dt][n] = *reinterpret_cast<const bf16x8*>(vs + (dt * 32 + j) * (LX_STEP * 2) + ((quarter * 4 + 2 * n + hb) ^ swizzle(j, 16)) * 16);
+    __builtin_amdgcn_sched_barrier(0);
     if (!(key0 + 31 <= full_hi && key0 >= full_lo)) {  // the same in all lanes
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -236,12 +255,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         sc[v] = key <= pos && key >= lo ? sc[v] : -INFINITY;
       }
     }
-    float top = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-    top = fmaxf(top, fmaxf(fmaxf(fmaxf(sc[8], sc[9]), fmaxf(sc[10], sc[11])), fmaxf(fmaxf(sc[12], sc[13]), fmaxf(sc[14], sc[15]))));
+    float top = max3(max3(sc[0], sc[1], sc[2]), max3(sc[3], sc[4], sc[5]), max3(sc[6], sc[7], sc[8]));
+    top = max3(top, max3(sc[9], sc[10], sc[11]), max3(sc[12], sc[13], max3(sc[14], sc[15], sc[15])));
     {
       const unsigned u = __float_as_uint(top);
       const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // the column's other lane
-      top = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+      top = max3(__uint_as_float(halves[0]), __uint_as_float(halves[1]), __uint_as_float(halves[1]));
     }
     const float m_new = fmaxf(m, top * a.scale2);  // (the scale is positive)
     const float alpha = __builtin_amdgcn_exp2f(m - m_new);
@@ -262,13 +281,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
     }
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(vs + (dt * 32 + j) * (LX_STEP * 2) + ((quarter * 4 + 2 * n + hb) ^ (j & 7)) * 16);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, p[n], acc[dt], 0, 0, 0);
-      }
-    }
+      for (int n = 0; n < 2; ++n) acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(values[dt][n], p[n], acc[dt], 0, 0, 0);
   }
   __syncthreads();  // everybody has read the last step
 
