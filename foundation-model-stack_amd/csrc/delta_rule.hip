@@ -9,7 +9,7 @@
 //   delta_prepare:  the short causal convolution over time of the q, k and v channels (inputs before the step come
 //                   from the sequence's state, zeros before its start), silu, unit vectors per q and k head, q's scale,
 //                   beta = sigmoid, g = exp(-exp(A_log) softplus(a + dt_bias)).
-//   conv_state:     the last (taps - 1) inputs of every sequence go into its state.
+//   conv_state:     the last (taps - 1) inputs of every sequence go into its state (a decode step's delta_prepare does that itself).
 //   delta_rule:     the recurrence.  Columns of S never mix (each value channel is a recurrence of its own), so a wave
 //                   owns a few columns of one head of one sequence: 16 (or 32) lanes share a column, each with a run of
 //                   its rows in registers.  The wave walks over the sequence's tokens; q, k and g of a run of tokens are
@@ -28,8 +28,8 @@
 
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.f / (1.f + expf(-z)); }
 
-// Blocks of 1024 threads for steps of few tokens (a decode step has a block per token and nothing else to hide a
-// load's latency behind: the fewer passes a thread makes, the fewer round trips to memory follow one another).
+// Blocks of 1024 threads for steps of few tokens (short prompts, and callers that do not say where sequences start: a block per token
+// and nothing else to hide a load's latency behind: the fewer passes a thread makes, the fewer round trips to memory follow one another).
 template <typename W>
 __global__ void __launch_bounds__(1024)
     delta_prepare_kernel(const float* __restrict__ proj, long ld, int col_b, const float* __restrict__ a, long lda, int col_a,
@@ -46,8 +46,7 @@ __global__ void __launch_bounds__(1024)
   const int C = 2 * G * D + H * Dv;
   const int have = tokens_before(seq_of_token, t, seq, taps);
   const float* state = conv_state + (size_t)slot * (taps - 1) * C;
-  // two channels a thread and pass, all their taps asked for before any is used: a decode step has a block per token
-  // and nothing else to hide a load's latency behind
+  // two channels a thread and pass, all their taps asked for before any is used
   for (int c0 = threadIdx.x; c0 < C; c0 += 2 * blockDim.x) {
     float x[2][DELTA_MAX_TAPS], w[2][DELTA_MAX_TAPS];
 #pragma unroll
@@ -213,6 +212,108 @@ __global__ void __launch_bounds__(256)
     const int col = (c < D ? 0 : G * D - D) + unit * D + c;
     for (int i = 0; i < n; ++i)
       if (own[i] >= 0) qkv[(size_t)(tb + i) * C + col] = y[i * stride + c] * inv[c < D ? 0 : 1][i];
+  }
+}
+
+// The same for a decode step, which also moves the convolution's state on: a block takes a sequence and the channels of a q head and
+// its k head, blockDim value channels, or as many decays (and the betas).  A channel's window of inputs belongs to one thread, which
+// reads it from the state, walks the sequence's tokens (one in a decode step) and writes it back, so no second kernel has to follow
+// the last reader.  What bounds such a step is the chain of round trips of a block and the launches, not the bytes: a block of all
+// channels takes them in passes.  8 sequences of 4096 channels (16 value heads of 128): 12.1 us and 4.5 us for the state behind it,
+// 4.9 us here.
+template <typename W>
+__global__ void __launch_bounds__(512)
+    delta_prepare_seqs_kernel(const float* __restrict__ proj, long ld, int col_b, const float* __restrict__ a, long lda, int col_a,
+                              const W* __restrict__ conv_w, int taps, const float* __restrict__ a_log,
+                              const float* __restrict__ dt_bias, float* __restrict__ conv_state, const int* __restrict__ seq_starts,
+                              const int* __restrict__ seq_of_token, const int* __restrict__ slot_ids, float* __restrict__ qkv,
+                              float* __restrict__ beta, float* __restrict__ decay, float* __restrict__ kq, int H, int G, int D, int Dv,
+                              int per_channel, float q_scale) {
+  extern __shared__ float y[];  // q and k of a token
+  __shared__ float inv[2];
+  const int b = blockIdx.x, tid = threadIdx.x, threads = blockDim.x;
+  const int C = 2 * G * D + H * Dv, v_units = (H * Dv + threads - 1) / threads;
+  const int unit = blockIdx.y;
+  const int t0 = seq_starts[b], t1 = seq_starts[b + 1];
+  const int slot_b = slot_ids[b];
+  if (t0 >= t1) return;
+
+  if (unit >= G + v_units) {  // decays and betas
+    const int per = per_channel ? D : 1, c = (unit - G - v_units) * threads + tid;
+    for (int t = t0; t < t1; ++t) {
+      if (seq_of_token[t] < 0) continue;
+      if (unit == G + v_units)
+        for (int h = tid; h < H; h += threads) beta[(size_t)t * H + h] = sigmoid_f32(proj[(size_t)t * ld + col_b + h]);
+      if (c < H * per)
+        decay[(size_t)t * H * per + c] = expf(-expf(a_log[c / per]) * softplus_f32(a[(size_t)t * lda + col_a + c] + dt_bias[c]));
+    }
+    return;
+  }
+
+  const bool values = unit >= G;
+  int c = -1;  // this thread's channel
+  if (values) {
+    const int v = (unit - G) * threads + tid;
+    if (v < H * Dv) c = 2 * G * D + v;
+  } else if (tid < 2 * D) {
+    c = (tid < D ? 0 : G * D - D) + unit * D + tid;
+  }
+  const bool live = c >= 0;
+  float w[DELTA_MAX_TAPS], x[DELTA_MAX_TAPS] = {};  // x: the inputs a token's taps meet, the token's own last
+#pragma unroll
+  for (int j = 0; j < DELTA_MAX_TAPS; ++j) w[j] = j < taps && live ? to_f32(conv_w[(size_t)c * taps + j]) : 0.f;
+  float* state = nullptr;
+  int before = -1;  // the last token's sequence
+  for (int t = t0; t < t1; ++t) {
+    const float fresh = live ? proj[(size_t)t * ld + c] : 0.f;
+    const int seq = seq_of_token[t];
+    const bool first = seq != before;
+    before = seq;
+    if (seq < 0) continue;
+    if (first) {
+      state = conv_state + (size_t)(seq == b ? slot_b : slot_ids[seq]) * (taps - 1) * C;
+#pragma unroll
+      for (int j = 0; j < DELTA_MAX_TAPS - 1; ++j) x[j] = j < taps - 1 && live ? state[(size_t)j * C + c] : 0.f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < DELTA_MAX_TAPS - 1; ++j) x[j] = x[j + 1];
+    }
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < DELTA_MAX_TAPS; ++j) {
+      x[j] = j == taps - 1 ? fresh : x[j];
+      acc = fmaf(w[j], x[j], acc);
+    }
+    const float out = acc / (1.f + expf(-acc));
+    if (values) {
+      if (live) qkv[(size_t)t * C + c] = out;
+      continue;
+    }
+    if (live) y[tid] = out;
+    __syncthreads();
+    const int lane = tid & 63, wave = tid >> 6;
+    if (wave < 2) {  // of the q head, of the k head
+      const float* v = y + wave * D;
+      float s = 0.f;
+      for (int i = lane; i < D; i += WAVE) s = fmaf(v[i], v[i], s);
+      s = wave_sum(s);
+      if (lane == 0) inv[wave] = (wave == 0 ? q_scale : 1.f) / sqrtf(s + 1e-6f);
+    }
+    __syncthreads();
+    const float iq = inv[0], ik = inv[1];
+    if (live) qkv[(size_t)t * C + c] = out * (tid < D ? iq : ik);
+    if (wave == 0) {  // k . q of the finished vectors
+      float s = 0.f;
+      for (int i = lane; i < D; i += WAVE) s = fmaf(y[i] * iq, y[D + i] * ik, s);
+      s = wave_sum(s);
+      if (lane == 0) kq[(size_t)t * G + unit] = s;
+    }
+    if (t + 1 < t1) __syncthreads();  // y and inv are read
+  }
+  if (before >= 0 && live) {
+#pragma unroll
+    for (int j = 1; j < DELTA_MAX_TAPS; ++j)
+      if (j < taps) state[(size_t)(j - 1) * C + c] = x[j];
   }
 }
 
@@ -460,11 +561,20 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
   const bool pays = dim > 128 ? long_seqs && work >= 8000000
                               : columns >= 8192 || (long_seqs && (columns >= 6144 || work >= 5000000 || (columns >= 4096 && n_tokens >= 512)));
   const bool by_tokens = n_tokens > 64 && dim <= 256 && units <= 65535 && pays;
+  // A sequence a block, and no kernel for the state behind it, where sequences bring a token each on average (a decode step).
+  // More tokens a sequence would follow one another in a block that the others spread over blocks.
+  const int seq_threads = dim <= 128 ? 256 : 512;
+  const long seq_units = kv_heads + (heads * (long)vdim + seq_threads - 1) / seq_threads + (decays + seq_threads - 1) / seq_threads;
+  const bool by_seqs = seq_starts != nullptr && n_tokens <= n_seqs && dim <= 256 && seq_units <= 65535;
   const dim3 grid(ceil_div(n_tokens, PREP_TOKENS), (unsigned)units);
   const size_t token_lds = (size_t)PREP_TOKENS * (2 * dim + 4) * sizeof(float);
 #define FMS_PREP(W)                                                                                                   \
   do {                                                                                                                \
-    if (by_tokens)                                                                                                    \
+    if (by_seqs)                                                                                                      \
+      delta_prepare_seqs_kernel<W><<<dim3(n_seqs, (unsigned)seq_units), seq_threads, 2 * dim * sizeof(float), stream>>>( \
+          proj, ld, col_b, a, lda, col_a, (const W*)conv_w, taps, a_log, dt_bias, conv_state, seq_starts, seq_of_token, slot_ids, qkv, \
+          beta, decay, kq, heads, kv_heads, dim, vdim, per_channel, q_scale);                                         \
+    else if (by_tokens)                                                                                               \
       delta_prepare_tokens_kernel<W><<<grid, 256, token_lds, stream>>>(proj, ld, col_b, a, lda, col_a, (const W*)conv_w, taps, a_log, \
                                                                        dt_bias, conv_state, seq_of_token, slot_ids, qkv, beta, decay, \
                                                                        kq, n_tokens, heads, kv_heads, dim, vdim, per_channel, q_scale); \
@@ -478,7 +588,7 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
   else FMS_REQUIRE(false, "delta_prepare: unknown dtype %d", conv_dtype);
 #undef FMS_PREP
   FMS_LAUNCH_CHECK("delta_prepare");
-  if (taps > 1) {
+  if (taps > 1 && !by_seqs) {
     move_conv_state(proj, ld, taps, conv_state, seq_of_token, slot_ids, n_tokens, (int)C, threads, seq_starts, n_seqs, stream);
     FMS_LAUNCH_CHECK("conv_state");
   }

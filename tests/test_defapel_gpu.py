@@ -605,6 +605,37 @@ def test_delta_prepare_of_long_sequences(lib, sizes):
     assert torch.equal(left, want_left)
 
 
+@pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (2, 2, 256, 80, 8, True), (3, 3, 40, 130, 1, False), (33, 3, 24, 9, 3, True), (1, 1, 129, 5, 2, False)])
+def test_delta_prepare_of_a_decode_step(lib, sizes):
+    """A block of a sequence's tokens, which moves the state on itself: single tokens, a sequence of none, of three, and a row of
+    padding, beside the kernel that takes a token a block (which runs where no starts are given).  The same sums in the same order."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, taps, per_channel = sizes
+    C = 2 * G * D + H * V
+    lens = [1, 0, 3, 1, 1, 0]
+    T = sum(lens)
+    gen = torch.Generator().manual_seed(D)
+    proj, a = torch.randn(T, C + H + 5, generator=gen).to(DEV), torch.randn(T, H * (D if per_channel else 1) + 2, generator=gen).to(DEV)
+    conv_w = (0.5 * torch.randn(C, taps, generator=gen)).to(DEV)
+    a_log, dt_bias = (torch.randn(H, generator=gen) - 1).to(DEV), torch.randn(H * (D if per_channel else 1), generator=gen).to(DEV)
+    state = torch.randn(8, max(taps - 1, 1), C, generator=gen).to(DEV)
+    slots = torch.tensor([5, 3, 0, 6, 1, 2], dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32)
+    seq[4] = -1  # the fourth sequence is padding
+    starts = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=DEV)
+
+    def run(conv_state, **how):
+        return ops.delta_prepare(proj, C + 2, a, 1, conv_w, a_log, dt_bias, conv_state, seq.to(DEV), slots, H, G, D, V, per_channel, D ** -0.5, **how)
+
+    left, want_left = state.clone(), state.clone()
+    got, want = run(left, seq_starts=starts, n_seqs=len(lens)), run(want_left)
+    kept = (seq >= 0).to(DEV)
+    for x, y in zip(got, want):
+        torch.testing.assert_close(x[kept], y[kept], atol=1e-7, rtol=5e-7)  # a last bit or two: sums the compiler may contract otherwise
+    assert torch.equal(left, want_left)
+
+
 def test_a_lost_state_shows(lib):
     """The recurrence's memory matters: a value written long ago, read by a matching query much later, with decays near one."""
     from fms_amd.kernels import ops
