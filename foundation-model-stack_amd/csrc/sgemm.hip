@@ -1,351 +1,448 @@
 // The true 32-bit product y = x W^T (+ bias): float32 rows of x and W (K contiguous), float32 result.
 //
-// Sums of 16 products each in float32, added up in float64: what a long K costs is the rounding of short sums, not of
-// every partial sum on the way.  The products and the short sums are the matrix unit's (mfma 32x32x2 and 16x16x4, float32
-// throughout), the sums over the runs the vector unit's, side by side.
+// A float32 number is the sum of three bfloat16 numbers, each the rounded rest of the one before: 24 bits are 8 + 8 + 8, so the sum
+// is exact.  Of the nine products of two such sums the six largest are multiplied, each exactly, on the matrix unit; what
+// the other three would add is less than 2^-26 of a product, and 2^-29 in the mean, below the rounding of the product itself (2^-24).  Six bfloat16
+// products take 96 clocks for 16 x 16 results and 32 k-values where float32 ones take 256, and vector instructions run beside them.
+//
+// Sums of 32 products each in float32, small terms first, added up in float64.  The matrix unit's sums round down, not to nearest, which
+// would add up over many of them (relative error 8.2e-8 at K = 4096, 1.2e-7 at 11008): every other run's x is negated and its sum subtracted,
+// so that what rounds down in one rounds up in the next (4.5e-8 at both; float32 products in sums of 16 had 7.8e-8).
 //
 // Every kernel here adds in one order, so that a row's bits do not depend on how many rows there are, on the columns beside an
 // element or on alignment:
-//   * within a run k, k + 4, k + 8, k + 12 for k = 0 .. 3 (one 16x16x4 instruction, or two of 32x32x2, a k);
-//   * the even runs in their order, the odd runs in theirs, then the two sums.
+//   * a run of 32 k-values: (x3, w1), (x1, w3), (x2, w2), (x2, w1), (x1, w2), (x1, w1), one 16x16x32 instruction each;
+//   * the even runs in their order, the odd runs in theirs, then the first sum less the second.
+//
+// A sum that is no finite number (an infinity among the factors, whose second part would be a NaN, or a number that rounds to one)
+// is formed again, the element by itself, from products and sums in float64.
+// Below 2^-109 a number's third part begins to leave bfloat16's range: what is lost is less than 2^-134, the unit keeps subnormal numbers.
 #include "common.h"
 #include "fmsamd.h"
 #include "tile_product_lds.h"
 
-#define SG_RUN 16  // products of a float32 sum
+#define SG_RUN 32  // products of a float32 sum
 
-// A product of TILE x TILE results, two (TILE 32) or four k-values; lane l of the result has column l % TILE and these rows.
-template <int TILE>
-__device__ __forceinline__ auto sgemm_mfma(float x, float w, float __attribute__((ext_vector_type(TILE * TILE / WAVE))) sum) {
-  if constexpr (TILE == 32)
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, sum, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, w, sum, 0, 0, 0);
-}
-template <int TILE>
-__device__ __forceinline__ int sgemm_row(int group, int e) {  // group: lane / TILE
-  return TILE == 32 ? 8 * (e / 4) + 4 * group + e % 4 : 4 * group + e;
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));  // the unit asks for no more
+typedef unsigned u32x4_parts __attribute__((ext_vector_type(4)));
+struct SgemmParts {
+  bf16x8 p[3];
+};
+
+// Two numbers at a time: 11 instructions where conversions by element take 15.
+__device__ __forceinline__ SgemmParts sgemm_split(f32x8 v) {
+  u32x4_parts w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      unsigned pair;
+      asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pair) : "v"(a), "v"(b));
+      w[p][i] = pair;
+      if (p < 2) a -= __uint_as_float(pair << 16), b -= __uint_as_float(pair & 0xffff0000u);
+    }
+  }
+  SgemmParts parts;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) parts.p[p] = __builtin_bit_cast(bf16x8, w[p]);
+  return parts;
 }
 
-// Few rows (TILE 16), and rows that are not 16-byte aligned (VEC false).  A block's tile is TILE rows of x by TILE rows of W; its KS
-// waves share K: of a step's RUNS * KS runs wave ks takes ks, ks + KS, ...  The step's rows wait in LDS while the next
-// step's are on their way from memory in registers.  Rows of LDS are padded by four floats: the 16-byte reads of eight
-// neighbouring rows then cover all banks.
-// Two waves have the even and the odd runs and keep their sums.  Eight waves (one run each) hand the short sums over through LDS,
-// where the step's rows were, and a thread adds up every second one of one element.  (Room of their own for the short sums
-// leaves three blocks a compute unit where four fit: 64 rows by 4096 of K = 4096 take 55 us instead of 47.)
-template <int TILE, int KS, int RUNS, bool VEC>
-__global__ void __launch_bounds__(KS* WAVE)
-    sgemm_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
-                 float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
-  constexpr bool HAND_OVER = KS > 2;
-  static_assert(KS == 2 || (RUNS == 1 && KS % 2 == 0 && KS * WAVE == 2 * TILE * TILE), "a thread for the even or the odd runs of an element");
-  constexpr int THREADS = KS * WAVE, BM = TILE, BN = TILE, BK = SG_RUN * RUNS * KS, LD = BK + 4;
-  constexpr int PIECES = (BM + BN) * (BK / 4);  // of 16 bytes a step
-  constexpr int LOADS = (PIECES + THREADS - 1) / THREADS;
-  constexpr int ACC = TILE * TILE / WAVE;
-  typedef float accv __attribute__((ext_vector_type(ACC)));
-  constexpr int STEP = (BM + BN) * LD;  // floats
-  static_assert(KS * TILE * TILE <= STEP, "the short sums, or the odd runs' sums in 64 bits, where a step's rows were");
-  __shared__ __attribute__((aligned(16))) float lds[2 * STEP];
+// A run of 16 rows of x by TN tiles of 16 rows of W; lane l of a result has column l % 16 and rows 4 (l / 16) + e.
+template <int TN>
+__device__ __forceinline__ void sgemm_run(const bf16x8 (&x)[3], const SgemmParts (&w)[TN], f32x4 (&sum)[TN]) {
+  constexpr int ORDER[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+  for (int j = 0; j < TN; ++j) sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 6; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[ORDER[i][0]], w[j].p[ORDER[i][1]], sum[j], 0, 0, 0);
+}
+
+// The result c of the rows x and w, if it is no finite number.
+__device__ __forceinline__ void sgemm_again(float* c, const float* x, const float* w, const float* bias, int K) {
+  if (fabsf(*c) < INFINITY) return;
+  double sum = 0.0;
+#pragma nounroll
+  for (int k = 0; k < K; ++k) sum += (double)x[k] * (double)w[k];
+  *c = (float)(sum + (bias ? *bias : 0.f));
+}
+
+// Few rows, and rows that are not 16-byte aligned or very far apart.  A block's tile is 16 TM rows of x by 16 TN rows of W; its eight
+// waves share K, wave i has the runs i, i + 8, ...  A lane asks for its eight k-values of each row itself, a run ahead, and splits
+// them.  The waves hand their short sums over through LDS, and a thread adds up the even or the odd runs of an element.
+template <int TM, int TN>
+__global__ void __launch_bounds__(8 * WAVE)
+    sgemm_few_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
+                     float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
+  constexpr int WAVES = 8, THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
+  constexpr int OWN = 2 * ELEMENTS / THREADS;  // sums of a thread: (chain, element) threadIdx.x, + THREADS, ...
+  __shared__ __attribute__((aligned(16))) float lds[2][WAVES][ELEMENTS];
 
   // The tiles of x that share a tile of W follow one another on one of the eight dies (blocks are dealt to the dies in
   // turn), so that W comes from memory once.
   const int per_die = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_die || tile >= tiles) return;
-  const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * BN;
+  const int m0 = (tile % m_tiles) * 16 * TM, n0 = (tile / m_tiles) * 16 * TN;
+  const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int r = lane % 16, o = lane / 16;
 
-  const int lane = threadIdx.x & (WAVE - 1), ks = threadIdx.x / WAVE;
-  const int r = lane % TILE, kq = lane / TILE;  // a lane's row and which four of a group of k-values it holds
-
-  f32x4 ahead[LOADS];
-  auto fetch = [&](int k0) {
+  const float* src[TM + TN];  // a row that is not there is the last one
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int p = threadIdx.x + i * THREADS;
-      const int row = p / (BK / 4), k = k0 + (p % (BK / 4)) * 4;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (p < PIECES) {
-        const bool of_x = row < BM;
-        const int at = of_x ? m0 + row : n0 + row - BM;
-        if (at < (of_x ? M : N)) {
-          const float* src = of_x ? a + (size_t)at * lda : w + (size_t)at * K;
-          if constexpr (VEC) {
-            if (k < K) v = *reinterpret_cast<const f32x4*>(src + k);
-          } else {
+  for (int u = 0; u < TM; ++u) src[u] = a + (size_t)min(m0 + u * 16 + r, M - 1) * lda + o * 8;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (k + e < K) v[e] = src[k + e];
-          }
+  for (int u = 0; u < TN; ++u) src[TM + u] = w + (size_t)min(n0 + u * 16 + r, N - 1) * K + o * 8;
+  f32x8 ahead[TM + TN];
+  auto fetch = [&](int run) {
+    const int k0 = run * SG_RUN;
+    const bool whole = k0 + SG_RUN <= K;  // uniform
+#pragma unroll
+    for (int u = 0; u < TM + TN; ++u) {
+      f32x8 v = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (whole) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4_at4 q = *reinterpret_cast<const f32x4_at4*>(src[u] + k0 + h * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[h * 4 + e] = q[e];
         }
-      }
-      ahead[i] = v;
-    }
-  };
-  auto put = [&](int buffer) {
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int p = threadIdx.x + i * THREADS;
-      if (p < PIECES) *reinterpret_cast<f32x4*>(lds + buffer * STEP + (p / (BK / 4)) * LD + (p % (BK / 4)) * 4) = ahead[i];
-    }
-  };
-
-  constexpr int OWN = HAND_OVER ? 1 : ACC;  // elements that a thread keeps the sum of
-  double total[OWN];
-#pragma unroll
-  for (int e = 0; e < OWN; ++e) total[e] = 0.0;
-  // HAND_OVER: element threadIdx.x % (TILE * TILE) in the order in which the lanes hold them, even runs or odd ones
-  const int odd = threadIdx.x / (TILE * TILE), element = threadIdx.x % (TILE * TILE);
-  auto add = [&](int buffer) {
-#pragma unroll
-    for (int i = 0; i < KS / 2; ++i) total[0] += (double)lds[buffer * STEP + (2 * i + odd) * TILE * TILE + element];
-  };
-
-  fetch(0);
-  put(0);
-  __syncthreads();
-  int buffer = 0;
-  for (int k0 = 0; k0 < K; k0 += BK, buffer ^= 1) {
-    const bool more = k0 + BK < K;
-    if (more) fetch(k0 + BK);
-    if (HAND_OVER && k0 > 0) add(buffer ^ 1);
-    constexpr int GROUP = 4 * (WAVE / TILE), PARTS = SG_RUN / GROUP;  // k-values of one 16-byte piece a lane, such pieces of a run
-#pragma unroll
-    for (int i = 0; i < RUNS; ++i) {
-      const float* sx = lds + buffer * STEP + r * LD + (i * KS + ks) * SG_RUN + kq * 4;
-      f32x4 xv[PARTS], wv[PARTS];
-#pragma unroll
-      for (int g = 0; g < PARTS; ++g) {
-        xv[g] = *reinterpret_cast<const f32x4*>(sx + g * GROUP);
-        wv[g] = *reinterpret_cast<const f32x4*>(sx + BM * LD + g * GROUP);
-      }
-      accv acc;
-#pragma unroll
-      for (int e = 0; e < ACC; ++e) acc[e] = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int g = 0; g < PARTS; ++g) acc = sgemm_mfma<TILE>(xv[g][e], wv[g][e], acc);
-      if constexpr (HAND_OVER) {
-        __syncthreads();  // everybody has read the step's rows, and the short sums of the step before
-        *reinterpret_cast<accv*>(lds + buffer * STEP + ks * TILE * TILE + lane * ACC) = acc;
       } else {
 #pragma unroll
-        for (int e = 0; e < ACC; ++e) total[e] += (double)acc[e];
+        for (int e = 0; e < 8; ++e)
+          if (k0 + o * 8 + e < K) v[e] = src[u][k0 + e];
       }
+      ahead[u] = v;
     }
-    if (more) put(buffer ^ 1);
+  };
+
+  double total[OWN];
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) total[i] = 0.0;
+  const int rounds = (K + WAVES * SG_RUN - 1) / (WAVES * SG_RUN);
+  fetch(wave);
+  for (int t = 0; t < rounds; ++t) {
+    SgemmParts x[TM], y[TN];
+#pragma unroll
+    for (int u = 0; u < TM; ++u) x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u]);
+#pragma unroll
+    for (int u = 0; u < TN; ++u) y[u] = sgemm_split(ahead[TM + u]);
+    if (t + 1 < rounds) fetch((t + 1) * WAVES + wave);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      f32x4 sum[TN];
+      sgemm_run<TN>(x[i].p, y, sum);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(&lds[t & 1][wave][(i * TN + j) * 256 + lane * 4]) = sum[j];
+    }
+    __syncthreads();  // and everybody is done with the sums of the round before the last
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int q = threadIdx.x + i * THREADS;
+#pragma unroll
+      for (int run = 0; run < WAVES / 2; ++run) total[i] += (double)lds[t & 1][2 * run + q / ELEMENTS][q % ELEMENTS];
+    }
+  }
+
+  if constexpr (OWN == 1) {  // the odd runs' sums, to the threads that have the even ones'
+    double* const shared = reinterpret_cast<double*>(lds[rounds & 1]);  // nobody reads there any more
+    if (threadIdx.x >= ELEMENTS) shared[threadIdx.x - ELEMENTS] = total[0];
     __syncthreads();
+    if (threadIdx.x >= ELEMENTS) return;
+    total[0] -= shared[threadIdx.x];
   }
-  if (HAND_OVER) add(buffer ^ 1);
-
-  // the odd runs' sums, to the threads that have the even ones'
-  double* const shared = reinterpret_cast<double*>(lds + buffer * STEP) + (HAND_OVER ? element : lane);
-  const bool even = HAND_OVER ? odd == 0 : ks == 0;
-  if (!even) {
+  bool again = false;
+  constexpr int RESULTS = (OWN + 1) / 2;
+  auto place = [&](int i, int& m, int& n) {
+    const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;  // the lane that had it
+    m = m0 + element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = n0 + element / 256 % TN * 16 + of % 16;
+    return m < M && n < N;
+  };
 #pragma unroll
-    for (int e = 0; e < OWN; ++e) shared[e * WAVE] = total[e];
+  for (int i = 0; i < RESULTS; ++i) {
+    int m, n;
+    if (!place(i, m, n)) continue;
+    const float v = (float)((OWN == 1 ? total[i] : total[i] - total[i + OWN / 2]) + (bias ? bias[n] : 0.f));
+    c[(size_t)m * ldc + n] = v;
+    again |= !(fabsf(v) < INFINITY);
   }
-  __syncthreads();
-  if (!even) return;
-#pragma unroll
-  for (int e = 0; e < OWN; ++e) {
-    const int of = HAND_OVER ? element / ACC : lane;  // the lane that had the element in the matrix unit's result
-    const int m = m0 + sgemm_row<TILE>(of / TILE, HAND_OVER ? element % ACC : e), n = n0 + of % TILE;
-    if (m < M && n < N) c[(size_t)m * ldc + n] = (float)(total[e] + shared[e * WAVE] + (bias ? bias[n] : 0.f));
+  if (again) {
+#pragma nounroll
+    for (int i = 0; i < RESULTS; ++i) {
+      int m, n;
+      if (place(i, m, n)) sgemm_again(c + (size_t)m * ldc + n, a + (size_t)m * lda, w + (size_t)n * K, bias ? bias + n : nullptr, K);
+    }
   }
 }
 
-template <int TILE, int KS, int RUNS, bool VEC>
-static void sgemm_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
-                         hipStream_t stream) {
-  const int m_tiles = ceil_div(M, TILE), tiles = m_tiles * ceil_div(N, TILE);
-  sgemm_kernel<TILE, KS, RUNS, VEC><<<8 * ceil_div(tiles, 8), KS * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
+template <int TM, int TN>
+static void sgemm_few_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
+                             hipStream_t stream) {
+  const int m_tiles = ceil_div(M, 16 * TM), tiles = m_tiles * ceil_div(N, 16 * TN);
+  sgemm_few_kernel<TM, TN><<<8 * ceil_div(tiles, 8), 8 * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
-// The same for 16-byte aligned rows: the rows go from memory straight into LDS (tile_product_lds.h), STAGES - 1 steps of 32
-// k-values ahead, in rows of 128 bytes whose pieces of 16 bytes are XOR-swizzled with the row.  WM x WN places of TILE x TILE results,
-// two waves each: one has the even run of a step, the other the odd one.  The short sums of a step are converted and added
-// while the matrix unit works on the next.
-// A vector instruction costs a float32 product its own time (on this GPU a 64-bit one or a conversion 4.4 clocks, a 32-bit one 2.6, in
-// kernels of nothing else, beside the 64 of a 32x32x2 product), so the loop has little but the two a result and run that the sums in 64 bits
-// need: the steps are unrolled, so that places in LDS are constants and short sums stay where they are, and addresses advance in
-// the scalar unit.
-template <int TILE, int WM, int WN, int STAGES>
-__global__ void __launch_bounds__(2 * WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(TILE == 32 ? 4 : 6)))
+// Many 16-byte aligned rows: 16 MT rows of x by 16 NT WN rows of W a block, two waves for each 16 NT of them: one has the even runs, the
+// other the odd ones.  A wave has its rows of W to itself and a share of the rows of x: both go straight into its own LDS (tile_product_lds.h), up to
+// three runs ahead, in rows of 128 bytes whose pieces of 16 bytes are XOR-swizzled with the row.  What it has of x it splits for
+// all waves of its runs, into LDS, once a block; W it splits into registers.  A run's split stands beside the products of the run before it.
+template <int MT, int NT, int WN>
+__global__ void __launch_bounds__(2 * WN* WAVE)
     sgemm_lds_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
                      float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
-  constexpr int WAVES = 2 * WM * WN, BM = TILE * WM, BN = TILE * WN, BK = 2 * SG_RUN;
-  constexpr int LOADS = (BM + BN) / 8 / WAVES;  // of 1 KB a step and wave, 8 rows each
-  constexpr int STAGE = (BM + BN) * BK;         // floats
-  constexpr int ACC = TILE * TILE / WAVE;
-  typedef float accv __attribute__((ext_vector_type(ACC)));
-  static_assert((BM + BN) % (8 * WAVES) == 0 && BM % 8 == 0, "whole rounds of loads, of x or of W");
-  static_assert(BM * BN * 8 <= STAGES * STAGE * 4, "the waves of a place meet in the same LDS");
-  __shared__ __attribute__((aligned(16))) float lds[STAGES * STAGE];
+  static_assert(MT % WN == 0 && MT >= 2 && NT <= MT, "every wave has as many rows of x; a tile of W is split beside a tile of x");
+  constexpr int BM = 16 * MT, BN = 16 * NT * WN, UNITS = NT + MT / WN, LOADS = 2 * UNITS;
+  constexpr int RAW = UNITS * 2048;                 // bytes of a wave's run: units of 16 rows of 32 k-values, of W, then of x
+  constexpr int PLANE = MT * 1024;                  // one of the three parts of a run of x: 16-byte pieces in the order of the lanes
+  constexpr int PLANES = 2 * WN * 2 * RAW;          // where the parts begin
+  constexpr int BYTES = PLANES + 2 * 2 * 3 * PLANE;
+  static_assert(BM * BN * 8 <= BYTES, "the waves of a place meet in the same LDS");
+  __shared__ __attribute__((aligned(16))) char lds[BYTES];
   const int per_die = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_die || tile >= tiles) return;
   const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * BN;
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int ks = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
-  const int r = lane % TILE, kq = lane / TILE;
+  const int odd = wave / WN, wn = wave % WN;
+  const int r = lane % 16, o = lane / 16;
 
-  auto swizzle = [](int row) { return TILE == 32 ? (row >> 1) & 7 : row & 7; };
-  const char* base[LOADS];  // the same in all lanes: of the block's first row of x or of W
-  unsigned from[LOADS];     // bytes from there to this lane's piece (sgemm asks whether 32 bits hold them)
-  int piece[LOADS];
-  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
+  unsigned from[LOADS];  // bytes from the block's first row to this lane's piece (sgemm asks whether 32 bits hold them)
+  int piece[2];          // which k-value that is
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int first = (wave * LOADS + i) * 8;  // of x, then of W
-    const bool of_x = first < BM;              // uniform
-    const int row = (of_x ? first : first - BM) + (lane >> 3), there = of_x ? M - m0 : N - n0;
-    piece[i] = ((lane & 7) ^ swizzle(row)) * 4;
-    base[i] = (const char*)(of_x ? a + (size_t)m0 * lda : w + (size_t)n0 * K);
-    from[i] = (unsigned)((row < there ? row : 0) * (of_x ? lda : (long)K) + piece[i]) * 4;  // a row that is not there is the first one
+  for (int h = 0; h < 2; ++h) {
+    const int row16 = h * 8 + (lane >> 3);
+    piece[h] = ((lane & 7) ^ (row16 >> 1)) * 4 + odd * SG_RUN;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int row = (u < NT ? wn * NT + u : wn * (MT / WN) + u - NT) * 16 + row16, there = u < NT ? N - n0 : M - m0;
+      from[u * 2 + h] = (unsigned)((row < there ? row : 0) * (u < NT ? (long)K : lda) + piece[h]) * 4;  // a row that is not there is the first one
+    }
   }
+  const char* const first_w = (const char*)(w + (size_t)n0 * K);
+  const char* const first_x = (const char*)(a + (size_t)m0 * lda);
+  const unsigned mine = wave * 2 * RAW, lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds + mine;
+  constexpr int BK = 2 * SG_RUN;
   auto fetch = [&](int s, int stage) {  // past the end: zeros, so that every step has the same number of loads under way
     const int k0 = s * BK;
-    const unsigned to = lds0 + stage * (STAGE * 4) + wave * LOADS * 1024;
     if (k0 + BK <= K) {  // uniform
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) load_to_lds(base[i] + (size_t)k0 * 4, from[i], to + i * 1024);
+      for (int i = 0; i < LOADS; ++i)
+        load_to_lds((i < 2 * NT ? first_w : first_x) + (size_t)k0 * 4, from[i], lds0 + stage * RAW + i * 1024);
     } else {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i)
-        load_to_lds(k0 + piece[i] < K ? (const void*)(base[i] + (size_t)k0 * 4 + from[i]) : (const void*)tile_zeros, to + i * 1024);
+        load_to_lds(k0 + piece[i & 1] < K ? (const void*)((i < 2 * NT ? first_w : first_x) + (size_t)k0 * 4 + from[i]) : (const void*)tile_zeros,
+                    lds0 + stage * RAW + i * 1024);
+    }
+  };
+  const unsigned at0 = mine + r * 128 + ((2 * o) ^ (r >> 1)) * 16, at1 = mine + r * 128 + ((2 * o + 1) ^ (r >> 1)) * 16;
+  f32x8 raw[UNITS];
+  auto read = [&](int stage) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(lds + stage * RAW + u * 2048 + at0);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(lds + stage * RAW + u * 2048 + at1);
+      raw[u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  auto put = [&](int stage) {
+#pragma unroll
+    for (int u = 0; u < MT / WN; ++u) {
+      const SgemmParts parts = sgemm_split(odd ? -raw[NT + u] : raw[NT + u]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<bf16x8*>(lds + PLANES + ((stage * 2 + odd) * 3 + p) * PLANE + (wn * (MT / WN) + u) * 1024 + lane * 16) = parts.p[p];
     }
   };
 
-  double total[ACC];
-  accv sums[2];  // the short sums of this step and of the one before
+  double total[MT][NT][4];
+  f32x4 last[NT];  // the short sums of the tiles before
 #pragma unroll
-  for (int e = 0; e < ACC; ++e) total[e] = 0.0, sums[0][e] = sums[1][e] = 0.f;
-  const int steps = (K + BK - 1) / BK;
-  for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
-  constexpr int PARTS = TILE / 16;  // pieces of 16 bytes that a lane has of its row's run
-  int x_at[PARTS], w_at[PARTS];
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-  for (int g = 0; g < PARTS; ++g) {
-    const int at = r * BK + ((ks * 4 + g * (WAVE / TILE) + kq) ^ swizzle(r)) * 4;
-    x_at[g] = wm * TILE * BK + at, w_at[g] = (BM + wn * TILE) * BK + at;
-  }
-  auto step = [&](int s, int stage, accv& sum, const accv& last) {
-    tile_wait<(STAGES - 2) * LOADS>();  // step s is there, and everybody is done with step s - 1
-    fetch(s + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
-    f32x4 xv[PARTS], wv[PARTS];
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int g = 0; g < PARTS; ++g) {
-      xv[g] = *reinterpret_cast<const f32x4*>(lds + stage * STAGE + x_at[g]);
-      wv[g] = *reinterpret_cast<const f32x4*>(lds + stage * STAGE + w_at[g]);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // all pieces are asked for before the first product (5% at 128 rows by 32000)
+      for (int e = 0; e < 4; ++e) total[i][j][e] = 0.0, last[j][e] = 0.f;
+  auto add = [&](int i) {
 #pragma unroll
-    for (int e = 0; e < ACC; ++e) sum[e] = 0.f;
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int g = 0; g < PARTS; ++g) sum = sgemm_mfma<TILE>(xv[g][e], wv[g][e], sum);
-#pragma unroll
-    for (int e = 0; e < ACC; ++e) total[e] += (double)last[e];
+      for (int e = 0; e < 4; ++e) total[i][j][e] += (double)last[j][e];
   };
-  constexpr int ROUND = STAGES % 2 ? 2 * STAGES : STAGES;  // steps after which places and short sums are where they were
-  for (int s0 = 0; s0 < steps; s0 += ROUND) {
+
+  SgemmParts parts[2][NT];
+  fetch(0, 0);
+  fetch(1, 1);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+  read(0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next run is written there
+  fetch(2, 0);
 #pragma unroll
-    for (int u = 0; u < ROUND; ++u)
-      if (s0 + u < steps) step(s0 + u, u % STAGES, sums[u & 1], sums[~u & 1]);  // uniform
+  for (int j = 0; j < NT; ++j) parts[0][j] = sgemm_split(raw[j]);
+  put(0);
+  const int steps = (K + BK - 1) / BK;
+  auto step = [&](int s, int stage) {
+    tile_wait<LOADS>();  // run s + 1 is there, the parts of x of run s too, and everybody is done with those of s - 1
+    const char* const at = lds + PLANES + (stage * 2 + odd) * 3 * PLANE + lane * 16;
+    bf16x8 x[3], next[3];
+#pragma unroll
+    for (int p = 2; p >= 0; --p) x[p] = *reinterpret_cast<const bf16x8*>(at + p * PLANE);
+    read(stage ^ 1);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if (i + 1 < MT) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) next[p] = *reinterpret_cast<const bf16x8*>(at + p * PLANE + (i + 1) * 1024);
+      }
+      f32x4 sum[NT];
+      sgemm_run<NT>(x, parts[stage], sum);
+      add(i ? i - 1 : MT - 1);
+      if (i == (MT > NT ? MT - NT - 1 : 0)) put(stage ^ 1);
+      if (i >= MT - NT) parts[stage ^ 1][i - MT + NT] = sgemm_split(raw[i - MT + NT]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) last[j] = sum[j];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) x[p] = next[p];
+      // a product of 16 clocks, then four vector instructions (5% against the compiler's order)
+#pragma unroll
+      for (int p = 0; p < 6 * NT; ++p) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    fetch(s + 3, stage ^ 1);
+  };
+  for (int s = 0; s < steps; s += 2) {
+    step(s, 0);
+    if (s + 1 < steps) step(s + 1, 1);  // uniform
   }
-  if (steps & 1) {
-#pragma unroll
-    for (int e = 0; e < ACC; ++e) total[e] += (double)sums[0][e];
-  } else {
-#pragma unroll
-    for (int e = 0; e < ACC; ++e) total[e] += (double)sums[1][e];
-  }
+  add(MT - 1);
   tile_wait<0>();
 
   // the odd runs' sums, to the waves that have the even ones'
-  double* const shared = reinterpret_cast<double*>(lds) + (size_t)(wm * WN + wn) * TILE * TILE + lane;
-  if (ks == 1) {
+  double* const shared = reinterpret_cast<double*>(lds) + (size_t)wn * MT * NT * 256 + lane;
+  if (odd) {
 #pragma unroll
-    for (int e = 0; e < ACC; ++e) shared[e * WAVE] = total[e];
+    for (int i = 0; i < MT * NT * 4; ++i) shared[i * WAVE] = total[i / (4 * NT)][i / 4 % NT][i % 4];
   }
   __syncthreads();
-  const int n = n0 + wn * TILE + r;
-  if (ks == 1 || n >= N) return;
-  const float b = bias ? bias[n] : 0.f;
+  if (odd) return;
+  bool again = false;
 #pragma unroll
-  for (int e = 0; e < ACC; ++e) {
-    const int m = m0 + wm * TILE + sgemm_row<TILE>(kq, e);
-    if (m < M) c[(size_t)m * ldc + n] = (float)(total[e] + shared[e * WAVE] + b);
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + (wn * NT + j) * 16 + r;
+    const float b = bias && n < N ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + i * 16 + o * 4 + e;
+        const float v = (float)(total[i][j][e] - shared[((i * NT + j) * 4 + e) * WAVE] + b);
+        if (m < M && n < N) {
+          c[(size_t)m * ldc + n] = v;
+          again |= !(fabsf(v) < INFINITY);
+        }
+      }
+  }
+  if (again) {
+#pragma nounroll
+    for (int i = 0; i < MT * NT * 4; ++i) {
+      const int m = m0 + i / (4 * NT) * 16 + o * 4 + i % 4, n = n0 + (wn * NT + i / 4 % NT) * 16 + r;
+      if (m < M && n < N) sgemm_again(c + (size_t)m * ldc + n, a + (size_t)m * lda, w + (size_t)n * K, bias ? bias + n : nullptr, K);
+    }
   }
 }
 
-template <int TILE, int WM, int WN, int STAGES>
+template <int MT, int NT, int WN>
 static void sgemm_lds_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
                              hipStream_t stream) {
-  const int m_tiles = ceil_div(M, TILE * WM), tiles = m_tiles * ceil_div(N, TILE * WN);
-  sgemm_lds_kernel<TILE, WM, WN, STAGES><<<8 * ceil_div(tiles, 8), 2 * WM * WN * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
+  const int m_tiles = ceil_div(M, 16 * MT), tiles = m_tiles * ceil_div(N, 16 * NT * WN);
+  sgemm_lds_kernel<MT, NT, WN><<<8 * ceil_div(tiles, 8), 2 * WN * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
-// The tile shape.  What a compute unit needs for its blocks was measured at K = 4096 (8 to 512 rows of x, 4096 to 32000 of W):
-// the first block costs `first` microseconds, every further one `next`, whatever the rows.  Small tiles fill the chip where
-// there are few rows, large ones read less from LDS and the caches per product (301 rows by 32000: 73 TFLOP/s of 16 x 16, 85 of 32 x 32, 92 of
-// 32 x 64; blocks of 64 x 64 and of 64 x 32 are within two per cent of the last, with four stages it takes a tenth longer).  Rows that are not 16-byte aligned have
-// tiles of their own.
+// At most SG_SHORT products: a thread has a row of W and 16 rows of x, sums in float64.  Bound by the results' bytes.
+#define SG_SHORT 16
+template <int KMAX>
+__global__ void __launch_bounds__(256)
+    sgemm_short_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
+                       float* __restrict__ c, long ldc, int M, int N, int K, int n_blocks) {
+  const int n = blockIdx.x % n_blocks * 256 + threadIdx.x, m0 = blockIdx.x / n_blocks * 16;
+  if (n >= N) return;
+  float y[KMAX];
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) y[k] = k < K ? w[(size_t)n * K + k] : 0.f;
+  const float b = bias ? bias[n] : 0.f;
+  for (int m = m0; m < min(m0 + 16, M); ++m) {
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) sum += (double)a[(size_t)m * lda + k] * (double)y[k];  // uniform
+    c[(size_t)m * ldc + n] = (float)(sum + b);
+  }
+}
+
+// The tile shape.  What a compute unit needs for its blocks was measured at K = 4096 (1 to 301 rows of x, 4096 to 32000 of W): the first
+// block costs `first` microseconds, every further one `next`, whatever the rows.  Small tiles fill the chip where there are few rows, and their
+// waves share K; large ones split each number less often (301 rows by 12288 of W: 793 us of 16 x 16, 436 of 32 x 32, 285 of 32 x 64, 268 of 64 x 64, 209 of
+// 64 x 128; 16 rows by 4096: 21, 32, 53, 67, 97).  Those through LDS want 16-byte aligned rows.
 struct SgemmShape {
   int bm, bn;
   float first, next;
 };
-static const SgemmShape SGEMM_SHAPES[3] = {{16, 16, 22.f, 8.5f}, {32, 32, 39.f, 24.f}, {32, 64, 58.f, 45.f}};
-static const SgemmShape SGEMM_UNALIGNED[2] = {{16, 16, 34.f, 28.f}, {32, 32, 126.f, 45.f}};
+#define SGEMM_FEW 4  // shapes that take any rows
+static const SgemmShape SGEMM_SHAPES[7] = {{16, 16, 21.f, 14.5f}, {16, 32, 27.5f, 21.5f}, {16, 64, 41.5f, 40.f}, {32, 32, 34.5f, 28.5f},
+                                           {32, 64, 54.f, 33.f},  {64, 64, 68.f, 67.f},   {64, 128, 102.f, 106.f}};
 #define SGEMM_COMPUTE_UNITS 256
 
-static int sgemm_rounds(const SgemmShape& s, int M, int N) {
-  return (int)ceil_div((long)ceil_div(M, s.bm) * ceil_div(N, s.bn), SGEMM_COMPUTE_UNITS);
-}
-
-template <int SHAPES>
-static int sgemm_shape(const SgemmShape (&shapes)[SHAPES], int M, int N) {
+static int sgemm_shape(int shapes, int M, int N) {
   int best = 0;
   float least = 0.f;
-  for (int i = 0; i < SHAPES; ++i) {
-    const float cost = shapes[i].first + shapes[i].next * (float)(sgemm_rounds(shapes[i], M, N) - 1);
+  for (int i = 0; i < shapes; ++i) {
+    const SgemmShape& s = SGEMM_SHAPES[i];
+    const long rounds = ceil_div((long)ceil_div(M, s.bm) * ceil_div(N, s.bn), SGEMM_COMPUTE_UNITS);
+    const float cost = s.first + s.next * (float)(rounds - 1);
     if (i == 0 || cost < least) best = i, least = cost;
   }
   return best;
 }
 
-#define SGEMM_NEAR (1 << 23)  // 64 rows of so many floats
+#define SGEMM_NEAR (1 << 22)  // 128 rows of so many floats lie within 32 bits of bytes
 static void sgemm(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K, bool aligned,
                   hipStream_t stream) {
-  if (aligned) {
-    const bool near = lda < SGEMM_NEAR && K < SGEMM_NEAR;  // a tile's rows lie within 32 bits of bytes
-    switch (near ? sgemm_shape(SGEMM_SHAPES, M, N) : 0) {
-      case 0: sgemm_launch<16, 8, 1, true>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-      case 1: sgemm_lds_launch<16, 2, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-      default: sgemm_lds_launch<32, 1, 2, 3>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    }
-  } else if (sgemm_shape(SGEMM_UNALIGNED, M, N) == 0) {
-    sgemm_launch<16, 8, 1, false>(a, lda, w, bias, c, ldc, M, N, K, stream);
-  } else if (sgemm_rounds(SGEMM_UNALIGNED[1], M, N) <= 2) {
-    // a block or two a compute unit: long steps (128 rows by 4096 of K = 4095 150 us, 184 in short ones); more of them
-    // hide one another's waits in short steps (301 rows: 423 against 290)
-    sgemm_launch<32, 2, 4, false>(a, lda, w, bias, c, ldc, M, N, K, stream);
-  } else {
-    sgemm_launch<32, 2, 1, false>(a, lda, w, bias, c, ldc, M, N, K, stream);
+  if (K <= SG_SHORT) {
+    const int n_blocks = ceil_div(N, 256), blocks = n_blocks * ceil_div(M, 16);
+    if (K <= 4)
+      sgemm_short_kernel<4><<<blocks, 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
+    else
+      sgemm_short_kernel<SG_SHORT><<<blocks, 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
+    return;
+  }
+  const bool any = aligned && lda < SGEMM_NEAR && K < SGEMM_NEAR;
+  switch (sgemm_shape(any ? 7 : SGEMM_FEW, M, N)) {
+    case 0: sgemm_few_launch<1, 1>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 1: sgemm_few_launch<1, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 2: sgemm_few_launch<1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 3: sgemm_few_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 4: sgemm_lds_launch<2, 2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 5: sgemm_lds_launch<4, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    default: sgemm_lds_launch<4, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
   }
 }
 
 // What one launch takes: its threads are counted in 32 bits (and wrap round silently), at most two for a result.
 #define SGEMM_LAUNCH_TILES (1 << 22)  // of 16 x 16 results
 
-// Bound by the matrix unit's float32 rate (154 TFLOP/s for the vendor's product of 8192^3) and the vector instructions beside it, which
-// take its time: with the 32 that the sums in 64 bits are for a run of 32 x 32 results some 120 would be left, and 110 are reached
-// for 2048 rows (99 with the 57 of a loop that moved short sums and addresses); with few rows by the weights' bytes.  301 rows, K 4096: 630 us for 22016 rows of W (705),
-// 134 for 4096 (144); 160 rows: 326 for 22016 (370), 82 for 4096 (85); 8 rows: 39 us for 12288 rows of W (5.0 TB/s), 23 for 4096.
+// Many rows: bound by the vector instructions of the split and of the sums in 64 bits, which overlap with the products only in part: a step of
+// 64 x 128 results and 64 k-values takes 1.5 us, of which the products alone are 0.64 (1.8 PFLOP/s in bfloat16), the sums about 0.5, the splits 0.4.
+// Few rows: the weights' bytes.  Against float32 products, K 4096 (us): 301 rows by 22016 rows of W 604 -> 408, by 4096 131 -> 103;
+// 128 rows by 12288 148 -> 103; 48 by 32000 193 -> 116; 24 by 4096 31 -> 29; 8 by 4096 23 -> 20, by 12288 37 -> 39 and by 32000 92 -> 95
+// (x's rows are split by every block); 8 by 4096 of K = 11008 52 -> 42; rows that are not aligned, 301 by 4096 of K = 4095: 302 -> 160.
 extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
                                int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;

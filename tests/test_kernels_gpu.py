@@ -589,9 +589,9 @@ def test_gemm_f32(ops, M, N, K):
     torch.testing.assert_close(out, (x.double() @ w.double().t() + b.double()).float(), atol=1e-4, rtol=1e-5)
 
 
-# every tile shape with rows, columns and K past its last whole tile.  Aligned: 16x16 (17 by 300, 48 by 4100), 32x32 (130 by 4100,
-# 64 by 8190, 301 by 8200), 32x64 (513 by 16390).  Rows that are not 16-byte aligned (odd K, odd stride): 16x16, 32x32 in long
-# steps (130 by 3000: two rounds of blocks) and in short ones (301 by 8200)
+# tile shapes with rows, columns and K past the last whole tile.  Aligned: 16x16 (17 by 300), 32x32 (48 by 4100), 32x64 (130 by
+# 3000 and 4100), 64x64 (64 by 8190), 64x128 (301 by 8200, 513 by 16390).  Rows that are not 16-byte aligned (odd K, odd stride): tiles of
+# 16x16 (17 by 300), 16x32 (8 by 4096) and 32x32 (from 130 by 3000 on).  K up to 16: sums in float64
 @pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
@@ -607,9 +607,8 @@ def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
 
 @pytest.mark.parametrize("K", [7, 36, 1000, 1028])
 def test_gemm_f32_rows_keep_their_bits(ops, K):
-    """A row has the same bits whatever else is in the product: tiles of 16x16 (1, 8 and 33 rows, and 301 by 100), 32x32 (17) and
-    32x64 (61, 130 and 301), rows that are not 16-byte aligned (an odd stride, an odd K) in tiles of 16x16 (1 and 8), 32x32 in
-    long steps (17) and in short ones (from 33 on)."""
+    """A row has the same bits whatever else is in the product: tiles of 16x64 (1 and 8 rows), 32x64 (17), 64x64 (33 and 61), 64x128
+    (130 and 301) and 16x16 (301 by 100), rows that are not 16-byte aligned (an odd stride, an odd K) in tiles of 16x64 and 32x32."""
     torch.manual_seed(62)
     N = 12790
     x, w, b = dev(torch.randn(301, K)), dev(torch.randn(N, K)), dev(torch.randn(N))
@@ -620,6 +619,30 @@ def test_gemm_f32_rows_keep_their_bits(ops, K):
         assert torch.equal(ops.linear(odd[:M], w, b), whole[:M]), M
     assert torch.equal(ops.linear(odd, w, b), whole)
     assert torch.equal(ops.linear(x, w[:100], b[:100]), whole[:, :100])
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 300, 64), (40, 4096, 132), (301, 4096, 256), (301, 4096, 131), (40, 300, 13)])
+def test_gemm_f32_of_numbers_that_are_not_finite_or_nearly(ops, M, N, K):
+    """Infinities and numbers that bfloat16 rounds to one show where 64 bits show them, and change no other result's bits; subnormal
+    thirds of small numbers are kept to 2^-134."""
+    torch.manual_seed(65)
+    x, w, b = torch.randn(M, K), torch.randn(N, K), torch.randn(N)
+    clean = ops.linear(dev(x), dev(w), dev(b)).cpu()
+    y, v = x.clone(), w.clone()
+    y[1, 5], y[2, 6], y[3, 7], v[9, 8], v[10] = math.inf, math.nan, 3.4028e38, -math.inf, 0.0
+    got = ops.linear(dev(y), dev(v), dev(b)).cpu()
+    want = (y.double() @ v.double().t() + b.double()).float()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[got.isinf()])
+    torch.testing.assert_close(got[3][want[3].isfinite()], want[3][want[3].isfinite()], rtol=2.0 ** -22, atol=1e-4)
+    rows, cols = [0] + list(range(4, M)), [n for n in range(N) if n not in (9, 10)]
+    assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
+    small = ops.linear(dev(x * 2.0 ** -120), dev(w), None).cpu().double()
+    exact = (x * 2.0 ** -120).double() @ w.double().t()
+    # the bound of the tile shapes' test, and what the third parts lose
+    bound = 2.0 ** -24 * (16.5 * exact.abs().new_tensor(2.0 ** -120) * (x.abs().double() @ w.abs().double().t()) + exact.abs())
+    bound += 2.0 ** -134 * w.abs().double().sum(1) + 2.0 ** -148
+    assert float(((small - exact).abs() / bound).max()) <= 1.0
 
 
 def test_gemm_f32_of_rows_far_apart(ops):
