@@ -355,7 +355,7 @@ long fmsamd_delta_runs_workspace(int n_tokens, int n_seqs, int heads, int dim, i
 int fmsamd_delta_runs(const float* qkv, const float* beta, const float* decay, float* state, float* out, const int* seq_starts,
                       const int* seq_of_token, const int* slot_ids, int n_tokens, int n_seqs, int heads, int kv_heads, int dim,
                       int vdim, int per_channel, void* workspace, long workspace_bytes, hipStream_t stream);
-// out[t, h, :] = o[t, h, :] / rms * weight * act(gate[t, h, :]) * out_scale
+// out[t, h, :] = o[t, h, :] / rms * weight * act(gate[t, h, :]) * out_scale; rows of no sequence become zeros
 int fmsamd_gated_head_norm(const float* o, const float* gate, long ldg, const void* weight, int weight_dtype, float eps,
                            int act, float out_scale, void* out, int out_dtype, long ldo, const int* seq_of_token,
                            int n_tokens, int heads, int vdim, hipStream_t stream);

@@ -1693,7 +1693,8 @@ def delta_rule(qkv: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, kq: t
 def gated_head_norm(o: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, eps: float, activation: str, heads: int, vdim: int,
                     out_dtype: torch.dtype, seq_of_token: torch.Tensor, scale: float = 1.0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """o float32 [T, heads*vdim]: every head divided by its root mean square, times weight [vdim], times act(gate)
-    (float32 logits [T, heads*vdim], rows of any stride), times scale -> out_dtype (into `out`, rows of any stride)."""
+    (float32 logits [T, heads*vdim], rows of any stride), times scale -> out_dtype (into `out`, rows of any stride).
+    Rows of no sequence (seq_of_token < 0) become zeros."""
     _need_cuda(o, gate, weight, seq_of_token, out)
     _rows2d("gate", gate)
     _need_i32("seq_of_token", seq_of_token)

@@ -28,6 +28,8 @@ from .linear import Linear
 
 
 class GatedDeltaRule(Mixer):
+    writes_padding_rows = True  # zeros
+
     def __init__(
         self,
         width: int,

@@ -691,6 +691,21 @@ def test_head_norm_with_a_gate(lib, dtype, sizes):
     assert float(out[:, :8].float().abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("vdim", [5, 64, 130])
+def test_gated_head_norm_of_padding_rows(lib, vdim):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(2)
+    T, H = 7, 3
+    o, gate = torch.randn(T, H * vdim, generator=gen), torch.randn(T, H * vdim, generator=gen)
+    o[2], gate[2] = math.nan, math.inf
+    seq = torch.tensor([0, 1, -1, 2, 3, -1, 4], dtype=torch.int32)
+    out = torch.full((T, H * vdim + 8), math.nan, dtype=torch.bfloat16, device=DEV)
+    ops.gated_head_norm(o.to(DEV), gate.to(DEV), torch.ones(vdim, device=DEV), 1e-5, "silu", H, vdim, torch.bfloat16, seq.to(DEV), out=out[:, 8:])
+    assert float(out[:, 8:][(seq < 0).to(DEV)].abs().max()) == 0.0
+    assert bool(out[:, 8:][(seq >= 0).to(DEV)].isfinite().all()) and bool(out[:, :8].isnan().all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_norm_over_whole_projections_gate_and_scales(lib, dtype):
     from fms_amd.kernels import ops
