@@ -532,6 +532,34 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The same for heads of 64, 128 or 256 and aligned rows: a lane has four neighbours, a wave 256 columns.  Bound by its bytes.  2277 tokens of 16 heads of 128: 13 us where the kernel above takes 21; of 32 of 64: 14 and 28.
+template <typename T, typename W, int LANES>
+__global__ void __launch_bounds__(256)
+    gated_head_norm4_kernel(const float* __restrict__ o, const float* __restrict__ gate, long ldg, const W* __restrict__ weight,
+                            float eps, int act, float out_scale, T* __restrict__ out, long ldo, const int* __restrict__ seq_of_token,
+                            int n_tokens, int H) {
+  constexpr int DV = 4 * LANES, PER = WAVE / LANES;
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, j = lane % LANES * 4;
+  const long pair = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * PER + lane / LANES;
+  if (pair >= (long)n_tokens * H) return;
+  const int t = (int)(pair / H), h = (int)(pair % H);
+  T* const to = out + (size_t)t * ldo + (size_t)h * DV + j;
+  if (seq_of_token[t] < 0) {
+    *(T4*)to = T4{};
+    return;
+  }
+  const f32x4 v = *(const f32x4*)(o + (size_t)pair * DV + j), g = *(const f32x4*)(gate + (size_t)t * ldg + (size_t)h * DV + j);
+  float s = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], v[3] * v[3])));
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, WAVE);
+  const float inv = 1.f / sqrtf(s / (float)DV + eps);
+  T4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = from_f32<T>(v[e] * inv * to_f32(weight[j + e]) * fms_activate(g[e], act) * out_scale);
+  *(T4*)to = r;
+}
+
 // --------------------------------------------------------------------------
 extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const float* a, long lda, int col_a, const void* conv_w,
                                     int conv_dtype, int taps, const float* a_log, const float* dt_bias, float* conv_state,
@@ -645,16 +673,32 @@ extern "C" int fmsamd_gated_head_norm(const float* o, const float* gate, long ld
   FMS_REQUIRE(n_tokens > 0 && heads > 0 && vdim > 0 && ldg >= (long)heads * vdim && ldo >= (long)heads * vdim,
               "gated_head_norm: bad sizes heads=%d vdim=%d", heads, vdim);
   FMS_REQUIRE(act >= 0 && act <= FMS_ACT_LAST, "gated_head_norm: unknown activation %d", act);
-  const int blocks = ceil_div((long)n_tokens * heads, 4);
+  const size_t out_piece = out_dtype == FMS_F32 ? 16 : 8;
+  const bool fours = (vdim == 64 || vdim == 128 || vdim == 256) && ldg % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)o | (uintptr_t)gate) % 16 == 0 &&
+                     (uintptr_t)out % out_piece == 0;
+  const int blocks = ceil_div((long)n_tokens * heads, fours ? 1024 / vdim : 4);
+#define FMS_GHN4(T, W, LANES)                                                                                                  \
+  gated_head_norm4_kernel<T, W, LANES><<<blocks, 256, 0, stream>>>(o, gate, ldg, (const W*)weight, eps, act, out_scale, (T*)out, ldo, \
+                                                                   seq_of_token, n_tokens, heads)
 #define FMS_GHN(T, W)                                                                                                          \
-  gated_head_norm_kernel<T, W><<<blocks, 256, 0, stream>>>(o, gate, ldg, (const W*)weight, eps, act, out_scale, (T*)out, ldo, \
-                                                           seq_of_token, n_tokens, heads, vdim)
+  do {                                                                                                                         \
+    if (fours && vdim == 64)                                                                                                   \
+      FMS_GHN4(T, W, 16);                                                                                                      \
+    else if (fours && vdim == 128)                                                                                             \
+      FMS_GHN4(T, W, 32);                                                                                                      \
+    else if (fours)                                                                                                            \
+      FMS_GHN4(T, W, 64);                                                                                                      \
+    else                                                                                                                       \
+      gated_head_norm_kernel<T, W><<<blocks, 256, 0, stream>>>(o, gate, ldg, (const W*)weight, eps, act, out_scale, (T*)out, ldo, \
+                                                               seq_of_token, n_tokens, heads, vdim);                           \
+  } while (0)
   if (out_dtype == FMS_F32 && weight_dtype == FMS_F32) FMS_GHN(float, float);
   else if (out_dtype == FMS_BF16 && weight_dtype == FMS_F32) FMS_GHN(bf16, float);
   else if (out_dtype == FMS_BF16 && weight_dtype == FMS_BF16) FMS_GHN(bf16, bf16);
   else if (out_dtype == FMS_F32 && weight_dtype == FMS_BF16) FMS_GHN(float, bf16);
   else FMS_REQUIRE(false, "gated_head_norm: unknown dtypes %d, %d", out_dtype, weight_dtype);
 #undef FMS_GHN
+#undef FMS_GHN4
   FMS_LAUNCH_CHECK("gated_head_norm");
   return 0;
 }

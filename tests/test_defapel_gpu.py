@@ -691,6 +691,26 @@ def test_head_norm_with_a_gate(lib, dtype, sizes):
     assert float(out[:, :8].float().abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,V", [(3, 64), (1, 128), (5, 128), (3, 256)])
+@pytest.mark.parametrize("shift", [0, 2])  # of the gate's columns: aligned rows, and rows that are not
+def test_head_norm_of_aligned_rows(lib, dtype, H, V, shift):
+    from fms_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(V + H)
+    T = 11
+    o, gate, w = torch.randn(T, H * V, generator=gen) * 3, torch.randn(T, H * V + 4, generator=gen), 1 + 0.3 * torch.randn(V, generator=gen)
+    seq = torch.tensor([0, 0, 1, -1, 2, 3, 4, -1, 5, 6, 7], dtype=torch.int32)
+    out = torch.full((T, H * V + 8), math.nan, dtype=dtype, device=DEV)
+    g = gate[:, shift : shift + H * V]
+    ops.gated_head_norm(o.to(DEV), gate.to(DEV)[:, shift : shift + H * V], w.to(DEV), 1e-5, "silu", H, V, dtype, seq.to(DEV), scale=0.7, out=out[:, 8:])
+    want = (P.rms(o.view(T, H, V), 1e-5) * w).view(T, H * V) * g * torch.sigmoid(g) * 0.7
+    want[seq < 0] = 0.0
+    # float32: a sum of V squares in any order, a root, six products; bfloat16: one rounding more
+    torch.testing.assert_close(out[:, 8:].float().cpu(), want, atol=1e-6, rtol=1e-5 if dtype == torch.float32 else 2.0 ** -8)
+    assert bool(out[:, :8].isnan().all())
+
+
 @pytest.mark.parametrize("vdim", [5, 64, 130])
 def test_gated_head_norm_of_padding_rows(lib, vdim):
     from fms_amd.kernels import ops
