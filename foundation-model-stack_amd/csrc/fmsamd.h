@@ -121,7 +121,7 @@ int fmsamd_attn_decode_bf16(const void* q, long q_stride, void* out, long out_st
                             float soft_cap, int chunk, const float* sink, int keep_first, const float* dist_bias,
                             int dist_len, hipStream_t stream);
 
-// c[M, N] = a[M, K] w[N, K]^T (+ bias[N])
+// c[M, N] = a[M, K] w[N, K]^T (+ bias[N]), rows of any alignment
 int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N,
                     int K, hipStream_t stream);
 int fmsamd_gemm_bf16(const void* a, long lda, const void* w, const void* bias, int bias_dtype, void* c, int out_dtype,

@@ -63,12 +63,12 @@ __device__ __forceinline__ void sgemm_run(const bf16x8 (&x)[3], const SgemmParts
       sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[ORDER[i][0]], w[j].p[ORDER[i][1]], sum[j], 0, 0, 0);
 }
 
-// The result c of the rows x and w, if it is no finite number.
+// The result c of the rows x and w, if it is no finite number (a NaN stays one, so nothing behind it is looked at).
 __device__ __forceinline__ void sgemm_again(float* c, const float* x, const float* w, const float* bias, int K) {
   if (fabsf(*c) < INFINITY) return;
   double sum = 0.0;
 #pragma nounroll
-  for (int k = 0; k < K; ++k) sum += (double)x[k] * (double)w[k];
+  for (int k = 0; k < K && sum == sum; ++k) sum += (double)x[k] * (double)w[k];
   *c = (float)(sum + (bias ? *bias : 0.f));
 }
 
