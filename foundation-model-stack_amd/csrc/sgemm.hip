@@ -26,11 +26,14 @@
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));  // the unit asks for no more
 typedef unsigned u32x4_parts __attribute__((ext_vector_type(4)));
+typedef float f32x2_parts __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_parts __attribute__((ext_vector_type(2)));
 struct SgemmParts {
   bf16x8 p[3];
 };
 
-// Two numbers at a time: 11 instructions where conversions by element take 15.
+// Two numbers at a time: 11 instructions where conversions by element take 15.  (The compiler forms the conversion: it does not look
+// into inline assembly for registers that a matrix instruction in flight still reads or writes, and so puts no wait in front of it.)
 __device__ __forceinline__ SgemmParts sgemm_split(f32x8 v) {
   u32x4_parts w[3];
 #pragma unroll
@@ -38,8 +41,7 @@ __device__ __forceinline__ SgemmParts sgemm_split(f32x8 v) {
     float a = v[2 * i], b = v[2 * i + 1];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      unsigned pair;
-      asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pair) : "v"(a), "v"(b));
+      const unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2_parts{a, b}), bf16x2_parts));
       w[p][i] = pair;
       if (p < 2) a -= __uint_as_float(pair << 16), b -= __uint_as_float(pair & 0xffff0000u);
     }

@@ -4,6 +4,7 @@ generation loop's decisions.  None of this needs a GPU."""
 import json
 import os
 import random
+import re
 
 import pytest
 import torch
@@ -1134,3 +1135,14 @@ def test_embedding_leaves_a_norm_of_somebody_elses_to_that_norm(monkeypatch):
         assert embedding.forward_normed(ids, norm, torch.float32) is None
     assert embedding.forward_normed(ids, ParameterizedNorm(8), torch.float32) == "one kernel"
     assert embedding.forward_normed(ids, ParameterizedNorm(8), torch.bfloat16) is None
+
+
+@pytest.mark.parametrize("name", ["sgemm.hip"])
+def test_vector_instructions_are_the_compilers(name):
+    """The compiler puts waits between a matrix instruction and whatever reads or writes its registers, but does not look into inline
+    assembly: none of it may hold vector arithmetic beside matrix instructions."""
+    from fms_amd.kernels.build import CSRC
+
+    with open(os.path.join(CSRC, name)) as f:
+        found = re.findall(r"asm\s*(?:volatile)?\s*\(\s*\"[^\"]*\bv_[^\"]*", f.read())
+    assert not found, found
