@@ -172,32 +172,21 @@ __device__ __forceinline__ float biased(float raw, int distance, const ScoreExtr
 // the maximum that a partial result of the decode kernel carries when it holds no key at all
 #define DECODE_EMPTY -1e30f
 
-// Maxima as single instructions.  fmaxf() first passes each operand through a max with itself (it must quiet a
-// signalling NaN), which tripled the instructions of the score maxima; the scores here come out of the matrix unit
-// and are never signalling NaNs.
-__device__ __forceinline__ float max2f(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
+// (fmaxf and not inline assembly: the compiler puts the wait between a matrix instruction and the first read of its result, and does
+// not look into assembly for that.  It forms v_max3_f32, and passes only what comes out of a lane swap through a maximum with itself.)
+__device__ __forceinline__ float max2f(float a, float b) { return fmaxf(a, b); }
 // The maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (a score column's four lane groups), in all four:
 // two swaps of lane halves and rows between a register and its copy, in the vector unit (a shuffle through
 // LDS takes a round trip to LDS for each of the two steps, in the middle of the softmax's chain).
 __device__ __forceinline__ float max_over_lane_groups(float x) {
   const unsigned u = __float_as_uint(x);
   const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // [lo, lo] and [hi, hi]
-  float m;
-  asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(__uint_as_float(halves[0])), "v"(__uint_as_float(halves[1])));
+  const float m = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
   const unsigned um = __float_as_uint(m);
   const auto rows = __builtin_amdgcn_permlane16_swap(um, um, false, false);  // rows [0, 0, 2, 2] and [1, 1, 3, 3]
-  asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(__uint_as_float(rows[0])), "v"(__uint_as_float(rows[1])));
-  return m;
+  return fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
 }
-__device__ __forceinline__ float max3f(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+__device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 // ==========================================================================
 // MFMA core.  One wave owns 16*QT query columns and walks over pages of keys.

@@ -96,13 +96,9 @@ struct PromptArgs {
   float scale2;  // times log2(e)
 };
 
-// In one instruction: fmaxf passes every operand through a maximum with itself first, to quiet a signalling NaN, which the matrix unit
-// does not make.
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// (fmaxf and not inline assembly: the compiler forms v_max3_f32, behind the wait between a matrix instruction and the first read of its
+// result, which it does not put in front of assembly)
+__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 // Scores S^T = K Q^T of 32 keys by 32 queries, O^T += V^T P^T, both 32x32x16: the lane layout is that of the prompts' attention with
 // head sizes up to 128 (attention.hip).  A block is 64 queries of one head and walks 128 keys a step: two runs of 32 queries by four
@@ -256,11 +252,11 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
     }
     float top = max3(max3(sc[0], sc[1], sc[2]), max3(sc[3], sc[4], sc[5]), max3(sc[6], sc[7], sc[8]));
-    top = max3(top, max3(sc[9], sc[10], sc[11]), max3(sc[12], sc[13], max3(sc[14], sc[15], sc[15])));
+    top = max3(top, max3(sc[9], sc[10], sc[11]), max3(sc[12], sc[13], fmaxf(sc[14], sc[15])));
     {
       const unsigned u = __float_as_uint(top);
       const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // the column's other lane
-      top = max3(__uint_as_float(halves[0]), __uint_as_float(halves[1]), __uint_as_float(halves[1]));
+      top = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
     }
     const float m_new = fmaxf(m, top * a.scale2);  // (the scale is positive)
     const float alpha = __builtin_amdgcn_exp2f(m - m_new);

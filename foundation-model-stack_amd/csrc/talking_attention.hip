@@ -97,17 +97,9 @@ __global__ void __launch_bounds__(TALK_THREADS)
 #define TALK_KEYS 32 // keys of a tile
 
 __device__ __forceinline__ bf16x8 talk_load8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
-// maxima as single instructions: the scores come out of the matrix unit and are never signalling NaNs
-__device__ __forceinline__ float talk_max2(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ float talk_max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// (fmaxf and not inline assembly: the compiler puts the wait between a matrix instruction and the first read of its result)
+__device__ __forceinline__ float talk_max2(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ float talk_max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 struct TalkArgs {
   const bf16* q;

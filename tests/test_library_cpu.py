@@ -1137,12 +1137,14 @@ def test_embedding_leaves_a_norm_of_somebody_elses_to_that_norm(monkeypatch):
     assert embedding.forward_normed(ids, ParameterizedNorm(8), torch.bfloat16) is None
 
 
-@pytest.mark.parametrize("name", ["sgemm.hip"])
-def test_vector_instructions_are_the_compilers(name):
+def test_vector_instructions_are_the_compilers():
     """The compiler puts waits between a matrix instruction and whatever reads or writes its registers, but does not look into inline
-    assembly: none of it may hold vector arithmetic beside matrix instructions."""
+    assembly: none of it may hold vector arithmetic, which could stand beside matrix instructions."""
     from fms_amd.kernels.build import CSRC
 
-    with open(os.path.join(CSRC, name)) as f:
-        found = re.findall(r"asm\s*(?:volatile)?\s*\(\s*\"[^\"]*\bv_[^\"]*", f.read())
-    assert not found, found
+    found = {}
+    for name in sorted(os.listdir(CSRC)):
+        if name.endswith((".hip", ".h")):
+            with open(os.path.join(CSRC, name)) as f:
+                found[name] = re.findall(r"asm\s*(?:volatile)?\s*\(\s*\"[^\"]*\bv_[^\"]*", f.read())
+    assert not any(found.values()) and "sgemm.hip" in found, found
