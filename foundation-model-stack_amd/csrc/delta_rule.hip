@@ -565,7 +565,7 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
                                     int conv_dtype, int taps, const float* a_log, const float* dt_bias, float* conv_state,
                                     const int* seq_of_token, const int* slot_ids, float* qkv, float* beta, float* decay,
                                     float* kq, int n_tokens, int heads, int kv_heads, int dim, int vdim, int per_channel,
-                                    float q_scale, const int* seq_starts, int n_seqs, hipStream_t stream) {
+                                    float q_scale, const int* seq_starts, int n_seqs, int single_tokens, hipStream_t stream) {
   if (n_tokens == 0) return 0;
   FMS_REQUIRE(n_tokens > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0,
               "delta_prepare: bad sizes heads=%d kv_heads=%d dim=%d vdim=%d", heads, kv_heads, dim, vdim);
@@ -593,11 +593,12 @@ extern "C" int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const
   const bool pays = dim > 128 ? long_seqs && work >= 8000000
                               : columns >= 8192 || (long_seqs && (columns >= 6144 || work >= 5000000 || (columns >= 4096 && n_tokens >= 512)));
   const bool by_tokens = n_tokens > 64 && dim <= 256 && units <= 65535 && pays;
-  // A sequence a block, and no kernel for the state behind it, where sequences bring a token each on average (a decode step).
-  // More tokens a sequence would follow one another in a block that the others spread over blocks.
+  // A sequence a block, and no kernel for the state behind it, where sequences bring a token each (a decode step, with or without
+  // rows of padding behind its sequences, so that it is the same kernel in a captured step and in an eager one) or less on average.  More
+  // tokens a sequence would follow one another in a block that the others spread over blocks.
   const int seq_threads = dim <= 128 ? 256 : 512;
   const long seq_units = kv_heads + (heads * (long)vdim + seq_threads - 1) / seq_threads + (decays + seq_threads - 1) / seq_threads;
-  const bool by_seqs = seq_starts != nullptr && n_tokens <= n_seqs && dim <= 256 && seq_units <= 65535;
+  const bool by_seqs = seq_starts != nullptr && (single_tokens || n_tokens <= n_seqs) && dim <= 256 && seq_units <= 65535;
   const dim3 grid(ceil_div(n_tokens, PREP_TOKENS), (unsigned)units);
   const size_t token_lds = (size_t)PREP_TOKENS * (2 * dim + 4) * sizeof(float);
 #define FMS_PREP(W)                                                                                                   \

@@ -6,7 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
-#define FMSAMD_ABI_VERSION 14
+#define FMSAMD_ABI_VERSION 15
 
 // element types
 #define FMS_F32 0
@@ -335,13 +335,14 @@ int fmsamd_cast_cols(const float* x, long ldx, void* out, int out_dtype, long ld
 // convolution and whose columns col_b .. col_b + heads are the logits of beta; a: rows with the decay's input at col_a
 // (heads columns, or heads*dim if per_channel); conv_w [C, taps]; conv_state [slots][taps-1][C] is read, then updated.
 // Writes qkv [T, C] (convolved, silu, q and k unit vectors per head, q times q_scale), beta [T, heads] and
-// (seq_starts [n_seqs + 1] or null: where the sequences start; the state is then moved on by their last tokens' blocks only)
+// (seq_starts [n_seqs + 1] or null: where the sequences start; the state is then moved on by their last tokens' blocks only;
+// single_tokens != 0: no sequence brings more than one token)
 // decay [T, heads (*dim)] = exp(-exp(a_log) softplus(a + dt_bias)), and kq [T, kv_heads] = k . q of the finished vectors.
 int fmsamd_delta_prepare(const float* proj, long ld, int col_b, const float* a, long lda, int col_a, const void* conv_w,
                          int conv_dtype, int taps, const float* a_log, const float* dt_bias, float* conv_state,
                          const int* seq_of_token, const int* slot_ids, float* qkv, float* beta, float* decay, float* kq,
                          int n_tokens, int heads, int kv_heads, int dim, int vdim, int per_channel, float q_scale,
-                         const int* seq_starts, int n_seqs, hipStream_t stream);
+                         const int* seq_starts, int n_seqs, int single_tokens, hipStream_t stream);
 // The recurrence over every sequence's tokens of the step (seq_starts [n_seqs + 1]); state [slots][heads][vdim][dim]
 // is read and written; out [T, heads*vdim].  single_tokens != 0: the caller knows that no sequence brings more than one
 // token, and the kernel stages accordingly (the result is the same either way).

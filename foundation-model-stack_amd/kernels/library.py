@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads libamdhip64 before our library asks for it)
 
 from . import build as _build
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
@@ -79,7 +79,7 @@ _SIGNATURES = {
     "fmsamd_value_head_norm": [P, L, I, I, I, F, P, I, L, P, I, P],
     "fmsamd_scale_f32": [P, L, F, P],
     "fmsamd_cast_cols": [P, L, P, I, L, I, I, P],
-    "fmsamd_delta_prepare": [P, L, I, P, L, I, P, I, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, P, I, P],
+    "fmsamd_delta_prepare": [P, L, I, P, L, I, P, I, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, P, I, I, P],
     "fmsamd_delta_runs": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, L, P],
     "fmsamd_delta_rule": [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
     "fmsamd_gated_head_norm": [P, P, L, P, I, F, I, F, P, I, L, P, I, I, I, P],

@@ -1602,13 +1602,14 @@ DELTA_RUN_LONGEST = 128
 def delta_prepare(proj: torch.Tensor, col_b: int, a: torch.Tensor, col_a: int, conv_w: torch.Tensor, a_log: torch.Tensor,
                   dt_bias: torch.Tensor, conv_state: torch.Tensor, seq_of_token: torch.Tensor, slot_ids: torch.Tensor, heads: int,
                   kv_heads: int, dim: int, vdim: int, per_channel: bool, q_scale: float, seq_starts: Optional[torch.Tensor] = None,
-                  n_seqs: int = 0):
+                  n_seqs: int = 0, single_tokens: bool = False):
     """What the recurrence of a step reads, from the float32 projections of its tokens: (qkv [T, C], beta [T, heads],
     decay [T, heads] or [T, heads*dim], kq [T, kv_heads] = k . q), all float32.  The first C = 2*kv_heads*dim + heads*vdim columns of `proj` pass the
     short causal convolution (conv_w [C, taps]; the inputs before the step come from conv_state [slots, taps-1, C], which
     is then moved on), silu, and q and k become unit vectors per head (q times q_scale); beta = sigmoid(proj[:, col_b:]);
     decay = exp(-exp(a_log) * softplus(a[:, col_a:] + dt_bias)).  seq_starts [n_seqs + 1]: where the sequences' rows start
-    (the convolution's state is then moved on by their last tokens' blocks only)."""
+    (the convolution's state is then moved on by their last tokens' blocks only).  single_tokens: every sequence brings one token (a
+    decode step, which may have rows of padding behind them)."""
     _need_cuda(proj, a, conv_w, a_log, dt_bias, conv_state, seq_of_token, slot_ids, seq_starts)
     if seq_starts is not None:
         _need_i32("seq_starts", seq_starts)
@@ -1644,7 +1645,7 @@ def delta_prepare(proj: torch.Tensor, col_b: int, a: torch.Tensor, col_a: int, c
                                       _code(conv_w.dtype), taps, a_log.data_ptr(), dt_bias.data_ptr(), conv_state.data_ptr(),
                                       seq_of_token.data_ptr(), slot_ids.data_ptr(), qkv.data_ptr(), beta.data_ptr(), decay.data_ptr(),
                                       kq.data_ptr(), T, heads, kv_heads, dim, vdim, int(bool(per_channel)), float(q_scale),
-                                      _ptr(seq_starts), int(n_seqs), _stream()))
+                                      _ptr(seq_starts), int(n_seqs), int(bool(single_tokens)), _stream()))
     return qkv, beta, decay, kq
 
 

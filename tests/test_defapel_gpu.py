@@ -636,6 +636,30 @@ def test_delta_prepare_of_a_decode_step(lib, sizes):
     assert torch.equal(left, want_left)
 
 
+@pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (2, 2, 256, 80, 8, True), (33, 3, 24, 9, 3, True)])
+def test_delta_prepare_of_an_eager_decode_step(lib, sizes):
+    """Three sequences of one token and a row of padding behind them: what the captured step of four sequences gives, bit for bit."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, taps, per_channel = sizes
+    C, per = 2 * G * D + H * V, D if per_channel else 1
+    gen = torch.Generator().manual_seed(D + 1)
+    proj, a = torch.randn(4, C + H, generator=gen).to(DEV), torch.randn(4, H * per, generator=gen).to(DEV)
+    conv_w, state = torch.randn(C, taps, generator=gen).to(DEV), torch.randn(5, taps - 1, C, generator=gen).to(DEV)
+    a_log, dt_bias = torch.randn(H, generator=gen).to(DEV), torch.randn(H * per, generator=gen).to(DEV)
+    seq = torch.tensor([0, 1, 2, -1], dtype=torch.int32, device=DEV)
+
+    def run(conv_state, n_seqs, **how):
+        starts, slots = torch.arange(n_seqs + 1, dtype=torch.int32, device=DEV), torch.tensor([3, 1, 4, 0][:n_seqs], dtype=torch.int32, device=DEV)
+        return ops.delta_prepare(proj, C, a, 0, conv_w, a_log, dt_bias, conv_state, seq, slots, H, G, D, V, per_channel, D ** -0.5,
+                                 seq_starts=starts, n_seqs=n_seqs, **how)
+
+    left, want_left = state.clone(), state.clone()
+    for x, y in zip(run(left, 3, single_tokens=True), run(want_left, 4)):
+        assert torch.equal(x[:3], y[:3])
+    assert torch.equal(left, want_left) and not torch.equal(left, state)
+
+
 def test_a_lost_state_shows(lib):
     """The recurrence's memory matters: a value written long ago, read by a matching query much later, with decays near one."""
     from fms_amd.kernels import ops
@@ -1062,6 +1086,30 @@ def test_long_decoding_through_graphs_and_eager_steps(lib, folders, dtype):
             engine.end_sequence(s)
         engine.cache.check()
         assert bool(engine.graph_captures) == use_graphs
+
+
+@pytest.mark.parametrize("name", sorted(CONFIGS))
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_eager_and_replayed_steps_have_the_same_bits(lib, folders, name, dtype):
+    """Three sequences and a row of padding: the eager step has the shape of the captured one and runs the same kernels."""
+    from fms_amd.engine import Engine
+    from fms_amd.sampling import SamplingParams
+
+    cfg, _ = plain(folders, name)
+    model = get(lib, folders, name, dtype)
+    seqs = [tokens_for(cfg["vocab"], n, 70 + n) for n in (90, 33, 17)]
+    got = {}
+    for use_graphs in (True, False):
+        engine = Engine(model, max_tokens=64 * 6, max_slots=3, use_graphs=use_graphs)
+        slots = [engine.new_sequence() for _ in seqs]
+        engine.step(slots, [s[:-12] for s in seqs], "last")
+        for i in range(12):
+            feed = [s[len(s) - 12 + i] for s in seqs]
+            if use_graphs:
+                engine.decode_and_choose(slots, feed, SamplingParams(do_sample=False))
+                got[i] = engine.last_graph.logits[: len(seqs)].clone()
+            else:
+                assert torch.equal(engine.step(slots, [[t] for t in feed], "last"), got[i]), i
 
 
 @pytest.mark.parametrize("name", sorted(CONFIGS))
