@@ -264,10 +264,16 @@ __global__ void __launch_bounds__(512)
   for (int j = 0; j < DELTA_MAX_TAPS; ++j) w[j] = j < taps && live ? to_f32(conv_w[(size_t)c * taps + j]) : 0.f;
   float* state = nullptr;
   int before = -1;  // the last token's sequence
+  auto leave = [&]() {  // the last inputs of a sequence, into its state
+#pragma unroll
+    for (int j = 1; j < DELTA_MAX_TAPS; ++j)
+      if (j < taps && live) state[(size_t)(j - 1) * C + c] = x[j];
+  };
   for (int t = t0; t < t1; ++t) {
     const float fresh = live ? proj[(size_t)t * ld + c] : 0.f;
     const int seq = seq_of_token[t];
     const bool first = seq != before;
+    if (first && before >= 0) leave();  // a range may end in padding, or in another sequence's token
     before = seq;
     if (seq < 0) continue;
     if (first) {
@@ -310,11 +316,7 @@ __global__ void __launch_bounds__(512)
     }
     if (t + 1 < t1) __syncthreads();  // y and inv are read
   }
-  if (before >= 0 && live) {
-#pragma unroll
-    for (int j = 1; j < DELTA_MAX_TAPS; ++j)
-      if (j < taps) state[(size_t)(j - 1) * C + c] = x[j];
-  }
+  if (before >= 0) leave();
 }
 
 // --------------------------------------------------------------------------

@@ -636,6 +636,33 @@ def test_delta_prepare_of_a_decode_step(lib, sizes):
     assert torch.equal(left, want_left)
 
 
+@pytest.mark.parametrize("rows", [[[0, -1], [1], [2], [3], []], [[0, 2], [1], [], [3]], [[0, 0, -1], [-1, 1], [], [3], [], []]])
+def test_delta_prepare_of_ranges_that_end_in_other_rows(lib, rows):
+    """In a step of no more tokens than sequences a sequence's rows may end in padding, or hold another sequence's token: every state is
+    moved on, as where no starts are given."""
+    from fms_amd.kernels import ops
+
+    H, G, D, V, taps = 4, 2, 24, 20, 4
+    C = 2 * G * D + H * V
+    gen = torch.Generator().manual_seed(9)
+    seq = torch.tensor([i for r in rows for i in r], dtype=torch.int32)
+    T = len(seq)
+    proj, a = torch.randn(T, C + H, generator=gen).to(DEV), torch.randn(T, H, generator=gen).to(DEV)
+    conv_w, state = torch.randn(C, taps, generator=gen).to(DEV), torch.randn(7, taps - 1, C, generator=gen).to(DEV)
+    a_log, dt_bias = torch.randn(H, generator=gen).to(DEV), torch.randn(H, generator=gen).to(DEV)
+    slots = torch.tensor([5, 3, 0, 6, 1, 2][: len(rows)], dtype=torch.int32, device=DEV)
+    starts = torch.tensor([0] + list(np.cumsum([len(r) for r in rows])), dtype=torch.int32, device=DEV)
+
+    def run(conv_state, **how):
+        return ops.delta_prepare(proj, C, a, 0, conv_w, a_log, dt_bias, conv_state, seq.to(DEV), slots, H, G, D, V, False, D ** -0.5, **how)
+
+    left, want_left = state.clone(), state.clone()
+    got, want = run(left, seq_starts=starts, n_seqs=len(rows)), run(want_left)
+    for x, y in zip(got, want):
+        torch.testing.assert_close(x[(seq >= 0).to(DEV)], y[(seq >= 0).to(DEV)], atol=1e-7, rtol=5e-7)
+    assert torch.equal(left, want_left)
+
+
 @pytest.mark.parametrize("sizes", [(16, 8, 128, 128, 4, False), (2, 2, 256, 80, 8, True), (33, 3, 24, 9, 3, True)])
 def test_delta_prepare_of_an_eager_decode_step(lib, sizes):
     """Three sequences of one token and a row of padding behind them: what the captured step of four sequences gives, bit for bit."""
