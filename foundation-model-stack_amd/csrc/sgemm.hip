@@ -15,7 +15,7 @@
 //   * the even runs in their order, the odd runs in theirs, then the first sum less the second.
 //
 // A sum that is no finite number (an infinity among the factors, whose second part would be a NaN, or a number that rounds to one)
-// is formed again, the element by itself, from products and sums in float64.
+// is formed again, the element by itself, from products and sums in float64 (sgemm_tile_f64).
 // Below 2^-109 a number's third part begins to leave bfloat16's range: what is lost is less than 2^-134, the unit keeps subnormal numbers.
 #include "common.h"
 #include "fmsamd.h"
@@ -65,13 +65,31 @@ __device__ __forceinline__ void sgemm_run(const bf16x8 (&x)[3], const SgemmParts
       sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[ORDER[i][0]], w[j].p[ORDER[i][1]], sum[j], 0, 0, 0);
 }
 
-// The result c of the rows x and w, if it is no finite number (a NaN stays one, so nothing behind it is looked at).
-__device__ __forceinline__ void sgemm_again(float* c, const float* x, const float* w, const float* bias, int K) {
-  if (fabsf(*c) < INFINITY) return;
-  double sum = 0.0;
-#pragma nounroll
-  for (int k = 0; k < K && sum == sum; ++k) sum += (double)x[k] * (double)w[k];
-  *c = (float)(sum + (bias ? *bias : 0.f));
+// 16 x 16 results of rows m0 .. of x and n0 .. of W from products and sums in float64, by a wave: lane l has column l % 16 and rows
+// l / 16 + 4 e.  For results that the bfloat16 parts cannot give.  Bound by the matrix unit in float64 and the round trips in front of it; a
+// product of nothing but such results takes some six times as long as another: 301 rows by 4096 of K = 4096 770 us instead of 120
+// (by a thread for each result, K in series: 15800), 8 rows 99 instead of 15 (406); with one infinity in x 274 (960), in W 424 (5860).
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f64x4 sgemm_tile_f64(const float* a, long lda, const float* w, int m0, int n0, int M, int N, int K) {
+  const int lane = threadIdx.x & (WAVE - 1), r = lane % 16, o = lane / 16;
+  const float* const x = a + (size_t)min(m0 + r, M - 1) * lda;  // a row that is not there is the last one
+  const float* const y = w + (size_t)min(n0 + r, N - 1) * K;
+  f64x4 sum = {0.0, 0.0, 0.0, 0.0};
+  int k = o * 4;
+#pragma unroll 4
+  for (; k - o * 4 + 16 <= K; k += 16) {  // uniform
+    const f32x4_at4 u = *reinterpret_cast<const f32x4_at4*>(x + k), v = *reinterpret_cast<const f32x4_at4*>(y + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)u[e], (double)v[e], sum, 0, 0, 0);
+  }
+  if (K % 16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = k + e < K;
+      sum = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? (double)x[k + e] : 0.0, in ? (double)y[k + e] : 0.0, sum, 0, 0, 0);
+    }
+  }
+  return sum;
 }
 
 // Few rows, and rows that are not 16-byte aligned or very far apart.  A block's tile is 16 TM rows of x by 16 TN rows of W; its eight
@@ -157,26 +175,27 @@ __global__ void __launch_bounds__(8 * WAVE)
     if (threadIdx.x >= ELEMENTS) return;
     total[0] -= shared[threadIdx.x];
   }
-  bool again = false;
   constexpr int RESULTS = (OWN + 1) / 2;
-  auto place = [&](int i, int& m, int& n) {
-    const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;  // the lane that had it
-    m = m0 + element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = n0 + element / 256 % TN * 16 + of % 16;
-    return m < M && n < N;
-  };
+  unsigned again = 0;  // bit i: the thread's result i
 #pragma unroll
   for (int i = 0; i < RESULTS; ++i) {
-    int m, n;
-    if (!place(i, m, n)) continue;
+    const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;  // the lane that had it
+    const int m = m0 + element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = n0 + element / 256 % TN * 16 + of % 16;
+    if (m >= M || n >= N) continue;
     const float v = (float)((OWN == 1 ? total[i] : total[i] - total[i + OWN / 2]) + (bias ? bias[n] : 0.f));
     c[(size_t)m * ldc + n] = v;
-    again |= !(fabsf(v) < INFINITY);
+    again |= fabsf(v) < INFINITY ? 0u : 1u << i;
   }
-  if (again) {
+  if (__any(again)) {  // the wave has four rows of a tile: rows 4 e + lane % 4, columns lane / 4
 #pragma nounroll
     for (int i = 0; i < RESULTS; ++i) {
-      int m, n;
-      if (place(i, m, n)) sgemm_again(c + (size_t)m * ldc + n, a + (size_t)m * lda, w + (size_t)n * K, bias ? bias + n : nullptr, K);
+      if (!__any(again >> i & 1)) continue;
+      const int tile16 = (wave * WAVE + i * THREADS) / 256, e = wave % 4;
+      const int mt = m0 + tile16 / TN * 16, nt = n0 + tile16 % TN * 16;
+      const f64x4 sum = sgemm_tile_f64(a, lda, w, mt, nt, M, N, K);
+      const int m = mt + 4 * e + o, n = nt + r;
+      if (__shfl((int)(again >> i & 1), r * 4 + o))
+        c[(size_t)m * ldc + n] = (float)((e == 0 ? sum[0] : e == 1 ? sum[1] : e == 2 ? sum[2] : sum[3]) + (bias ? bias[n] : 0.f));
     }
   }
 }
@@ -335,7 +354,8 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   }
   __syncthreads();
   if (odd) return;
-  bool again = false;
+  unsigned again = 0;  // bit 4 (j MT + i) + e
+  static_assert(MT * NT * 4 <= 32, "a bit for every result");
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = n0 + (wn * NT + j) * 16 + r;
@@ -348,15 +368,21 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
         const float v = (float)(total[i][j][e] - shared[((i * NT + j) * 4 + e) * WAVE] + b);
         if (m < M && n < N) {
           c[(size_t)m * ldc + n] = v;
-          again |= !(fabsf(v) < INFINITY);
+          again |= fabsf(v) < INFINITY ? 0u : 1u << (4 * (j * MT + i) + e);
         }
       }
   }
-  if (again) {
+  if (__any(again)) {
 #pragma nounroll
-    for (int i = 0; i < MT * NT * 4; ++i) {
-      const int m = m0 + i / (4 * NT) * 16 + o * 4 + i % 4, n = n0 + (wn * NT + i / 4 % NT) * 16 + r;
-      if (m < M && n < N) sgemm_again(c + (size_t)m * ldc + n, a + (size_t)m * lda, w + (size_t)n * K, bias ? bias + n : nullptr, K);
+    for (int t = 0; t < MT * NT; ++t) {
+      const int bits = again >> (4 * t) & 15;
+      if (!__any(bits)) continue;
+      const int mt = m0 + t % MT * 16, nt = n0 + (wn * NT + t / MT) * 16;
+      const f64x4 sum = sgemm_tile_f64(a, lda, w, mt, nt, M, N, K);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)  // row 4 e + o: lane 16 e + r had it, as its result o
+        if (__shfl(bits, 16 * e + r) >> o & 1)
+          c[(size_t)(mt + 4 * e + o) * ldc + nt + r] = (float)(sum[e] + (bias ? bias[nt + r] : 0.f));
     }
   }
 }

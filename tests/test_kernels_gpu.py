@@ -646,6 +646,31 @@ def test_gemm_f32_of_numbers_that_are_not_finite_or_nearly(ops, M, N, K):
     assert float(((small - exact).abs() / bound).max()) <= 1.0
 
 
+@pytest.mark.parametrize("M,N", [(301, 4096), (8, 4096)])
+def test_gemm_f32_of_results_that_are_not_finite_costs_little(ops, M, N):
+    """A product whose results all overflow, or are all infinite, takes a few times as long as another."""
+    torch.manual_seed(66)
+    K = 4096
+    x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
+
+    def time(rows, weights):
+        ops.linear(rows, weights, None)
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(3):
+            ops.linear(rows, weights, None)
+        end.record()
+        end.synchronize()
+        return start.elapsed_time(end)
+
+    usual = time(x, w)
+    endless, large = x.clone(), x.abs() * 1e30
+    endless[:, 7] = math.inf
+    assert time(endless, w.abs()) < 12 * usual
+    assert bool(ops.linear(large, w.abs() * 1e30, None).isinf().all())
+    assert time(large, w.abs() * 1e30) < 12 * usual
+
+
 def test_gemm_f32_of_rows_far_apart(ops):
     """Rows of x 2^23 floats apart and one float less: a tile's rows lie past 32 bits of bytes, and just within them."""
     if torch.cuda.mem_get_info()[0] < 8e9:
