@@ -16,7 +16,8 @@
 //
 // A sum that is no finite number (an infinity among the factors, whose second part would be a NaN, or a number that rounds to one)
 // is formed again, the element by itself, from products and sums in float64 (sgemm_tile_f64).
-// Below 2^-109 a number's third part begins to leave bfloat16's range: what is lost is less than 2^-134, the unit keeps subnormal numbers.
+// Below 2^-109 a number's third part begins to leave bfloat16's range (the unit keeps subnormal numbers).  Results of a row with a number
+// that its parts do not hold exactly are formed again like those that are not finite.
 #include "common.h"
 #include "fmsamd.h"
 #include "tile_product_lds.h"
@@ -34,7 +35,8 @@ struct SgemmParts {
 
 // Two numbers at a time: 11 instructions where conversions by element take 15.  (The compiler forms the conversion: it does not look
 // into inline assembly for registers that a matrix instruction in flight still reads or writes, and so puts no wait in front of it.)
-__device__ __forceinline__ SgemmParts sgemm_split(f32x8 v) {
+// lost: its lower half becomes other than zero if the third rest of a number has bits that bfloat16 has not.
+__device__ __forceinline__ SgemmParts sgemm_split(f32x8 v, unsigned& lost) {
   u32x4_parts w[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -45,11 +47,19 @@ __device__ __forceinline__ SgemmParts sgemm_split(f32x8 v) {
       w[p][i] = pair;
       if (p < 2) a -= __uint_as_float(pair << 16), b -= __uint_as_float(pair & 0xffff0000u);
     }
+    lost |= __float_as_uint(a) | __float_as_uint(b);
   }
   SgemmParts parts;
 #pragma unroll
   for (int p = 0; p < 3; ++p) parts.p[p] = __builtin_bit_cast(bf16x8, w[p]);
   return parts;
+}
+
+// Which of the 16 rows that a wave's lanes have split (lane l: row l % 16) have lost bits.
+__device__ __forceinline__ unsigned sgemm_lost_rows(unsigned lost) {
+  const unsigned long long lanes = __ballot((lost & 0xffffu) != 0);
+  const unsigned half = (unsigned)lanes | (unsigned)(lanes >> 32);
+  return (half | half >> 16) & 0xffffu;
 }
 
 // A run of 16 rows of x by TN tiles of 16 rows of W; lane l of a result has column l % 16 and rows 4 (l / 16) + e.
@@ -102,6 +112,7 @@ __global__ void __launch_bounds__(8 * WAVE)
   constexpr int WAVES = 8, THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
   constexpr int OWN = 2 * ELEMENTS / THREADS;  // sums of a thread: (chain, element) threadIdx.x, + THREADS, ...
   __shared__ __attribute__((aligned(16))) float lds[2][WAVES][ELEMENTS];
+  __shared__ __attribute__((aligned(16))) unsigned lost_rows[TM + TN][WAVES];
 
   // The tiles of x that share a tile of W follow one another on one of the eight dies (blocks are dealt to the dies in
   // turn), so that W comes from memory once.
@@ -143,15 +154,21 @@ __global__ void __launch_bounds__(8 * WAVE)
   double total[OWN];
 #pragma unroll
   for (int i = 0; i < OWN; ++i) total[i] = 0.0;
+  unsigned lost[TM + TN] = {};
   const int rounds = (K + WAVES * SG_RUN - 1) / (WAVES * SG_RUN);
   fetch(wave);
   for (int t = 0; t < rounds; ++t) {
     SgemmParts x[TM], y[TN];
 #pragma unroll
-    for (int u = 0; u < TM; ++u) x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u]);
+    for (int u = 0; u < TM; ++u) x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u], lost[u]);
 #pragma unroll
-    for (int u = 0; u < TN; ++u) y[u] = sgemm_split(ahead[TM + u]);
-    if (t + 1 < rounds) fetch((t + 1) * WAVES + wave);
+    for (int u = 0; u < TN; ++u) y[u] = sgemm_split(ahead[TM + u], lost[TM + u]);
+    if (t + 1 < rounds) {
+      fetch((t + 1) * WAVES + wave);
+    } else {
+#pragma unroll
+      for (int u = 0; u < TM + TN; ++u) lost_rows[u][wave] = sgemm_lost_rows(lost[u]);
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       f32x4 sum[TN];
@@ -184,7 +201,11 @@ __global__ void __launch_bounds__(8 * WAVE)
     if (m >= M || n >= N) continue;
     const float v = (float)((OWN == 1 ? total[i] : total[i] - total[i + OWN / 2]) + (bias ? bias[n] : 0.f));
     c[(size_t)m * ldc + n] = v;
-    again |= fabsf(v) < INFINITY ? 0u : 1u << i;
+    unsigned rows = 0, cols = 0;
+#pragma unroll
+    for (int of_wave = 0; of_wave < WAVES; ++of_wave)
+      rows |= lost_rows[element / 256 / TN][of_wave], cols |= lost_rows[TM + element / 256 % TN][of_wave];
+    again |= fabsf(v) < INFINITY && ((rows >> (m & 15) | cols >> (n & 15)) & 1) == 0 ? 0u : 1u << i;
   }
   if (__any(again)) {  // the wave has four rows of a tile: rows 4 e + lane % 4, columns lane / 4
 #pragma nounroll
@@ -223,6 +244,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   constexpr int BYTES = PLANES + 2 * 2 * 3 * PLANE;
   static_assert(BM * BN * 8 <= BYTES, "the waves of a place meet in the same LDS");
   __shared__ __attribute__((aligned(16))) char lds[BYTES];
+  __shared__ unsigned lost_rows[MT + NT * WN][2];  // of x, of W, in the even and the odd runs
   const int per_die = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_die || tile >= tiles) return;
@@ -262,6 +284,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   };
   const unsigned at0 = mine + r * 128 + ((2 * o) ^ (r >> 1)) * 16, at1 = mine + r * 128 + ((2 * o + 1) ^ (r >> 1)) * 16;
   f32x8 raw[UNITS];
+  unsigned lost[UNITS] = {};
   auto read = [&](int stage) {
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
@@ -273,7 +296,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   auto put = [&](int stage) {
 #pragma unroll
     for (int u = 0; u < MT / WN; ++u) {
-      const SgemmParts parts = sgemm_split(odd ? -raw[NT + u] : raw[NT + u]);
+      const SgemmParts parts = sgemm_split(odd ? -raw[NT + u] : raw[NT + u], lost[NT + u]);
 #pragma unroll
       for (int p = 0; p < 3; ++p)
         *reinterpret_cast<bf16x8*>(lds + PLANES + ((stage * 2 + odd) * 3 + p) * PLANE + (wn * (MT / WN) + u) * 1024 + lane * 16) = parts.p[p];
@@ -303,7 +326,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next run is written there
   fetch(2, 0);
 #pragma unroll
-  for (int j = 0; j < NT; ++j) parts[0][j] = sgemm_split(raw[j]);
+  for (int j = 0; j < NT; ++j) parts[0][j] = sgemm_split(raw[j], lost[j]);
   put(0);
   const int steps = (K + BK - 1) / BK;
   auto step = [&](int s, int stage) {
@@ -323,7 +346,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
       sgemm_run<NT>(x, parts[stage], sum);
       add(i ? i - 1 : MT - 1);
       if (i == (MT > NT ? MT - NT - 1 : 0)) put(stage ^ 1);
-      if (i >= MT - NT) parts[stage ^ 1][i - MT + NT] = sgemm_split(raw[i - MT + NT]);
+      if (i >= MT - NT) parts[stage ^ 1][i - MT + NT] = sgemm_split(raw[i - MT + NT], lost[i - MT + NT]);
 #pragma unroll
       for (int j = 0; j < NT; ++j) last[j] = sum[j];
 #pragma unroll
@@ -345,6 +368,9 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   }
   add(MT - 1);
   tile_wait<0>();
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u)
+    lost_rows[u < NT ? MT + wn * NT + u : wn * (MT / WN) + u - NT][odd] = sgemm_lost_rows(lost[u]);
 
   // the odd runs' sums, to the waves that have the even ones'
   double* const shared = reinterpret_cast<double*>(lds) + (size_t)wn * MT * NT * 256 + lane;
@@ -360,17 +386,20 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   for (int j = 0; j < NT; ++j) {
     const int n = n0 + (wn * NT + j) * 16 + r;
     const float b = bias && n < N ? bias[n] : 0.f;
+    const unsigned col = (lost_rows[MT + wn * NT + j][0] | lost_rows[MT + wn * NT + j][1]) >> r & 1;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i) {
+      const unsigned rows = (lost_rows[i][0] | lost_rows[i][1]) >> (o * 4) | (col ? 15u : 0u);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int m = m0 + i * 16 + o * 4 + e;
         const float v = (float)(total[i][j][e] - shared[((i * NT + j) * 4 + e) * WAVE] + b);
         if (m < M && n < N) {
           c[(size_t)m * ldc + n] = v;
-          again |= fabsf(v) < INFINITY ? 0u : 1u << (4 * (j * MT + i) + e);
+          again |= (rows >> e & 1) == 0 && fabsf(v) < INFINITY ? 0u : 1u << (4 * (j * MT + i) + e);
         }
       }
+    }
   }
   if (__any(again)) {
 #pragma nounroll

@@ -624,8 +624,8 @@ def test_gemm_f32_rows_keep_their_bits(ops, K):
 
 @pytest.mark.parametrize("M,N,K", [(8, 300, 64), (40, 4096, 132), (301, 4096, 256), (301, 4096, 131), (40, 300, 13)])
 def test_gemm_f32_of_numbers_that_are_not_finite_or_nearly(ops, M, N, K):
-    """Infinities and numbers that bfloat16 rounds to one show where 64 bits show them, and change no other result's bits; subnormal
-    thirds of small numbers are kept to 2^-134."""
+    """Infinities and numbers that bfloat16 rounds to one show where 64 bits show them, and change no other result's bits; small numbers,
+    whose third parts bfloat16 does not hold, count whole."""
     torch.manual_seed(65)
     x, w, b = torch.randn(M, K), torch.randn(N, K), torch.randn(N)
     clean = ops.linear(dev(x), dev(w), dev(b)).cpu()
@@ -640,10 +640,34 @@ def test_gemm_f32_of_numbers_that_are_not_finite_or_nearly(ops, M, N, K):
     assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
     small = ops.linear(dev(x * 2.0 ** -120), dev(w), None).cpu().double()
     exact = (x * 2.0 ** -120).double() @ w.double().t()
-    # the bound of the tile shapes' test, and what the third parts lose
+    # the bound of the tile shapes' test
     bound = 2.0 ** -24 * (16.5 * exact.abs().new_tensor(2.0 ** -120) * (x.abs().double() @ w.abs().double().t()) + exact.abs())
-    bound += 2.0 ** -134 * w.abs().double().sum(1) + 2.0 ** -148
+    bound += 2.0 ** -148
     assert float(((small - exact).abs() / bound).max()) <= 1.0
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 300, 40), (8, 12288, 132), (16, 4100, 520), (40, 4096, 132), (130, 4100, 260), (301, 4096, 256), (40, 4096, 131)])
+@pytest.mark.parametrize("down", [-105, -115, -125, -140])
+def test_gemm_f32_of_small_numbers(ops, M, N, K, down):
+    """Rows of x and of W with a small number, or all small, beside large factors: float32's 24 bits count, down to its subnormal numbers,
+    and the rows beside them keep their bits."""
+    torch.manual_seed(67)
+    x, w = torch.randn(M, K), torch.randn(N, K) * 2.0 ** 60
+    clean = ops.linear(dev(x), dev(w), None).cpu()
+    y, v = x.clone(), w.clone()
+    y[1] *= 2.0 ** down
+    y[3, K - 1] *= 2.0 ** down
+    v[7] *= 2.0 ** (down - 60)
+    v[N - 1, 0] *= 2.0 ** (down - 60)
+    got = ops.linear(dev(y), dev(v), None).cpu()
+    exact = y.double() @ v.double().t()
+    # the bound of the tile shapes' test, and half a step of the smallest numbers
+    bound = 2.0 ** -24 * (16.5 * (y.abs().double() @ v.abs().double().t()) + exact.abs()) + 2.0 ** -149
+    assert float(((got.double() - exact).abs() / bound).max()) <= 1.0
+    rows, cols = [m for m in range(M) if m not in (1, 3)], [n for n in range(N) if n not in (7, N - 1)]
+    assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
+    for few in (1, 2, 4):  # the same bits in the tiles of fewer rows
+        assert torch.equal(ops.linear(dev(y[:few]), dev(v), None).cpu(), got[:few])
 
 
 @pytest.mark.parametrize("M,N", [(301, 4096), (8, 4096)])
