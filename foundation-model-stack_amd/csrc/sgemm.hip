@@ -13,6 +13,7 @@
 // element or on alignment:
 //   * a run of 32 k-values: (x3, w1), (x1, w3), (x2, w2), (x2, w1), (x1, w2), (x1, w1), one 16x16x32 instruction each;
 //   * the even runs in their order, the odd runs in theirs, then the first sum less the second.
+// Short rows (sgemm_is_short: by K alone) are summed in float64.
 //
 // A sum that is no finite number (an infinity among the factors, whose second part would be a NaN, or a number that rounds to one)
 // is formed again, the element by itself, from products and sums in float64 (sgemm_tile_f64).
@@ -82,20 +83,20 @@ __device__ __forceinline__ void sgemm_run(const bf16x8 (&x)[3], const SgemmParts
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f64x4 sgemm_tile_f64(const float* a, long lda, const float* w, int m0, int n0, int M, int N, int K) {
   const int lane = threadIdx.x & (WAVE - 1), r = lane % 16, o = lane / 16;
-  const float* const x = a + (size_t)min(m0 + r, M - 1) * lda;  // a row that is not there is the last one
-  const float* const y = w + (size_t)min(n0 + r, N - 1) * K;
+  const float* const x = a + (size_t)min(m0 + r, M - 1) * lda + o * 4;  // a row that is not there is the last one
+  const float* const y = w + (size_t)min(n0 + r, N - 1) * K + o * 4;
   f64x4 sum = {0.0, 0.0, 0.0, 0.0};
-  int k = o * 4;
-#pragma unroll 4
-  for (; k - o * 4 + 16 <= K; k += 16) {  // uniform
+  int k = 0;
+#pragma unroll 2
+  for (; k + 16 <= K; k += 16) {
     const f32x4_at4 u = *reinterpret_cast<const f32x4_at4*>(x + k), v = *reinterpret_cast<const f32x4_at4*>(y + k);
 #pragma unroll
     for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)u[e], (double)v[e], sum, 0, 0, 0);
   }
-  if (K % 16) {
+  if (k < K) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const bool in = k + e < K;
+      const bool in = k + o * 4 + e < K;
       sum = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? (double)x[k + e] : 0.0, in ? (double)y[k + e] : 0.0, sum, 0, 0, 0);
     }
   }
@@ -112,7 +113,8 @@ __global__ void __launch_bounds__(8 * WAVE)
   constexpr int WAVES = 8, THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
   constexpr int OWN = 2 * ELEMENTS / THREADS;  // sums of a thread: (chain, element) threadIdx.x, + THREADS, ...
   __shared__ __attribute__((aligned(16))) float lds[2][WAVES][ELEMENTS];
-  __shared__ __attribute__((aligned(16))) unsigned lost_rows[TM + TN][WAVES];
+  static_assert(TM <= 4 && TN <= 4, "a bit of 64 for every row");
+  __shared__ unsigned long long lost_rows[WAVES][2];  // of x, of W
 
   // The tiles of x that share a tile of W follow one another on one of the eight dies (blocks are dealt to the dies in
   // turn), so that W comes from memory once.
@@ -154,20 +156,27 @@ __global__ void __launch_bounds__(8 * WAVE)
   double total[OWN];
 #pragma unroll
   for (int i = 0; i < OWN; ++i) total[i] = 0.0;
-  unsigned lost[TM + TN] = {};
+  unsigned long long lost[2] = {};  // rows of x, of W (in scalar registers: vector ones would cost the block beside this one its place)
   const int rounds = (K + WAVES * SG_RUN - 1) / (WAVES * SG_RUN);
   fetch(wave);
   for (int t = 0; t < rounds; ++t) {
     SgemmParts x[TM], y[TN];
 #pragma unroll
-    for (int u = 0; u < TM; ++u) x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u], lost[u]);
+    for (int u = 0; u < TM; ++u) {
+      unsigned bits = 0;
+      x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u], bits);
+      lost[0] |= (unsigned long long)sgemm_lost_rows(bits) << (u * 16);
+    }
 #pragma unroll
-    for (int u = 0; u < TN; ++u) y[u] = sgemm_split(ahead[TM + u], lost[TM + u]);
+    for (int u = 0; u < TN; ++u) {
+      unsigned bits = 0;
+      y[u] = sgemm_split(ahead[TM + u], bits);
+      lost[1] |= (unsigned long long)sgemm_lost_rows(bits) << (u * 16);
+    }
     if (t + 1 < rounds) {
       fetch((t + 1) * WAVES + wave);
     } else {
-#pragma unroll
-      for (int u = 0; u < TM + TN; ++u) lost_rows[u][wave] = sgemm_lost_rows(lost[u]);
+      lost_rows[wave][0] = lost[0], lost_rows[wave][1] = lost[1];
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -201,11 +210,18 @@ __global__ void __launch_bounds__(8 * WAVE)
     if (m >= M || n >= N) continue;
     const float v = (float)((OWN == 1 ? total[i] : total[i] - total[i + OWN / 2]) + (bias ? bias[n] : 0.f));
     c[(size_t)m * ldc + n] = v;
-    unsigned rows = 0, cols = 0;
+    again |= fabsf(v) < INFINITY ? 0u : 1u << i;
+  }
+  unsigned long long rows = 0, cols = 0;
 #pragma unroll
-    for (int of_wave = 0; of_wave < WAVES; ++of_wave)
-      rows |= lost_rows[element / 256 / TN][of_wave], cols |= lost_rows[TM + element / 256 % TN][of_wave];
-    again |= fabsf(v) < INFINITY && ((rows >> (m & 15) | cols >> (n & 15)) & 1) == 0 ? 0u : 1u << i;
+  for (int of_wave = 0; of_wave < WAVES; ++of_wave) rows |= lost_rows[of_wave][0], cols |= lost_rows[of_wave][1];
+  if (rows | cols) {  // the same in the block
+#pragma unroll
+    for (int i = 0; i < RESULTS; ++i) {
+      const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;
+      const int m = element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = element / 256 % TN * 16 + of % 16;
+      if (m0 + m < M && n0 + n < N) again |= (unsigned)((rows >> m | cols >> n) & 1) << i;
+    }
   }
   if (__any(again)) {  // the wave has four rows of a tile: rows 4 e + lane % 4, columns lane / 4
 #pragma nounroll
@@ -380,39 +396,54 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
   }
   __syncthreads();
   if (odd) return;
-  unsigned again = 0;  // bit 4 (j MT + i) + e
+  auto result = [&](int i, int j, int e, float b) { return (float)(total[i][j][e] - shared[((i * NT + j) * 4 + e) * WAVE] + b); };
+  float finite = 0.f;  // or a NaN
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + (wn * NT + j) * 16 + r;
+    const float b = bias && n < N ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + i * 16 + o * 4 + e;
+        const float v = result(i, j, e, b);
+        finite = fmaf(v, 0.f, finite);
+        if (m < M && n < N) c[(size_t)m * ldc + n] = v;
+      }
+  }
+  unsigned rows[MT + NT], any = 0;
+#pragma unroll
+  for (int u = 0; u < MT + NT; ++u) {
+    const int of = u < MT ? u : u + wn * NT;
+    any |= rows[u] = lost_rows[of][0] | lost_rows[of][1];
+  }
+  if (any == 0 && !__any(finite != 0.f)) return;  // the same in the wave
+  unsigned again = 0;                             // bit 4 (j MT + i) + e
   static_assert(MT * NT * 4 <= 32, "a bit for every result");
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = n0 + (wn * NT + j) * 16 + r;
     const float b = bias && n < N ? bias[n] : 0.f;
-    const unsigned col = (lost_rows[MT + wn * NT + j][0] | lost_rows[MT + wn * NT + j][1]) >> r & 1;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const unsigned rows = (lost_rows[i][0] | lost_rows[i][1]) >> (o * 4) | (col ? 15u : 0u);
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + i * 16 + o * 4 + e;
-        const float v = (float)(total[i][j][e] - shared[((i * NT + j) * 4 + e) * WAVE] + b);
-        if (m < M && n < N) {
-          c[(size_t)m * ldc + n] = v;
-          again |= (rows >> e & 1) == 0 && fabsf(v) < INFINITY ? 0u : 1u << (4 * (j * MT + i) + e);
-        }
+        const bool lost_bits = (rows[i] >> (o * 4 + e) | rows[MT + j] >> r) & 1;
+        if (m0 + i * 16 + o * 4 + e < M && n < N && (lost_bits || !(fabsf(result(i, j, e, b)) < INFINITY)))
+          again |= 1u << (4 * (j * MT + i) + e);
       }
-    }
   }
-  if (__any(again)) {
 #pragma nounroll
-    for (int t = 0; t < MT * NT; ++t) {
-      const int bits = again >> (4 * t) & 15;
-      if (!__any(bits)) continue;
-      const int mt = m0 + t % MT * 16, nt = n0 + (wn * NT + t / MT) * 16;
-      const f64x4 sum = sgemm_tile_f64(a, lda, w, mt, nt, M, N, K);
+  for (int t = 0; t < MT * NT; ++t) {
+    const int bits = again >> (4 * t) & 15;
+    if (!__any(bits)) continue;
+    const int mt = m0 + t % MT * 16, nt = n0 + (wn * NT + t / MT) * 16;
+    const f64x4 sum = sgemm_tile_f64(a, lda, w, mt, nt, M, N, K);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)  // row 4 e + o: lane 16 e + r had it, as its result o
-        if (__shfl(bits, 16 * e + r) >> o & 1)
-          c[(size_t)(mt + 4 * e + o) * ldc + nt + r] = (float)(sum[e] + (bias ? bias[nt + r] : 0.f));
-    }
+    for (int e = 0; e < 4; ++e)  // row 4 e + o: lane 16 e + r had it, as its result o
+      if (__shfl(bits, 16 * e + r) >> o & 1)
+        c[(size_t)(mt + 4 * e + o) * ldc + nt + r] = (float)(sum[e] + (bias ? bias[nt + r] : 0.f));
   }
 }
 
@@ -423,26 +454,101 @@ static void sgemm_lds_launch(const float* a, long lda, const float* w, const flo
   sgemm_lds_kernel<MT, NT, WN><<<8 * ceil_div(tiles, 8), 2 * WN * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
-// At most SG_SHORT products: a thread has a row of W and 16 rows of x, sums in float64.  Bound by the results' bytes.
-#define SG_SHORT 16
-template <int KMAX>
+// At most four products: a thread has a row of W and 16 rows of x, sums in float64.  Bound by the results' bytes.
+#define SG_TINY 4
 __global__ void __launch_bounds__(256)
-    sgemm_short_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
-                       float* __restrict__ c, long ldc, int M, int N, int K, int n_blocks) {
+    sgemm_tiny_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
+                      float* __restrict__ c, long ldc, int M, int N, int K, int n_blocks) {
   const int n = blockIdx.x % n_blocks * 256 + threadIdx.x, m0 = blockIdx.x / n_blocks * 16;
   if (n >= N) return;
-  float y[KMAX];
+  float y[SG_TINY];
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) y[k] = k < K ? w[(size_t)n * K + k] : 0.f;
+  for (int k = 0; k < SG_TINY; ++k) y[k] = k < K ? w[(size_t)n * K + k] : 0.f;
   const float b = bias ? bias[n] : 0.f;
   for (int m = m0; m < min(m0 + 16, M); ++m) {
     double sum = 0.0;
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k)
+    for (int k = 0; k < SG_TINY; ++k)
       if (k < K) sum += (double)a[(size_t)m * lda + k] * (double)y[k];  // uniform
     c[(size_t)m * ldc + n] = (float)(sum + b);
   }
 }
+
+// Short rows: 16 TM rows of x by 16 TN rows of W a wave, products and sums on the matrix unit in float64, four of 4 k-values at a time.
+// Lane l asks for four k-values of row l % 16 at a time, from memory to registers.  Bound by the matrix unit (4.6 us for 16 k-values of
+// 2048 by 4096 results) and the results' bytes.  A wave of 64 x 64 results has its unit to itself, and nothing else to do while it stores:
+// 2048 by 4096 of K = 32 22 us, as waves of 32 x 32 19, of 16 x 16 22; 301 by 4096 10.9, 6.6, 5.6.
+template <int TM, int TN>
+__global__ void __launch_bounds__(256)
+    sgemm_short_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
+                       float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
+  const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int tile = blockIdx.x * 4 + wave;
+  if (tile >= tiles) return;
+  const int m0 = tile % m_tiles * 16 * TM, n0 = tile / m_tiles * 16 * TN;
+  const int r = lane % 16, o = lane / 16;
+  const float* src[TM + TN];  // a row that is not there is the last one
+#pragma unroll
+  for (int u = 0; u < TM; ++u) src[u] = a + (size_t)min(m0 + u * 16 + r, M - 1) * lda + o * 4;
+#pragma unroll
+  for (int u = 0; u < TN; ++u) src[TM + u] = w + (size_t)min(n0 + u * 16 + r, N - 1) * K + o * 4;
+  f32x4 ahead[TM + TN];
+  auto fetch = [&](int k0) {
+    if (k0 + 16 <= K) {  // uniform
+#pragma unroll
+      for (int u = 0; u < TM + TN; ++u) ahead[u] = *reinterpret_cast<const f32x4_at4*>(src[u] + k0);
+    } else {
+#pragma unroll
+      for (int u = 0; u < TM + TN; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ahead[u][e] = k0 + o * 4 + e < K ? src[u][k0 + e] : 0.f;
+    }
+  };
+  f64x4 sum[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) sum[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+  fetch(0);
+  for (int k0 = 0; k0 < K; k0 += 16) {
+    f32x4 v[TM + TN];
+#pragma unroll
+    for (int u = 0; u < TM + TN; ++u) v[u] = ahead[u];
+    if (k0 + 16 < K) fetch(k0 + 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          sum[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)v[i][e], (double)v[TM + j][e], sum[i][j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + j * 16 + r;
+    if (n >= N) continue;
+    const float b = bias ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + i * 16 + 4 * e + o;
+        if (m < M) c[(size_t)m * ldc + n] = (float)(sum[i][j][e] + b);
+      }
+  }
+}
+
+template <int TM, int TN>
+static void sgemm_short_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
+                               hipStream_t stream) {
+  const int m_tiles = ceil_div(M, 16 * TM), tiles = m_tiles * ceil_div(N, 16 * TN);
+  sgemm_short_kernel<TM, TN><<<ceil_div(tiles, 4), 4 * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
+}
+
+// Which rows are short goes with K alone, so that a row's bits go with nothing else.  Beside the kernels of three parts, which take a whole run
+// of 32 and the ends of a block however short the rows are, 2048 by 4096: K = 16 13 us and 28, 32 19 and 29, 64 27 and 29, 96 37 and 38, 128 47 and 36; rows that
+// cannot all be aligned, K = 17 19 and 60, 129 50 and 70, 255 89 and 96, 321 110 and 106.
+static bool sgemm_is_short(int K) { return K <= (K % 4 == 0 ? 96 : 256); }
 
 // The tile shape.  What a compute unit needs for its blocks was measured at K = 4096 (1 to 301 rows of x, 4096 to 32000 of W): the first
 // block costs `first` microseconds, every further one `next`, whatever the rows.  Small tiles fill the chip where there are few rows, and their
@@ -469,15 +575,19 @@ static int sgemm_shape(int shapes, int M, int N) {
   return best;
 }
 
+#define SGEMM_SHORT_TILES 16384  // from here on waves of 32 x 32 results fill the chip
 #define SGEMM_NEAR (1 << 22)  // 128 rows of so many floats lie within 32 bits of bytes
 static void sgemm(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K, bool aligned,
                   hipStream_t stream) {
-  if (K <= SG_SHORT) {
-    const int n_blocks = ceil_div(N, 256), blocks = n_blocks * ceil_div(M, 16);
-    if (K <= 4)
-      sgemm_short_kernel<4><<<blocks, 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
-    else
-      sgemm_short_kernel<SG_SHORT><<<blocks, 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
+  if (sgemm_is_short(K)) {
+    if (K <= SG_TINY) {
+      const int n_blocks = ceil_div(N, 256);
+      sgemm_tiny_kernel<<<n_blocks * ceil_div(M, 16), 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
+    } else if ((long)ceil_div(M, 16) * ceil_div(N, 16) >= SGEMM_SHORT_TILES) {
+      sgemm_short_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream);
+    } else {
+      sgemm_short_launch<1, 1>(a, lda, w, bias, c, ldc, M, N, K, stream);
+    }
     return;
   }
   const bool any = aligned && lda < SGEMM_NEAR && K < SGEMM_NEAR;

@@ -590,9 +590,12 @@ def test_gemm_f32(ops, M, N, K):
 
 
 # every tile shape with rows, columns and K past its last whole tile.  Aligned: 16x16 (17 by 300), 16x64 (48 by 4100), 32x64 (130 by
-# 3000, 64 by 8190), 64x64 (130 by 4100, 301 by 8200), 64x128 (513 by 16390).  Rows that are not 16-byte aligned (odd K, odd stride):
-# 16x16 (8 by 4096, 17 by 300), 16x64 (48 by 4100), 32x32 (from 130 rows on).  K up to 16: sums in float64
-@pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7)])
+# 3000, 64 by 8190), 64x64 (130 and 301 by 8200 of K = 260), 64x128 (513 by 16390 of K = 100).  Rows that are not 16-byte aligned (odd
+# stride, K = 261): 16x16 (17 by 300), 16x64 (48 by 4100), 32x32 (from 130 rows on).  K up to 96, odd K up to 256: sums in float64, waves
+# of 16x16 (8 by 4096, 130 by 4100) and 32x32 (from 301 by 8200 on)
+@pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7),
+                                   (17, 300, 261), (48, 4100, 261), (130, 4100, 261), (130, 8200, 260), (301, 8200, 260), (513, 16390, 100),
+                                   (301, 8200, 96), (301, 8200, 255), (17, 300, 255)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     torch.manual_seed(61)
@@ -605,11 +608,11 @@ def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     assert float(((out - want).abs() / bound).max()) <= 1.0
 
 
-@pytest.mark.parametrize("K", [7, 36, 1000, 1028])
+@pytest.mark.parametrize("K", [3, 7, 36, 96, 100, 255, 257, 1000, 1028])
 def test_gemm_f32_rows_keep_their_bits(ops, K):
     """A row has the same bits whatever else is in the product: tiles of 16x64 (1 and 8 rows), 32x64 (17 and 130), 64x64 (33 and 61),
     64x128 (301) and 16x16 (301 by 100), rows that are not 16-byte aligned (an odd stride, an odd K) in tiles of 16x64 (1 and 8),
-    16x32 (33) and 32x32."""
+    16x32 (33) and 32x32; short rows (K up to 96, odd ones up to 256) in waves of 16x16 (up to 33 rows) and 32x32."""
     torch.manual_seed(62)
     N = 12790
     x, w, b = dev(torch.randn(301, K)), dev(torch.randn(N, K)), dev(torch.randn(N))
