@@ -111,7 +111,9 @@ __global__ void __launch_bounds__(8 * WAVE)
     sgemm_few_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
                      float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
   constexpr int WAVES = 8, THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
-  constexpr int OWN = 2 * ELEMENTS / THREADS;  // sums of a thread: (chain, element) threadIdx.x, + THREADS, ...
+  // A thread adds up the even and the odd runs of its elements threadIdx.x, + THREADS, ...; with one tile the even or the odd ones.
+  constexpr bool BOTH = ELEMENTS >= THREADS;
+  constexpr int RESULTS = (ELEMENTS + THREADS - 1) / THREADS;
   __shared__ __attribute__((aligned(16))) float lds[2][WAVES][ELEMENTS];
   static_assert(TM <= 4 && TN <= 4, "a bit of 64 for every row");
   __shared__ unsigned long long lost_rows[WAVES][2];  // of x, of W
@@ -153,9 +155,9 @@ __global__ void __launch_bounds__(8 * WAVE)
     }
   };
 
-  double total[OWN];
+  double total[RESULTS], odd[RESULTS];
 #pragma unroll
-  for (int i = 0; i < OWN; ++i) total[i] = 0.0;
+  for (int i = 0; i < RESULTS; ++i) total[i] = odd[i] = 0.0;
   unsigned long long lost[2] = {};  // rows of x, of W (in scalar registers: vector ones would cost the block beside this one its place)
   const int rounds = (K + WAVES * SG_RUN - 1) / (WAVES * SG_RUN);
   fetch(wave);
@@ -187,28 +189,31 @@ __global__ void __launch_bounds__(8 * WAVE)
     }
     __syncthreads();  // and everybody is done with the sums of the round before the last
 #pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-      const int q = threadIdx.x + i * THREADS;
+    for (int i = 0; i < RESULTS; ++i) {
+      const int q = BOTH ? threadIdx.x + i * THREADS : threadIdx.x % ELEMENTS;
+      if (ELEMENTS % THREADS != 0 && q >= ELEMENTS) continue;  // the same in the wave
 #pragma unroll
-      for (int run = 0; run < WAVES / 2; ++run) total[i] += (double)lds[t & 1][2 * run + q / ELEMENTS][q % ELEMENTS];
+      for (int run = 0; run < WAVES / 2; ++run) {
+        total[i] += (double)lds[t & 1][2 * run + (BOTH ? 0 : threadIdx.x / ELEMENTS)][q];
+        if (BOTH) odd[i] += (double)lds[t & 1][2 * run + 1][q];
+      }
     }
   }
 
-  if constexpr (OWN == 1) {  // the odd runs' sums, to the threads that have the even ones'
+  if constexpr (!BOTH) {  // the odd runs' sums, to the threads that have the even ones'
     double* const shared = reinterpret_cast<double*>(lds[rounds & 1]);  // nobody reads there any more
     if (threadIdx.x >= ELEMENTS) shared[threadIdx.x - ELEMENTS] = total[0];
     __syncthreads();
     if (threadIdx.x >= ELEMENTS) return;
-    total[0] -= shared[threadIdx.x];
+    odd[0] = shared[threadIdx.x];
   }
-  constexpr int RESULTS = (OWN + 1) / 2;
   unsigned again = 0;  // bit i: the thread's result i
 #pragma unroll
   for (int i = 0; i < RESULTS; ++i) {
     const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;  // the lane that had it
     const int m = m0 + element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = n0 + element / 256 % TN * 16 + of % 16;
-    if (m >= M || n >= N) continue;
-    const float v = (float)((OWN == 1 ? total[i] : total[i] - total[i + OWN / 2]) + (bias ? bias[n] : 0.f));
+    if ((ELEMENTS % THREADS != 0 && element >= ELEMENTS) || m >= M || n >= N) continue;
+    const float v = (float)(total[i] - odd[i] + (bias ? bias[n] : 0.f));
     c[(size_t)m * ldc + n] = v;
     again |= fabsf(v) < INFINITY ? 0u : 1u << i;
   }
@@ -220,7 +225,7 @@ __global__ void __launch_bounds__(8 * WAVE)
     for (int i = 0; i < RESULTS; ++i) {
       const int element = threadIdx.x + i * THREADS, of = element % 256 / 4;
       const int m = element / 256 / TN * 16 + of / 16 * 4 + element % 4, n = element / 256 % TN * 16 + of % 16;
-      if (m0 + m < M && n0 + n < N) again |= (unsigned)((rows >> m | cols >> n) & 1) << i;
+      if ((ELEMENTS % THREADS == 0 || element < ELEMENTS) && m0 + m < M && n0 + n < N) again |= (unsigned)((rows >> m | cols >> n) & 1) << i;
     }
   }
   if (__any(again)) {  // the wave has four rows of a tile: rows 4 e + lane % 4, columns lane / 4
@@ -558,9 +563,10 @@ struct SgemmShape {
   int bm, bn;
   float first, next;
 };
-#define SGEMM_FEW 4  // shapes that take any rows
-static const SgemmShape SGEMM_SHAPES[7] = {{16, 16, 21.f, 14.5f}, {16, 32, 27.5f, 21.5f}, {16, 64, 41.5f, 40.f}, {32, 32, 34.5f, 28.5f},
-                                           {32, 64, 54.f, 33.f},  {64, 64, 68.f, 67.f},   {64, 128, 102.f, 106.f}};
+#define SGEMM_FEW 5     // shapes that take any rows
+#define SGEMM_SHAPES_N 8
+static const SgemmShape SGEMM_SHAPES[SGEMM_SHAPES_N] = {{16, 16, 21.f, 14.5f}, {16, 32, 27.5f, 21.5f}, {16, 48, 38.f, 34.f},  {16, 64, 41.5f, 40.f},
+                                                        {32, 32, 34.5f, 28.5f}, {32, 64, 54.f, 33.f},  {64, 64, 68.f, 67.f}, {64, 128, 102.f, 106.f}};
 #define SGEMM_COMPUTE_UNITS 256
 
 static int sgemm_shape(int shapes, int M, int N) {
@@ -591,13 +597,14 @@ static void sgemm(const float* a, long lda, const float* w, const float* bias, f
     return;
   }
   const bool any = aligned && lda < SGEMM_NEAR && K < SGEMM_NEAR;
-  switch (sgemm_shape(any ? 7 : SGEMM_FEW, M, N)) {
+  switch (sgemm_shape(any ? SGEMM_SHAPES_N : SGEMM_FEW, M, N)) {
     case 0: sgemm_few_launch<1, 1>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
     case 1: sgemm_few_launch<1, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 2: sgemm_few_launch<1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 3: sgemm_few_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 4: sgemm_lds_launch<2, 2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 5: sgemm_lds_launch<4, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 2: sgemm_few_launch<1, 3>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 3: sgemm_few_launch<1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 4: sgemm_few_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 5: sgemm_lds_launch<2, 2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 6: sgemm_lds_launch<4, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
     default: sgemm_lds_launch<4, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
   }
 }
