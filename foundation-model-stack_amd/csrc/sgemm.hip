@@ -7,12 +7,13 @@
 //
 // Sums of 32 products each in float32, small terms first, added up in float64.  The matrix unit's sums round down, not to nearest, which
 // would add up over many of them (relative error 8.2e-8 at K = 4096, 1.2e-7 at 11008): every other run's x is negated and its sum subtracted,
-// so that what rounds down in one rounds up in the next (4.5e-8 at both; float32 products in sums of 16 had 7.8e-8).
+// so that what rounds down in one rounds up in the next (4.5e-8 at both; float32 products in sums of 16 had 7.8e-8).  The runs' signs are
+// + - - + over and over, so that the same holds where every other run is zero (9.2e-8 at 11008 with + -).
 //
 // Every kernel here adds in one order, so that a row's bits do not depend on how many rows there are, on the columns beside an
 // element or on alignment:
 //   * a run of 32 k-values: (x3, w1), (x1, w3), (x2, w2), (x2, w1), (x1, w2), (x1, w1), one 16x16x32 instruction each;
-//   * the even runs in their order, the odd runs in theirs, then the first sum less the second.
+//   * the even runs in their order, the odd runs in theirs, every other one negated, then the first sum less the second.
 // Short rows (sgemm_is_short: by K alone) are summed in float64.
 //
 // A sum that is no finite number (an infinity among the factors, whose second part would be a NaN, or a number that rounds to one)
@@ -166,7 +167,7 @@ __global__ void __launch_bounds__(8 * WAVE)
 #pragma unroll
     for (int u = 0; u < TM; ++u) {
       unsigned bits = 0;
-      x[u] = sgemm_split(wave & 1 ? -ahead[u] : ahead[u], bits);
+      x[u] = sgemm_split((wave ^ wave >> 1) & 1 ? -ahead[u] : ahead[u], bits);
       lost[0] |= (unsigned long long)sgemm_lost_rows(bits) << (u * 16);
     }
 #pragma unroll
@@ -194,8 +195,12 @@ __global__ void __launch_bounds__(8 * WAVE)
       if (ELEMENTS % THREADS != 0 && q >= ELEMENTS) continue;  // the same in the wave
 #pragma unroll
       for (int run = 0; run < WAVES / 2; ++run) {
-        total[i] += (double)lds[t & 1][2 * run + (BOTH ? 0 : threadIdx.x / ELEMENTS)][q];
-        if (BOTH) odd[i] += (double)lds[t & 1][2 * run + 1][q];
+        const double sum = (double)lds[t & 1][2 * run + (BOTH ? 0 : threadIdx.x / ELEMENTS)][q];
+        total[i] = run & 1 ? total[i] - sum : total[i] + sum;
+        if (BOTH) {
+          const double other = (double)lds[t & 1][2 * run + 1][q];
+          odd[i] = run & 1 ? odd[i] - other : odd[i] + other;
+        }
       }
     }
   }
@@ -314,10 +319,10 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
       raw[u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   };
-  auto put = [&](int stage) {
+  auto put = [&](int stage) {  // (a run's stage is whether its number among its wave's runs is odd)
 #pragma unroll
     for (int u = 0; u < MT / WN; ++u) {
-      const SgemmParts parts = sgemm_split(odd ? -raw[NT + u] : raw[NT + u], lost[NT + u]);
+      const SgemmParts parts = sgemm_split(odd ^ stage ? -raw[NT + u] : raw[NT + u], lost[NT + u]);
 #pragma unroll
       for (int p = 0; p < 3; ++p)
         *reinterpret_cast<bf16x8*>(lds + PLANES + ((stage * 2 + odd) * 3 + p) * PLANE + (wn * (MT / WN) + u) * 1024 + lane * 16) = parts.p[p];
@@ -332,11 +337,14 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) total[i][j][e] = 0.0, last[j][e] = 0.f;
-  auto add = [&](int i) {
+  auto add = [&](int i, int stage) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) total[i][j][e] += (double)last[j][e];
+      for (int e = 0; e < 4; ++e) {
+        const double sum = (double)last[j][e];
+        total[i][j][e] = stage ? total[i][j][e] - sum : total[i][j][e] + sum;
+      }
   };
 
   SgemmParts parts[2][NT];
@@ -365,7 +373,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
       }
       f32x4 sum[NT];
       sgemm_run<NT>(x, parts[stage], sum);
-      add(i ? i - 1 : MT - 1);
+      add(i ? i - 1 : MT - 1, i ? stage : stage ^ 1);
       if (i == (MT > NT ? MT - NT - 1 : 0)) put(stage ^ 1);
       if (i >= MT - NT) parts[stage ^ 1][i - MT + NT] = sgemm_split(raw[i - MT + NT], lost[i - MT + NT]);
 #pragma unroll
@@ -387,7 +395,7 @@ __global__ void __launch_bounds__(2 * WN* WAVE)
     step(s, 0);
     if (s + 1 < steps) step(s + 1, 1);  // uniform
   }
-  add(MT - 1);
+  add(MT - 1, (steps - 1) & 1);
   tile_wait<0>();
 #pragma unroll
   for (int u = 0; u < UNITS; ++u)
