@@ -263,7 +263,8 @@ int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long ldo, void*
 
 // ---- the same for prompts, with keys and values expanded for the step (latent_expanded.hip) ----------------------------
 // q: rows of every head's dim + rot elements, not yet rotated; uk [nheads * dim, rank], uv [nheads * vdim, rank]; keys and values:
-// room for n_seqs * pages * nheads * 64 * dim and * vdim elements, pages even and at least what the longest sequence holds.
+// room for n_seqs * pages * nheads * 64 * dim and * vdim elements, pages even and at least what the step's tokens of a sequence look at
+// (with a window from the even page on that the sequence's first token of the step sees).
 // qblock_start, qblock_len: the step's tokens in blocks of at most 64 of one sequence.  Bfloat16; gate: float32 logits, a row a token.
 int fmsamd_latent_prompt_fits(int dim, int rot, int vdim, int rank);
 int fmsamd_latent_prompt(const void* q, long ldq, void* out, long ldo, const void* cache, const void* uk, const void* uv,

@@ -7,7 +7,8 @@
 // for its result, so it is for steps that bring most of the tokens that they look at.
 //
 //   latent_expand:  keys [seq][page][H][token][D] and values, transposed, [seq][page][H][V][token] of every row that the
-//                   step's sequences hold; rows behind a sequence's last token are zeros, up to an even number of pages
+//                   step's tokens look at (with a window from the pair of pages on that the sequence's first token of the step sees);
+//                   rows behind a sequence's last token are zeros, up to an even number of pages
 //   latent_prompt:  causal softmax attention over them: rotation of the queries on the way in, the gate on the way out
 #include "common.h"
 #include "fmsamd.h"
@@ -21,8 +22,13 @@ struct ExpandArgs {
   const bf16 *uk, *uv;  // [H * D, R], [H * V, R]
   bf16 *keys, *values;
   const int *positions, *seq_starts, *block_table;
-  int table_stride, pages, H, D, V, R;
+  int table_stride, pages, H, D, V, R, window;
 };
+
+// The first pair of pages that a sequence's tokens of the step look at, which its room begins with.
+__device__ __forceinline__ int first_pair(int first_position, int window) {
+  return window > 0 && first_position - window + 1 > 0 ? (first_position - window + 1) / LX_STEP : 0;
+}
 
 // A block: 128 tokens (two pages) by 128 columns of Uk, or 128 rows of Uv by 128 tokens, so that either result is written in runs
 // of 64 bytes.  K is the latent's size, eight steps for R = 512, so a block is mostly its first loads and its stores and two of them
@@ -36,12 +42,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) l
   const int seq = blockIdx.x / (a.pages / 2), pair = blockIdx.x % (a.pages / 2);
   const bool of_keys = (int)blockIdx.y < col_tiles;
   const int n0 = ((int)blockIdx.y - (of_keys ? 0 : col_tiles)) * COLS;
-  const int last = uniform_load(a.seq_starts + seq + 1) - 1;
-  const int context = last < uniform_load(a.seq_starts + seq) ? 0 : uniform_load(a.positions + last) + 1;
-  const int first = pair * LX_STEP;
+  const int begin = uniform_load(a.seq_starts + seq), last = uniform_load(a.seq_starts + seq + 1) - 1;
+  if (last < begin) return;  // uniform
+  const int context = uniform_load(a.positions + last) + 1;
+  const int of_sequence = first_pair(uniform_load(a.positions + begin), a.window) + pair, first = of_sequence * LX_STEP;
   if (first >= context) return;  // uniform
-  const int* bt = a.block_table + (size_t)seq * a.table_stride;
-  const size_t page0 = readable_page(bt[2 * pair]), page1 = readable_page(bt[2 * pair + (first + PAGE_TOKENS < context ? 1 : 0)]);
+  const int* bt = a.block_table + (size_t)seq * a.table_stride + 2 * of_sequence;
+  const size_t page0 = readable_page(bt[0]), page1 = readable_page(bt[first + PAGE_TOKENS < context ? 1 : 0]);
   auto token_row = [&](int i) { return a.cache + ((i < PAGE_TOKENS ? page0 : page1) * PAGE_TOKENS + i % PAGE_TOKENS) * a.width; };
   const int rows = a.H * (of_keys ? a.D : a.V);
   const bf16* const w = of_keys ? a.uk : a.uv;
@@ -89,7 +96,7 @@ struct PromptArgs {
   bf16* out;  // [T, ldo]: head h's V elements at h V
   long ldo;
   const bf16 *keys, *values, *cache;
-  const int *positions, *seq_of_token, *qblock_start, *qblock_len, *block_table;
+  const int *positions, *seq_of_token, *seq_starts, *qblock_start, *qblock_len, *block_table;
   const float *cos_t, *sin_t, *sink, *gate;  // gate: logits [T, ldg] or null
   long ldg;
   int n_qblocks, table_stride, pages, H, rank, window;
@@ -181,14 +188,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int d = (wave * V_LOADS + n) * 4 + (lane >> 4), piece = (lane & 15) ^ swizzle(d, 16);
     v_from[n] = (unsigned)((piece >> 3) * page_values + d * PAGE_TOKENS + (piece & 7) * 8) * 2;
   }
+  const int room_first = a.window > 0 ? first_pair(uniform_load(a.positions + uniform_load(a.seq_starts + seq)), a.window) : 0;
   const char* const own_keys = (const char*)(a.keys + ((size_t)seq * a.pages + half) * page_keys + (size_t)h * PAGE_TOKENS * D);
   const char* const own_values = (const char*)(a.values + (size_t)seq * a.pages * page_values + (size_t)h * V * PAGE_TOKENS);
   // (the second page of the last step may not be there: nobody sees its keys)
   auto entry_of = [&](int step) { return RC > 0 ? uniform_load(bt + step * 2 + (step * LX_STEP + half * PAGE_TOKENS <= blk_last ? half : 0)) : 0; };
   auto fetch = [&](int step, int buffer, int entry) {
     const unsigned to = lds0 + buffer * STAGE;
-    const char* const kp = own_keys + (size_t)step * 2 * page_keys * 2;
-    const char* const vp = own_values + (size_t)step * 2 * page_values * 2;
+    const char* const kp = own_keys + (size_t)(step - room_first) * 2 * page_keys * 2;
+    const char* const vp = own_values + (size_t)(step - room_first) * 2 * page_values * 2;
 #pragma unroll
     for (int n = 0; n < KN_LOADS; ++n) load_to_lds(kp, kn_from[n], to + (wave * KN_LOADS + n) * 1024);
     if constexpr (RC > 0) {
@@ -332,7 +340,7 @@ extern "C" int fmsamd_latent_prompt_fits(int dim, int rot, int vdim, int rank) {
   return dim == 128 && (rot == 64 || rot == 0) && vdim == 128 && rank >= TL_BK && rank % 8 == 0;
 }
 
-// pages: of every sequence in keys and values, even, at least as many as the longest sequence holds.
+// pages: of every sequence in keys and values, even, at least as many as the step's tokens of any sequence look at, from an even page on.
 // Every row of q belongs to a query block (qblock_start, qblock_len: at most 64 tokens of one sequence each).
 extern "C" int fmsamd_latent_prompt(const void* q, long ldq, void* out, long ldo, const void* cache, const void* uk, const void* uv,
                                     void* keys, void* values, const int* positions, const int* seq_of_token, const int* seq_starts,
@@ -356,11 +364,11 @@ extern "C" int fmsamd_latent_prompt(const void* q, long ldq, void* out, long ldo
                   (long)n_qblocks * nheads < (1l << 31) && nheads <= 16384,
               "latent_prompt: too much for one launch");
   const ExpandArgs e{(const bf16*)cache, rank + rot, (const bf16*)uk, (const bf16*)uv, (bf16*)keys, (bf16*)values, positions, seq_starts,
-                     block_table, table_stride, pages, nheads, dim, vdim, rank};
+                     block_table, table_stride, pages, nheads, dim, vdim, rank, window};
   latent_expand_kernel<<<dim3(n_seqs * (pages / 2), ceil_div((long)nheads * dim, 128) + ceil_div((long)nheads * vdim, 128)), 256, 0, stream>>>(e);
   FMS_LAUNCH_CHECK("latent_expand");
   const PromptArgs a{(const bf16*)q, ldq, (bf16*)out, ldo, (const bf16*)keys, (const bf16*)values, (const bf16*)cache, positions, seq_of_token,
-                     qblock_start, qblock_len, block_table, cos_t, sin_t, sink, gate, ldg, n_qblocks, table_stride, pages, nheads, rank, window,
+                     seq_starts, qblock_start, qblock_len, block_table, cos_t, sin_t, sink, gate, ldg, n_qblocks, table_stride, pages, nheads, rank, window,
                      scale * 1.4426950408889634f};
 #define LAUNCH_PROMPT(RC)                                                                                                     \
   do {                                                                                                                        \

@@ -1191,23 +1191,53 @@ def latent_prompt_pages(longest: int) -> int:
     return -(-longest // (2 * PAGE_TOKENS)) * 2
 
 
-def latent_prompt_pays(starts: Sequence[int], lengths: Sequence[int], nheads: int, dim: int, rot: int, vdim: int, rank: int) -> bool:
+def latent_prompt_longest(starts: Sequence[int], lengths: Sequence[int], window: int = 0) -> int:
+    """The most rows that the tokens of a sequence of the step (position of the first one, how many) look at, counted from the first
+    row of a pair of pages."""
+    return max(latent_prompt_rows(starts, lengths, window))
+
+
+def latent_prompt_rows(starts: Sequence[int], lengths: Sequence[int], window: int = 0) -> list:
+    """The same of every sequence."""
+    pair = 2 * PAGE_TOKENS
+    return [s + n - (max(s - window + 1, 0) // pair * pair if window > 0 else 0) for s, n in zip(starts, lengths)]
+
+
+def latent_prompt_pays(starts: Sequence[int], lengths: Sequence[int], nheads: int, dim: int, rot: int, vdim: int, rank: int,
+                       window: int = 0) -> bool:
     """True if a step of these sequences (position of the first token, tokens) is faster with expanded keys and values than in the
-    latent space.  Expanding costs what the rows cost, every sequence's as many as the longest one's; measured 5 ns a row for 16 heads
-    of 128 and a latent of 512.  In the latent space the products in and out are launches of their own (10 us more than here for a
-    few tokens), every pair of query and key is a product over the latent twice, and a block of four (token, 16 heads) takes its sequences one after the
-    other, 24 ns a key.  Measured, us, expanded and not: one prompt of 32 tokens 18, 29, of 300 22, 40, of 2048 64, 190; 2 tokens behind
-    8000 180, 427; 100 tokens beside four single ones behind 2000 each 124, 414, beside sixteen of them 403, 426; thirty single
-    tokens behind 100 beside two of 20 tokens 66, 57.
+    latent space, in microseconds of 16 heads of 128 + 64 and 128 and a latent of 512.  Expanded: 7.7 ns for every row that the step's tokens look
+    at (whole pairs of pages), written and read once, then 13 ns a key of the longest sequence, or of
+    every block of 64 tokens and a head, with 7 us for the block, on 256 compute units.  In the latent space: the products in and out are launches of their own, a block of four
+    (token, 16 heads) takes its sequences one after the other, 50 ns a key, or the products, 3.4 times as many.  Measured, us, expanded and
+    not: one prompt of 32 tokens 21, 39, sixteen of them 28, 39, one of 2048 69, 178; 64 tokens behind 8000 168, 434, four times that 374, 445,
+    eight times 623, 452; with a window of 1024: one prompt of 8192 245, 628, 64 tokens behind 30000 38, 78, 16 times 64 tokens behind 4000 143,
+    107, 30 times 8 tokens behind 2000 319, 85, 20 tokens beside 15 single ones behind 2000 each 140, 236; with one of 128 20 tokens beside 60
+    single ones behind 500 each 157, 62.
     """
-    contexts = [s + n for s, n in zip(starts, lengths)]
-    rows = len(contexts) * latent_prompt_pages(max(contexts)) * PAGE_TOKENS
-    if rows * nheads * (dim + vdim) * 2 > LATENT_PROMPT_ROOM:
+    spans = latent_prompt_rows(starts, lengths, window)
+    longest = max(spans)
+    if len(spans) * latent_prompt_pages(longest) * PAGE_TOKENS * nheads * (dim + vdim) * 2 > LATENT_PROMPT_ROOM:
         return False
-    expand = rows * nheads * (dim + vdim) * rank / (16 * 256 * 512) * 5e-3
-    chain = max(max(contexts), sum(sorted((c for c, n in zip(contexts, lengths) if n < 4), reverse=True)[:4]))
-    pairs = sum(n * c - n * (n - 1) // 2 for c, n in zip(contexts, lengths))
-    return expand <= 10 + 24e-3 * chain + pairs * nheads * (2 * rank + rot) * 2 / 5.5e8
+    rows = sum(latent_prompt_pages(r) for r in spans) * PAGE_TOKENS
+    seen = [min(s + n, window + 3) if window > 0 else s + n for s, n in zip(starts, lengths)]  # keys of a block's four tokens
+    chain = max(max(seen), sum(sorted((c for c, n in zip(seen, lengths) if n < 4), reverse=True)[:4]))
+    pairs = latent_prompt_pairs(starts, lengths, window)
+    size = nheads * (dim + vdim) * rank / (16 * 256 * 512)
+    blocks = sum(-(-n // LATENT_PROMPT_QBLOCK) * (7 + 13e-3 * (p / n + LATENT_PROMPT_QBLOCK / 2)) for p, n in zip(pairs, lengths)) * nheads / 256
+    expanded = 14 + 7.7e-3 * rows * size + max(13e-3 * longest, blocks)
+    latent = 39 + 12e-3 * sum(lengths) * size + max(50e-3 * chain, sum(pairs) * nheads * (2 * rank + rot) * 2 / 5.5e8)
+    return 1.1 * expanded <= latent
+
+
+def latent_prompt_pairs(starts: Sequence[int], lengths: Sequence[int], window: int = 0) -> list:
+    """Pairs of query and key of every sequence of the step."""
+    pairs = []
+    for s, n in zip(starts, lengths):
+        beyond = max(s + n - window, 0) if window > 0 else 0  # the last token sees so many keys less, the one in front of it one less, ...
+        over = min(beyond, n)
+        pairs.append(n * (s + n) - n * (n - 1) // 2 - (over * beyond - over * (over - 1) // 2))
+    return pairs
 
 
 def latent_prompt_aligned(q, uk, uv, cache, cos, sin, out) -> bool:
@@ -1223,7 +1253,8 @@ def latent_prompt_attention(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor,
     """Causal attention of a prompt step over the latent cache, with the keys [Uk c | shared part] and values Uv c of every cached
     row of the step's sequences formed first.  q: bfloat16 rows of every head's dim + rot elements, not rotated; uk
     [nheads * dim, rank], uv [nheads * vdim, rank]; gate: float32 logits [T, >= nheads] whose sigmoid multiplies a head's result, or
-    None; longest: at least what the longest sequence holds with this step.  Returns [T, nheads * vdim] (into `out`, rows of any
+    None; longest: at least the rows that a sequence's tokens look at (latent_prompt_longest; what the longest sequence holds is
+    enough).  Returns [T, nheads * vdim] (into `out`, rows of any
     stride)."""
     _need_cuda(q, uk, uv, positions, seq_of_token, seq_starts, qblock_start, qblock_len, block_table, cache, cos, sin, sink, gate, out)
     _rows2d("q", q)

@@ -97,3 +97,26 @@ def test_a_block_that_norms_its_branches_keeps_the_branch_norm_for_the_next_read
         stream.add_branch("another", post_norm=post)
     assert stream.normed(Norm(), torch.float32) == "normed" and calls == [("mixer output", post, None)]
     assert stream.pending is None and stream.pending_norm is None
+
+
+@pytest.mark.parametrize("window", [0, 1, 40, 128, 1024])
+def test_expanded_keys_are_counted_as_the_window_leaves_them(window):
+    """The rows, from a pair of pages on, and the pairs of query and key that a step's tokens see, against a count one by one."""
+    from fms_amd.kernels import ops
+
+    for starts, lengths in (([0], [1]), ([30000], [64]), ([100, 0, 2000], [3, 500, 1]), ([1023], [2]), ([1024, 5], [300, 1])):
+        seen = [[range(max(p - window + 1, 0) if window else 0, p + 1) for p in range(s, s + n)] for s, n in zip(starts, lengths)]
+        assert ops.latent_prompt_longest(starts, lengths, window) == max(r[-1].stop - r[0].start // 128 * 128 for r in seen)
+        assert ops.latent_prompt_pairs(starts, lengths, window) == [sum(len(keys) for keys in r) for r in seen]
+
+
+@pytest.mark.parametrize("runs,window,pays", [
+    ([(0, 32)], 0, True), ([(0, 32)] * 16, 0, True), ([(0, 2048)], 0, True), ([(8000, 64)], 0, True), ([(8000, 64)] * 4, 0, True),
+    ([(8000, 64)] * 8, 0, False), ([(0, 2048)], 1024, True), ([(0, 8192)], 1024, True), ([(30000, 64)], 1024, True),
+    ([(4000, 100)] * 4, 1024, True), ([(4000, 64)] * 16, 1024, False), ([(2000, 8)] * 30, 1024, False),
+    ([(2000, 1)] * 15 + [(2000, 20)], 1024, True), ([(500, 1)] * 60 + [(0, 20)], 128, False), ([(100000, 64)], 0, False)])
+def test_keys_are_expanded_where_that_was_measured_to_be_faster(runs, window, pays):
+    """The steps that the rule's comment names (and one without room): both ways were timed."""
+    from fms_amd.kernels import ops
+
+    assert ops.latent_prompt_pays([s for s, _ in runs], [n for _, n in runs], 16, 128, 64, 128, 512, window) == pays

@@ -427,10 +427,26 @@ def test_latent_attention_of_prompts(lib, heads, rot, runs, window):
 @pytest.mark.parametrize("runs,window", [([(0, 1)], 0), ([(0, 63), (0, 65), (0, 64)], 0), ([(0, 129), (127, 3), (128, 1), (200, 70)], 0),
                                          ([(300, 150), (0, 31)], 40), ([(0, 257)], 100)])
 def test_latent_attention_with_expanded_keys(lib, heads, rot, gated, runs, window):
+    expanded_keys(heads, rot, gated, runs, window, 72, max(s + n for s, n in runs))
+
+
+# a latent of the registered models' size, longer contexts, and with a window no more room than the step looks at
+@pytest.mark.parametrize("rot,gated", [(64, False), (0, True)])
+@pytest.mark.parametrize("runs,window", [([(0, 1030)], 0), ([(1900, 65), (3, 2), (1000, 1)], 0), ([(1000, 70), (640, 130)], 100),
+                                         ([(1500, 64)], 128), ([(900, 3), (2000, 200), (0, 40)], 1024)])
+def test_latent_attention_with_expanded_keys_of_long_contexts(lib, rot, gated, runs, window):
+    from fms_amd.kernels import ops
+
+    longest = ops.latent_prompt_longest([s for s, _ in runs], [n for _, n in runs], window)
+    assert longest <= min(max(s + n for s, n in runs), window + 127 + max(n for _, n in runs) if window else 1 << 30)
+    expanded_keys(2, rot, gated, runs, window, 512, longest)
+
+
+def expanded_keys(heads, rot, gated, runs, window, R, longest):
     from fms_amd.kernels import ops
 
     gen = torch.Generator().manual_seed(17 * heads + rot)
-    D, V, R, scale = 128, 128, 72, 0.06
+    D, V, scale = 128, 128, 0.06
     pages_of = [-(-(s + n) // 64) for s, n in runs]
     order = torch.randperm(sum(pages_of) + 1, generator=gen).tolist()
     table = torch.full((len(runs), max(pages_of)), -1, dtype=torch.int32)
@@ -451,20 +467,21 @@ def test_latent_attention_with_expanded_keys(lib, heads, rot, gated, runs, windo
     uk, uv = ((torch.randn(heads * size, R, generator=gen) * R ** -0.5).to(torch.bfloat16) for size in (D, V))
     sink = torch.randn(heads, generator=gen) if gated else None
     gate = torch.randn(T, heads + 2, generator=gen) if gated else None
-    angles = torch.arange(512)[:, None] * 10000.0 ** (-torch.arange(rot // 2) / max(rot // 2, 1))[None]
+    angles = torch.arange(4096)[:, None] * 10000.0 ** (-torch.arange(rot // 2) / max(rot // 2, 1))[None]
     cos, sin = torch.cos(angles).contiguous(), torch.sin(angles).contiguous()
     dev = lambda t: None if t is None else t.to(DEV)
     wide = torch.full((T, heads * V + 8), 7.0, dtype=torch.bfloat16, device=DEV)
     got = ops.latent_prompt_attention(dev(q), dev(uk), dev(uv), dev(pos), dev(seq), dev(starts), dev(torch.tensor([b for b, _ in blocks], dtype=torch.int32)),
                                       dev(torch.tensor([n for _, n in blocks], dtype=torch.int32)), dev(table), dev(cache),
                                       dev(cos) if rot else None, dev(sin) if rot else None, dev(sink), dev(gate), heads, D, rot, V, R, scale, window,
-                                      n_seqs=len(runs), longest=max(s + n for s, n in runs), out=wide[:, : heads * V]).double().cpu()
+                                      n_seqs=len(runs), longest=longest, out=wide[:, : heads * V]).double().cpu()
     assert bool((wide[:, heads * V:] == 7.0).all())
     want = torch.zeros(T, heads * V, dtype=torch.float64)
     for t in range(T):
         i, p = int(seq[t]), int(pos[t])
         lo = max(0, p - window + 1) if window else 0
-        rows = torch.stack([cache[int(table[i, k // 64]), 0, k % 64] for k in range(lo, p + 1)]).double()
+        places = torch.arange(lo, p + 1)
+        rows = cache[table[i, places // 64].long(), 0, places % 64].double()
         qt = q[t].double().view(heads, D + rot)
         if rot:
             u, w, c, s_ = qt[:, D::2], qt[:, D + 1 :: 2], cos[p].double(), sin[p].double()
