@@ -1246,15 +1246,26 @@ def latent_prompt_aligned(q, uk, uv, cache, cos, sin, out) -> bool:
             and (out is None or (out.data_ptr() % 8 == 0 and out.stride(0) % 4 == 0)))
 
 
+def latent_prompt_room(n_seqs: int, longest: int, nheads: int, dim: int, vdim: int, dtype: torch.dtype, device):
+    """Room for the expanded keys and values of a step's sequences, or None where the GPU has none left: the latent space takes such a
+    step with less."""
+    pages = n_seqs * latent_prompt_pages(longest)
+    try:
+        return (torch.empty(pages, nheads, PAGE_TOKENS, dim, dtype=dtype, device=device),
+                torch.empty(pages, nheads, vdim, PAGE_TOKENS, dtype=dtype, device=device))
+    except torch.OutOfMemoryError:
+        return None
+
+
 def latent_prompt_attention(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor, positions, seq_of_token, seq_starts, qblock_start, qblock_len,
                             block_table, cache: torch.Tensor, cos, sin, sink: Optional[torch.Tensor], gate: Optional[torch.Tensor],
                             nheads: int, dim: int, rot: int, vdim: int, rank: int, scale: float, window: int = 0, *, n_seqs: int,
-                            longest: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                            longest: int, out: Optional[torch.Tensor] = None, room=None) -> torch.Tensor:
     """Causal attention of a prompt step over the latent cache, with the keys [Uk c | shared part] and values Uv c of every cached
     row of the step's sequences formed first.  q: bfloat16 rows of every head's dim + rot elements, not rotated; uk
     [nheads * dim, rank], uv [nheads * vdim, rank]; gate: float32 logits [T, >= nheads] whose sigmoid multiplies a head's result, or
     None; longest: at least the rows that a sequence's tokens look at (latent_prompt_longest; what the longest sequence holds is
-    enough).  Returns [T, nheads * vdim] (into `out`, rows of any
+    enough); room: a latent_prompt_room of these sizes, or a new one.  Returns [T, nheads * vdim] (into `out`, rows of any
     stride)."""
     _need_cuda(q, uk, uv, positions, seq_of_token, seq_starts, qblock_start, qblock_len, block_table, cache, cos, sin, sink, gate, out)
     _rows2d("q", q)
@@ -1283,8 +1294,14 @@ def latent_prompt_attention(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor,
     pages = latent_prompt_pages(longest)
     if longest <= 0 or -(-longest // PAGE_TOKENS) > block_table.shape[1]:
         raise ValueError(f"sequences of {longest} tokens do not fit a block table of {block_table.shape[1]} pages")
-    keys = torch.empty(n_seqs * pages, nheads, PAGE_TOKENS, dim, dtype=q.dtype, device=q.device)
-    values = torch.empty(n_seqs * pages, nheads, vdim, PAGE_TOKENS, dtype=q.dtype, device=q.device)
+    if room is None:
+        room = latent_prompt_room(n_seqs, longest, nheads, dim, vdim, q.dtype, q.device)
+        if room is None:
+            raise torch.OutOfMemoryError(f"no room for the expanded keys and values of {n_seqs * pages} pages")
+    keys, values = room
+    for name, t, shape in (("keys", keys, (n_seqs * pages, nheads, PAGE_TOKENS, dim)), ("values", values, (n_seqs * pages, nheads, vdim, PAGE_TOKENS))):
+        if t.dtype != q.dtype or tuple(t.shape) != shape or t.device != q.device or not t.is_contiguous():
+            raise ValueError(f"room for {name} is a contiguous {q.dtype} {shape} tensor")
     check(load().fmsamd_latent_prompt(q.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0), cache.data_ptr(), uk.data_ptr(), uv.data_ptr(),
                                       keys.data_ptr(), values.data_ptr(), positions.data_ptr(), seq_of_token.data_ptr(), seq_starts.data_ptr(),
                                       qblock_start.data_ptr(), qblock_len.data_ptr(), qblock_start.numel(), block_table.data_ptr(),

@@ -152,15 +152,18 @@ class LatentAttention(Mixer):
             q = down[:, : self.q_cols] if down.dtype == x.dtype else ops.cast_cols(down, 0, self.q_cols, x.dtype)
         gate = down[:, self.gate_col : self.gate_col + self.gate_cols] if self.has_gate else None
         qb_start, qb_len = batch.qblocks.get(ops.LATENT_PROMPT_QBLOCK, (None, None))
+        room = None
         if (self._expands and not batch.is_decode and qb_start is not None
                 and ops.latent_prompt_aligned(q, self.w["uk.weight"], self.w["uv.weight"], cache.keys, cos, sin, out)
                 and ops.latent_prompt_pays(batch.starts, batch.q_lens, H, D, P, V, R, self.window)):
+            longest = ops.latent_prompt_longest(batch.starts, batch.q_lens, self.window)
+            room = ops.latent_prompt_room(batch.n_seqs, longest, H, D, V, q.dtype, q.device)
+        if room is not None:
             by_head = gate if self.gate_cols == H else None
             into = out if gate is by_head else None
             mixed = ops.latent_prompt_attention(q, self.w["uk.weight"], self.w["uv.weight"], batch.positions, batch.seq_of_token,
                                                 batch.seq_starts, qb_start, qb_len, table, cache.keys, cos, sin, self._sink, by_head, H, D, P, V, R,
-                                                self.scale, self.window, n_seqs=batch.n_seqs,
-                                                longest=ops.latent_prompt_longest(batch.starts, batch.q_lens, self.window), out=into)
+                                                self.scale, self.window, n_seqs=batch.n_seqs, longest=longest, out=into, room=room)
             if gate is not by_head:  # a gate per output element
                 mixed = ops.gate_mul(mixed, gate, "sigmoid", out=out)
             return BranchOutput(mixed, self.o)

@@ -120,3 +120,24 @@ def test_keys_are_expanded_where_that_was_measured_to_be_faster(runs, window, pa
     from fms_amd.kernels import ops
 
     assert ops.latent_prompt_pays([s for s, _ in runs], [n for _, n in runs], 16, 128, 64, 128, 512, window) == pays
+
+
+def test_no_memory_for_expanded_keys_is_an_answer(monkeypatch):
+    """A step that finds no memory for expanded keys and values is told so, and not refused; other errors stay errors."""
+    from fms_amd.kernels import ops
+
+    keys, values = ops.latent_prompt_room(3, 129, 2, 128, 64, torch.bfloat16, "cpu")
+    assert tuple(keys.shape) == (12, 2, 64, 128) and tuple(values.shape) == (12, 2, 64, 64)
+    taken, empty = [], torch.empty
+
+    def full(*sizes, **how):
+        if taken:
+            raise torch.OutOfMemoryError("none left")
+        taken.append(sizes)
+        return empty(*sizes, **how)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", full)
+        assert ops.latent_prompt_room(3, 129, 2, 128, 64, torch.bfloat16, "cpu") is None
+    with pytest.raises(RuntimeError):
+        ops.latent_prompt_room(3, 129, -2, 128, 64, torch.bfloat16, "cpu")
