@@ -91,6 +91,11 @@ CONFIGS = {
         layer(chunked(2, 2, 96, 96, 33, 48, factor=4.0, softcap=12.0), 64),
         layer(latent(2, 64, 32, 32, 128, 200, base=100.0), None),
     ]),
+    # head sizes whose prompts in bfloat16 attend to expanded keys and values: a window within the test sequences, one beyond them
+    "E": dict(vocab=300, width=192, norm={"eps": 1e-6}, embedding={"scale": 5.0}, max_positions=2048, layers=[
+        layer(latent(2, 128, 64, 128, 128, 20, scale=0.07), 128),
+        layer(latent(3, 128, 64, 128, 64, 500, scale=0.07), 192),
+    ]),
 }
 
 
@@ -409,6 +414,22 @@ def test_whole_sequence(lib, folders, name, dtype):
     judge(engine.step([slot], [ids], "all"), want, dtype)
     engine.end_sequence(slot)
     engine.cache.check()
+
+
+def test_prompts_with_a_window_and_a_gate_per_element_expand_keys(lib, folders, monkeypatch):
+    """Portions that start inside a window, behind pages that it has given back, through the expanded keys in every layer."""
+    from fms_amd.engine import Engine
+    from fms_amd.kernels import ops
+
+    ids, want = expected_for(folders, "E", 400, 3, "bfloat16")
+    model = get(lib, folders, "E", "bfloat16")
+    expanded, attention = [], ops.latent_prompt_attention
+    monkeypatch.setattr(ops, "latent_prompt_attention", lambda *args, **how: expanded.append((args[0].shape[0], how["longest"])) or attention(*args, **how))
+    engine = Engine(model, max_tokens=512, max_slots=1)
+    slot = engine.new_sequence()
+    got = [engine.step([slot], [ids[a:b]], "all") for a, b in ((0, 130), (130, 333), (333, 400))]
+    judge(torch.cat(got), want, "bfloat16")
+    assert expanded == [(130, 130), (130, 130), (203, 333), (203, 333), (67, 400 - 256), (67, 400)]
 
 
 @pytest.mark.parametrize("name", sorted(CONFIGS))

@@ -89,6 +89,11 @@ CONFIGS = {
         layer(recurrent(384, 3, 4), moe(8, 4, 3, 128, count=4, keep=2, scale=2.5, shared=128)),
         layer(attention(4, 128, 64, 64, 0.08), moe(0, 4, 2, 0, count=2, keep=1, scale=1.0, shared=256)),
     ]),
+    # head sizes whose prompts in bfloat16 attend to expanded keys and values
+    "D": dict(vocab=300, width=192, norm={"eps": 1e-6, "groups": 2}, canon={"taps": 3}, max_positions=1024, layers=[
+        layer(attention(3, 128, 128, 128, 0.08), {"kind": "dense", "ff": 256}),
+        layer(attention(2, 128, 128, 64, 0.08), {"kind": "dense", "ff": 128}),
+    ]),
 }
 
 

@@ -56,6 +56,7 @@ def layer(m, mlp):
 _mA = dict(heads=4, dim=16, rot=8, vdim=24, q_rank=48, kv_rank=40, scale=0.2)
 _mB = dict(heads=3, dim=12, rot=4, vdim=20, q_rank=36, kv_rank=28, scale=0.31)
 _mC = dict(heads=8, dim=64, rot=32, vdim=48, q_rank=128, kv_rank=128, scale=0.1)
+_mD = dict(heads=3, dim=128, rot=64, vdim=128, q_rank=96, kv_rank=128, scale=0.07)
 CONFIGS = {
     # two layers read the first one's latent; a layer without a feed-forward; experts with and without a shared one,
     # one of them choosing all its experts
@@ -76,6 +77,11 @@ CONFIGS = {
     "C": dict(vocab=512, width=256, norm={"eps": 1e-6}, embedding={"scale": 16.0}, max_positions=2048, layers=[
         layer(mixer(**_mC), {"kind": "dense", "ff": 512}),
         layer(mixer(**_mC, kv_from=0), moe(8, 2, 128, 2.0, shared=(128, 4.0))),
+    ]),
+    # head sizes whose prompts in bfloat16 attend to expanded keys and values, of a latent of their own and of another layer's
+    "D": dict(vocab=300, width=192, norm={"eps": 1e-6}, embedding={"scale": 8.0}, max_positions=1024, layers=[
+        layer(mixer(**_mD), {"kind": "dense", "ff": 256}),
+        layer(mixer(**_mD, kv_from=0), {"kind": "dense", "ff": 128}),
     ]),
 }
 
@@ -688,6 +694,41 @@ def test_whole_sequence_and_every_layer(lib, folders, name, dtype):
     judge(engine.step([slot], [ids], "all"), want, dtype)
     engine.end_sequence(slot)
     engine.cache.check()
+
+
+def test_prompts_expand_keys_where_there_is_room(lib, folders, monkeypatch):
+    """A prompt, portions behind it and sequences side by side go through the expanded keys in every layer; without room, and with less
+    memory than that takes, through the latent space; both are as near to the plain implementation."""
+    from fms_amd.engine import Engine
+    from fms_amd.kernels import ops
+
+    ids, want = expected_for(folders, "D", 150, 1, "bfloat16")
+    model = get(lib, folders, "D", "bfloat16")
+    expanded, attention = [], ops.latent_prompt_attention
+    monkeypatch.setattr(ops, "latent_prompt_attention", lambda *args, **how: expanded.append(args[0].shape[0]) or attention(*args, **how))
+
+    def run(cuts):
+        expanded.clear()
+        engine = Engine(model, max_tokens=256, max_slots=2)
+        slot = engine.new_sequence()
+        got = [engine.step([slot], [ids[a:b]], "all") for a, b in zip(cuts, cuts[1:])]
+        judge(torch.cat(got), want, "bfloat16")
+        return expanded[:]
+
+    assert run([0, 150]) == [150, 150]
+    assert run([0, 100, 101, 150]) == [100, 100, 49, 49]
+    with monkeypatch.context() as m:
+        m.setattr(ops, "LATENT_PROMPT_ROOM", 0)
+        assert run([0, 150]) == []
+    with monkeypatch.context() as m:
+        m.setattr(ops, "latent_prompt_room", lambda *sizes: None)
+        assert run([0, 150]) == []
+    engine = Engine(model, max_tokens=256, max_slots=2)
+    slots, expanded[:] = [engine.new_sequence(), engine.new_sequence()], []
+    got = engine.step(slots, [ids[:70], ids[:33]], "all")
+    judge(got[:70], want[:70], "bfloat16")
+    judge(got[70:], want[:33], "bfloat16")
+    assert expanded == [103, 103]
 
 
 @pytest.mark.parametrize("name", ["A", "C"])
