@@ -2,7 +2,9 @@
 //
 // A float32 number is the sum of three bfloat16 numbers, each the rounded rest of the one before: 24 bits are 8 + 8 + 8, so the sum
 // is exact.  Of the nine products of two such sums the six largest are multiplied, each exactly, on the matrix unit; what
-// the other three would add is less than 2^-26 of a product, and 2^-29 in the mean, below the rounding of the product itself (2^-24).  Six bfloat16
+// the other three would add is less than 2^-24 of a product, which is what its rounding to float32 may take (2^-28 in the mean, of either sign).
+// Numbers that all have the largest second and third parts, and those of one sign, lose it every time: rows and weights of 1 to 2 with such parts
+// lie 3.5e-8 to 5.2e-8 from 64 bits, where float32 instructions have 2.6e-8 to 4.1e-8 (of either sign 4.9e-8 and 7.9e-8).  Six bfloat16
 // products take 96 clocks for 16 x 16 results and 32 k-values where float32 ones take 256, and vector instructions run beside them.
 //
 // Sums of 32 products each in float32, small terms first, added up in float64.  The matrix unit's sums round down, not to nearest, which

@@ -603,7 +603,9 @@ def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     x = wide[:, :K]
     out = ops.linear(dev(wide)[:, :K], dev(w), dev(b)).cpu().double()
     want = x.double() @ w.double().t() + b.double()
-    # a float32 sum of 16 products is off by at most 16 roundings of the sum of their sizes; the float64 sum's one rounding at the end
+    # what a float32 sum of 16 products is off by at most (16 roundings of the sum of their sizes), and the float64 sum's one rounding at the
+    # end.  The bfloat16 products are held to the same: the three that are left out are one rounding of a product (2^-24), the others are
+    # exact, and a run of 32 is rounded in six instructions, five of them on sums of 2^-8 of its size
     bound = 2.0 ** -24 * (16.5 * (x.abs().double() @ w.abs().double().t()) + want.abs()) + 1e-30
     assert float(((out - want).abs() / bound).max()) <= 1.0
 
@@ -648,6 +650,23 @@ def test_gemm_f32_of_numbers_that_are_not_finite_or_nearly(ops, M, N, K):
     bound = 2.0 ** -24 * (16.5 * exact.abs().new_tensor(2.0 ** -120) * (x.abs().double() @ w.abs().double().t()) + exact.abs())
     bound += 2.0 ** -148
     assert float(((small - exact).abs() / bound).max()) <= 1.0
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 300, 132), (301, 4096, 4096), (301, 8200, 256)])
+@pytest.mark.parametrize("signs", [False, True])
+def test_gemm_f32_of_the_largest_products_left_out(ops, M, N, K, signs):
+    """Numbers whose second and third parts are as large as they get, 2^-8 and -2^-17 beside a first part of 1 to 2: the products of the two,
+    which are not formed, are then 2^-24 each pair of factors, all of one sign where the factors are, and add up."""
+    torch.manual_seed(69)
+    rest = 2.0 ** -8 - 2.0 ** -17
+    x, w = (1.0 + torch.randint(0, 128, shape).float() / 128 + rest for shape in ((M, K), (N, K)))
+    if signs:
+        x, w = x * (torch.randint(0, 2, x.shape) * 2 - 1), w * (torch.randint(0, 2, w.shape) * 2 - 1)
+    got, exact, size = ops.linear(dev(x), dev(w), None).cpu().double(), x.double() @ w.double().t(), x.abs().double() @ w.abs().double().t()
+    # what is left out is 2^-24 of a pair of ones at most; the runs' own roundings as in the tile shapes' test
+    assert float(((got - exact).abs() / (2.0 ** -24 * (K + 15.5 * size + exact.abs()))).max()) <= 1.0
+    # and the result as a whole no further off than half of float32's last bit, one rounding of every product
+    assert float((got - exact).norm() / exact.norm()) < 2.0 ** -24 * (1.5 if signs else 1.0)
 
 
 @pytest.mark.parametrize("M,N", [(8, 512), (130, 1024), (301, 4096)])
