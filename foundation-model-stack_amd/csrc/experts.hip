@@ -409,10 +409,12 @@ __device__ __forceinline__ bool expert_place(const ExpertArgs& a, int max_tiles,
 }
 
 // Are the weight rows of this tile loaded as bytes that are not read again?  Where a tile of 32 rows is the only one of its expert,
-// nobody else reads them; the other tiles of a popular expert do.  And with fewer blocks than compute units such loads take
-// longer.  Gate, up and down of 32 experts, 4 a token, width 2048, hidden 1024 (measured when all blocks walked K from its start): 32 tokens 80 us (88 without the mark), one token 28
-// (33 with it), 128 tokens of which most go to a few experts 104 (118 with every load marked, 113 with none); 64 experts, 8 a token,
-// hidden 768, 128 such tokens 134 (163, 157).
+// nobody else reads them; the other tiles of a popular expert do.  And with fewer blocks than compute units (of which each can take four) such loads
+// take longer.  Grouping, gate, up and down together, us, weights out of memory, with this rule, no load marked and every load marked: 32 experts, 4 a
+// token, width 2048, hidden 1024, 4 tokens 42, 46, 41, 32 tokens 69, 77, 68, 128 tokens 74, 84, 73, 128 tokens of which most go to a few
+// experts 101, 103, 109; 64 experts, 8 a token, hidden 768, 32 tokens 110, 121, 110, 128 such tokens 123, 135, 139, one token (192 and 256
+// blocks) 30, 27, 30; 8 experts, 2 a token, width 768, hidden 2048, 256 tokens 49, 48, 55.  Two or four times as many blocks as the line: a token
+// of the 64 experts 27, 4 to 32 tokens of the 32 up to 77.
 template <int BM>
 __device__ __forceinline__ bool expert_reads_once(const ExpertArgs& a, int max_tiles, int col_blocks, int tile, int e) {
   if (BM != TILE_SMALL_ROWS) return false;

@@ -733,15 +733,16 @@ def test_gemm_f32_of_results_that_are_not_finite_costs_little(ops, M, N):
     assert time(large, w.abs() * 1e30) < 12 * usual
 
 
-def test_gemm_f32_of_rows_far_apart(ops):
-    """Rows of x 2^23 floats apart and one float less: a tile's rows lie past 32 bits of bytes, and just within them."""
-    if torch.cuda.mem_get_info()[0] < 8e9:
-        pytest.skip("needs 8 GB of memory")
+@pytest.mark.parametrize("M,N,K", [(130, 8200, 128), (513, 16390, 128), (130, 4100, 64)])
+def test_gemm_f32_of_rows_far_apart(ops, M, N, K):
+    """Rows of x so far apart that a tile's lie just within the 32 bits of bytes that the kernels through LDS count in (64x64 and 64x128: 2^22
+    floats less four), just past them (2^22, to the registers' kernels), and on either side of 32 bits for one of 128 rows; short rows beside them."""
+    if torch.cuda.mem_get_info()[0] < 40e9:
+        pytest.skip("needs 40 GB of memory")
     torch.manual_seed(64)
-    M, N, K = 130, 4100, 64
     x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
     want = ops.linear(x, w, None)
-    for stride in ((1 << 23) + 4, (1 << 23) - 4):
+    for stride in ((1 << 22) - 4, 1 << 22, (1 << 23) + 4, (1 << 23) - 4):
         far = torch.empty(M * stride, device="cuda").as_strided((M, K), (stride, 1)).copy_(x)
         assert torch.equal(ops.linear(far, w, None), want)
         del far
