@@ -469,24 +469,38 @@ static void sgemm_lds_launch(const float* a, long lda, const float* w, const flo
   sgemm_lds_kernel<MT, NT, WN><<<8 * ceil_div(tiles, 8), 2 * WN * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
-// At most four products: a thread has a row of W and 16 rows of x, sums in float64.  Bound by the results' bytes.
+// At most SG_TINY products: a thread has a row of W and 16 rows of x, sums in float64.  Bound by the launch and the results' bytes: all of x is
+// asked for at once (a row after the other, each a round trip: 48 rows by 768 of K = 4 5.1 us, now 3.6; 2048 by 4096 12.7 and 10.7).
 #define SG_TINY 4
+template <int K>
 __global__ void __launch_bounds__(256)
     sgemm_tiny_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
-                      float* __restrict__ c, long ldc, int M, int N, int K, int n_blocks) {
-  const int n = blockIdx.x % n_blocks * 256 + threadIdx.x, m0 = blockIdx.x / n_blocks * 16;
+                      float* __restrict__ c, long ldc, int M, int N, int n_blocks) {
+  constexpr int ROWS = 16;
+  const int n = blockIdx.x % n_blocks * 256 + threadIdx.x, m0 = blockIdx.x / n_blocks * ROWS;
   if (n >= N) return;
-  float y[SG_TINY];
+  float x[ROWS][K], y[K];
 #pragma unroll
-  for (int k = 0; k < SG_TINY; ++k) y[k] = k < K ? w[(size_t)n * K + k] : 0.f;
+  for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+    for (int k = 0; k < K; ++k) x[i][k] = a[(size_t)min(m0 + i, M - 1) * lda + k];  // a row that is not there is the last one
+#pragma unroll
+  for (int k = 0; k < K; ++k) y[k] = w[(size_t)n * K + k];
   const float b = bias ? bias[n] : 0.f;
-  for (int m = m0; m < min(m0 + 16, M); ++m) {
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    if (m0 + i >= M) break;  // uniform
     double sum = 0.0;
 #pragma unroll
-    for (int k = 0; k < SG_TINY; ++k)
-      if (k < K) sum += (double)a[(size_t)m * lda + k] * (double)y[k];  // uniform
-    c[(size_t)m * ldc + n] = (float)(sum + b);
+    for (int k = 0; k < K; ++k) sum += (double)x[i][k] * (double)y[k];
+    c[(size_t)(m0 + i) * ldc + n] = (float)(sum + b);
   }
+}
+
+template <int K>
+static void sgemm_tiny_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, hipStream_t stream) {
+  const int n_blocks = ceil_div(N, 256);
+  sgemm_tiny_kernel<K><<<n_blocks * ceil_div(M, 16), 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, n_blocks);
 }
 
 // Short rows: 16 TM rows of x by 16 TN rows of W a wave, products and sums on the matrix unit in float64, four of 4 k-values at a time.
@@ -597,8 +611,12 @@ static void sgemm(const float* a, long lda, const float* w, const float* bias, f
                   hipStream_t stream) {
   if (sgemm_is_short(K)) {
     if (K <= SG_TINY) {
-      const int n_blocks = ceil_div(N, 256);
-      sgemm_tiny_kernel<<<n_blocks * ceil_div(M, 16), 256, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, n_blocks);
+      switch (K) {
+        case 1: sgemm_tiny_launch<1>(a, lda, w, bias, c, ldc, M, N, stream); break;
+        case 2: sgemm_tiny_launch<2>(a, lda, w, bias, c, ldc, M, N, stream); break;
+        case 3: sgemm_tiny_launch<3>(a, lda, w, bias, c, ldc, M, N, stream); break;
+        default: sgemm_tiny_launch<SG_TINY>(a, lda, w, bias, c, ldc, M, N, stream); break;
+      }
     } else if ((long)ceil_div(M, 16) * ceil_div(N, 16) >= SGEMM_SHORT_TILES) {
       sgemm_short_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream);
     } else {

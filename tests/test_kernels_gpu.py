@@ -592,10 +592,11 @@ def test_gemm_f32(ops, M, N, K):
 # every tile shape with rows, columns and K past its last whole tile.  Aligned: 16x16 (17 by 300), 16x48 (9 by 12250), 16x64 (48 by 4100), 32x64 (130 by
 # 3000, 64 by 8190), 64x64 (130 and 301 by 8200 of K = 260), 64x128 (513 by 16390 of K = 100).  Rows that are not 16-byte aligned (odd
 # stride, K = 261): 16x16 (17 by 300), 16x64 (48 by 4100), 32x32 (from 130 rows on).  K up to 96, odd K up to 256: sums in float64, waves
-# of 16x16 (8 by 4096, 130 by 4100) and 32x32 (from 301 by 8200 on)
+# of 16x16 (8 by 4096, 130 by 4100) and 32x32 (from 301 by 8200 on); K up to 4: a row of W a thread
 @pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7),
                                    (17, 300, 261), (48, 4100, 261), (130, 4100, 261), (130, 8200, 260), (301, 8200, 260), (513, 16390, 100),
-                                   (301, 8200, 96), (301, 8200, 255), (17, 300, 255), (9, 12250, 260), (13, 12250, 261)])
+                                   (301, 8200, 96), (301, 8200, 255), (17, 300, 255), (9, 12250, 260), (13, 12250, 261),
+                                   (1, 300, 1), (17, 256, 2), (33, 255, 3), (16, 257, 4), (130, 1, 4)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     torch.manual_seed(61)
