@@ -106,14 +106,17 @@ __device__ __forceinline__ f64x4 sgemm_tile_f64(const float* a, long lda, const 
   return sum;
 }
 
-// Few rows, and rows that are not 16-byte aligned or very far apart.  A block's tile is 16 TM rows of x by 16 TN rows of W; its eight
-// waves share K, wave i has the runs i, i + 8, ...  A lane asks for its eight k-values of each row itself, a run ahead, and splits
-// them.  The waves hand their short sums over through LDS, and a thread adds up the even or the odd runs of an element.
-template <int TM, int TN>
-__global__ void __launch_bounds__(8 * WAVE)
+// Few rows, and rows that are not 16-byte aligned or very far apart.  A block's tile is 16 TM rows of x by 16 TN rows of W; its
+// waves share K, wave i has the runs i, i + WAVES, ...  A lane asks for its eight k-values of each row itself, a run ahead, and splits
+// them.  The waves hand their short sums over through LDS, and a thread adds up the even or the odd runs of an element.  Eight waves where K is
+// long; with four of them few runs leave no wave idle and a compute unit has room for twice the blocks: one row by 32000 of K = 128 9.6 us
+// and 6.5, of K = 320 18.3 and 12.6; 2048 rows by 4096 of K = 321 123 and 101.
+template <int TM, int TN, int WAVES>
+__global__ void __launch_bounds__(WAVES * WAVE)
     sgemm_few_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
                      float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
-  constexpr int WAVES = 8, THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
+  static_assert(WAVES % 4 == 0, "a wave's runs have one sign");
+  constexpr int THREADS = WAVES * WAVE, TILES = TM * TN, ELEMENTS = TILES * 256;
   // A thread adds up the even and the odd runs of its elements threadIdx.x, + THREADS, ...; with one tile the even or the odd ones.
   constexpr bool BOTH = ELEMENTS >= THREADS;
   constexpr int RESULTS = (ELEMENTS + THREADS - 1) / THREADS;
@@ -249,11 +252,11 @@ __global__ void __launch_bounds__(8 * WAVE)
   }
 }
 
-template <int TM, int TN>
+template <int TM, int TN, int WAVES>
 static void sgemm_few_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
                              hipStream_t stream) {
   const int m_tiles = ceil_div(M, 16 * TM), tiles = m_tiles * ceil_div(N, 16 * TN);
-  sgemm_few_kernel<TM, TN><<<8 * ceil_div(tiles, 8), 8 * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
+  sgemm_few_kernel<TM, TN, WAVES><<<8 * ceil_div(tiles, 8), WAVES * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
 // Many 16-byte aligned rows: 16 MT rows of x by 16 NT WN rows of W a block, two waves for each 16 NT of them: one has the even runs, the
@@ -574,32 +577,37 @@ static void sgemm_short_launch(const float* a, long lda, const float* w, const f
   sgemm_short_kernel<TM, TN><<<ceil_div(tiles, 4), 4 * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
-// Which rows are short goes with K alone, so that a row's bits go with nothing else.  Beside the kernels of three parts, which take a whole run
-// of 32 and the ends of a block however short the rows are, 2048 by 4096: K = 16 13 us and 28, 32 19 and 29, 64 27 and 29, 96 37 and 38, 128 47 and 36; rows that
-// cannot all be aligned, K = 17 19 and 60, 129 50 and 70, 255 89 and 96, 321 110 and 106.
-static bool sgemm_is_short(int K) { return K <= (K % 4 == 0 ? 96 : 256); }
+// Which rows are short goes with K alone, so that a row's bits go with nothing else.  Against the best block of three parts, us: 2048 by 4096 of K = 80
+// 34 and 38, 48 by 11008 6.2 and 6.8; with K = 96 three parts take 10 to 15% less.  Rows that cannot all be aligned: 2048 by 4096 of K = 97 46 and 55, 129 55
+// and 68, 193 73 and 73, 48 by 11008 8.6, 9.9, 12.5 and 7.5, 9.5, 10.2.
+static bool sgemm_is_short(int K) { return K <= (K % 4 == 0 ? 80 : 128); }
 
-// The tile shape.  What a compute unit needs for its blocks was measured at K = 4096 (1 to 301 rows of x, 4096 to 32000 of W): the first
-// block costs `first` microseconds, every further one `next`, whatever the rows.  Small tiles fill the chip where there are few rows, and their
-// waves share K; large ones split each number less often (301 rows by 12288 of W: 793 us of 16 x 16, 436 of 32 x 32, 285 of 32 x 64, 268 of 64 x 64, 209 of
-// 64 x 128; 16 rows by 4096: 21, 32, 53, 67, 97).  Those through LDS want 16-byte aligned rows.
+// The block: its results, the k-values of its steps and what it costs, in microseconds: the first round of blocks over the compute units and each
+// of its steps, every further round and each of its steps, fitted to 3100 products (1 to 2048 rows of x by 64 to 32000 of W, K from 84 to 8192); the
+// block that is chosen by them takes 1% longer than the fastest in the mean, the slowest hundredth 15%.  Small tiles fill the chip where there are few rows,
+// and their waves share K; large ones split each number less often (301 rows by 12288 of W of K = 4096: 793 us of 16 x 16, 436 of 32 x 32, 285 of 32 x 64, 268 of
+// 64 x 64, 209 of 64 x 128; 16 rows by 4096: 21, 32, 53, 67, 97).  Those through LDS (the last three) want 16-byte aligned rows.
 struct SgemmShape {
-  int bm, bn;
-  float first, next;
+  int bm, bn, step;
+  float first, first_step, next, next_step;
 };
-#define SGEMM_FEW 5     // shapes that take any rows
-#define SGEMM_SHAPES_N 8
-static const SgemmShape SGEMM_SHAPES[SGEMM_SHAPES_N] = {{16, 16, 21.f, 14.5f}, {16, 32, 27.5f, 21.5f}, {16, 48, 38.f, 34.f},  {16, 64, 41.5f, 40.f},
-                                                        {32, 32, 34.5f, 28.5f}, {32, 64, 54.f, 33.f},  {64, 64, 68.f, 67.f}, {64, 128, 102.f, 106.f}};
+#define SGEMM_FEW 8  // shapes that take any rows
+#define SGEMM_SHAPES_N 11
+static const SgemmShape SGEMM_SHAPES[SGEMM_SHAPES_N] = {
+    {16, 16, 256, 3.28f, 0.93f, 0.17f, 0.77f}, {16, 32, 256, 3.29f, 1.52f, 0.24f, 1.42f}, {16, 48, 256, 3.27f, 2.33f, 1.58f, 2.02f},
+    {16, 64, 256, 3.64f, 2.60f, 1.50f, 2.68f}, {32, 32, 256, 3.60f, 2.01f, 0.52f, 1.80f}, {16, 16, 128, 3.17f, 0.60f, 0.14f, 0.37f},
+    {16, 32, 128, 3.37f, 0.99f, 0.21f, 0.60f}, {32, 32, 128, 3.73f, 1.27f, 0.54f, 0.83f}, {32, 64, 64, 5.00f, 0.82f, 1.70f, 0.54f},
+    {64, 64, 64, 5.47f, 1.18f, 3.54f, 1.11f},  {64, 128, 64, 8.32f, 1.68f, 5.57f, 1.59f}};
 #define SGEMM_COMPUTE_UNITS 256
 
-static int sgemm_shape(int shapes, int M, int N) {
+static int sgemm_shape(int shapes, int M, int N, int K) {
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < shapes; ++i) {
     const SgemmShape& s = SGEMM_SHAPES[i];
     const long rounds = ceil_div((long)ceil_div(M, s.bm) * ceil_div(N, s.bn), SGEMM_COMPUTE_UNITS);
-    const float cost = s.first + s.next * (float)(rounds - 1);
+    const float steps = (float)ceil_div(K, s.step);
+    const float cost = s.first + s.first_step * steps + (float)(rounds - 1) * (s.next + s.next_step * steps);
     if (i == 0 || cost < least) best = i, least = cost;
   }
   return best;
@@ -625,14 +633,17 @@ static void sgemm(const float* a, long lda, const float* w, const float* bias, f
     return;
   }
   const bool any = aligned && lda < SGEMM_NEAR && K < SGEMM_NEAR;
-  switch (sgemm_shape(any ? SGEMM_SHAPES_N : SGEMM_FEW, M, N)) {
-    case 0: sgemm_few_launch<1, 1>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 1: sgemm_few_launch<1, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 2: sgemm_few_launch<1, 3>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 3: sgemm_few_launch<1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 4: sgemm_few_launch<2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 5: sgemm_lds_launch<2, 2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
-    case 6: sgemm_lds_launch<4, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+  switch (sgemm_shape(any ? SGEMM_SHAPES_N : SGEMM_FEW, M, N, K)) {
+    case 0: sgemm_few_launch<1, 1, 8>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 1: sgemm_few_launch<1, 2, 8>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 2: sgemm_few_launch<1, 3, 8>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 3: sgemm_few_launch<1, 4, 8>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 4: sgemm_few_launch<2, 2, 8>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 5: sgemm_few_launch<1, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 6: sgemm_few_launch<1, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 7: sgemm_few_launch<2, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 8: sgemm_lds_launch<2, 2, 2>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
+    case 9: sgemm_lds_launch<4, 1, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
     default: sgemm_lds_launch<4, 2, 4>(a, lda, w, bias, c, ldc, M, N, K, stream); break;
   }
 }

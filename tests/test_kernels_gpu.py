@@ -589,14 +589,20 @@ def test_gemm_f32(ops, M, N, K):
     torch.testing.assert_close(out, (x.double() @ w.double().t() + b.double()).float(), atol=1e-4, rtol=1e-5)
 
 
-# every tile shape with rows, columns and K past its last whole tile.  Aligned: 16x16 (17 by 300), 16x48 (9 by 12250), 16x64 (48 by 4100), 32x64 (130 by
-# 3000, 64 by 8190), 64x64 (130 and 301 by 8200 of K = 260), 64x128 (513 by 16390 of K = 100).  Rows that are not 16-byte aligned (odd
-# stride, K = 261): 16x16 (17 by 300), 16x64 (48 by 4100), 32x32 (from 130 rows on).  K up to 96, odd K up to 256: sums in float64, waves
-# of 16x16 (8 by 4096, 130 by 4100) and 32x32 (from 301 by 8200 on); K up to 4: a row of W a thread
+# every tile shape with rows, columns and K past its last whole tile, in blocks of eight waves: 16x16 (9 by 300 of K = 2052, 17 by 300 of 516), 16x32 (9 by
+# 4100 of 516), 16x48 (9 by 8200 of 516, 513 by 300 of 132), 16x64 (33 by 4100 of 132, 48 of 1028), 32x32 (17 by 8190 of 132, 513 by 300 of
+# 516), the same with K one more (not 16-byte aligned); of four: 16x16 (1 by 300 of 261, 61 of 260), 16x32 (33 by 8200 of 129, 48 by 4100 of 260 and 261), 32x32
+# (17 by 8190 of 84 and 261, 130 by 8200 of 261); through LDS: 32x64 (130 by 3000 of 132, 17 by 8200 of 132), 64x64 (301 by 8200 of 260, 33 of 1028), 64x128
+# (513 by 16390 of 100, 130 by 8200 of 260).  Rows at an odd stride: those of eight and four waves.  K up to 80, odd K up to 128: sums in
+# float64, waves of 16x16 (8 by 4096, 130 by 4100) and 32x32 (from 301 by 8200 on); K up to 4: a row of W a thread
 @pytest.mark.parametrize("M,N,K", [(1, 17, 130), (8, 4096, 33), (17, 300, 516), (48, 4100, 260), (130, 3000, 132), (130, 4100, 65), (130, 4100, 68), (64, 8190, 100), (301, 8200, 36), (513, 16390, 20), (513, 16390, 7),
                                    (17, 300, 261), (48, 4100, 261), (130, 4100, 261), (130, 8200, 260), (301, 8200, 260), (513, 16390, 100),
                                    (301, 8200, 96), (301, 8200, 255), (17, 300, 255), (9, 12250, 260), (13, 12250, 261),
-                                   (1, 300, 1), (17, 256, 2), (33, 255, 3), (16, 257, 4), (130, 1, 4)])
+                                   (1, 300, 1), (17, 256, 2), (33, 255, 3), (16, 257, 4), (130, 1, 4),
+                                   (9, 300, 2052), (9, 300, 2053), (9, 4100, 516), (9, 4100, 517), (9, 8200, 516), (513, 300, 132), (513, 300, 133),
+                                   (33, 4100, 132), (33, 4100, 133), (48, 4100, 1028), (48, 4100, 1029), (17, 8190, 132), (17, 8190, 133), (513, 300, 516),
+                                   (1, 300, 261), (61, 300, 260), (33, 8200, 129), (17, 8190, 84), (17, 8190, 261), (17, 8200, 132), (33, 8200, 1028),
+                                   (130, 8200, 80), (301, 8200, 127), (17, 300, 81)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     torch.manual_seed(61)
@@ -611,11 +617,11 @@ def test_gemm_f32_tile_shapes(ops, M, N, K, pad):
     assert float(((out - want).abs() / bound).max()) <= 1.0
 
 
-@pytest.mark.parametrize("K", [3, 7, 36, 96, 100, 255, 257, 1000, 1028])
+@pytest.mark.parametrize("K", [3, 7, 36, 80, 96, 100, 127, 129, 255, 257, 1000, 1028, 2049])
 def test_gemm_f32_rows_keep_their_bits(ops, K):
-    """A row has the same bits whatever else is in the product: tiles of 16x64 (1 and 8 rows), 32x64 (17 and 130), 64x64 (33 and 61),
-    64x128 (301) and 16x16 (301 by 100), rows that are not 16-byte aligned (an odd stride, an odd K) in tiles of 16x64 (1 and 8),
-    16x32 (33) and 32x32; short rows (K up to 96, odd ones up to 256) in waves of 16x16 (up to 33 rows) and 32x32."""
+    """A row has the same bits whatever else is in the product: blocks of 16x16 to 32x32 results whose four and eight waves share K, of 32x64, 64x64 and
+    64x128 through LDS, and for rows that are not 16-byte aligned (an odd stride, an odd K) the former alone; short rows (K up to 80, odd ones up to
+    128) in waves of 16x16 (up to 33 rows) and 32x32."""
     torch.manual_seed(62)
     N = 12790
     x, w, b = dev(torch.randn(301, K)), dev(torch.randn(N, K)), dev(torch.randn(N))
@@ -626,7 +632,8 @@ def test_gemm_f32_rows_keep_their_bits(ops, K):
         assert torch.equal(ops.linear(odd[:M], w, b), whole[:M]), M
     assert torch.equal(ops.linear(odd, w, b), whole)
     assert torch.equal(ops.linear(x, w[:100], b[:100]), whole[:, :100])
-    assert torch.equal(ops.linear(x[:9], w[:12200], b[:12200]), whole[:9, :12200])  # 16x48
+    for N in (4096, 8200, 12200):  # 16x32, 16x48 of eight waves
+        assert torch.equal(ops.linear(x[:9], w[:N], b[:N]), whole[:9, :N]), N
 
 
 @pytest.mark.parametrize("M,N,K", [(8, 300, 64), (40, 4096, 132), (301, 4096, 256), (301, 4096, 131), (40, 300, 13)])
@@ -734,9 +741,9 @@ def test_gemm_f32_of_results_that_are_not_finite_costs_little(ops, M, N):
     assert time(large, w.abs() * 1e30) < 12 * usual
 
 
-@pytest.mark.parametrize("M,N,K", [(130, 8200, 128), (513, 16390, 128), (130, 4100, 64)])
+@pytest.mark.parametrize("M,N,K", [(130, 3000, 132), (301, 8200, 260), (513, 16390, 128), (130, 4100, 64)])
 def test_gemm_f32_of_rows_far_apart(ops, M, N, K):
-    """Rows of x so far apart that a tile's lie just within the 32 bits of bytes that the kernels through LDS count in (64x64 and 64x128: 2^22
+    """Rows of x so far apart that a tile's lie just within the 32 bits of bytes that the kernels through LDS count in (32x64, 64x64, 64x128: 2^22
     floats less four), just past them (2^22, to the registers' kernels), and on either side of 32 bits for one of 128 rows; short rows beside them."""
     if torch.cuda.mem_get_info()[0] < 40e9:
         pytest.skip("needs 40 GB of memory")
