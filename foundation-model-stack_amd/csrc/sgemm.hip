@@ -515,7 +515,7 @@ __global__ void __launch_bounds__(256)
     sgemm_short_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
                        float* __restrict__ c, long ldc, int M, int N, int K, int m_tiles, int tiles) {
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int tile = blockIdx.x * 4 + wave;
+  const int tile = blockIdx.x * (blockDim.x / WAVE) + wave;
   if (tile >= tiles) return;
   const int m0 = tile % m_tiles * 16 * TM, n0 = tile / m_tiles * 16 * TN;
   const int r = lane % 16, o = lane / 16;
@@ -570,11 +570,15 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Up to so many tiles a block is one wave, which spreads them over the compute units: 16 rows by 4096 of K = 64 (256 tiles) 4.2 us as blocks of four
+// waves, 3.9; by 12288 (768) 4.5 either way.
+#define SGEMM_SHORT_ALONE 512
 template <int TM, int TN>
 static void sgemm_short_launch(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K,
                                hipStream_t stream) {
   const int m_tiles = ceil_div(M, 16 * TM), tiles = m_tiles * ceil_div(N, 16 * TN);
-  sgemm_short_kernel<TM, TN><<<ceil_div(tiles, 4), 4 * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
+  const int waves = tiles <= SGEMM_SHORT_ALONE ? 1 : 4;  // of a block
+  sgemm_short_kernel<TM, TN><<<ceil_div(tiles, waves), waves * WAVE, 0, stream>>>(a, lda, w, bias, c, ldc, M, N, K, m_tiles, tiles);
 }
 
 // Which rows are short goes with K alone, so that a row's bits go with nothing else.  Against the best block of three parts, us: 2048 by 4096 of K = 80
@@ -613,7 +617,9 @@ static int sgemm_shape(int shapes, int M, int N, int K) {
   return best;
 }
 
-#define SGEMM_SHORT_TILES 16384  // from here on waves of 32 x 32 results fill the chip
+// From so many tiles of 16 x 16 results on waves of 32 x 32 fill the chip: 96 by 32000 of K = 64 (12000 tiles) 17.3
+// us as waves of 16 x 16, 13.9 of 32 x 32; 512 by 4096 (8192) 11.9 and 10.6, of K = 24 9.1 and 9.0; 96 by 11008 (4128) 8.7 and 9.8.
+#define SGEMM_SHORT_TILES 8192
 #define SGEMM_NEAR (1 << 22)  // 128 rows of so many floats lie within 32 bits of bytes
 static void sgemm(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M, int N, int K, bool aligned,
                   hipStream_t stream) {
