@@ -423,11 +423,12 @@ __device__ __forceinline__ bool expert_reads_once(const ExpertArgs& a, int max_t
   return alone && a.tiles[3 * max_tiles - 2] * col_blocks >= EXPERT_COMPUTE_UNITS;
 }
 
-// The step of K that a block starts with: weight rows lie a multiple of kilobytes apart, and blocks that walk them in step crowd into few
-// memory channels (32 tokens of the above: gate and up 42 us instead of 60).  It goes with the expert and the columns alone (in the width of the large tiles' blocks), so
-// that a pair has the same bits in any tile.
-#define TILE_BIG_COLS 256
-__device__ __forceinline__ int expert_first_step(int e, int cols, int K) { return (5 * cols + 3 * e) % ((K + TL_BK - 1) / TL_BK); }
+// The step of K that a block starts with: weight rows lie a multiple of kilobytes apart, and the blocks of all experts in step crowd into few
+// memory channels.  It goes with the expert alone: the blocks of a tile share its rows, and those of an expert its weights, while they are in
+// an L2.  Grouping, gate, up and down together, us, all blocks at the start of K, this, and another start for every column: 32 experts, 4 a token, width
+// 2048, hidden 1024, 32 tokens 85, 75, 76, 2048 tokens 205, 199, 203; 4 experts, 2 a token, width 4096, hidden 3584, 1024 tokens 275, 273, 309, 4096 tokens
+// 895, 895, 1065.  And a pair has the same bits in any tile.
+__device__ __forceinline__ int expert_first_step(int e, int K) { return 3 * e % ((K + TL_BK - 1) / TL_BK); }
 
 template <int WM, int WN, int TM, int TN, int ST, bool GATED>
 __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_eu(2))) expert_gate_up_lds_kernel(ExpertArgs a, int max_tiles, int col_blocks) {
@@ -456,7 +457,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
     const int c = n0 + (GATED ? ((t / TN) * (TN / 2) + t % (TN / 2)) * 32 + n % 32 : n);
     return (up ? wu : wg) + (size_t)(c < a.N ? c : 0) * a.K;
   };
-  const int first = expert_first_step(e, n0 / (TILE_BIG_COLS / (GATED ? 2 : 1)), a.K);
+  const int first = expert_first_step(e, a.K);
   if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
     tile_product_lds<WM, WN, TM, TN, ST, true, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
   else
@@ -505,7 +506,7 @@ __global__ void __launch_bounds__(WM* WN* WAVE) __attribute__((amdgpu_waves_per_
   const bool works = (int)(threadIdx.x / WAVE) / WN * TM * 32 < rows;
   auto a_row = [&](int m) { return x + (size_t)(start + (m < rows ? m : 0)) * a.ldx; };
   auto w_row = [&](int n) { return w + (size_t)(n0 + n < a.N ? n0 + n : 0) * a.K; };
-  const int first = expert_first_step(e, n0 / TILE_BIG_COLS, a.K);
+  const int first = expert_first_step(e, a.K);
   if (expert_reads_once<S::BM>(a, max_tiles, col_blocks, tile, e))
     tile_product_lds<WM, WN, TM, TN, ST, true, (TM * WM > 1)>(a_row, w_row, a.K, lds, acc, works, first);
   else
