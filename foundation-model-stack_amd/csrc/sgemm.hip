@@ -659,9 +659,9 @@ static void sgemm(const float* a, long lda, const float* w, const float* bias, f
 
 // Many rows: bound by the vector instructions of the split and of the sums in 64 bits, which overlap with the products only in part: a step of
 // 64 x 128 results and 64 k-values takes 1.5 us, of which the products alone are 0.64 (1.8 PFLOP/s in bfloat16), the sums about 0.5, the splits 0.4.
-// Few rows: the weights' bytes.  Against float32 products, K 4096 (us): 301 rows by 22016 rows of W 604 -> 408, by 4096 131 -> 103;
-// 128 rows by 12288 148 -> 103; 48 by 32000 193 -> 116; 24 by 4096 31 -> 29; 8 by 4096 23 -> 20, by 12288 37 -> 39 and by 32000 92 -> 95
-// (x's rows are split by every block); 8 by 4096 of K = 11008 52 -> 42; rows that are not aligned, 301 by 4096 of K = 4095: 302 -> 160.
+// Few rows: the weights' bytes.  Against float32 products, K 4096, weights out of memory (us): 301 rows by 22016 rows of W 604 -> 420, by 4096 131 -> 106;
+// 130 rows by 12288 190 -> 160; 48 by 32000 196 -> 137; 17 by 4096 30 -> 27; 8 by 4096 27 -> 20, by 11008 39 -> 40, by 12288 39 -> 43 and by 32000
+// 92 -> 99 (x's rows are split by every block); 8 by 4096 of K = 11008 73 -> 52; rows that are not aligned, 301 by 4096 of K = 4095: 302 -> 160.
 extern "C" int fmsamd_gemm_f32(const float* a, long lda, const float* w, const float* bias, float* c, long ldc, int M,
                                int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;
