@@ -150,6 +150,14 @@ int fmsamd_gemm_skinny_gated_bf16(const void* x, long ldx, const void* w, const 
                                   int out_dtype, long ldo, int M, int hidden, int K, int act,
                                   const fmsamd_gate_clamp* clamp, const fmsamd_row_scale* row_scale, void* workspace, long workspace_bytes,
                                   hipStream_t stream);
+// The same two products for more rows than that, in tiles of up to 256 x 256: N and ldo multiples of 8, K a multiple of 128 and at
+// least 256, 16-byte addresses.  pays: 1 where they are expected to be faster than the vendor library's.
+int fmsamd_gemm_tall_pays(int M, int N, int K, int gated);
+int fmsamd_gemm_tall_plan(int M, int N, int K, int gated);  // which tiles it takes, 0 to 4
+int fmsamd_gemm_tall_bf16(const void* x, long ldx, const void* w, const void* bias, int bias_dtype, void* out, int out_dtype, long ldo, int M,
+                          int N, int K, hipStream_t stream);
+int fmsamd_gemm_tall_gated_bf16(const void* x, long ldx, const void* w, const void* bias, int bias_dtype, void* out, long ldo, int M, int hidden,
+                                int K, int act, const fmsamd_gate_clamp* clamp, hipStream_t stream);
 // resid += x W^T (+ bias) in float32; scaled = resid * norm_w in bfloat16; partials[M, partial_count] = sums
 // of squares of resid by groups of columns (partial_count as fmsamd_gemm_skinny_residual_partials(M, N, K) says;
 // every entry is written).  At most 192 rows.

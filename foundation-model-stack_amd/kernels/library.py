@@ -45,6 +45,10 @@ _SIGNATURES = {
     "fmsamd_gemm_skinny_workspace": [I, I, I],
     "fmsamd_gemm_skinny_bf16": [P, L, P, P, I, P, I, L, I, I, I, I, P, P, L, P],
     "fmsamd_gemm_skinny_gated_bf16": [P, L, P, P, I, P, I, L, I, I, I, I, P, P, P, L, P],
+    "fmsamd_gemm_tall_pays": [I, I, I, I],
+    "fmsamd_gemm_tall_plan": [I, I, I, I],
+    "fmsamd_gemm_tall_bf16": [P, L, P, P, I, P, I, L, I, I, I, P],
+    "fmsamd_gemm_tall_gated_bf16": [P, L, P, P, I, P, L, I, I, I, I, P, P],
     "fmsamd_gemm_skinny_residual_partials": [I, I, I],
     "fmsamd_gemm_skinny_residual_bf16": [P, L, P, P, I, P, L, P, I, P, L, P, I, I, I, I, P, P, L, P],
     "fmsamd_sample": [P, L, I, I, I, F, I, P, P, P],

@@ -594,6 +594,12 @@ _PLAIN_ACTIVATIONS = ("identity", "relu", "relu2")  # what the skinny kernels fi
 SKINNY_FAST_ROWS = 192
 
 
+def _tall_fits(x: torch.Tensor, weight: torch.Tensor, cols: int, gated: bool) -> bool:
+    """True if the kernel for many rows takes this bfloat16 product and is expected to be faster than the vendor library's."""
+    return (x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and max(x.stride(0), 4 * cols) < 1 << 22 and load().fmsamd_gemm_tall_pays(x.shape[0], cols, x.shape[1], int(gated)) == 1)
+
+
 def linear(
     x: torch.Tensor,
     weight: torch.Tensor,
@@ -607,9 +613,9 @@ def linear(
     other activation and kernel is followed by the activation kernel.
 
     float32 x float32: the float32 matrix-core kernel (true 32-bit).  bfloat16 x bfloat16: the weight-streaming
-    skinny kernels up to 192 rows; above that the vendor library (hipBLASLt through torch.matmul,
-    as the reference's nn.Linear does; for float32 output with the float32 sums as they are), or this
-    package's MFMA kernel when allow_library is False.
+    skinny kernels up to 192 rows; above that the kernel for many rows, and where few tiles share a long K, or widths or
+    addresses do not fit it, the vendor library (hipBLASLt through torch.matmul, as the reference's nn.Linear does; for
+    float32 output with the float32 sums as they are); this package's first MFMA kernel when allow_library is False.
     A float32 weight with bfloat16 activations (a tensor the checkpoint keeps in 32-bit) runs the
     float32 kernel on up-cast activations.
     """
@@ -660,6 +666,11 @@ def linear(
         check(lib.fmsamd_gemm_skinny_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias), bcode, out.data_ptr(),
                                           _code(out_dtype), out.stride(0), M, N, K, ACTIVATIONS[activation], _row_scale(row_norm, M), _ptr(ws),
                                           ws_bytes, _stream()))
+        return out
+    if allow_library and _tall_fits(x, weight, N, False):
+        out = torch.empty(M, N, dtype=out_dtype, device=x.device)
+        check(lib.fmsamd_gemm_tall_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias), bcode, out.data_ptr(), _code(out_dtype),
+                                        out.stride(0), M, N, K, _stream()))
         return out
     if allow_library and out_dtype in (torch.bfloat16, torch.float32):
         # vendor library GEMM, float32 accumulation; float32 results (the logits of many rows) come straight from the
@@ -748,6 +759,16 @@ def gated_linear(
         return out
     if row_norm is not None:
         raise ValueError(f"a deferred row norm goes with the bfloat16 product of at most {SKINNY_FAST_ROWS} rows")
+    if (allow_library and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2
+            and weight.shape[1] == x.shape[1] and weight.is_contiguous()
+            and (bias is None or (bias.shape == (2 * hidden,) and bias.is_contiguous())) and _tall_fits(x, weight, hidden, True)):
+        _need_cuda(x, weight, bias)
+        rows = _rows_out(out, M, hidden, torch.bfloat16, x.device)
+        if rows.stride(0) % 8 == 0 and rows.stride(0) < 1 << 21 and rows.data_ptr() % 16 == 0:
+            check(load().fmsamd_gemm_tall_gated_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias),
+                                                     _code(bias.dtype) if bias is not None else 0, rows.data_ptr(), rows.stride(0), M, hidden,
+                                                     x.shape[1], ACTIVATIONS[activation], _clamp(clamp), _stream()))
+            return rows
     gu = linear(x, weight, None, allow_library=allow_library)
     return gated_act(gu, bias, activation, clamp, out)
 
