@@ -26,53 +26,154 @@
 #define ROUTE_MAX_EXPERTS 1024
 #define ROUTE_MAX_TOP 64
 
-// One wave per token.
-__global__ void __launch_bounds__(256)
-    route_kernel(const float* __restrict__ logits, long ld, int n_tokens, int n_experts, int top, int score, int* __restrict__ ids,
-                 float* __restrict__ weights) {
-  extern __shared__ float lds[];  // 4 waves x (n_experts + top)
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= n_tokens) return;
-  float* z = lds + (size_t)wave * (n_experts + top);
-  float* chosen = z + n_experts;
-  for (int e = lane; e < n_experts; e += WAVE) z[e] = logits[(size_t)t * ld + e];
-  __builtin_amdgcn_wave_barrier();
+// The largest of a wave's values, in all lanes: rows of 16 lanes in the vector unit, then their four results.
+__device__ __forceinline__ float route_max(float v) {
+#define ROUTE_DPP_MAX(ctrl) v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, true)))
+  ROUTE_DPP_MAX(0xB1);   // quad_perm [1, 0, 3, 2]
+  ROUTE_DPP_MAX(0x4E);   // quad_perm [2, 3, 0, 1]
+  ROUTE_DPP_MAX(0x141);  // row_half_mirror
+  ROUTE_DPP_MAX(0x140);  // row_mirror
+#undef ROUTE_DPP_MAX
+  auto of = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); };
+  return fmaxf(fmaxf(of(0), of(16)), fmaxf(of(32), of(48)));
+}
+
+// The `top` largest of the values z(e), e < n_experts <= 64 PER, and their weights, by a wave that keeps them in registers: a round is the largest
+// value, the lanes that have it and the lowest index among them (a chain of shuffles through LDS with value and index takes 0.6 us a round).
+template <int PER, typename Value>
+__device__ __forceinline__ void route_row(Value z, int lane, int n_experts, int top, int score, int* ids, float* weights) {
+  float v[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) v[i] = lane + i * WAVE < n_experts ? z(lane + i * WAVE) : 0.f;
+  float mine = 0.f;  // lane j: the j-th chosen one
+  int my_id = 0;
   for (int j = 0; j < top; ++j) {
     float best = -INFINITY;
     int at = 0x7fffffff;
-    for (int e = lane; e < n_experts; e += WAVE) {
-      const float v = z[e];
-      if (v > best || (v == best && e < at)) best = v, at = e;
-    }
-    if (at == 0x7fffffff) at = lane < n_experts ? lane : 0;  // only NaNs or -inf left in this lane's share
 #pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, WAVE);
-      const int oa = __shfl_xor(at, off, WAVE);
-      if (ov > best || (ov == best && oa < at)) best = ov, at = oa;
+    for (int i = 0; i < PER; ++i) {
+      const int e = lane + i * WAVE;
+      if (e < n_experts && (v[i] > best || (v[i] == best && e < at))) best = v[i], at = e;
     }
-    if (lane == 0) {
-      ids[(size_t)t * top + j] = at;
-      chosen[j] = best;
-      z[at] = -INFINITY;
+    if (at == 0x7fffffff) at = lane < n_experts ? lane : 0;  // only NaNs left in this lane's share
+    const float largest = route_max(best);
+    unsigned long long have = __ballot(best == largest);
+    int chosen = 0x7fffffff;
+    for (; have != 0; have &= have - 1) {  // one lane, but for ties
+      const int other = __builtin_amdgcn_readlane(at, __builtin_ctzll(have));
+      chosen = other < chosen ? other : chosen;
     }
-    __builtin_amdgcn_wave_barrier();
-    __threadfence_block();
+    if (lane == j) mine = largest, my_id = chosen;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = lane + i * WAVE == chosen ? -INFINITY : v[i];
   }
-  if (lane == 0) {
-    if (score == FMS_ROUTE_SOFTMAX) {
-      const float m = chosen[0];  // the largest comes first
+  auto of = [&](float x, int j) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), j)); };
+  const float m = of(mine, 0);  // the largest comes first
+  // softmax over the chosen ones, or sigmoid scores (the order of the logits is the order of their sigmoids); sums in the order of j
+  const float one = score == FMS_ROUTE_SOFTMAX ? expf(mine - m) : 1.f / (1.f + expf(-mine));
+  float sum = 0.f;
+  for (int j = 0; j < top; ++j) sum += of(one, j);
+  const float norm = score == FMS_ROUTE_SIGMOID_NORMED ? 1.f / sum : 1.f;
+  if (lane < top) {
+    ids[lane] = my_id;
+    weights[lane] = score == FMS_ROUTE_SOFTMAX ? one / sum : norm / (1.f + expf(-mine));
+  }
+}
+
+// One wave per token.
+template <int PER>
+__global__ void __launch_bounds__(256)
+    route_kernel(const float* __restrict__ logits, long ld, int n_tokens, int n_experts, int top, int score, int* __restrict__ ids,
+                 float* __restrict__ weights) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + wave;
+  if (t >= n_tokens) return;
+  route_row<PER>([&](int e) { return logits[(size_t)t * ld + e]; }, lane, n_experts, top, score, ids + (size_t)t * top, weights + (size_t)t * top);
+}
+
+// The smallest number of values a lane that a kernel is built for.
+#define ROUTE_PER(n_experts, CALL)     \
+  do {                                 \
+    if ((n_experts) <= WAVE) CALL(1);  \
+    else if ((n_experts) <= 4 * WAVE) CALL(4); \
+    else CALL(16);                     \
+  } while (0)
+static_assert(ROUTE_MAX_EXPERTS <= 16 * WAVE && ROUTE_MAX_TOP <= WAVE, "values a lane, and a lane for every choice");
+
+// The router's product and the choice as one kernel, for the few tokens of a decode step: a block of sixteen waves a token, a row of W a wave
+// at a time, three rows asked for at once.  Bound by a launch, the round trip for x and W together and the chain of the choice.  Width 2048, 33
+// outputs, 4 chosen, us, the two kernels and this one: 1 token 5.6 and 4.8, 8 5.6 and 5.0, 32 7.4 and 5.1, 128 10.9 and 5.3 (the
+// two with the choice's shuffles through LDS 7.9, 9.3, 10.5, 14.1).  Every token reads all of W: 128 outputs of width 1024 7.5 and 7.7 for 16
+// tokens, 8.1 and 7.7 for 32; 65 of width 4096 10 and 14.
+#define ROUTER_WAVES 16
+#define ROUTER_WIDEST 2048
+// CHUNKS: of 512 elements of a row; PER: route_row's
+template <int CHUNKS, int PER>
+__global__ void __launch_bounds__(ROUTER_WAVES* WAVE)
+    router_kernel(const bf16* __restrict__ x, long ldx, const bf16* __restrict__ w, int K, int n_out, int n_experts, int top, int score,
+                  float* __restrict__ logits, int* __restrict__ ids, float* __restrict__ weights) {
+  __shared__ float z[PER * WAVE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x & (WAVE - 1), t = blockIdx.x;
+  const bf16x8 zero = __builtin_bit_cast(bf16x8, f32x4{0.f, 0.f, 0.f, 0.f});
+  auto row = [&](const bf16* from, bf16x8 (&to)[CHUNKS]) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int k = c * 512 + lane * 8;
+      to[c] = k < K ? *reinterpret_cast<const bf16x8*>(from + k) : zero;
+    }
+  };
+  bf16x8 v[CHUNKS];
+  row(x + (size_t)t * ldx, v);
+  constexpr int AT_ONCE = 3;
+  for (int n0 = wave; n0 < n_out; n0 += ROUTER_WAVES * AT_ONCE) {
+    bf16x8 u[AT_ONCE][CHUNKS];
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) row(w + (size_t)(n0 + i * ROUTER_WAVES < n_out ? n0 + i * ROUTER_WAVES : n0) * K, u[i]);
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) {
       float sum = 0.f;
-      for (int j = 0; j < top; ++j) sum += expf(chosen[j] - m);
-      for (int j = 0; j < top; ++j) weights[(size_t)t * top + j] = expf(chosen[j] - m) / sum;
-    } else {  // sigmoid scores (the order of the logits is the order of their sigmoids)
-      float sum = 0.f;
-      for (int j = 0; j < top; ++j) sum += 1.f / (1.f + expf(-chosen[j]));
-      const float norm = score == FMS_ROUTE_SIGMOID_NORMED ? 1.f / sum : 1.f;
-      for (int j = 0; j < top; ++j) weights[(size_t)t * top + j] = norm / (1.f + expf(-chosen[j]));
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum = fmaf((float)v[c][e], (float)u[i][c][e], sum);
+      sum = row16_sum(sum);
+      sum += __shfl_xor(sum, 16, WAVE);
+      sum += __shfl_xor(sum, 32, WAVE);
+      const int n = n0 + i * ROUTER_WAVES;
+      if (lane == 0 && n < n_out) {
+        logits[(size_t)t * n_out + n] = sum;
+        if (n < n_experts) z[n] = sum;
+      }
     }
   }
+  __syncthreads();
+  if (wave == 0) route_row<PER>([&](int e) { return z[e]; }, lane, n_experts, top, score, ids + (size_t)t * top, weights + (size_t)t * top);
+}
+
+// logits [n_tokens, n_out] = x W^T in float32 (bfloat16 x and W, K a multiple of 8 up to 4096, 16-byte addresses), and the choice among
+// the first n_experts of them as fmsamd_moe_route makes it.
+extern "C" int fmsamd_moe_router(const void* x, long ldx, const void* w, int n_tokens, int K, int n_out, int n_experts, int top, int score,
+                                 float* logits, int* ids, float* weights, hipStream_t stream) {
+  if (n_tokens == 0) return 0;
+  FMS_REQUIRE(n_tokens > 0 && n_experts > 0 && n_experts <= n_out && n_out <= ROUTE_MAX_EXPERTS + 1 && top > 0 && top <= n_experts && top <= ROUTE_MAX_TOP,
+              "moe_router: %d experts of %d outputs (at most %d), top %d (at most %d and the experts)", n_experts, n_out, ROUTE_MAX_EXPERTS, top,
+              ROUTE_MAX_TOP);
+  FMS_REQUIRE(K > 0 && K % 8 == 0 && K <= ROUTER_WIDEST && ldx >= K && ldx % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0,
+              "moe_router: K=%d (a multiple of 8, at most %d), row stride %ld", K, ROUTER_WIDEST, ldx);
+  FMS_REQUIRE(score >= FMS_ROUTE_SOFTMAX && score <= FMS_ROUTE_SIGMOID_NORMED, "moe_router: unknown score %d", score);
+#define FMS_ROUTER(CHUNKS, PER)                                                                                                             \
+  router_kernel<CHUNKS, PER><<<n_tokens, ROUTER_WAVES * WAVE, 0, stream>>>((const bf16*)x, ldx, (const bf16*)w, K, n_out, n_experts, top, score, \
+                                                                           logits, ids, weights)
+#define FMS_ROUTER_OF(PER)                   \
+  do {                                       \
+    if (K <= 1024) FMS_ROUTER(2, PER);       \
+    else FMS_ROUTER(4, PER);                 \
+  } while (0)
+  ROUTE_PER(n_experts, FMS_ROUTER_OF);
+#undef FMS_ROUTER_OF
+#undef FMS_ROUTER
+  FMS_LAUNCH_CHECK("moe_router");
+  return 0;
 }
 
 extern "C" int fmsamd_moe_route(const float* logits, long ld, int n_tokens, int n_experts, int top, int score, int* ids,
@@ -82,8 +183,9 @@ extern "C" int fmsamd_moe_route(const float* logits, long ld, int n_tokens, int 
               "moe_route: %d experts (at most %d), top %d (at most %d and the experts)", n_experts, ROUTE_MAX_EXPERTS, top, ROUTE_MAX_TOP);
   FMS_REQUIRE(ld >= n_experts, "moe_route: rows of %ld for %d experts", ld, n_experts);
   FMS_REQUIRE(score >= FMS_ROUTE_SOFTMAX && score <= FMS_ROUTE_SIGMOID_NORMED, "moe_route: unknown score %d", score);
-  const size_t lds = 4 * (size_t)(n_experts + top) * sizeof(float);
-  route_kernel<<<ceil_div(n_tokens, 4), 256, lds, stream>>>(logits, ld, n_tokens, n_experts, top, score, ids, weights);
+#define FMS_ROUTE(PER) route_kernel<PER><<<ceil_div(n_tokens, 4), 256, 0, stream>>>(logits, ld, n_tokens, n_experts, top, score, ids, weights)
+  ROUTE_PER(n_experts, FMS_ROUTE);
+#undef FMS_ROUTE
   FMS_LAUNCH_CHECK("moe_route");
   return 0;
 }

@@ -288,6 +288,8 @@ int fmsamd_latent_prompt(const void* q, long ldq, void* out, long ldo, const voi
 #define FMS_ROUTE_SOFTMAX 0
 #define FMS_ROUTE_SIGMOID 1
 #define FMS_ROUTE_SIGMOID_NORMED 2
+int fmsamd_moe_router(const void* x, long ldx, const void* w, int n_tokens, int K, int n_out, int n_experts, int top, int score,
+                      float* logits, int* ids, float* weights, hipStream_t stream);  // the router's product (bfloat16) and moe_route as one
 int fmsamd_moe_route(const float* logits, long ld, int n_tokens, int n_experts, int top, int score, int* ids, float* weights,
                      hipStream_t stream);
 // Rows of a tile of (token, choice) pairs of one expert: 32, or 128 where experts have many rows, for a product that the

@@ -67,6 +67,7 @@ _SIGNATURES = {
     "fmsamd_latent_attn_generic": [P, L, P, L, I, P, P, P, I, P, P, I, I, I, I, F, I, P],
     "fmsamd_latent_prompt_fits": [I, I, I, I],
     "fmsamd_latent_prompt": [P, L, P, L, P, P, P, P, P, P, P, P, P, P, I, P, I, I, P, P, P, P, L, I, I, I, I, I, I, F, I, P],
+    "fmsamd_moe_router": [P, L, P, I, I, I, I, I, I, P, P, P, P],
     "fmsamd_moe_route": [P, L, I, I, I, I, P, P, P],
     "fmsamd_moe_group": [P, I, I, P, P, I, I, P],
     "fmsamd_moe_experts": [I, P, L, P, P, P, I, P, P, I, I, I, I, I, F, F, F, P, I, P],

@@ -116,10 +116,13 @@ class ExpertsFeedForward(FeedForward):
             self._correction = self.w["correction"].to(torch.float32).contiguous()
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        logits = self.router.forward(x, out_dtype=torch.float32)
-        if self.score == "softmax_all":
+        if self.score != "softmax_all" and ops.moe_router_fits(x, self.router.w["weight"]):
+            ids, weights, logits = ops.moe_router(x, self.router.w["weight"], self.experts, self.top, self.score)
+        elif self.score == "softmax_all":
+            logits = self.router.forward(x, out_dtype=torch.float32)
             ids, weights = ops.moe_route_grouped(logits, self.outputs, self.top, self._correction, self.groups, self.keep, self.route_scale)
         else:
+            logits = self.router.forward(x, out_dtype=torch.float32)
             ids, weights = ops.moe_route(logits, self.experts, self.top, self.score)
         on_input = self.weight_on == "input"
         if self.experts:
