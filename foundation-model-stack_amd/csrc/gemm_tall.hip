@@ -121,11 +121,17 @@ __device__ __forceinline__ void tall_tiles(const TallArgs& g, int first, int las
         });
       });
     };
-    // (a choice for the whole tile: one for every element costs more than the products of a tile)
-    if (GATED && g.act.kind != FMS_ACT_SILU)
-      write([&](float gate, float up) { return sk_gated(gate, up, g.act); });
-    else  // (the reciprocal's last bit is far below the result's)
+    // (a choice for the whole tile: one for every element costs more than the products of a tile.  The fast exponential's and the
+    // reciprocal's last bits are far below the result's.)
+    if (!GATED || g.act.kind == FMS_ACT_SILU)
       write([&](float gate, float up) { return gate * __builtin_amdgcn_rcpf(1.f + __expf(-gate)) * up; });
+    else if (g.act.kind == FMS_ACT_CLAMPED_GATE)
+      write([&](float gate, float up) {
+        const float z = fminf(gate, g.act.limit), u = fminf(fmaxf(up, -g.act.limit), g.act.limit);
+        return z * __builtin_amdgcn_rcpf(1.f + __expf(-g.act.alpha * z)) * (u + g.act.shift);
+      });
+    else
+      write([&](float gate, float up) { return sk_gated(gate, up, g.act); });
   };
   ring_product<R>((unsigned)(g.ldx * 2), (unsigned)(g.K * 2), g.K, lds, place, finish);
 }

@@ -93,6 +93,7 @@ class ExpertsFeedForward(FeedForward):
         self.groups, self.keep, self.route_scale, self.has_correction = int(groups), int(keep), float(route_scale), bool(correction)
         self.shared_hidden_dim = int(shared_hidden_dim)
         self.shared_limit = float(shared_limit if shared_limit is not None else limit)
+        self._shared_unit = ops.GateClamp(self.shared_limit, self.alpha, self.shift)
         self.has_shared_gate = bool(shared_gate) and self.shared_hidden_dim > 0
         # the router's rows, and behind them the row of the shared expert's gate: one product, float32 logits
         self.router = self.add_child("router", Linear(width, self.outputs + (1 if self.has_shared_gate else 0)))
@@ -133,7 +134,10 @@ class ExpertsFeedForward(FeedForward):
         shared = gate = None
         if self.shared_hidden_dim:
             if self.expert_gate:
-                hidden = ops.clamped_gated_act(self.shared_gate_up.forward(x), self.shared_limit, self.alpha, self.shift)
+                if self.shared_limit > 0:
+                    hidden = ops.gated_linear(x, self.shared_gate_up.w["weight"], None, "silu", clamp=self._shared_unit)
+                else:
+                    hidden = ops.clamped_gated_act(self.shared_gate_up.forward(x), self.shared_limit, self.alpha, self.shift)
             else:
                 hidden = ops.activation(self.shared_up.forward(x), self.activation)
             shared = self.shared_down.forward(hidden)
