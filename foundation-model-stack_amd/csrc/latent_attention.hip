@@ -977,6 +977,108 @@ __global__ void __launch_bounds__(256, 1)
   latent_finish<RT, WC, true>(st, out, ldo, t, head, nheads, RANK, grp);
 }
 
+// --------------------------------------------------------------------------
+// bfloat16 single tokens with a latent of 512 (RT * 16 elements in rows of WC * 32): the parts, shares and arithmetic of the kernel above, bit
+// by bit.  A wave brings its tile of 32 keys straight into its own place in LDS, as whole rows, and reads both operands there: the keys as they
+// lie, the values transposed by the read (ds_read_b64_tr_b16), so that the latent comes from memory once and the transposed copy not at all.
+// Bound by the rows' bytes (64 sequences of 2000 tokens: 147 MB in 34 us without the merge's 6) and, for few, by the chain of lookups, first loads and
+// meeting.  Us with the merge, 16 heads, latent 512 + 64, the kernel above (keys and transposed latent through registers, 64 bytes of a row at a
+// time) and this one: 32 sequences of 128 to 2048 tokens 33.0 and 26.1, 64 of them 48.2 and 33.9, 64 of 2000 59.0 and 39.9, 8 of 2000 22.2
+// and 17.0, one of 100 19.0 and 14.2.  Operands asked for in other groups: the same within 3 %, whole rows of keys and 16 tiles of the latent
+// ahead 36.1 (registers).
+// The pieces of 16 bytes of a row are XOR-swizzled with the row on the address side of the loads, so that the reads of the 16 rows of an operand
+// cover all banks: a row of 1152 bytes begins half way round them after the row before, one of 1024 where that does.
+// --------------------------------------------------------------------------
+template <int RT, int WC>
+__global__ void __launch_bounds__(256, 1)
+    latent_attn_decode_kernel(const bf16* __restrict__ qa, long ldq, bf16* __restrict__ out, long ldo, float* __restrict__ ws,
+                              const int* __restrict__ positions, const int* __restrict__ seq_of_token, const int* __restrict__ block_table,
+                              int table_stride, const bf16* __restrict__ cache, const float* __restrict__ sink, int nheads, float scale,
+                              int window, int tiles_per_token, int n_parts) {
+  constexpr int RANK = RT * 16, WIDTH = WC * 32, ROW = WIDTH * 2, TILE = 32 * ROW, LOADS = TILE / 1024;
+  static_assert(ROW == 1152 || ROW == 1024, "the swizzles");
+  extern __shared__ __attribute__((aligned(1024))) bf16 lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int t = blockIdx.x / tiles_per_token, head0 = blockIdx.x % tiles_per_token * 16, head = head0 + col, block_part = blockIdx.y;
+  const bool valid = head < nheads;
+  const int seq = uniform_load(seq_of_token + t);
+  if (seq < 0) {
+    if (n_parts == 1 && valid)
+      for (int d = grp; d < RANK; d += 4) out[(size_t)t * ldo + (size_t)head * RANK + d] = (bf16)0.f;
+    return;
+  }
+  const int pos = uniform_load(positions + t), lo = window > 0 ? (pos - window + 1 > 0 ? pos - window + 1 : 0) : 0;
+  int first = lo / 32, end = pos / 32 + 1;
+  const int least = (end - first + n_parts - 1) / n_parts, share = n_parts > 1 && least < 4 ? 4 : least;  // a tile a wave
+  const int parts = (end - first + share - 1) / share;
+  if (n_parts > 1 && block_part == 0) {  // what the merge passes by
+    for (int i = parts + wave * 4 + grp; i < n_parts; i += 16)
+      if (valid) {
+        float* w = ws + (((size_t)t * nheads + head) * n_parts + i) * (RANK + 4);
+        w[0] = LAT_EMPTY, w[1] = LAT_NO_KEYS;
+      }
+  }
+  first += block_part * share;
+  end = end < first + share ? end : first + share;
+  const int used = end - first < 4 ? end - first : 4;
+  if (used <= 0) return;
+
+  bf16x8 q[WC];
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  const bf16* const qrow = qa + (size_t)t * ldq + (size_t)(valid ? head : 0) * WIDTH + grp * 8;
+#pragma unroll
+  for (int c = 0; c < WC; ++c) q[c] = valid ? *reinterpret_cast<const bf16x8*>(qrow + c * 32) : zero8;
+
+  // where a lane's 16 bytes of a load come from: the loads fill LDS in the order of the lanes, 72 (64) of them a row
+  constexpr int PIECES = ROW / 16, BASES = ROW == 1152 ? 9 : 1;  // nine loads are eight rows of 1152 bytes
+  unsigned from[BASES];
+#pragma unroll
+  for (int j = 0; j < BASES; ++j) {
+    const int at = j * 64 + lane, row = at / PIECES, piece = at % PIECES;
+    from[j] = row * ROW + (ROW == 1152 ? piece ^ (row >> 1 & 1) : piece) * 16;
+  }
+  const unsigned place = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)lds + wave * TILE;
+  // rows 8 g + i and 8 g + 4 + i (i < 4) have the same swizzle: of 1152 bytes bit 1 of i and the two of g, of 1024 the two of i and of g
+  auto swizzle = [](int g, int i) { return ROW == 1152 ? (i >> 1 & 1) | g << 1 : (i & 3) | g << 2; };
+  const char* const mine = reinterpret_cast<const char*>(lds) + wave * TILE;
+  const char* const key_row = mine + (8 * (col >> 2) + (col & 3)) * ROW;
+  const int key_swizzle = swizzle(col >> 2, col & 3);
+  // a transposing read: sixteen lanes ask for four keys, each a quarter of 16 elements, and lane l gets element l of the four
+  const unsigned value_row = place + (8 * grp + (col >> 2)) * ROW + (col & 1) * 8;
+  const int value_swizzle = swizzle(grp, col >> 2);
+
+  LatentState<RT, WC> st;
+#pragma unroll
+  for (int dt = 0; dt < RT; ++dt) st.acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  st.m = (sink && valid) ? sink[head] : LAT_EMPTY;
+  st.l = (sink && valid && block_part == 0 && wave == 0 && grp == 0) ? 1.f : 0.f;
+  const int* const bt = block_table + (size_t)seq * table_stride;
+  for (int kt = first + wave; kt < end; kt += 4) {
+    const int base = kt * 32;
+    const char* const rows = (const char*)(cache + (readable_page(uniform_load(bt + base / PAGE_TOKENS)) * PAGE_TOKENS + base % PAGE_TOKENS) * WIDTH);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tile before this one has been read
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int g = ROW == 1152 ? j / 9 : (j & 3) | (j >> 3) << 2;
+      load_to_lds(rows + (ROW == 1152 ? j / 9 * 9216 : j * 1024), from[ROW == 1152 ? j % 9 : 0] ^ (g << (ROW == 1152 ? 5 : 4)), place + j * 1024);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    typedef __attribute__((address_space(3))) bf16x4 LdsRow;
+    latent_tile<RT, WC, 6, 8, true>(
+        st, [&](int c) { return q[c]; },
+        [&](int which, int c) { return *reinterpret_cast<const bf16x8*>(key_row + which * 4 * ROW + ((c * 4 + grp) ^ key_swizzle) * 16); },
+        [&](int dt) {
+          const unsigned at = value_row + (((dt * 2 + (col >> 1 & 1)) ^ value_swizzle) * 16);
+          const bf16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((LdsRow*)(uintptr_t)at);
+          const bf16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((LdsRow*)(uintptr_t)(at + 4 * ROW));
+          return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+        },
+        base, lo, pos, RANK, WIDTH, scale, grp);
+  }
+  latent_meet<RT, WC, true>(st, reinterpret_cast<float*>(lds), out, ldo, ws, t, head0, nheads, RANK, n_parts, block_part, used);
+}
+
 // out[t, h, :] = sum_i acc_i exp(m_i - M) / sum_i l_i exp(m_i - M) over the parts i.  The parts' maxima and sums are
 // loaded side by side (a thread a part) and their weights left in LDS: no chain of dependent loads.
 #define LAT_MAX_PARTS 64
@@ -1099,6 +1201,25 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
     FMS_LAUNCH_CHECK("latent_attn_prompt");
     return 0;
   }
+  // single tokens with a latent of 512 (likewise)
+  const bool decode_kernel = n_splits > 0 && rank == 512 && (width == 576 || width == 512) && (uintptr_t)cache % 16 == 0;
+  if (decode_kernel) {
+#define LAUNCH_DECODE(RT, WC)                                                                                                      \
+  constexpr int tiles_bytes = 4 * 32 * WC * 64, meet_bytes = 4 * 16 * (RT * 16 + 4) * (int)sizeof(float);                          \
+  constexpr int bytes = tiles_bytes > meet_bytes ? tiles_bytes : meet_bytes;                                                       \
+  static const hipError_t sized = hipFuncSetAttribute((const void*)latent_attn_decode_kernel<RT, WC>,                              \
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                          \
+  FMS_REQUIRE(sized == hipSuccess, "latent_attn_mfma: the kernel's LDS could not be sized: %s", hipGetErrorString(sized));         \
+  latent_attn_decode_kernel<RT, WC><<<grid, 256, bytes, stream>>>((const bf16*)qa, ldq, (bf16*)out, ldo, (float*)workspace, positions, \
+                                                                  seq_of_token, block_table, table_stride, (const bf16*)cache, sink, nheads, \
+                                                                  scale, window, tiles_per_token, n_parts)
+    if (width == 576) {
+      LAUNCH_DECODE(32, 18);
+    } else {
+      LAUNCH_DECODE(32, 16);
+    }
+#undef LAUNCH_DECODE
+  } else
   // the sizes of the largest configuration exactly (a latent of 512 with a rotated part of 64, or with none) and the
   // smaller latents without a rotated part run without a question around any product; everything else in the smallest
   // configuration that holds it

@@ -1079,9 +1079,9 @@ def latent_attention_fits_mfma(rank: int, rot: int) -> bool:
 
 def latent_attention_splits(n_tokens: int, nheads: int, max_context: int) -> int:
     """Into how many parts at most the keys of a (token, 16 heads) of a decode step are cut: one round of 256 blocks in all, and no
-    block of four waves with fewer than four tiles of 32 keys at the context bound.  (Half as many parts again, or twice as many:
-    32 sequences of 128 to 2048 tokens 47 and 40 us instead of 32, 64 of them 58 and 56 instead of 47.5, of 2000 tokens each 78
-    and 67 instead of 58.)"""
+    block of four waves with fewer than four tiles of 32 keys at the context bound.  (Half as many parts again, or twice as many,
+    with the keys through registers: 32 sequences of 128 to 2048 tokens 47 and 40 us instead of 32, 64 of them 58 and 56 instead of
+    47.5, of 2000 tokens each 78 and 67 instead of 58.)"""
     tiles = n_tokens * -(-nheads // 16)
     return max(1, min(256 // tiles, -(-max_context // 128), 64))
 
