@@ -264,6 +264,62 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The same for few tokens (a decode step): a block has one token, so that its sequence, position and page come through the scalar unit, and a
+// thread QV elements of one head.  Bound by a launch and that chain of lookups, with more tokens by the values' 2-byte stores.  Us, the kernel above (whose
+// blocks are 64 tokens, so that it has a block a head) and this one, heads and kv heads of 128 in bfloat16: 16 and 4, 8 tokens 7.3 and 2.7, 64 9.9 and 3.0,
+// 256 10.8 and 5.6; 32 and 8, 8 tokens 7.4 and 3.0, 512 14.2 and 11.3; 32 and 32 in float32, 256 tokens 21.9 and 17.5, 512 33.1 and 32.6; 32 and 8 12.6 and 13.1.
+template <typename T, int QV>
+__global__ void __launch_bounds__(256)
+    rope_kv_few_kernel(T* __restrict__ qkv, long row_stride, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
+                       const int* __restrict__ block_table, int table_stride, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                       int rot_dim, int max_pos, T* __restrict__ k_cache, T* __restrict__ v_cache, int nheads, int kvheads, int head_dim) {
+  typedef typename VecOf<T, QV>::type vecq;
+  const int t = blockIdx.y, per_head = head_dim / QV, piece = blockIdx.x * blockDim.x + threadIdx.x, hh = piece / per_head;
+  if (hh >= nheads + (k_cache ? 2 * kvheads : 0)) return;
+  const int d0 = (piece - hh * per_head) * QV;
+  T* const p = qkv + (size_t)t * row_stride + (size_t)hh * head_dim + d0;
+  vecq v = *reinterpret_cast<const vecq*>(p);  // (of a padding row too: it is there)
+  const int seq = uniform_load(seq_of_token + t);
+  if (seq < 0) return;
+  const int pos = uniform_load(positions + t);
+  const int page = k_cache ? uniform_load(block_table + (size_t)seq * table_stride + pos / PAGE_TOKENS) : 0;
+  if (page < 0) return;  // as a padding row
+  const int rot_half = rot_dim / 2;
+  if (cos_t != nullptr && hh < nheads + kvheads) {
+    const int tpos = pos < 0 ? 0 : (pos < max_pos ? pos : max_pos - 1);  // the host has checked; never read outside the table
+    const int i0 = d0 / 2;  // the first pair (x[2i], x[2i+1]) of this piece
+    float c[QV / 2], sn[QV / 2];
+#pragma unroll
+    for (int j = 0; j < QV / 2; ++j) {
+      const bool rotates = i0 + j < rot_half;
+      c[j] = rotates ? cos_t[(size_t)tpos * rot_half + i0 + j] : 1.f;
+      sn[j] = rotates ? sin_t[(size_t)tpos * rot_half + i0 + j] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < QV / 2; ++j) {
+      if (i0 + j < rot_half) {
+        const float a = to_f32(v[2 * j]), b = to_f32(v[2 * j + 1]);
+        v[2 * j] = from_f32<T>(c[j] * a - sn[j] * b);
+        v[2 * j + 1] = from_f32<T>(sn[j] * a + c[j] * b);
+      }
+    }
+  }
+  if (hh < nheads) {
+    *reinterpret_cast<vecq*>(p) = v;
+    return;
+  }
+  const size_t at = (size_t)page * kvheads * PAGE_TOKENS * head_dim;
+  if (hh < nheads + kvheads) {
+    *reinterpret_cast<vecq*>(k_cache + at + ((size_t)(hh - nheads) * PAGE_TOKENS + pos % PAGE_TOKENS) * head_dim + d0) = v;
+  } else {
+    T* const to = v_cache + at + ((size_t)(hh - nheads - kvheads) * head_dim + d0) * PAGE_TOKENS + pos % PAGE_TOKENS;
+#pragma unroll
+    for (int j = 0; j < QV; ++j) to[(size_t)j * PAGE_TOKENS] = v[j];
+  }
+}
+
+#define ROPE_FEW_TOKENS 384
+
 extern "C" int fmsamd_rope_kv_write(void* qkv, int dtype, long row_stride, const int* positions,
                                     const int* seq_of_token, const int* block_table, int table_stride,
                                     const float* cos_t, const float* sin_t, int rot_dim, int max_pos, void* k_cache,
@@ -294,7 +350,17 @@ extern "C" int fmsamd_rope_kv_write(void* qkv, int dtype, long row_stride, const
     const bool by_eights = dtype == FMS_BF16 && head_dim % 8 == 0 && row_stride % 8 == 0 && (uintptr_t)qkv % 16 == 0 &&
                            (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0 && (uintptr_t)cos_t % 16 == 0 &&
                            (uintptr_t)sin_t % 16 == 0;
-    if (dtype == FMS_F32)
+    if (n_tokens <= ROPE_FEW_TOKENS) {
+      const int qv = by_eights ? 8 : 4;
+      const dim3 few(ceil_div((long)(nheads + 2 * kvheads) * (head_dim / qv), threads), n_tokens);
+#define FMS_ROPE_FEW(T, QV)                                                                                                             \
+  rope_kv_few_kernel<T, QV><<<few, threads, 0, stream>>>((T*)qkv, row_stride, positions, seq_of_token, block_table, table_stride, c, sin_t, \
+                                                         rot_dim, max_pos, (T*)k_cache, (T*)v_cache, nheads, kvheads, head_dim)
+      if (dtype == FMS_F32) FMS_ROPE_FEW(float, 4);
+      else if (by_eights) FMS_ROPE_FEW(bf16, 8);
+      else FMS_ROPE_FEW(bf16, 4);
+#undef FMS_ROPE_FEW
+    } else if (dtype == FMS_F32)
       rope_kv_tile_kernel<float, 4><<<grid, threads, lds, stream>>>(
           (float*)qkv, row_stride, positions, seq_of_token, block_table, table_stride, c, sin_t, rot_dim, max_pos,
           (float*)k_cache, (float*)v_cache, nheads, kvheads, head_dim, n_tokens);
