@@ -181,6 +181,55 @@ __global__ void __launch_bounds__(TILE_THREADS) headwise_mfma_kernel(HeadwiseArg
   }
 }
 
+// The same for few tokens: 16 tokens by 32 elements a block, whose four waves take every fourth of K's steps and meet in LDS.  Four times the blocks,
+// and one round of loads instead of several after each other.  Us, the kernel above and this one, 16 heads: 512 into 128, 8 tokens 7.6 and 3.5, 32 8.3
+// and 3.9, 192 (192 blocks above) 8.6 and 6.8; 128 into 512, 8 tokens 4.2 and 2.7, 32 4.4 and 3.4, 128 (512) 6.1 and 6.0; 64 into 128, 32 tokens
+// 3.7 and 2.8; 32 heads of 512 into 128, 128 tokens (256) 10.4 and 8.6, 192 (384) 16.4 and 16.3.
+#define HEADWISE_SPLIT_COLS 32
+__global__ void __launch_bounds__(256) headwise_split_kernel(HeadwiseArgs a) {
+  constexpr int NT = HEADWISE_SPLIT_COLS / 16, AHEAD = 4;
+  __shared__ __attribute__((aligned(16))) float parts[4][NT][256];  // lane l's four results of a tile at 4 l
+  const int t0 = blockIdx.x * TILE_ROWS, h = blockIdx.y, n0 = blockIdx.z * HEADWISE_SPLIT_COLS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = (lane >> 4) * 8;
+  // a row that is not there is the first one: its results are not stored
+  const bf16* const x = (const bf16*)a.x + (size_t)h * a.xs + (size_t)(t0 + r < a.T ? t0 + r : t0) * a.ldx;
+  const bf16* w[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) w[t] = (const bf16*)a.w + ((size_t)h * a.N + (n0 + t * 16 + r < a.N ? n0 + t * 16 + r : n0)) * a.K;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int k0 = wave * 32; k0 < a.K; k0 += 128 * AHEAD) {
+    bf16x8 xv[AHEAD], wv[AHEAD][NT];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      const int k = k0 + 128 * s + kq;
+      xv[s] = k < a.K ? *reinterpret_cast<const bf16x8*>(x + k) : zero;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wv[s][t] = k < a.K ? *reinterpret_cast<const bf16x8*>(w[t] + k) : zero;
+    }
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[s], wv[s][t], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&parts[wave][t][lane * 4]) = acc[t];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {  // neighbouring threads: neighbouring elements of a token
+    const int at = i * 256 + threadIdx.x, row = at / HEADWISE_SPLIT_COLS, c = at % HEADWISE_SPLIT_COLS, t = t0 + row, n = n0 + c;
+    if (t >= a.T || n >= a.N) continue;
+    const int from = (row / 4 * 16 + c % 16) * 4 + row % 4;
+    float v = 0.f;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) v += parts[p][c / 16][from];
+    if (a.gate) v *= 1.f / (1.f + expf(-a.gate[(size_t)t * a.ldg + h]));
+    ((bf16*)a.y)[(size_t)t * a.ldy + (size_t)h * a.ys + n] = (bf16)v;
+  }
+}
+
 // The same for steps of many tokens, through LDS (tile_product_lds.h): tiles of 128 tokens by 128 elements, two blocks a compute
 // unit.  K is short (a head's size or the latent's), so a block is mostly its first loads and its stores.  2048 tokens, 16 heads
 // of 128 into a latent of 512 and back: 24.8 us on average (29.7 in tiles of 64 tokens whose operands came straight from memory).
@@ -212,6 +261,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) h
 }
 
 #define HEADWISE_COMPUTE_UNITS 256
+#define HEADWISE_SPLIT_K 64        // (two steps)
+#define HEADWISE_SPLIT_BLOCKS 384  // of the kernel without the split
 
 extern "C" int fmsamd_headwise_linear(const void* x, long ldx, long x_head_stride, const void* w, void* y, long ldy,
                                       long y_head_stride, const float* gate, long ldg, int dtype, int n_tokens, int nheads,
@@ -236,6 +287,9 @@ extern "C" int fmsamd_headwise_linear(const void* x, long ldx, long x_head_strid
                       (double)n_tokens * nheads * N * K >= 2e8;
     if (aligned && K >= TL_BK && full && grid.z <= 65535)  // (and tiles that fit a launch)
       headwise_lds_kernel<<<grid, 256, 0, stream>>>(a);
+    else if (aligned && K >= HEADWISE_SPLIT_K && (long)row_tiles * nheads * ceil_div(N, TILE_MFMA_COLS) <= HEADWISE_SPLIT_BLOCKS &&
+             ceil_div(N, HEADWISE_SPLIT_COLS) <= 65535)
+      headwise_split_kernel<<<dim3(row_tiles, nheads, ceil_div(N, HEADWISE_SPLIT_COLS)), 256, 0, stream>>>(a);
     else if (aligned)
       headwise_mfma_kernel<<<dim3(row_tiles, nheads, ceil_div(N, TILE_MFMA_COLS)), TILE_THREADS, 0, stream>>>(a);
     else
