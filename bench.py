@@ -453,16 +453,18 @@ def design_comparison(args, design) -> int:
             T, n_seqs = a[0].shape[0], a[9]
             vector_flops = 5.0 * T * H * D * V
             return T * 4 * a[0].shape[1] + nbytes(kw.get("up_t"), out) + 2 * n_seqs * (st.numel() // st.shape[0]) * 4, vector_flops * mfma_flops / PEAK_FLOPS["fp32"]
-        if name == "latent_attention":  # one row of rank + rot a key, and the latent once more as values
+        if name == "latent_attention":  # one row of rank + rot a key, and the latent once more as values (not for single tokens with a latent of 512)
             H, R, P = a[6], a[7], a[8]
             read, loaded = keys_of_call(a, kw)
-            return 2 * loaded * (2 * R + P) + nbytes(a[0]) + 2 * a[0].shape[0] * H * R, 2.0 * read * H * (2 * R + P)
+            return 2 * loaded * (R + P if R == 512 and kw.get("decode") else 2 * R + P) + nbytes(a[0]) + 2 * a[0].shape[0] * H * R, 2.0 * read * H * (2 * R + P)
         if name == "rglru_gates":  # two block-diagonal products on the float32 vector units, priced like the delta rule's passes
             u, ra = a[0], a[1]
             vector_flops = 4.0 * u.shape[0] * ra.numel()
             return nbytes(u, ra, a[3]) + 2 * u.numel() * 4, vector_flops * mfma_flops / PEAK_FLOPS["fp32"]
         if name == "rglru_scan":  # a, b and the other branch read once, the result written once
             return nbytes(a[0], a[1]) + a[0].numel() * 4 + nbytes(out), 0.0
+        if name == "moe_router":  # the product's rows and weights, and the choice's few bytes
+            return nbytes(a[0], a[1], *out), 2.0 * a[0].shape[0] * a[1].numel()
         if name == "moe_experts" and a[2] is None:  # experts without a gate
             x, ids, _, u, d = a[:5]
             used = min(u.shape[0], ids.numel())
@@ -475,12 +477,12 @@ def design_comparison(args, design) -> int:
         return nbytes(*[t for t in tensors if t.dim() == 2 and t.shape[0] == tensors[0].shape[0]]), 0.0
 
     watched = ["linear", "gated_linear", "linear_into_stream", "headwise_linear", "attention", "latent_attention", "moe_experts",
-               "moe_route", "moe_combine", "add_norm", "norm_add_norm", "rms_norm_cols", "rope_kv_write", "qkv_rope_write",
+               "moe_router", "moe_route", "moe_combine", "add_norm", "norm_add_norm", "rms_norm_cols", "rope_kv_write", "qkv_rope_write",
                "latent_kv_write", "latent_q_rotate", "activation", "clamped_gated_act", "gated_act", "embed", "norm_add_norm_affine",
                "delta_rule", "delta_prepare", "gated_head_norm", "qk_projection_norm", "gate_mul", "scale_", "cast", "cast_cols",
                "rglru_gates", "rglru_scan", "short_conv", "group_norm_chain", "poly_norm", "moe_route_grouped", "talking_attention", "ssd", "ssd_step",
                "gated_group_norm", "value_head_norm", "stream_rows", "linear_recurrence", "stream_enter", "soft_cap_"]
-    small = {"moe_route", "moe_combine", "add_norm", "norm_add_norm", "norm_add_norm_affine", "rms_norm_cols", "rope_kv_write", "latent_kv_write",
+    small = {"moe_router", "moe_route", "moe_combine", "add_norm", "norm_add_norm", "norm_add_norm_affine", "rms_norm_cols", "rope_kv_write", "latent_kv_write",
              "latent_q_rotate", "activation", "clamped_gated_act", "gated_act", "embed", "delta_prepare", "gated_head_norm",
              "qk_projection_norm", "gate_mul", "scale_", "cast", "cast_cols", "short_conv", "group_norm_chain", "poly_norm",
              "moe_route_grouped", "gated_group_norm", "value_head_norm", "stream_rows", "stream_enter", "soft_cap_"}
