@@ -2,7 +2,8 @@
 
 torch tensors are used as device buffers only; every computation below is a
 HIP kernel of this package, with one exception that is named where it happens
-(large bfloat16 matrix products go to the vendor library through
+(bfloat16 matrix products of more than 192 rows that the kernel for many rows
+does not take, or would take longer for, go to the vendor library through
 ``torch.matmul``, as the reference's linear layers do).  Each wrapper checks on
 the host what its kernel and grid assume before launching.
 """
@@ -589,8 +590,8 @@ def prefill_qblock(nheads: int, kvheads: int, head_dim: int, n_tokens: int) -> i
 # --------------------------------------------------------------------------
 SKINNY_MAX_ROWS = 192
 _PLAIN_ACTIVATIONS = ("identity", "relu", "relu2")  # what the skinny kernels finish a plain product with
-# Up to this many rows the skinny kernel, with the norms, rotation and activation fused into it, beats the
-# vendor library followed by those as kernels of their own.
+# Up to this many rows the skinny kernel, with the norms, rotation and activation fused into it, beats a
+# product for many rows followed by those as kernels of their own.
 SKINNY_FAST_ROWS = 192
 
 
