@@ -154,6 +154,7 @@ int fmsamd_gemm_skinny_gated_bf16(const void* x, long ldx, const void* w, const 
 // least 256, 16-byte addresses.  pays: 1 where they are expected to be faster than the vendor library's.
 int fmsamd_gemm_tall_pays(int M, int N, int K, int gated);
 int fmsamd_gemm_tall_plan(int M, int N, int K, int gated);  // which tiles it takes, 0 to 4
+long fmsamd_gemm_tall_stores(int M, int N, long ldo, int size, int gated, int tiles);  // stores walked through on the host, -1: one lies outside
 int fmsamd_gemm_tall_bf16(const void* x, long ldx, const void* w, const void* bias, int bias_dtype, void* out, int out_dtype, long ldo, int M,
                           int N, int K, hipStream_t stream);
 int fmsamd_gemm_tall_gated_bf16(const void* x, long ldx, const void* w, const void* bias, int bias_dtype, void* out, long ldo, int M, int hidden,

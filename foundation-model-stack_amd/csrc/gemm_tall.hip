@@ -32,23 +32,42 @@ struct TallArgs {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// The tiles from `first` to `last`, cut into PARTS parts each (2: rows in halves; 4: columns as well), dealt to the blocks: in every
-// round the blocks of one XCD (block % 8) take neighbours, which share rows of x and of W in its L2.
+// The tiles from `first` to `last`, cut into `parts` parts each (2: rows in halves; 4: columns as well), dealt to the blocks: in every
+// round the blocks of one XCD (block % 8) take neighbours, which share rows of x and of W in its L2.  The corner of the n-th part of a
+// block, of bm rows and bn columns; false behind the last one.  A part may lie behind the last row or column as a whole.
+__host__ __device__ __forceinline__ bool tall_corner(const TallArgs& g, int first, int last, int parts, int bm, int bn, int blocks, int block, int n,
+                                                     int& m0, int& n0) {
+  const int row_parts = parts > 1 ? 2 : 1, col_parts = parts / row_parts, xcd = block % 8, nth = block / 8, count = (last - first) * parts;
+  const int left = count - n * blocks, per = ((left < blocks ? left : blocks) + 7) / 8, in_round = xcd * per + nth;
+  if (nth >= per || in_round >= left) return false;
+  const int u = n * blocks + in_round;
+  const int t = first + u / parts, part = u % parts;
+  const int top = t / (g.group * g.col_tiles) * g.group, rows = g.row_tiles - top < g.group ? g.row_tiles - top : g.group;
+  const int in = t - top * g.col_tiles;
+  m0 = ((top + in % rows) * row_parts + part % row_parts) * bm;
+  n0 = ((in / rows) * col_parts + part / row_parts) * bn;
+  return true;
+}
+
+// How many bytes of out a part of bm rows may store to, from its first result on: to the end of its last row that exists.  What lies
+// behind is left out by the store.  None for a part without rows or columns.  (The store takes the number as unsigned: it must not be
+// negative, as it would be for one row whose columns all lie behind N.)  Below 2^31, so that TALL_ABSENT lies behind it.
+__host__ __device__ __forceinline__ unsigned tall_reach(const TallArgs& g, int m0, int n0, int bm, int size) {
+  const int rows = g.M - m0 < bm ? g.M - m0 : bm;
+  return rows <= 0 || n0 >= g.N ? 0 : (unsigned)((rows * g.ldo - n0) * size);
+}
+
+// Where in there a piece of eight results is stored: of columns that do not exist, behind the reach.
+#define TALL_ABSENT 0x80000000u
+__host__ __device__ __forceinline__ unsigned tall_offset(const TallArgs& g, int n0, int row, int col, int size) {
+  return n0 + col < g.N ? (unsigned)(((long)row * g.ldo + col) * size) : TALL_ABSENT;
+}
+
 template <typename R, bool GATED, typename O, int PARTS>
 __device__ __forceinline__ void tall_tiles(const TallArgs& g, int first, int last, char* lds) {
-  constexpr int BN = GATED ? R::HN : R::BN, ROW_PARTS = PARTS > 1 ? 2 : 1, COL_PARTS = PARTS / ROW_PARTS;
-  const int blocks = gridDim.x, xcd = blockIdx.x % 8, nth = blockIdx.x / 8;
-  const int count = (last - first) * PARTS;
+  constexpr int BN = GATED ? R::HN : R::BN;
   auto corner = [&](int n, int& m0, int& n0) __attribute__((always_inline)) {
-    const int left = count - n * blocks, per = ((left < blocks ? left : blocks) + 7) / 8, in_round = xcd * per + nth;
-    if (nth >= per || in_round >= left) return false;
-    const int u = n * blocks + in_round;
-    const int t = first + u / PARTS, part = u % PARTS;
-    const int top = t / (g.group * g.col_tiles) * g.group, rows = g.row_tiles - top < g.group ? g.row_tiles - top : g.group;
-    const int in = t - top * g.col_tiles;
-    m0 = ((top + in % rows) * ROW_PARTS + part % ROW_PARTS) * R::BM;
-    n0 = ((in / rows) * COL_PARTS + part / ROW_PARTS) * BN;
-    return true;
+    return tall_corner(g, first, last, PARTS, R::BM, BN, gridDim.x, blockIdx.x, n, m0, n0);
   };
   auto bytes = [](long there, int most, long stride) { return (unsigned)((there < 0 ? 0 : there < most ? there : most) * stride * 2); };
   auto place = [&](int n, RingTile& t) __attribute__((always_inline)) {
@@ -72,10 +91,9 @@ __device__ __forceinline__ void tall_tiles(const TallArgs& g, int first, int las
     const int row0 = (wave / R::WN) * R::QM * 16 + r, col0 = (wave % R::WN) * R::QN * 32 + h * 8;
     int m0, n0;
     corner(n, m0, n0);
-    const int rows = g.M - m0 < R::BM ? g.M - m0 : R::BM;
-    // a store that lies behind the buffer's end is left out
-    const auto to = __builtin_amdgcn_make_buffer_rsrc((O*)g.out + (long)m0 * g.ldo + n0, 0, rows <= 0 ? 0 : (int)((rows * g.ldo - n0) * sizeof(O)),
-                                                      0x00020000);
+    const unsigned reach = tall_reach(g, m0, n0, R::BM, sizeof(O));
+    if (reach == 0) return;
+    const auto to = __builtin_amdgcn_make_buffer_rsrc((O*)g.out + (long)m0 * g.ldo + n0, 0, (int)reach, 0x00020000);
     auto store = [&](u32x4 v, unsigned offset) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b128(v, to, offset, 0, 0); };
     auto write = [&](auto unit) __attribute__((always_inline)) {
       ring_for<(GATED ? 1 : 2) * R::QN>([&](auto bjc) __attribute__((always_inline)) {
@@ -97,8 +115,7 @@ __device__ __forceinline__ void tall_tiles(const TallArgs& g, int first, int las
         ring_for<2 * R::QM>([&](auto aic) __attribute__((always_inline)) {
           constexpr int a = decltype(aic)::value / R::QM, i = decltype(aic)::value % R::QM;
           const int row = row0 + a * R::HM + i * 16;
-          // (rows that do not exist lie behind the end of the buffer, columns that do not far behind it)
-          const unsigned offset = there ? (unsigned)(((long)row * g.ldo + col) * sizeof(O)) : 0x80000000u;
+          const unsigned offset = tall_offset(g, n0, row, col, sizeof(O));
           float v[8];
           const f32x4 lo = sums[R::at(a, b, i, j)], hi = sums[R::at(a, b, i, j + 1)];
 #pragma unroll
@@ -205,20 +222,26 @@ extern "C" int fmsamd_gemm_tall_pays(int M, int N, int K, int gated) {
   return ideal >= tall_plan(M, N, K, gated != 0).us * share * (gated ? 0.5 : 1.0);
 }
 
-template <typename R, bool GATED, typename O>
-static int tall_launch(TallArgs g, int split, hipStream_t stream) {
-  g.row_tiles = ceil_div(g.M, R::BM);
-  g.col_tiles = ceil_div(g.N, GATED ? R::HN : R::BN);
+// The tiles, of bm rows and bn columns, that a product is cut into, and how many of them stay whole.
+static int tall_cut(TallArgs& g, int bm, int bn, int split) {
+  g.row_tiles = ceil_div(g.M, bm);
+  g.col_tiles = ceil_div(g.N, bn);
   g.group = ceil_div(g.row_tiles, ceil_div(g.row_tiles, 8));
   const int tiles = g.row_tiles * g.col_tiles, units = TALL_COMPUTE_UNITS;
   g.split = split;
   g.full = split == 1 ? tiles : tiles / units * units;
+  const long parts = (long)tiles * split;
+  return parts < units ? ((int)parts + 7) / 8 * 8 : units;  // blocks
+}
+
+template <typename R, bool GATED, typename O>
+static int tall_launch(TallArgs g, int split, hipStream_t stream) {
+  const int blocks = tall_cut(g, R::BM, GATED ? R::HN : R::BN, split);
   auto kernel = tall_kernel<R, GATED, O>;
   // more than 64 KB of LDS a block has to be asked for, once a kernel
   static const hipError_t sized = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, R::LDS_BYTES);
   FMS_REQUIRE(sized == hipSuccess, "gemm_tall: %d bytes of LDS refused: %s", R::LDS_BYTES, hipGetErrorString(sized));
-  const long parts = (long)tiles * split;
-  kernel<<<parts < units ? ((int)parts + 7) / 8 * 8 : units, R::THREADS, R::LDS_BYTES, stream>>>(g);
+  kernel<<<blocks, R::THREADS, R::LDS_BYTES, stream>>>(g);
   FMS_LAUNCH_CHECK("gemm_tall");
   return 0;
 }
@@ -263,4 +286,33 @@ extern "C" int fmsamd_gemm_tall_gated_bf16(const void* x, long ldx, const void* 
   const TallArgs g{(const bf16*)x, (const bf16*)w, bias, bias_dtype == FMS_F32, out, ldx, ldo, M, hidden, K, 0, 0, 0, 0, 0, unit};
   if (tall_check("gemm_tall_gated_bf16", g, 2)) return -1;
   return tall_choose<true, bf16>(g, stream);
+}
+
+// How many pieces of eight results a product of this kind of tiles (as fmsamd_gemm_tall_plan names them) stores, walked through on the host
+// with what the kernels compute their stores from: M N / 8.  -1: one would lie outside its row, behind the last row or behind its part's reach.
+extern "C" long fmsamd_gemm_tall_stores(int M, int N, long ldo, int size, int gated, int tiles) {
+  TallArgs g{};
+  g.M = M, g.N = N, g.ldo = ldo;
+  const int split = tiles == 1 ? 2 : tiles == 2 ? 4 : 1, bn = (tiles < 3 ? 256 : tiles == 3 ? 192 : 128) / (gated ? 2 : 1);
+  const int blocks = tall_cut(g, 256, bn, split);
+  long stored = 0;
+  for (int rest = 0; rest < 2; ++rest) {  // the whole tiles, and the parts of the others
+    const int first = rest ? g.full : 0, last = rest ? g.row_tiles * g.col_tiles : g.full, parts = rest ? split : 1;
+    const int part_rows = parts > 1 ? 128 : 256, part_cols = parts == 4 ? bn / 2 : bn;
+    for (int block = 0; block < blocks; ++block) {
+      int m0, n0;
+      for (int n = 0; tall_corner(g, first, last, parts, part_rows, part_cols, blocks, block, n, m0, n0); ++n) {
+        const unsigned reach = tall_reach(g, m0, n0, part_rows, size);
+        if (reach > TALL_ABSENT) return -1;
+        for (int row = 0; row < part_rows; ++row)
+          for (int col = 0; col < part_cols; col += 8) {
+            const unsigned offset = tall_offset(g, n0, row, col, size);
+            if (offset >= reach) continue;
+            if (m0 + row >= M || n0 + col + 8 > N || offset + 8u * size > reach) return -1;
+            ++stored;
+          }
+      }
+    }
+  }
+  return stored;
 }

@@ -47,6 +47,7 @@ _SIGNATURES = {
     "fmsamd_gemm_skinny_gated_bf16": [P, L, P, P, I, P, I, L, I, I, I, I, P, P, P, L, P],
     "fmsamd_gemm_tall_pays": [I, I, I, I],
     "fmsamd_gemm_tall_plan": [I, I, I, I],
+    "fmsamd_gemm_tall_stores": [I, I, L, I, I, I],
     "fmsamd_gemm_tall_bf16": [P, L, P, P, I, P, I, L, I, I, I, P],
     "fmsamd_gemm_tall_gated_bf16": [P, L, P, P, I, P, L, I, I, I, I, P, P],
     "fmsamd_gemm_skinny_residual_partials": [I, I, I],
@@ -161,6 +162,7 @@ def load(verbose: bool = True) -> ctypes.CDLL:
         lib.fmsamd_argmax_workspace.argtypes = [I, I]
         lib.fmsamd_attn_decode_workspace.restype = c_long
         lib.fmsamd_gemm_skinny_workspace.restype = c_long
+        lib.fmsamd_gemm_tall_stores.restype = c_long
         lib.fmsamd_attn_decode_workspace.argtypes = [I, I, I, I]
         lib.path = path
         _lib = lib

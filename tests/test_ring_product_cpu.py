@@ -48,3 +48,21 @@ def test_a_product_that_pays_is_one_that_fits(gated):
     for M, N, K in ((2048, 4096, 4096), (2048, 6144, 4096), (4689, 14336, 4096)):
         assert lib.fmsamd_gemm_tall_pays(M, N, K, gated) == 1
         assert 0 <= lib.fmsamd_gemm_tall_plan(M, N, K, gated) <= 4
+
+
+@pytest.mark.parametrize("tiles", range(5))
+@pytest.mark.parametrize("gated", [0, 1])
+@pytest.mark.parametrize("size", [2, 4])
+def test_every_store_of_a_product_lies_inside_its_output(tiles, gated, size):
+    """Every result is stored and nothing else, whatever rows and columns are left for the last tiles and their halves and quarters."""
+    from fms_amd.kernels.library import load
+
+    lib = load()
+    for rows in (193, 255, 256, 257, 384, 385, 513, 640, 641, 642, 1921, 2049, 2561, 3201, 4097):
+        for cols in (128, 136, 248, 256, 264, 384, 392, 1360, 2048, 4368, 6176):
+            for ldo in (cols, cols + 8, 3 * cols):
+                assert lib.fmsamd_gemm_tall_stores(rows, cols, ldo, size, gated, tiles) == rows * cols // 8, (rows, cols, ldo)
+    # the longest rows that are taken
+    longest = (1 << 22) // size - 8
+    for rows, cols in ((193, longest), (257, 264), (641, 4368)):
+        assert lib.fmsamd_gemm_tall_stores(rows, cols, longest, size, gated, tiles) == rows * cols // 8

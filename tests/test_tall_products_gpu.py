@@ -90,6 +90,32 @@ def test_gated(M, N, K, tiles, kind):
     assert bool((wide[M] == 7).all()) and bool((wide[:M, :8] == 7).all()) and bool((wide[:M, 8 + N :] == 7).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(641, 4368, 2048), (2049, 1360, 2048), (2561, 6176, 2048)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_one_row_and_no_column_for_the_last_quarter(M, N, K, out_dtype):
+    from fms_amd.kernels import ops
+
+    assert library().fmsamd_gemm_tall_pays(M, N, K, 0) == 1 and library().fmsamd_gemm_tall_plan(M, N, K, 0) == 2
+    x, w = rows_of(M, K, 0, 11).contiguous(), rows_of(N, K, 0, 12).contiguous()
+    want, size = sums(x, w, None)
+    allowed = size * (K / 16) * 2.0 ** -24 + (want.abs() * 2.0 ** -8 if out_dtype == torch.bfloat16 else 0)
+    assert float(((ops.linear(x, w, out_dtype=out_dtype).double() - want).abs() - allowed).max()) <= 0
+
+
+def test_one_row_and_no_column_for_the_last_quarter_of_a_gated_product():
+    from fms_amd.kernels import ops
+
+    M, N, K = 3201, 136, 1024
+    assert library().fmsamd_gemm_tall_pays(M, N, K, 1) == 1 and library().fmsamd_gemm_tall_plan(M, N, K, 1) == 2
+    x, w = rows_of(M, K, 0, 13).contiguous(), (rows_of(2 * N, K, 0, 14) * 0.1).contiguous()
+    s, size = sums(x, w, None)
+    gate, up = s[:, :N], s[:, N:]
+    act = gate * torch.sigmoid(gate)
+    want, loose = act * up, size * (K / 16) * 2.0 ** -24  # allowed: as in test_gated
+    allowed = want.abs() * 2.0 ** -8 + 2 * loose[:, :N] * up.abs() + loose[:, N:] * act.abs() + 2.0 ** -20 * (gate.abs() + 1) * (up.abs() + 1)
+    assert float(((ops.gated_linear(x, w, None, "silu").double() - want).abs() - allowed).max()) <= 0
+
+
 def test_rows_keep_their_own_infinities():
     """An infinity or NaN in a row of x or W stays in its row or column, also where a tile has rows that do not exist."""
     from fms_amd.kernels import ops
