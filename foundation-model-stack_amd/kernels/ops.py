@@ -596,8 +596,9 @@ SKINNY_FAST_ROWS = 192
 
 
 def _tall_fits(x: torch.Tensor, weight: torch.Tensor, cols: int, gated: bool) -> bool:
-    """True if the kernel for many rows takes this bfloat16 product and is expected to be faster than the vendor library's."""
-    return (x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+    """True if the kernel for many rows takes this bfloat16 product and is expected to be faster than the vendor library's (which
+    takes rows that overlap, too)."""
+    return (x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1] and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and max(x.stride(0), 4 * cols) < 1 << 22 and load().fmsamd_gemm_tall_pays(x.shape[0], cols, x.shape[1], int(gated)) == 1)
 
 

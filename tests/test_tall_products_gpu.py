@@ -156,6 +156,22 @@ def test_entry_points_take_what_they_took():
     assert ops.linear(x, w[:120].contiguous()).shape == (M, 120) and ops.linear(x, w[:300].contiguous()).shape == (M, 300)
 
 
+@pytest.mark.parametrize("step", [0, 8, 2040])
+def test_rows_may_overlap(step):
+    """Rows of x that are one row many times over, or a window that slides along."""
+    from fms_amd.kernels import ops
+
+    M, N, K = 2048, 2048, 2048
+    flat = torch.randn(step * (M - 1) + K, generator=torch.Generator(device="cuda").manual_seed(15), device="cuda").to(torch.bfloat16)
+    x, w = flat.as_strided((M, K), (step, 1)), (rows_of(N, K, 0, 16) * 0.05).contiguous()
+    for out_dtype in (torch.bfloat16, torch.float32):
+        want, size = sums(x, w, None)
+        allowed = size * (K / 16) * 2.0 ** -24 + want.abs() * 2.0 ** -8
+        assert float(((ops.linear(x, w, out_dtype=out_dtype).double() - want).abs() - allowed).max()) <= 0
+    gated, same = ops.gated_linear(x, w, None, "silu"), ops.gated_linear(x.contiguous(), w, None, "silu")
+    assert float((gated.float() - same.float()).norm() / same.float().norm()) < 2.0 ** -7
+
+
 def test_a_captured_product_replays():
     from fms_amd.kernels import ops
 
