@@ -174,6 +174,16 @@ def _rows_out(out: Optional[torch.Tensor], rows: int, cols: int, dtype: torch.dt
     return out
 
 
+def _spans_meet(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """True if the memory from a's first to its last element and that of b have a byte in common (rows with a contiguous last dimension)."""
+    def span(t):
+        first = t.data_ptr()
+        return first, first + ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) * t.element_size()
+
+    (a0, a1), (b0, b1) = span(a), span(b)
+    return a0 < b1 and b0 < a1
+
+
 def gated_act(gu: torch.Tensor, bias: Optional[torch.Tensor], activation: str, clamp: Optional[GateClamp] = None,
               out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """[T, 2*hidden] (gate first) -> act(gate + b) * (up + b) [T, hidden], or the clamped unit of the two sums.  out: rows of
@@ -766,7 +776,8 @@ def gated_linear(
             and (bias is None or (bias.shape == (2 * hidden,) and bias.is_contiguous())) and _tall_fits(x, weight, hidden, True)):
         _need_cuda(x, weight, bias)
         rows = _rows_out(out, M, hidden, torch.bfloat16, x.device)
-        if rows.stride(0) % 8 == 0 and rows.stride(0) < 1 << 21 and rows.data_ptr() % 16 == 0:
+        # (results over rows of x that other blocks still read are left to the two kernels below, which are done with x by then)
+        if rows.stride(0) % 8 == 0 and rows.stride(0) < 1 << 21 and rows.data_ptr() % 16 == 0 and not (out is not None and _spans_meet(rows, x)):
             check(load().fmsamd_gemm_tall_gated_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias),
                                                      _code(bias.dtype) if bias is not None else 0, rows.data_ptr(), rows.stride(0), M, hidden,
                                                      x.shape[1], ACTIVATIONS[activation], _clamp(clamp), _stream()))

@@ -172,6 +172,21 @@ def test_rows_may_overlap(step):
     assert float((gated.float() - same.float()).norm() / same.float().norm()) < 2.0 ** -7
 
 
+@pytest.mark.parametrize("shift", [0, 2048])
+def test_results_may_take_the_place_of_the_rows(shift):
+    """A gated product whose results go where its rows stand reads them all first, also where it has tiles for several rounds of blocks."""
+    from fms_amd.kernels import ops
+
+    M, N, K = 8192, 2048, 4096
+    x, w = rows_of(M, K, 0, 17).contiguous(), (rows_of(2 * N, K, 0, 18) * 0.05).contiguous()
+    assert library().fmsamd_gemm_tall_pays(M, N, K, 1) == 1
+    gu = x.float() @ w.float().T.contiguous()
+    want = torch.nn.functional.silu(gu[:, :N]) * gu[:, N:]
+    out = x[:, shift : shift + N]
+    assert ops.gated_linear(x, w, None, "silu", out=out).data_ptr() == out.data_ptr()
+    assert float((x[:, shift : shift + N].float() - want).norm() / want.norm()) < 2.0 ** -7  # three roundings of 2^-9, gate and up among them
+
+
 def test_a_captured_product_replays():
     from fms_amd.kernels import ops
 
