@@ -213,8 +213,15 @@ extern "C" int fmsamd_gemm_tall_plan(int M, int N, int K, int gated) {
 
 // Whether a product is better here than in the vendor library, which cuts K where rows and columns give few tiles: from the share of
 // the chip that the tiles here use.  Of shapes timed in turn, 512 rows by 4096 columns of K = 2048 are equal (16 us, a share of 0.31), 1024
-// by 4096 of K = 4096 too (39 us, 0.56), and of K = 14336 3000 rows lose (292 us, library 249; 0.77) where 2048 win (181, 196; 0.84).  Around
-// the line either is up to a tenth faster.  A gated product saves the kernel behind it and its bytes as well: half of the share will do.
+// by 4096 of K = 4096 too (39 us, 0.56), and of K = 14336 3000 rows lose (292 us, library 249; 0.77) where 2048 win (181, 196; 0.84).  A
+// gated product saves the kernel behind it and its bytes as well: half of the share will do.
+//
+// The products of every registered configuration at 33 numbers of rows from 193 to 4689, between a kernel that writes x and one that
+// reads the results: of 1556 that are taken 960 are more than 3 % faster here and 245 slower, 7.7 % faster on average.  The slower ones are
+// whole squares of bfloat16 results with many rows (3000 x 4096 x 4096 84, library 76; K = 5120 and 128256 columns are 4 to 18 % faster
+// here: equal on average) and 256 x 128 tiles with a share below 0.55 (5 % slower on average).  Leaving the first to the library
+// makes a pass of 8 layers of 4096 wide 0.3 % slower to 1.3 % faster (2277 to 4096 rows), the second one of 2048 wide 1.0 % slower to
+// 0.5 % faster (512 to 1280 rows): the kernels behind read the library's results more slowly.  So there is no line for them.
 extern "C" int fmsamd_gemm_tall_pays(int M, int N, int K, int gated) {
   if (M <= FMS_SKINNY_MAX_ROWS || N < 128 || K < 256 || N % 8 || K % 128 || K >= TALL_LONGEST || !tall_countable(M, N)) return 0;
   const double ideal = (double)M * N * (gated ? 2 : 1) / (256. * 256 * TALL_COMPUTE_UNITS) * (K / 64) * 1.36;
