@@ -786,6 +786,14 @@ def gated_linear(
     return gated_act(gu, bias, activation, clamp, out)
 
 
+def clamped_product_pays(rows: int, weight: torch.Tensor) -> bool:
+    """True if a clamped gated unit of these rows is formed faster by `gated_linear` than by the product and `clamped_gated_act`.  Not for
+    17 to 32 rows by a small weight, whose plain product runs in the kernel for up to 16 rows, two tiles a wave, and the gated one in the one for
+    up to 192: 2 x 128 by 256 6.0 us and 5.2, 2 x 512 by 512 6.3 and 5.7, 2 x 384 by 1024 7.1 and 6.4; 2 x 1024 by 1024 6.5 and 6.7, 2 x 2048 by 2048 10.0
+    and 10.1.  (Fewer rows 3.1 and 5.1, 6.5 and 8.4 for the smallest and the largest of them, more 6.1 and 7.7, 10 and 13.)"""
+    return not (16 < rows <= 32 and weight.numel() < 1 << 20)
+
+
 # --------------------------------------------------------------------------
 # norms behind a branch, further activations
 # --------------------------------------------------------------------------

@@ -134,8 +134,9 @@ class ExpertsFeedForward(FeedForward):
         shared = gate = None
         if self.shared_hidden_dim:
             if self.expert_gate:
-                if self.shared_limit > 0:
-                    hidden = ops.gated_linear(x, self.shared_gate_up.w["weight"], None, "silu", clamp=self._shared_unit)
+                gate_up = self.shared_gate_up.w["weight"]
+                if self.shared_limit > 0 and ops.clamped_product_pays(x.shape[0], gate_up):
+                    hidden = ops.gated_linear(x, gate_up, None, "silu", clamp=self._shared_unit)
                 else:
                     hidden = ops.clamped_gated_act(self.shared_gate_up.forward(x), self.shared_limit, self.alpha, self.shift)
             else:
