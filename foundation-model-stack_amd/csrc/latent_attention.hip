@@ -760,7 +760,7 @@ __global__ void __launch_bounds__(256)
       if (base + 32 <= last_pos) fetch(base + 32);
       // (a condition that all lanes of the wave share: matrix instructions take their operands from every lane)
       if (tile < n_tiles && seq >= 0 && base <= pos) {
-        latent_tile<RT, WC, (WC <= 10 ? WC : (WC % 8 == 0 ? 8 : 6)), (RT <= 16 ? RT : 8), EXACT>(
+        latent_tile<RT, WC, (WC <= 10 ? WC : 6), (RT <= 16 ? RT : 8), EXACT>(
             st, load_q,
             [&](int which, int c) {
               return (EXACT || c * 32 + grp * 8 < width) ? *reinterpret_cast<const bf16x8*>(k_lds + (key_a + 4 * which) * ks + c * 32 + grp * 8) : zero8;
@@ -786,8 +786,8 @@ __global__ void __launch_bounds__(256)
       const bf16* vt = vt_cache + (page * rank + col) * PAGE_TOKENS + in_page + grp * 8;
       // straight from global memory (guarded products of the largest sizes, and blocks of a prompt whose tiles lie in several
       // sequences, have no registers for loads that far ahead)
-      constexpr bool AHEAD = !LDS && (EXACT || RT <= 16);
-      latent_tile<RT, WC, (!AHEAD && WC > 10 ? (WC % 8 == 0 ? 8 : 9) : WC), (AHEAD && RT > 8 ? 8 : RT <= 16 ? RT : 16), EXACT, AHEAD>(
+      constexpr bool AHEAD = !LDS && RT <= 16;
+      latent_tile<RT, WC, (WC > 10 ? 9 : WC), (AHEAD && RT > 8 ? 8 : RT <= 16 ? RT : 16), EXACT, AHEAD>(
           st, load_q,
           [&](int which, int c) {
             return (EXACT || c * 32 + grp * 8 < width) ? *reinterpret_cast<const bf16x8*>(ka + which * 4 * (size_t)width + c * 32) : zero8;
@@ -1292,14 +1292,9 @@ extern "C" int fmsamd_latent_attn_mfma(const void* qa, long ldq, void* out, long
     }
 #undef LAUNCH_DECODE
   } else
-  // the sizes of the largest configuration exactly (a latent of 512 with a rotated part of 64, or with none) and the
-  // smaller latents without a rotated part run without a question around any product; everything else in the smallest
-  // configuration that holds it
-  if (rank == 512 && width == 576) {
-    LAUNCH_LATENT(32, 18, true);
-  } else if (rank == 512 && width == 512) {
-    LAUNCH_LATENT(32, 16, true);
-  } else if (rank == 256 && width == 256) {
+  // the smaller latents without a rotated part run without a question around any product; everything else in the smallest
+  // configuration that holds it (also a latent of 512 whose cache does not start at a 16-byte address)
+  if (rank == 256 && width == 256) {
     LAUNCH_LATENT(16, 8, true);
   } else if (rank == 128 && width == 128) {
     LAUNCH_LATENT(8, 4, true);

@@ -45,3 +45,27 @@ def test_decode(rot, heads, sink, lengths, window):
                 s = torch.cat([s, sinks.double()[:, None]], dim=1)
             want = torch.softmax(s, dim=1)[:, : rows.shape[0]].contiguous() @ rows[:, :512].contiguous()
             assert float((got - want).abs().max()) <= 2.0 ** -8 * float(rows.abs().max()), (n, bound)
+
+
+@pytest.mark.parametrize("rot", [0, 64])
+@pytest.mark.parametrize("decode", [True, False])
+def test_a_cache_that_starts_between_16_byte_addresses(rot, decode):
+    """Such a cache runs the kernel for any sizes: the same averages, both within the bound above of the float64 ones."""
+    from fms_amd.kernels import ops
+
+    heads, width, pages = 17, 512 + rot, 3
+    g = torch.Generator(device="cuda").manual_seed(rot)
+    cache = torch.randn(pages, 1, 64, width, generator=g, device="cuda").to(torch.bfloat16)
+    flat = torch.zeros(cache.numel() + 4, dtype=torch.bfloat16, device="cuda")
+    shifted = flat[4:].view(cache.shape)
+    shifted.copy_(cache)
+    assert shifted.data_ptr() % 16 == 8
+    values = cache[:, :, :, :512].transpose(2, 3).contiguous()
+    lengths = [130, 65, 191] if decode else list(range(60, 71))
+    positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32, device="cuda")
+    seqs = torch.arange(3, dtype=torch.int32, device="cuda") if decode else torch.zeros(len(lengths), dtype=torch.int32, device="cuda")
+    table = torch.arange(pages, dtype=torch.int32, device="cuda").repeat(3, 1)
+    qa = (torch.randn(len(lengths), heads * width, generator=g, device="cuda") * 0.4).to(torch.bfloat16)
+    same, out = (ops.latent_attention(qa, positions, seqs, table, c, None, heads, 512, rot, 0.06, decode=decode, max_context=192, vt_cache=values)
+                 for c in (cache, shifted))
+    assert float((out.double() - same.double()).abs().max()) <= 2 * 2.0 ** -8 * float(cache.abs().max())
