@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(ROUTER_WAVES* WAVE)
   if (wave == 0) route_row<PER>([&](int e) { return z[e]; }, lane, n_experts, top, score, ids + (size_t)t * top, weights + (size_t)t * top);
 }
 
-// logits [n_tokens, n_out] = x W^T in float32 (bfloat16 x and W, K a multiple of 8 up to 4096, 16-byte addresses), and the choice among
+// logits [n_tokens, n_out] = x W^T in float32 (bfloat16 x and W, K a multiple of 8 up to 2048, 16-byte addresses), and the choice among
 // the first n_experts of them as fmsamd_moe_route makes it.
 extern "C" int fmsamd_moe_router(const void* x, long ldx, const void* w, int n_tokens, int K, int n_out, int n_experts, int top, int score,
                                  float* logits, int* ids, float* weights, hipStream_t stream) {

@@ -49,7 +49,9 @@ extern "C" int fmsamd_probe_read(const void* buffer, long bytes, int blocks, int
 }
 
 // Independent accumulators, so that the matrix unit never waits for a result.  LARGE: 32x32x16 products (four
-// accumulators of 16 registers), otherwise 16x16x32 (eight of 4); either is 2 * 16384 / 2 flops a lane group.
+// accumulators of 16 registers), otherwise 16x16x32 (eight of 4); either is 2 * 16384 / 2 flops a lane group.  The smaller ones sixteen
+// rounds at a time: the compiler moves the accumulators of a short loop from register to register, 55 moves for 8 products, which is
+// what such a loop measures (1.4 PFLOP/s with many waves a SIMD, so 2.1).
 template <bool LARGE>
 __global__ void __launch_bounds__(256) probe_mfma_kernel(int iterations, float* __restrict__ out) {
   const int lane = threadIdx.x & (WAVE - 1);
@@ -78,10 +80,16 @@ __global__ void __launch_bounds__(256) probe_mfma_kernel(int iterations, float* 
     f32x4 acc[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int it = 0; it < iterations; ++it) {
+    auto round = [&]() {
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[k], 0, 0, 0);
+    };
+    int it = 0;
+    for (; it + 16 <= iterations; it += 16) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) round();
     }
+    for (; it < iterations; ++it) round();
 #pragma unroll
     for (int k = 0; k < 8; ++k) sum += acc[k][0] + acc[k][1] + acc[k][2] + acc[k][3];
   }

@@ -1,5 +1,5 @@
-// A block's tile of C = A W^T for many rows: bfloat16 operands through LDS, 32x32x16 matrix instructions (they run at twice
-// the rate of 16x16x32 on this GPU).  Like tile_product.h, the rows are found through functions, so that they may be
+// A block's tile of C = A W^T for many rows: bfloat16 operands through LDS, 32x32x16 matrix instructions (half the
+// instructions and operand reads a product of 16x16x32).  Like tile_product.h, the rows are found through functions, so that they may be
 // gathered (tokens sorted by expert), strided or plain; K a multiple of 8 and rows aligned to 16 bytes.
 //
 // WM x WN waves, each with TM x TN tiles of 32 x 32.  A step is 64 k-values, cut into four products of 16.
