@@ -4,7 +4,8 @@
 //   * The tile is as large as the registers hold (256 x 256 results a block): every byte from the caches and from LDS then feeds the
 //     most products.  With random data it is the power of the chip that ends the rate, and bytes moved are power; so are sums, of which
 //     a 16x16x32 instruction reads and writes half as many a product as a 32x32x16 one (8192 x 8192 x 8192: 795 us with 32x32x16
-//     products, 720 with 16x16x32; with zeros for data, which take no power, 600 and 585).
+//     products, 720 with 16x16x32 in the same form; as it is now 725, with zeros for data, which take less power, 552, the vendor
+//     library 687 and 487).
 //   * A wave's tile is four quadrants, two halves of the block's rows of A by two halves of its rows of W.  A step is 64
 //     k-values of them in the order (A0 W0) (A0 W1) (A1 W1) (A1 W0): each quadrant needs one new half, which is read from LDS
 //     between the matrix instructions of the quadrant before it.
