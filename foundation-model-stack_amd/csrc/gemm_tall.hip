@@ -138,8 +138,9 @@ __device__ __forceinline__ void tall_tiles(const TallArgs& g, int first, int las
         });
       });
     };
-    // (a choice for the whole tile: one for every element costs more than the products of a tile.  The fast exponential's and the
-    // reciprocal's last bits are far below the result's.)
+    // (a choice for the whole tile: one for every element costs more than the products of a tile.  The fast exponential and the
+    // reciprocal are within 7e-6 of the sigmoid wherever it is above 2^-126, the result is rounded to 2^-9; expf and a division take
+    // 354 us instead of 342 for 2048 rows by 2 x 14336 of K = 4096, 809 instead of 778 for 4689.)
     if (!GATED || g.act.kind == FMS_ACT_SILU)
       write([&](float gate, float up) { return gate * __builtin_amdgcn_rcpf(1.f + __expf(-gate)) * up; });
     else if (g.act.kind == FMS_ACT_CLAMPED_GATE)
